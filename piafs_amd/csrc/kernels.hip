@@ -2986,25 +2986,24 @@ __global__ void __launch_bounds__(256) k_viscflux(CASE_ARGS) {
 // (ChemistrySolve.c:18-115, chemistry.h:30-127) with the photon density of
 // the Gaussian pulse at the stage time.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void viscous_par(const CaseDev &C, int i, int j, long p, double par[3]) {
+// component c (variable c + 1) of the parabolic term
+__device__ __forceinline__ double viscous_par(const CaseDev &C, int c, int i, int j, long p) {
   const Grid &G = C.G;
   const PhysParams &P = C.P;
   const long pl = (long)G.nxg * G.nyg;
   const double dxi = C.dxinv[G.g + i], dyi = C.dxinv[(G.nx + 2 * G.g) + G.g + j];
-  for (int c = 0; c < 3; c++) {
-    const double *Fx = C.FV + c * pl, *Fy = C.FV + (3 + c) * pl;
-    double dfx, dfy;
-    if (P.par4) {
-      const double t12 = 1.0 / 12.0;
-      dfx = (Fx[p - 2] - 8 * Fx[p - 1] + 8 * Fx[p + 1] - Fx[p + 2]) * t12;
-      dfy = (Fy[p - 2 * G.nxg] - 8 * Fy[p - G.nxg] + 8 * Fy[p + G.nxg] - Fy[p + 2 * G.nxg]) * t12;
-    } else {
-      dfx = 0.0 * Fx[p + 1] - (-1.0) * Fx[p] + (-1.0) * Fx[p - 1];
-      dfy = 0.0 * Fy[p + G.nxg] - (-1.0) * Fy[p] + (-1.0) * Fy[p - G.nxg];
-    }
-    par[c] = dxi * dfx;
-    par[c] = par[c] + dyi * dfy;
+  const double *Fx = C.FV + c * pl, *Fy = C.FV + (3 + c) * pl;
+  double dfx, dfy;
+  if (P.par4) {
+    const double t12 = 1.0 / 12.0;
+    dfx = (Fx[p - 2] - 8 * Fx[p - 1] + 8 * Fx[p + 1] - Fx[p + 2]) * t12;
+    dfy = (Fy[p - 2 * G.nxg] - 8 * Fy[p - G.nxg] + 8 * Fy[p + G.nxg] - Fy[p + 2 * G.nxg]) * t12;
+  } else {
+    dfx = 0.0 * Fx[p + 1] - (-1.0) * Fx[p] + (-1.0) * Fx[p - 1];
+    dfy = 0.0 * Fy[p + G.nxg] - (-1.0) * Fy[p] + (-1.0) * Fy[p - G.nxg];
   }
+  const double px = dxi * dfx;
+  return px + dyi * dfy;
 }
 
 // Sponge zones act as a source (BCSponge.c:29-74, called by
@@ -3030,184 +3029,155 @@ __device__ __forceinline__ double sponge(const CaseDev &C, int i, int j, int v, 
   return s;
 }
 
-// photon density reaching layer 0 at the stage time: the Gaussian pulse
-// (ChemistrySolve.c:36-43) times the beam map
-__device__ __forceinline__ double chem_nh0(const CaseDev &C, int stage, long p) {
+// the Gaussian pulse at the stage time (ChemistrySolve.c:36-43); the photon
+// density reaching layer 0 is its product with the beam map
+__device__ __forceinline__ double chem_pulse(const CaseDev &C, int stage) {
   const PhysParams &P = C.P;
   const double time = *C.time + C.c[stage] * C.dt;
-  double hs = 0.0;
-  if (time > P.t_start_norm) {
-    const double sigma = P.t_pulse_norm / 2.35482;
-    const double tp = time - (P.t_start_norm + P.t_pulse_norm);
-    hs = P.I0 * exp(-(tp * tp) / (2 * sigma * sigma));
-  }
-  return (hs * C.imap[p]) / P.hnu_den;
+  if (!(time > P.t_start_norm)) return 0.0;
+  const double sigma = P.t_pulse_norm / 2.35482;
+  const double tp = time - (P.t_start_norm + P.t_pulse_norm);
+  return P.I0 * exp(-(tp * tp) / (2 * sigma * sigma));
 }
 
-// sources of layer iz at point p (chemistry.h:30-127): its seven species s[]
-// and the energy term, for photon density nh reaching the layer
-__device__ __forceinline__ void chem_layer(const CaseDev &C, int iz, long p, double nh, double s[7], double &src_e) {
+// Photochemistry source of variable v at point p (chemistry.h:30-127,
+// ChemistrySolve.c:45-110): a species' own term, or the energy's, which is the
+// last layer's heating.  The other variables have none.  hs: the pulse at the
+// stage time (chem_pulse).
+__device__ __forceinline__ double chem_var(const CaseDev &C, int v, long p, double hs) {
   const PhysParams &P = C.P;
   const double *U = C.U;
   const long pl = C.G.plane;
-  const int nfv = P.nflow + P.z_stride * iz;
-  const double nO2 = U[(long)(nfv + 0) * pl + p], nO3 = U[(long)(nfv + 1) * pl + p];
-  const double n1D = U[(long)(nfv + 2) * pl + p], n1Dg = U[(long)(nfv + 3) * pl + p];
-  const double n3Su = U[(long)(nfv + 4) * pl + p], n1Sg = U[(long)(nfv + 5) * pl + p];
-  const double nCO2 = U[(long)(nfv + 6) * pl + p];
-  s[0] = 0.0;
-  s[1] = -(P.k0a + P.k0b) * nh * nO3 - (P.k2a + P.k2b) * nO3 * n1D - (P.k3a + P.k3b) * nO3 * n1Sg -
-         P.k5 * nO3 * n3Su - P.k6 * n1Dg * nO3;
-  s[2] = P.k0a * nh * nO3 - (P.k1a + P.k1b) * n1D * nO2 - (P.k2a + P.k2b) * n1D * nO3 - P.k4 * n1D * nCO2;
-  s[3] = P.k0a * nh * nO3 + P.k5 * nO3 * n3Su - P.k6 * n1Dg * nO3;
-  s[4] = P.k2a * nO3 * n1D - P.k5 * nO3 * n3Su;
-  s[5] = P.k1a * n1D * nO2 - (P.k3a + P.k3b) * nO3 * n1Sg;
-  s[6] = 0.0;
-  src_e = ((P.q0a * P.k0a + P.q0b * P.k0b) * nh * nO3 + (P.q1a * P.k1a + P.q1b * P.k1b) * nO2 * n1D +
-           (P.q2a * P.k2a + P.q2b * P.k2b) * nO3 * n1D + (P.q3a * P.k3a + P.q3b * P.k3b) * nO3 * n1Sg +
-           P.q4 * P.k4 * n1D * nCO2 + P.q5 * P.k5 * nO3 * n3Su + P.q6 * P.k6 * n1Dg * nO3) /
-          P.ch_gm1;
-}
-
-// rhs += chemistry source, layer by layer (ChemistrySolve.c:45-110); the
-// energy takes the last layer's term
-__device__ __forceinline__ void chem_source(const CaseDev &C, int stage, long p, double *udot, bool sp, int i,
-                                            int j) {
-  const Grid &G = C.G;
-  const PhysParams &P = C.P;
-  const long pl = G.plane;
-  double nh = chem_nh0(C, stage, p);
-  double src_e = 0.0;
-  for (int iz = 0; iz < P.nlayers; iz++) {
-    const int nfv = P.nflow + P.z_stride * iz;
-    if (iz > 0) nh = nh * (1.0 - P.damp_coef * C.U[(long)(P.nflow + P.z_stride * (iz - 1) + 1) * pl + p]);
-    double s[7];
-    chem_layer(C, iz, p, nh, s, src_e);
-    for (int m = 0; m < 7; m++) {
-      double *o = udot + (long)(nfv + m) * pl + p;
-      *o = *o + (sp ? sponge(C, i, j, nfv + m, p, s[m]) : s[m]);
-    }
+  const bool energy = v == P.nflow - 1;
+  const int iz = energy ? P.nlayers - 1 : (v - P.nflow) / P.z_stride, m = v - P.nflow - P.z_stride * iz;
+  if (!energy && (m == 0 || m == 6)) return 0.0;
+  auto n = [&](int q) { return U[(long)(P.nflow + P.z_stride * iz + q) * pl + p]; };
+  // photon density reaching layer iz
+  auto photons = [&]() {
+    double nh = (hs * C.imap[p]) / P.hnu_den;
+    for (int z = 0; z < iz; z++) nh = nh * (1.0 - P.damp_coef * U[(long)(P.nflow + P.z_stride * z + 1) * pl + p]);
+    return nh;
+  };
+  const double nO3 = n(1);
+  if (m == 4 && !energy) return P.k2a * nO3 * n(2) - P.k5 * nO3 * n(4);
+  if (m == 5 && !energy) return P.k1a * n(2) * n(0) - (P.k3a + P.k3b) * nO3 * n(5);
+  const double nh = photons();
+  if (energy) {
+    const double nO2 = n(0), n1D = n(2), n1Dg = n(3), n3Su = n(4), n1Sg = n(5), nCO2 = n(6);
+    return ((P.q0a * P.k0a + P.q0b * P.k0b) * nh * nO3 + (P.q1a * P.k1a + P.q1b * P.k1b) * nO2 * n1D +
+            (P.q2a * P.k2a + P.q2b * P.k2b) * nO3 * n1D + (P.q3a * P.k3a + P.q3b * P.k3b) * nO3 * n1Sg +
+            P.q4 * P.k4 * n1D * nCO2 + P.q5 * P.k5 * nO3 * n3Su + P.q6 * P.k6 * n1Dg * nO3) /
+           P.ch_gm1;
   }
-  double *o = udot + (long)(P.nflow - 1) * pl + p;
-  *o = *o + (sp ? sponge(C, i, j, P.nflow - 1, p, src_e) : src_e);
-}
-
-// The source term at interior point (i, j), ghosted offset p: chemistry,
-// then sponge zones (SourceFunction.c:21-60); rhs += source.
-__device__ __forceinline__ void add_source(const CaseDev &C, int stage, int i, int j, long p, double *udot) {
-  const bool sp = C.sponge && in_sponge(C, i, j);
-  if (C.P.chem) chem_source(C, stage, p, udot, sp, i, j);
-  if (!sp) return;
-  const int nplain = C.P.chem ? C.P.nflow - 1 : C.G.nv;  // variables chemistry leaves at zero
-  for (int v = 0; v < nplain; v++) {
-    double *o = udot + (long)v * C.G.plane + p;
-    *o = *o + sponge(C, i, j, v, p, 0.0);
+  if (m == 1)
+    return -(P.k0a + P.k0b) * nh * nO3 - (P.k2a + P.k2b) * nO3 * n(2) - (P.k3a + P.k3b) * nO3 * n(5) -
+           P.k5 * nO3 * n(4) - P.k6 * n(3) * nO3;
+  if (m == 2) {
+    const double n1D = n(2);
+    return P.k0a * nh * nO3 - (P.k1a + P.k1b) * n1D * n(0) - (P.k2a + P.k2b) * n1D * nO3 - P.k4 * n1D * n(6);
   }
+  return P.k0a * nh * nO3 + P.k5 * nO3 * n(4) - P.k6 * n(3) * nO3;  // m == 3
 }
 
+// rhs of variable v at interior point (i, j), ghosted offset p, with its
+// source added (SourceFunction.c:21-60): chemistry, then the sponge zones
+__device__ __forceinline__ double with_source(const CaseDev &C, int v, int i, int j, long p, double hs, double r) {
+  const bool chem = C.P.chem && v >= C.P.nflow - 1;
+  const double s = chem ? chem_var(C, v, p, hs) : 0.0;
+  if (C.sponge && in_sponge(C, i, j)) return r + sponge(C, i, j, v, p, s);
+  return chem ? r + s : r;
+}
+
+// One variable of one 32 x 32 tile per block, the tile's variables in
+// neighbouring blocks of one XCD (the species a source reads are shared in its
+// L2).  Bound by memory latency on small grids and by HBM on large ones.  A
+// block has one exchange through LDS (the y-sweep interfaces, which are
+// contiguous along y) and no serial walk over the variables: a tile's latency
+// is paid once, not once per variable, a grid of few tiles has nv times as many
+// blocks, and the source is added before the one store of a value.  With a tile
+// per block walking all variables (a load round and two barriers each, the
+// source a second pass over the stored values) a launch took, nv 11: 128 x 97
+// 53.3 -> 10.5 us, 600 x 343 59.4 -> 26, 1024^2 119 -> 115, 2048 x 1531 368 ->
+// 336 us.
 __global__ void __launch_bounds__(256) k_assemble(CASE_ARGS) {
   CASE_PREAMBLE
   if (stage >= C.nstages) return;
   const Grid &G = C.G;
   const int nv = G.nv;
   double *udot = C.Udot[stage];
+  const bool src = (C.P.chem || C.sponge) && (C.terms & 4);
   if (G.ndims == 1) {
-    if (t >= G.nx) return;
-    const int i = (int)t;
+    if (t >= (long)G.nx * nv) return;
+    const int v = (int)(t / G.nx), i = (int)(t % G.nx);
     const long p = i + G.g;
-    const double dxi = C.dxinv[G.g + i];
-    for (int v = 0; v < nv; v++) {
-      const long a = (long)v * (G.nx + 1) + i;
-      const double hyp = dxi * (C.fIx[a + 1] - C.fIx[a]);
-      udot[(long)v * G.plane + p] = (C.terms & 1) ? -hyp : 0.0;
-    }
-    if (C.terms & 4) add_source(C, stage, i, 0, p, udot);
+    const long a = (long)v * (G.nx + 1) + i;
+    const double hyp = C.dxinv[G.g + i] * (C.fIx[a + 1] - C.fIx[a]);
+    double r = (C.terms & 1) ? -hyp : 0.0;
+    if (src) r = with_source(C, v, i, 0, p, C.P.chem ? chem_pulse(C, stage) : 0.0, r);
+    udot[(long)v * G.plane + p] = r;
     return;
   }
-  // 2D: a 32 x 32 tile of points, four per thread
   __shared__ double tl[32][33];
   const int ntx = (G.nx + 31) / 32;
-  const int nb = ntx * ((G.ny + 31) / 32);  // tiles; the case's blocks are padded to a multiple of eight
+  const int nb = ntx * ((G.ny + 31) / 32) * nv;  // the case's blocks are padded to a multiple of eight
   const int id = xcd_order((int)(blockIdx.x - firstblock[cidx]), (nb + 7) & ~7, firstblock[cidx]);
   if (id >= nb) return;
-  const int i0 = (id % ntx) * 32, j0 = (id / ntx) * 32;
+  const int v = id % nv, tile = id / nv;
+  const int i0 = (tile % ntx) * 32, j0 = (tile / ntx) * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int i = i0 + tx;
-  const bool visc = C.P.viscous && (C.terms & 2);
-  double par[4][3];
+  // Points outside the grid read the nearest one inside and are not stored, so
+  // that every load is issued without a branch (a branch would wait for the
+  // loads before it).
+  const int ic = min(i, G.nx - 1);
+  auto jq = [&](int q) { return min(j0 + ty + 8 * q, G.ny - 1); };
+  // y-sweep interfaces of lines i0..i0+31, interfaces j0..j0+32
+  double fy[4], fy32 = 0.0;
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    fy[q] = C.fIy[((long)v * G.nx + min(i0 + ty + 8 * q, G.nx - 1)) * (G.ny + 1) + min(j0 + tx, G.ny)];
+  // interface j0 + 32 of line i0 + the thread's index, by the first 32 threads
+  if (threadIdx.x < 32) fy32 = C.fIy[((long)v * G.nx + ic) * (G.ny + 1) + min(j0 + 32, G.ny)];
+  const bool visc = C.P.viscous && (C.terms & 2) && v >= 1 && v <= 3;
+  double hx[4], add[4];
+  {
+    double x0[4], x1[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const long a = ((long)v * G.ny + jq(q)) * (G.nx + 1) + ic;
+      x0[q] = C.fIx[a];
+      x1[q] = C.fIx[a + 1];
+    }
+    const double dxi = C.dxinv[G.g + ic];
+#pragma unroll
+    for (int q = 0; q < 4; q++) hx[q] = dxi * (x1[q] - x0[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    add[q] = visc ? viscous_par(C, v - 1, ic, jq(q), (long)(jq(q) + G.gy) * G.nxg + (ic + G.g)) : 0.0;
+  double sv[4] = {0.0, 0.0, 0.0, 0.0};
+  const bool chem = C.P.chem && (C.terms & 4) && v >= C.P.nflow - 1;
+  if (chem) {
+    const double hs = chem_pulse(C, stage);
+#pragma unroll
+    for (int q = 0; q < 4; q++) sv[q] = chem_var(C, v, (long)(jq(q) + G.gy) * G.nxg + (ic + G.g), hs);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) tl[ty + 8 * q][tx] = fy[q];
+  if (threadIdx.x < 32) tl[threadIdx.x][32] = fy32;
+  lds_barrier();
 #pragma unroll
   for (int q = 0; q < 4; q++) {
-    const int j = j0 + ty + 8 * q;
-    par[q][0] = par[q][1] = par[q][2] = 0.0;
-    if (visc && i < G.nx && j < G.ny) viscous_par(C, i, j, (long)(j + G.gy) * G.nxg + (i + G.g), par[q]);
-  }
-  const double dxi = i < G.nx ? C.dxinv[G.g + i] : 0.0;
-#if PIAFS_ASM_PIPELINE
-  // y-sweep interfaces of lines i0..i0+31, interfaces j0..j0+32, of variable
-  // v: this thread's share (rows ty + 8q, interfaces tx and tx + 32), loaded
-  // one variable ahead so that the loads are in flight during the previous
-  // variable's work; the barriers order the LDS tile only, so that global
-  // loads and stores stay in flight across them
-  double fy[4][2];
-  auto load_y = [&](int v) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int ii = i0 + ty + 8 * q;
-      const double *row = C.fIy + ((long)v * G.nx + ii) * (G.ny + 1);
-#pragma unroll
-      for (int k = 0; k < 2; k++) {
-        const int a = tx + 32 * k, j = j0 + a;
-        fy[q][k] = (ii < G.nx && a < 33 && j <= G.ny) ? row[j] : 0.0;
-      }
-    }
-  };
-  load_y(0);
-  for (int v = 0; v < nv; v++) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      tl[ty + 8 * q][tx] = fy[q][0];
-      if (tx == 0) tl[ty + 8 * q][32] = fy[q][1];
-    }
-    lds_barrier();
-    if (v + 1 < nv) load_y(v + 1);
-#else
-  for (int v = 0; v < nv; v++) {
-    // y-sweep interfaces of lines i0..i0+31, interfaces j0..j0+32
-    for (int b = ty; b < 32; b += 8) {
-      const int ii = i0 + b;
-      if (ii < G.nx) {
-        const double *row = C.fIy + ((long)v * G.nx + ii) * (G.ny + 1);
-        for (int a = tx; a < 33; a += 32) {
-          const int j = j0 + a;
-          if (j <= G.ny) tl[b][a] = row[j];
-        }
-      }
-    }
-    __syncthreads();
-#endif
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int jl = ty + 8 * q, j = j0 + jl;
-      if (i < G.nx && j < G.ny) {
-        const long a = ((long)v * G.ny + j) * (G.nx + 1) + i;
-        double hyp = dxi * (C.fIx[a + 1] - C.fIx[a]);
-        hyp = hyp + C.dxinv[(G.nx + 2 * G.g) + G.g + j] * (tl[tx][jl + 1] - tl[tx][jl]);
-        double r = (C.terms & 1) ? -hyp : 0.0;
-        if (visc && v >= 1 && v <= 3) r = r + par[q][v - 1];
-        udot[(long)v * G.plane + (long)(j + G.gy) * G.nxg + (i + G.g)] = r;
-      }
-    }
-#if PIAFS_ASM_PIPELINE
-    lds_barrier();
-#else
-    __syncthreads();
-#endif
-  }
-  if ((C.P.chem || C.sponge) && (C.terms & 4)) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int j = j0 + ty + 8 * q;
-      if (i < G.nx && j < G.ny) add_source(C, stage, i, j, (long)(j + G.gy) * G.nxg + (i + G.g), udot);
+    const int jl = ty + 8 * q, j = j0 + jl;
+    const long p = (long)(j + G.gy) * G.nxg + (i + G.g);
+    const double hyp = hx[q] + C.dxinv[(G.nx + 2 * G.g) + G.g + jq(q)] * (tl[tx][jl + 1] - tl[tx][jl]);
+    double r = (C.terms & 1) ? -hyp : 0.0;
+    if (visc) r = r + add[q];
+    if (i < G.nx && j < G.ny) {
+      // chemistry, then the sponge zones (SourceFunction.c:21-60)
+      if (C.sponge && (C.terms & 4) && in_sponge(C, i, j)) r = r + sponge(C, i, j, v, p, sv[q]);
+      else if (chem) r = r + sv[q];
+      udot[(long)v * G.plane + p] = r;
     }
   }
 }
@@ -3618,7 +3588,7 @@ void case_blocks(const CaseDev &c, int blocks[K_NCLASS]) {
   const bool visc = two && c.P.viscous;
   blocks[K_QDERIV] = visc ? nb((long)G.nxg * G.nyg) : 0;
   blocks[K_VISCFLUX] = visc ? nb((long)G.nxg * G.nyg) : 0;
-  blocks[K_ASSEMBLE] = pad8(two ? ((G.nx + 31) / 32) * ((G.ny + 31) / 32) : nb(G.nx));
+  blocks[K_ASSEMBLE] = pad8(two ? ((G.nx + 31) / 32) * ((G.ny + 31) / 32) * G.nv : nb((long)G.nx * G.nv));
   blocks[K_UPDATE] = nb((long)G.nx * G.ny * G.nv);
 }
 

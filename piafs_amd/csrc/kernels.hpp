@@ -76,12 +76,6 @@ constexpr int kMaxRows = PIAFS_MAX_ROWS;
 #ifndef PIAFS_SCAN_DPP
 #define PIAFS_SCAN_DPP 1
 #endif
-// k_assemble loads each variable's y-interface tile one variable ahead and
-// synchronises on the LDS tile only (1), or loads and waits variable by
-// variable (0).
-#ifndef PIAFS_ASM_PIPELINE
-#define PIAFS_ASM_PIPELINE 1
-#endif
 // the tile kernels (k_assemble, k_stage with 32-point tiles) give each XCD a
 // contiguous band of tiles (1) or take tiles in workgroup order (0)
 #ifndef PIAFS_XCD_ORDER
