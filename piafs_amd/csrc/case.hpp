@@ -11,6 +11,7 @@
 #include "../../include/piafs_amd.h"
 #include "config.hpp"
 #include "kernels.hpp"
+#include "transfer.hpp"
 
 namespace piafs {
 
@@ -27,6 +28,7 @@ struct Case {
   double t = 0.0;       // host mirror of the simulation time (t += dt per step)
   std::string err;
   std::vector<void *> allocs;
+  std::shared_ptr<Staging> staging;  // pinned buffers of the device's cases
   double *uprev = nullptr, *partials = nullptr;
   int nparts = 0;
 
@@ -37,6 +39,8 @@ struct Case {
   int setup(int dev, hipStream_t st);
   int fail(int code, const std::string &msg);
   double *dalloc(size_t n, hipStream_t st);
+  // the interior state, point-major; upload returns when uh is no longer
+  // needed, its device side follows in stream order
   int upload(const double *uh, hipStream_t st);
   int download(double *uh, hipStream_t st, const double *src = nullptr);
   int write_binary(const std::string &path, hipStream_t st);

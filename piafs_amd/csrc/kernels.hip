@@ -3493,6 +3493,28 @@ __global__ void __launch_bounds__(TB) k_dev_planar(Grid G, const double *__restr
   out[p * G.nv + v] = nat[pn];
 }
 
+// Host states, point-major in pinned memory, to and from the planar layout
+// (see transfer.hpp).  Bound by the host link, so consecutive lanes take
+// consecutive values of the host side, and the planar side's short runs (the
+// few points a wave covers of every variable) merge in L2.
+__device__ __forceinline__ long pack_at(const Grid &G, long q0, unsigned e) {
+  const unsigned v = e % (unsigned)G.nv;
+  const long q = q0 + e / (unsigned)G.nv;
+  const int i = (int)(q % G.nx), j = (int)(q / G.nx);
+  return (long)v * G.plane + (long)(j + G.gy) * G.nxg + (i + G.g);
+}
+__global__ void __launch_bounds__(TB) k_pack(Grid G, const double *__restrict__ host, long q0, unsigned n,
+                                             double *__restrict__ u) {
+  const unsigned e = blockIdx.x * TB + threadIdx.x;
+  if (e < n) u[pack_at(G, q0, e)] = host[e];
+}
+__global__ void __launch_bounds__(TB) k_unpack(Grid G, const double *__restrict__ u, long q0, unsigned n,
+                                               double *__restrict__ host) {
+  const unsigned e = blockIdx.x * TB + threadIdx.x;
+  if (e < n) host[e] = u[pack_at(G, q0, e)];
+}
+__global__ void k_set_time(double *time, double t) { *time = t; }
+
 // Interface arrays of one sweep: reference layout <-> line-major
 // a[(v*nlines + l)*(N+1) + k].  One thread per (interface, line, variable).
 __global__ void __launch_bounds__(TB) k_dev_iface(int ndims, int dir, int nx, int N, int nl, int nv,
@@ -3690,6 +3712,20 @@ void launch_dev_planar(const Grid &G, const double *a, double *nat, double *tr, 
                        double *out, hipStream_t s) {
   const long n = (long)G.nxg * G.nyg * G.nv;
   hipLaunchKernelGGL(k_dev_planar, dim3(nblk(n)), dim3(TB), 0, s, G, a, nat, tr, to_planar, ghosts_only, out);
+}
+
+void launch_pack(const Grid &G, const double *host, long q0, long np, double *u, hipStream_t s) {
+  const long n = np * G.nv;
+  hipLaunchKernelGGL(k_pack, dim3(nblk(n)), dim3(TB), 0, s, G, host, q0, (unsigned)n, u);
+}
+
+void launch_unpack(const Grid &G, const double *u, long q0, long np, double *host, hipStream_t s) {
+  const long n = np * G.nv;
+  hipLaunchKernelGGL(k_unpack, dim3(nblk(n)), dim3(TB), 0, s, G, u, q0, (unsigned)n, host);
+}
+
+void launch_set_time(double *time, double t, hipStream_t s) {
+  hipLaunchKernelGGL(k_set_time, dim3(1), dim3(1), 0, s, time, t);
 }
 
 void launch_dev_iface(int ndims, int dir, int nx, int N, int nl, int nv, const double *src, double *dst,

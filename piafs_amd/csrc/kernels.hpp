@@ -245,6 +245,11 @@ void launch_dev_weights(const AosGrid &A, int model, double gamma, int dir, int 
 // ghosted reference-layout array <-> planar natural / transposed copies
 void launch_dev_planar(const Grid &G, const double *a, double *nat, double *tr, int to_planar, int ghosts_only,
                        double *out, hipStream_t s);
+// Interior points q0 .. q0+np-1 (x fastest) of a state: point-major values in
+// pinned host memory -> the planar ghosted layout, and back.
+void launch_pack(const Grid &G, const double *host, long q0, long np, double *u, hipStream_t s);
+void launch_unpack(const Grid &G, const double *u, long q0, long np, double *host, hipStream_t s);
+void launch_set_time(double *time, double t, hipStream_t s);
 // one sweep's interface array: reference layout <-> line-major
 void launch_dev_iface(int ndims, int dir, int nx, int N, int nl, int nv, const double *src, double *dst,
                       int to_lines, hipStream_t s);

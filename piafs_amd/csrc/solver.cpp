@@ -290,6 +290,8 @@ int Case::setup(int dev, hipStream_t st) {
   }
   t = (double)cfg.restart_iter * cfg.dt;
   HIPCHK(hipMemcpyAsync(D.time, &t, sizeof(double), hipMemcpyHostToDevice, st));
+  staging = Staging::of(device);
+  if (!staging->reserve((size_t)cfg.npts_int * nv * sizeof(double))) return fail(-2, "pinned host memory allocation failed");
   int rc = upload(cfg.u0.data(), st);
   if (rc) return rc;
   HIPCHK(hipStreamSynchronize(st));
@@ -326,30 +328,21 @@ Case::~Case() {
 
 // point-major interior (WriteBinary order) <-> natural planar ghosted
 int Case::upload(const double *uh, hipStream_t st) {
-  const Grid &G = h.G;
-  const int nv = cfg.nvars;
-  std::vector<double> buf((size_t)nv * G.plane, 0.0);
-  for (long q = 0; q < cfg.npts_int; q++) {
-    int i = (int)(q % G.nx), j = (int)(q / G.nx);
-    long p = (long)(j + G.gy) * G.nxg + (i + G.g);
-    for (int v = 0; v < nv; v++) buf[(size_t)v * G.plane + p] = uh[(size_t)q * nv + v];
-  }
-  HIPCHK(hipMemcpyAsync(h.u, buf.data(), buf.size() * sizeof(double), hipMemcpyHostToDevice, st));
-  HIPCHK(hipStreamSynchronize(st));
+  const hipError_t e = staging->upload(uh, cfg.npts_int, cfg.nvars, st, [&](long q0, long np, double *buf) {
+    launch_pack(h.G, buf, q0, np, h.u, st);
+  });
+  if (e != hipSuccess) return fail(-1, std::string("state upload: ") + hipGetErrorString(e));
+  HIPCHK(hipGetLastError());
   return 0;
 }
 
 int Case::download(double *uh, hipStream_t st, const double *src) {
-  const Grid &G = h.G;
-  const int nv = cfg.nvars;
-  std::vector<double> buf((size_t)nv * G.plane);
-  HIPCHK(hipMemcpyAsync(buf.data(), src ? src : h.u, buf.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
-  for (long q = 0; q < cfg.npts_int; q++) {
-    int i = (int)(q % G.nx), j = (int)(q / G.nx);
-    long p = (long)(j + G.gy) * G.nxg + (i + G.g);
-    for (int v = 0; v < nv; v++) uh[(size_t)q * nv + v] = buf[(size_t)v * G.plane + p];
-  }
+  const double *from = src ? src : h.u;
+  const hipError_t e = staging->download(uh, cfg.npts_int, cfg.nvars, st, [&](long q0, long np, double *buf) {
+    launch_unpack(h.G, from, q0, np, buf, st);
+  });
+  if (e != hipSuccess) return fail(-1, std::string("state download: ") + hipGetErrorString(e));
+  HIPCHK(hipGetLastError());
   return 0;
 }
 
@@ -915,8 +908,8 @@ int piafs_download_state(piafs_case *pc, double *u) {
 int piafs_set_time(piafs_case *pc, double t) {
   if (!pc || !pc->c) return 1;  // no case
   pc->c->t = t;
-  if (hipMemcpyAsync(pc->c->h.time, &t, sizeof(double), hipMemcpyHostToDevice, pc->eng.stream) != hipSuccess ||
-      hipStreamSynchronize(pc->eng.stream) != hipSuccess) {
+  launch_set_time(pc->c->h.time, t, pc->eng.stream);
+  if (hipGetLastError() != hipSuccess) {
     pc->err = "set_time failed";
     return -1;
   }
@@ -982,9 +975,10 @@ static int eval_pieces(piafs_case *pc, const double *u, double t, int last, int 
   if ((rc = c->upload(u, st))) return case_fail(pc, rc);
   if ((rc = piafs_set_time(pc, t))) return rc;
   int *dterms = &pc->eng.d_cases[0].terms;
+  if (hipStreamSynchronize(st) != hipSuccess) return -1;
   if (terms != 7 && hipMemcpy(dterms, &terms, sizeof(int), hipMemcpyHostToDevice) != hipSuccess) return -1;
-  // the stream is idle here (upload and set_time synchronise), so the
-  // blocking copies of the mask cannot race the kernels that read it
+  // the stream is idle here, so the blocking copies of the mask cannot race
+  // the kernels that read it
   rc = pc->eng.stage_only(0, last);
   if (!rc) rc = body();
   const int all = 7;

@@ -1,0 +1,184 @@
+#include "transfer.hpp"
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <map>
+
+namespace piafs {
+
+std::shared_ptr<Staging> Staging::of(int device) {
+  static std::mutex mu;
+  static std::map<int, std::weak_ptr<Staging>> known;
+  std::lock_guard<std::mutex> g(mu);
+  std::shared_ptr<Staging> s = known[device].lock();
+  if (!s) known[device] = s = std::make_shared<Staging>(device);
+  return s;
+}
+
+Staging::~Staging() {
+  {
+    std::lock_guard<std::mutex> g(m);
+    stop = true;
+  }
+  wake.notify_all();
+  for (std::thread &t : pool) t.join();
+  hipSetDevice(device);
+  release();
+}
+
+void Staging::release() {
+  for (Slot &s : slots) {
+    if (s.ev && s.pending) hipEventSynchronize(s.ev);
+    if (s.ev) hipEventDestroy(s.ev);
+    if (s.buf) hipHostFree(s.buf);
+    s = Slot();
+  }
+  nslots = 0;
+  cap = 0;
+}
+
+// Chunk size and buffers of a state: an eighth of it, within kMinChunk (below,
+// a chunk's fixed cost of a launch and an event exceeds its copy) and
+// kSlotBytes (above, the first chunk's copy delays the link).
+void Staging::shape(size_t bytes, size_t &chunk, int &n) {
+  chunk = std::min(std::max((bytes + kSlots - 1) / kSlots, kMinChunk), kSlotBytes);
+  n = (int)std::min<size_t>(kSlots, std::max<size_t>(1, (bytes + chunk - 1) / chunk));
+}
+
+bool Staging::grow(size_t bytes) {
+  size_t chunk;
+  int n;
+  shape(bytes, chunk, n);
+  if (chunk > cap || n > nslots) {
+    const size_t c = std::max(chunk, cap);
+    const int want = std::max(n, nslots);
+    release();
+    for (int k = 0; k < want; k++) {
+      void *p = nullptr;
+      if (hipHostMalloc(&p, c, hipHostMallocDefault) != hipSuccess) break;
+      slots[k].buf = (double *)p;
+      if (hipEventCreateWithFlags(&slots[k].ev, hipEventDisableTiming) != hipSuccess) {
+        hipHostFree(p);
+        slots[k] = Slot();
+        break;
+      }
+      nslots = k + 1;
+    }
+    if (nslots) cap = c;
+    hipGetLastError();  // a shortage of pinned memory leaves fewer buffers
+  }
+  while ((int)pool.size() < nslots - 1) {
+    const int id = (int)pool.size() + 1;
+    try {
+      pool.emplace_back([this, id] { worker(id); });
+    } catch (...) {
+      break;  // fewer threads
+    }
+  }
+  return nslots > 0;
+}
+
+bool Staging::reserve(size_t bytes) {
+  std::lock_guard<std::mutex> g(use);
+  try {
+    return grow(bytes);
+  } catch (...) {
+    return nslots > 0;
+  }
+}
+
+void Staging::worker(int id) {
+  hipSetDevice(device);
+  uint64_t seen = 0;
+  std::unique_lock<std::mutex> g(m);
+  for (;;) {
+    wake.wait(g, [&] { return stop || (round != seen && id <= helpers); });
+    if (stop) return;
+    seen = round;
+    const std::function<void(int)> *f = job;
+    g.unlock();
+    (*f)(id);
+    g.lock();
+    if (--busy == 0) idle.notify_one();
+  }
+}
+
+// body(chunk, slot) for every chunk, on the calling thread and the helpers,
+// each with its own slot.  A thread takes the next chunk when it is done with
+// one.
+hipError_t Staging::each(long nchunks, const std::function<hipError_t(long, Slot &)> &body) {
+  std::atomic<long> next{0};
+  std::atomic<int> err{(int)hipSuccess};
+  const std::function<void(int)> run = [&](int s) {
+    for (long c = next++; c < nchunks && err == (int)hipSuccess; c = next++) {
+      const hipError_t e = body(c, slots[s]);
+      if (e != hipSuccess) err = (int)e;
+    }
+  };
+  const int n = (int)std::min<long>({(long)nslots - 1, (long)pool.size(), nchunks - 1});
+  if (n > 0) {
+    {
+      std::lock_guard<std::mutex> g(m);
+      job = &run;
+      helpers = busy = n;
+      round++;
+    }
+    wake.notify_all();
+  }
+  run(0);
+  if (n > 0) {
+    std::unique_lock<std::mutex> g(m);
+    idle.wait(g, [&] { return busy == 0; });
+    helpers = 0;
+    job = nullptr;
+  }
+  return (hipError_t)err.load();
+}
+
+hipError_t Staging::upload(const double *src, long npts, int nv, hipStream_t st, const Kern &kernel) {
+  std::lock_guard<std::mutex> g(use);
+  const size_t bytes = (size_t)npts * nv * sizeof(double);
+  if (!grow(bytes)) return hipErrorOutOfMemory;
+  size_t chunk;
+  int n;
+  shape(bytes, chunk, n);
+  const long per = std::max<long>(1, (long)(chunk / (nv * sizeof(double))));
+  return each((npts + per - 1) / per, [&](long c, Slot &s) {
+    const long q0 = c * per, np = std::min(per, npts - q0);
+    if (s.pending) {
+      const hipError_t e = hipEventSynchronize(s.ev);
+      if (e != hipSuccess) return e;
+      s.pending = false;
+    }
+    memcpy(s.buf, src + q0 * nv, (size_t)np * nv * sizeof(double));
+    kernel(q0, np, s.buf);
+    s.pending = true;
+    return hipEventRecord(s.ev, st);
+  });
+}
+
+hipError_t Staging::download(double *dst, long npts, int nv, hipStream_t st, const Kern &kernel) {
+  std::lock_guard<std::mutex> g(use);
+  const size_t bytes = (size_t)npts * nv * sizeof(double);
+  if (!grow(bytes)) return hipErrorOutOfMemory;
+  size_t chunk;
+  int n;
+  shape(bytes, chunk, n);
+  const long per = std::max<long>(1, (long)(chunk / (nv * sizeof(double))));
+  return each((npts + per - 1) / per, [&](long c, Slot &s) {
+    const long q0 = c * per, np = std::min(per, npts - q0);
+    if (s.pending) {
+      const hipError_t e = hipEventSynchronize(s.ev);
+      if (e != hipSuccess) return e;
+      s.pending = false;
+    }
+    kernel(q0, np, s.buf);
+    hipError_t e = hipEventRecord(s.ev, st);
+    if (e == hipSuccess) e = hipEventSynchronize(s.ev);
+    if (e == hipSuccess) memcpy(dst + q0 * nv, s.buf, (size_t)np * nv * sizeof(double));
+    return e;
+  });
+}
+
+}  // namespace piafs

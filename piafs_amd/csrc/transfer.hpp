@@ -1,0 +1,72 @@
+// Host <-> device passage of solution states through pinned host memory.
+//
+// A state crosses in chunks.  Each chunk has a pinned buffer of its own; a
+// host thread copies between the caller's array and the buffer, and a kernel
+// (k_pack / k_unpack) moves the chunk between the buffer, over the host link,
+// and the planar device layout, so the change of layout costs no pass over
+// memory.  Several threads work on chunks at the same time, since one thread's
+// memory copy is several times slower than the link.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <condition_variable>
+#include <cstdint>
+#include <functional>
+#include <memory>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+namespace piafs {
+
+// The pinned buffers and copy threads of one device, shared by all its cases
+// (at most kSlots * kSlotBytes of pinned memory) and given back with the last
+// of them.  One transfer at a time; callers on other threads wait their turn.
+class Staging {
+ public:
+  static constexpr int kSlots = 8;
+  static constexpr size_t kSlotBytes = (size_t)2 << 20, kMinChunk = (size_t)128 << 10;
+
+  // the device's staging (created at the first call, while a holder lives)
+  static std::shared_ptr<Staging> of(int device);
+  explicit Staging(int dev) : device(dev) {}
+  ~Staging();
+  // pinned buffers for states of `bytes`, so that transfers allocate nothing
+  bool reserve(size_t bytes);
+  // n doubles from `src` (host) / to `dst` (host) in chunks of whole points of
+  // nv doubles: kernel(first point, points, buffer) enqueues the device side of
+  // a chunk on st.  upload returns when src is no longer needed (the kernels
+  // may still run), download when dst is complete.
+  typedef std::function<void(long q0, long np, double *buf)> Kern;
+  hipError_t upload(const double *src, long npts, int nv, hipStream_t st, const Kern &kernel);
+  hipError_t download(double *dst, long npts, int nv, hipStream_t st, const Kern &kernel);
+
+ private:
+  struct Slot {
+    double *buf = nullptr;
+    hipEvent_t ev = nullptr;
+    bool pending = false;  // a kernel may still be reading buf (ev recorded after it)
+  };
+  int device;
+  std::mutex use;
+  Slot slots[kSlots];
+  int nslots = 0;
+  size_t cap = 0;  // bytes of every slot's buffer
+
+  std::vector<std::thread> pool;
+  std::mutex m;
+  std::condition_variable wake, idle;
+  const std::function<void(int)> *job = nullptr;
+  uint64_t round = 0;
+  int helpers = 0, busy = 0;
+  bool stop = false;
+
+  static void shape(size_t bytes, size_t &chunk, int &n);
+  bool grow(size_t bytes);
+  void release();
+  void worker(int id);
+  hipError_t each(long nchunks, const std::function<hipError_t(long, Slot &)> &body);
+};
+
+}  // namespace piafs
