@@ -436,9 +436,7 @@ def main():
         if ktimes:
             # per-class average launch time (ms) x launches per step -> share of the step
             ns = inf.nstages
-            per_step = {"stage_bc": ns, "ghost": ns, "bflux": ns, "flux": ns, "recon_ends": ns, "recon": ns, "recon_full": ns, "recon_char": ns, "upwind": ns, "qderiv": ns,
-                        "viscflux": ns, "assemble": ns, "update": 1}
-            share = {k: v * per_step.get(k, 1) for k, v in ktimes.items()}
+            share = {k: v * (1 if k == "update" else ns) for k, v in ktimes.items()}
             dom = max(share.items(), key=lambda kv: kv[1])[0]
             paired = (not inf.characteristic) and dk.physics["upwinding"] in ("roe", "rusanov")
             io_byts = kernel_algorithmic_bytes(dom, nx, nx, nv, g, inf.nstages, True, paired)

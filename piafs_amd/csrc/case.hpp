@@ -92,7 +92,7 @@ struct Engine {
   void enqueue_step();         // eager launches of one full step
   int step(int n);             // n steps (graph replay when enabled)
   int stage_only(int s, int last = K_NCLASS);  // one stage, or its classes up to `last`
-  double time_class(int cls, int reps, int cls2 = -1);
+  double time_classes(const std::vector<int> &cls, int reps);
   int autotune(const int *cands, int ncand, int reps, int *best_rows, double *best_ms);
   int sync();
   void mark(int cls, bool begin, hipStream_t st);

@@ -68,6 +68,7 @@ int unit_prepare(piafs_case *pc, hipStream_t st) {
   UnitOps &un = *pc->unit;
   CaseDev d = c->h;
   d.paired = 0;
+  d.unit = 1;
   d.terms = 7;
   d.u = un.u;
   d.status = pc->eng.d_status;  // zero pivots reach the case's own status word (piafs_sync)
@@ -129,6 +130,10 @@ int piafs_dev_interp_interfaces(piafs_case *pc, double *fI, const double *fC, co
   if (dir < 0 || dir >= c->cfg.ndims) return fail(pc, 1, "dir must be 0 .. ndims-1");
   if (upw != 1 && upw != -1) return fail(pc, 1, "upw must be 1 or -1");
   const hipStream_t st = stream_of(pc, stream);
+  if (!c->h.R.crweno) {
+    launch_dev_weno(aos_grid(c), c->h.model, c->h.P.gamma, c->h.R, dir, upw > 0, fC, uflag ? fC : u_ghosted, fI, st);
+    return launched(pc);
+  }
   int rc = unit_prepare(pc, st);
   if (rc) return rc;
   UnitOps &un = *pc->unit;
@@ -141,7 +146,7 @@ int piafs_dev_interp_interfaces(piafs_case *pc, double *fI, const double *fC, co
   launch_class(un.eng.d_cases, un.eng.plan, K_FLUX, 0, st);
   if (!uflag)
     launch_dev_planar(G, fC, dir ? nullptr : d.flux_x, dir ? d.flux_y : nullptr, 1, 0, nullptr, st);
-  for (int cls : {K_ENDS, K_RECON, K_RECONF, K_RCHAR, K_CWROWS, K_CWSOLVE})
+  for (int cls : {K_ENDS, K_RECON, K_RECONF, K_LROWS, K_LSOLVE, K_CWROWS, K_CWSOLVE})
     launch_class(un.eng.d_cases, un.eng.plan, cls, 0, st);
   const int r = (uflag ? 0 : 2) + (upw > 0 ? 0 : 1);
   const SweepGeom &S = dir ? d.Sy : d.Sx;

@@ -5,7 +5,7 @@
 // file:line of the formula being restated is given at each device function),
 // and the library is compiled without floating-point contraction so that the
 // rounding of every +, -, *, / and sqrt matches the reference build.
-#include "kernels.hpp"
+#include "device.hpp"
 
 #include <cstdio>
 #include <type_traits>
@@ -17,346 +17,6 @@ namespace {
 constexpr int TB = 256;  // threads per block
 
 inline unsigned nblk(long n, int tb = TB) { return (unsigned)((n + tb - 1) / tb); }
-
-// ---------------------------------------------------------------------------
-// Quotient n / d for the WENO weights and the CRWENO5 multipliers: the
-// target's IEEE double division (a reciprocal estimate, two Newton-Raphson
-// refinements and one residual correction, Markstein's method) without its
-// range scaling and special-case fix-up steps, in three fewer instructions
-// and with no condition register between them.  Those steps are identities,
-// and the result is the IEEE quotient's bits, while n is +0 or of magnitude at
-// least 2^-969, d is normal and positive, and the quotient lies within
-// 2^-969 .. 2^1022: for the weights, whenever the smoothness indicators stay
-// within about 2^400 of epsilon (data of ordinary magnitude with the usual
-// epsilons).  Far outside (epsilon 1e-100 with data of 1e70), a weight below
-// about 1e-290 can differ in its last bits, and where a Z or YC ratio
-// overflows the row's weights are all NaN rather than partly NaN: the
-// interpolated value is still NaN as the reference's is, and a tiny weight's
-// term lies far below the last bit of a sum led by the large weights.
-// ---------------------------------------------------------------------------
-#ifndef PIAFS_FAST_WDIV
-#define PIAFS_FAST_WDIV 1
-#endif
-__device__ __forceinline__ double wdiv(double n, double d) {
-#if PIAFS_FAST_WDIV
-  const double r0 = __builtin_amdgcn_rcp(d);
-  const double e0 = __builtin_fma(-d, r0, 1.0);
-  const double r1 = __builtin_fma(r0, e0, r0);
-  const double e1 = __builtin_fma(-d, r1, 1.0);
-  const double r2 = __builtin_fma(r1, e1, r1);
-  const double q = n * r2;
-  const double t = __builtin_fma(-d, q, n);
-  return __builtin_fma(t, r2, q);
-#else
-  return n / d;
-#endif
-}
-
-// ---------------------------------------------------------------------------
-// WENO5 nonlinear weights, include/interpolation.h:255-490
-// (JS :255-281, mapped :309-341, Z (Borges) :420-450, YC :478-508)
-// ---------------------------------------------------------------------------
-template <int KIND>
-__device__ __forceinline__ void weno_w(double c1, double c2, double c3, double m3, double m2, double m1,
-                                       double p1, double p2, double eps, double &w1, double &w2, double &w3) {
-  const double t1312 = 13.0 / 12.0, q14 = 1.0 / 4.0;
-  const double d1 = m3 - 2 * m2 + m1, e1 = m3 - 4 * m2 + 3 * m1;
-  const double d2 = m2 - 2 * m1 + p1, e2 = m2 - p1;
-  const double d3 = m1 - 2 * p1 + p2, e3 = 3 * m1 - 4 * p1 + p2;
-  const double b1 = t1312 * d1 * d1 + q14 * e1 * e1;
-  const double b2 = t1312 * d2 * d2 + q14 * e2 * e2;
-  const double b3 = t1312 * d3 * d3 + q14 * e3 * e3;
-  double a1, a2, a3;
-  if (KIND == 2 || KIND == 3) {
-    double tau;
-    if (KIND == 2) {
-      tau = fabs(b3 - b1);
-    } else {
-      const double t = m3 - 4 * m2 + 6 * m1 - 4 * p1 + p2;
-      tau = t * t;
-    }
-    const double r1 = wdiv(tau, b1 + eps), r2 = wdiv(tau, b2 + eps), r3 = wdiv(tau, b3 + eps);
-    a1 = c1 * (1.0 + r1 * r1);
-    a2 = c2 * (1.0 + r2 * r2);
-    a3 = c3 * (1.0 + r3 * r3);
-  } else {
-    a1 = wdiv(c1, (b1 + eps) * (b1 + eps));
-    a2 = wdiv(c2, (b2 + eps) * (b2 + eps));
-    a3 = wdiv(c3, (b3 + eps) * (b3 + eps));
-  }
-  double s = wdiv(1.0, a1 + a2 + a3);
-  w1 = a1 * s;
-  w2 = a2 * s;
-  w3 = a3 * s;
-  if (KIND == 1) {
-    a1 = wdiv(w1 * (c1 + c1 * c1 - 3 * c1 * w1 + w1 * w1), c1 * c1 + w1 * (1.0 - 2.0 * c1));
-    a2 = wdiv(w2 * (c2 + c2 * c2 - 3 * c2 * w2 + w2 * w2), c2 * c2 + w2 * (1.0 - 2.0 * c2));
-    a3 = wdiv(w3 * (c3 + c3 * c3 - 3 * c3 * w3 + w3 * w3), c3 * c3 + w3 * (1.0 - 2.0 * c3));
-    s = wdiv(1.0, a1 + a2 + a3);
-    w1 = a1 * s;
-    w2 = a2 * s;
-    w3 = a3 * s;
-  }
-}
-
-__device__ __forceinline__ void weno_w_rt(int kind, double c1, double c2, double c3, double m3, double m2,
-                                          double m1, double p1, double p2, double eps, double &w1, double &w2,
-                                          double &w3) {
-  switch (kind) {
-    case 1: weno_w<1>(c1, c2, c3, m3, m2, m1, p1, p2, eps, w1, w2, w3); break;
-    case 2: weno_w<2>(c1, c2, c3, m3, m2, m1, p1, p2, eps, w1, w2, w3); break;
-    case 3: weno_w<3>(c1, c2, c3, m3, m2, m1, p1, p2, eps, w1, w2, w3); break;
-    default: weno_w<0>(c1, c2, c3, m3, m2, m1, p1, p2, eps, w1, w2, w3); break;
-  }
-}
-
-// Candidate stencils of WENO5 (Interp1PrimFifthOrderWENO.c:151-153) and of the
-// compact scheme (Interp1PrimFifthOrderCRWENO.c:176-179).
-__device__ __forceinline__ void weno5_cands(double m3, double m2, double m1, double p1, double p2, double &f1,
-                                            double &f2, double &f3) {
-  const double s6 = 1.0 / 6.0;
-  f1 = (2 * s6) * m3 + (-7 * s6) * m2 + (11 * s6) * m1;
-  f2 = (-s6) * m2 + (5 * s6) * m1 + (2 * s6) * p1;
-  f3 = (2 * s6) * m1 + (5 * s6) * p1 + (-s6) * p2;
-}
-__device__ __forceinline__ void crweno5_cands(double m2, double m1, double p1, double &f1, double &f2,
-                                              double &f3) {
-  const double s6 = 1.0 / 6.0;
-  f1 = (s6)*m2 + (5 * s6) * m1;
-  f2 = (5 * s6) * m1 + (s6)*p1;
-  f3 = (s6)*m1 + (5 * s6) * p1;
-}
-
-// Linear fifth-order upwind interpolation (upw5),
-// Interp1PrimFifthOrderUpwind.c:92-96 and :138-142, in the reference's
-// operation order (sums left to right).
-__device__ __forceinline__ double upw5_value(double m3, double m2, double m1, double p1, double p2) {
-  const double c30 = 1.0 / 30.0, c13 = 13.0 / 60.0, c47 = 47.0 / 60.0, c27 = 27.0 / 60.0, c20 = 1.0 / 20.0;
-  return c30 * m3 - c13 * m2 + c47 * m1 + c27 * p1 - c20 * p2;
-}
-
-// Coefficients of row k of one line system: A, B, C and the right-hand side
-// (for WENO5 and upw5, KIND 4, the right-hand side is the interface value
-// itself).
-template <int CR, int KIND>
-__device__ __forceinline__ void row_coeffs(int k, int N, bool left, const ReconParams &R, double w0, double w1,
-                                           double w2, double w3, double w4, double w5, double &Ak, double &Bk,
-                                           double &Ck, double &Rk) {
-  double m3, m2, m1, p1, p2;
-  if (left) { m3 = w0; m2 = w1; m1 = w2; p1 = w3; p2 = w4; }
-  else { m3 = w5; m2 = w4; m1 = w3; p1 = w2; p2 = w1; }
-  if (KIND == 4) {
-    Ak = 0.0; Bk = 1.0; Ck = 0.0;
-    Rk = upw5_value(m3, m2, m1, p1, p2);
-    return;
-  }
-  const bool bnd = (k == 0) || (k == N);
-  double c1, c2, c3;
-  if (CR && !bnd) { c1 = 0.2; c2 = 0.5; c3 = 0.3; }
-  else { c1 = 0.1; c2 = 0.6; c3 = 0.3; }
-  double a1, a2, a3;
-  if (R.no_limiting) { a1 = c1; a2 = c2; a3 = c3; }
-  else weno_w<KIND>(c1, c2, c3, m3, m2, m1, p1, p2, R.eps, a1, a2, a3);
-  double f1, f2, f3;
-  if (!CR || bnd) {
-    weno5_cands(m3, m2, m1, p1, p2, f1, f2, f3);
-    Ak = 0.0; Bk = 1.0; Ck = 0.0;
-  } else {
-    const double t3 = 1.0 / 3.0;
-    crweno5_cands(m2, m1, p1, f1, f2, f3);
-    const double lo = (2 * t3) * a1 + (t3)*a2;
-    Bk = (t3)*a1 + (2 * t3) * a2 + (2 * t3) * a3;
-    const double hi = (t3)*a3;
-    if (left) { Ak = lo; Ck = hi; } else { Ak = hi; Ck = lo; }
-  }
-  Rk = a1 * f1 + a2 * f2 + a3 * f3;
-}
-
-// ---------------------------------------------------------------------------
-// 1D Euler eigenstructure, euler1d.h:91-193
-// ---------------------------------------------------------------------------
-struct Eig3 {
-  double L[3][3], R[3][3], D[3];
-};
-
-__device__ __forceinline__ void euler1d_roeavg(double g, double rhoL, double muL, double eL, double rhoR,
-                                               double muR, double eR, double &r0, double &r1, double &r2) {
-  const double vL = muL / rhoL, PL = (eL - 0.5 * rhoL * vL * vL) * (g - 1.0), cLsq = g * PL / rhoL;
-  const double HL = 0.5 * vL * vL + cLsq / (g - 1.0);
-  const double vR = muR / rhoR, PR = (eR - 0.5 * rhoR * vR * vR) * (g - 1.0), cRsq = g * PR / rhoR;
-  const double HR = 0.5 * vR * vR + cRsq / (g - 1.0);
-  const double tL = sqrt(rhoL), tR = sqrt(rhoR);
-  const double rho = tL * tR, v = (tL * vL + tR * vR) / (tL + tR), H = (tL * HL + tR * HR) / (tL + tR);
-  const double csq = (g - 1.0) * (H - 0.5 * v * v), P = csq * rho / g;
-  r0 = rho;
-  r1 = rho * v;
-  r2 = P / (g - 1.0) + 0.5 * rho * v * v;
-}
-
-__device__ __forceinline__ void euler1d_eig(double g, double u0, double u1, double u2, Eig3 &E) {
-  const double rho = u0, v = u1 / rho, e = u2;
-  const double P = (e - 0.5 * rho * v * v) * (g - 1.0), c = sqrt(g * P / rho);
-  E.D[0] = v; E.D[1] = v - c; E.D[2] = v + c;
-  const double k = (g - 1) / (rho * c);
-  E.L[1][0] = k * (-(v * v) / 2 - c * v / (g - 1));
-  E.L[1][1] = k * (v + c / (g - 1));
-  E.L[1][2] = k * (-1);
-  E.L[0][0] = k * (rho * (-(v * v) / 2 + c * c / (g - 1)) / c);
-  E.L[0][1] = k * (rho * v / c);
-  E.L[0][2] = k * (-rho / c);
-  E.L[2][0] = k * ((v * v) / 2 - c * v / (g - 1));
-  E.L[2][1] = k * (-v + c / (g - 1));
-  E.L[2][2] = k * (1);
-  E.R[0][1] = -rho / (2 * c);
-  E.R[1][1] = -rho * (v - c) / (2 * c);
-  E.R[2][1] = -rho * ((v * v) / 2 + (c * c) / (g - 1) - c * v) / (2 * c);
-  E.R[0][0] = 1; E.R[1][0] = v; E.R[2][0] = v * v / 2;
-  E.R[0][2] = rho / (2 * c);
-  E.R[1][2] = rho * (v + c) / (2 * c);
-  E.R[2][2] = rho * ((v * v) / 2 + (c * c) / (g - 1) + c * v) / (2 * c);
-}
-
-// ---------------------------------------------------------------------------
-// 2D Navier-Stokes flow eigenstructure along direction DIR (0: x, 1: y).
-// Only the 4x4 flow block is formed: the species block of the reference's
-// n x n matrices is the identity (L, R) with eigenvalue vn.
-// ---------------------------------------------------------------------------
-// Roe average of two conserved flow states (navierstokes2d.h:115-160)
-__device__ __forceinline__ void ns2d_roeavg(double g, const double uL[4], const double uR[4], double ua[4]) {
-  const double rhoL = uL[0], vxL = uL[1] / rhoL, vyL = uL[2] / rhoL, eL = uL[3];
-  const double vsqL = (vxL * vxL) + (vyL * vyL), PL = (eL - 0.5 * rhoL * vsqL) * (g - 1.0);
-  const double cLsq = g * PL / rhoL, HL = 0.5 * (vxL * vxL + vyL * vyL) + cLsq / (g - 1.0);
-  const double rhoR = uR[0], vxR = uR[1] / rhoR, vyR = uR[2] / rhoR, eR = uR[3];
-  const double vsqR = (vxR * vxR) + (vyR * vyR), PR = (eR - 0.5 * rhoR * vsqR) * (g - 1.0);
-  const double cRsq = g * PR / rhoR, HR = 0.5 * (vxR * vxR + vyR * vyR) + cRsq / (g - 1.0);
-  const double tL = sqrt(rhoL), tR = sqrt(rhoR);
-  const double rA = tL * tR;
-  const double vxA = (tL * vxL + tR * vxR) / (tL + tR), vyA = (tL * vyL + tR * vyR) / (tL + tR);
-  const double HA = (tL * HL + tR * HR) / (tL + tR), vsqA = vxA * vxA + vyA * vyA;
-  const double csqA = (g - 1.0) * (HA - 0.5 * vsqA), PA = csqA * rA / g;
-  ua[0] = rA;
-  ua[1] = rA * vxA;
-  ua[2] = rA * vyA;
-  ua[3] = PA / (g - 1.0) + 0.5 * rA * vsqA;
-}
-
-// Flow eigenvalues, in the reference's order (navierstokes2d.h:161-184)
-template <int DIR>
-__device__ __forceinline__ void ns2d_eigvals(double g, const double u[4], double D[4]) {
-  const double rho = u[0], vx = (rho == 0) ? 0 : u[1] / rho, vy = (rho == 0) ? 0 : u[2] / rho, e = u[3];
-  const double vsq = (vx * vx) + (vy * vy), P = (e - 0.5 * rho * vsq) * (g - 1.0);
-  const double a = sqrt(g * P / rho), vn = DIR == 0 ? vx : vy;
-  D[0] = vn - a;
-  if (DIR == 0) { D[1] = vn + a; D[2] = vn; }
-  else { D[1] = vn; D[2] = vn + a; }
-  D[3] = vn;
-}
-
-// |v_n| of the Roe average of two cells with the Harten entropy fix
-// (delta = 1e-6, NavierStokes2DUpwind.c:75-78): the species' dissipation
-// coefficient of the Roe flux, as upwind_ns2d_roe computes it
-template <int DIR>
-__device__ __forceinline__ double ns2d_roe_dsp(double g, const double uLc[4], const double uRc[4]) {
-  double ua[4], D[4];
-  ns2d_roeavg(g, uLc, uRc, ua);
-  ns2d_eigvals<DIR>(g, ua, D);
-  const double vn = D[3];
-  const double delta = 0.000001, delta2 = delta * delta;
-  return fabs(vn) < delta ? (vn * vn + delta2) / (2 * delta) : fabs(vn);
-}
-
-// Left (rows) and right (columns) flow eigenvectors (navierstokes2d.h:186-311)
-template <int DIR>
-__device__ __forceinline__ void ns2d_eigvecs(double g, const double u[4], double L[4][4], double R[4][4]) {
-  const double gm1 = g - 1.0;
-  const double rho = u[0], vx = (rho == 0) ? 0 : u[1] / rho, vy = (rho == 0) ? 0 : u[2] / rho, e = u[3];
-  const double vsq = (vx * vx) + (vy * vy), P = (e - 0.5 * rho * vsq) * (g - 1.0);
-  const double a = sqrt(g * P / rho), ek = 0.5 * (vx * vx + vy * vy);
-  const double aa2 = 2 * a * a, aa = a * a;
-  if (DIR == 0) {
-    const double un = vx, nx = 1.0, ny = 0.0;
-    L[0][0] = (gm1 * ek + a * un) / aa2;
-    L[0][1] = ((-gm1) * vx - a * nx) / aa2;
-    L[0][2] = ((-gm1) * vy - a * ny) / aa2;
-    L[0][3] = gm1 / aa2;
-    L[3][0] = (aa - gm1 * ek) / aa;
-    L[3][1] = (gm1 * vx) / aa;
-    L[3][2] = (gm1 * vy) / aa;
-    L[3][3] = (-gm1) / aa;
-    L[1][0] = (gm1 * ek - a * un) / aa2;
-    L[1][1] = ((-gm1) * vx + a * nx) / aa2;
-    L[1][2] = ((-gm1) * vy + a * ny) / aa2;
-    L[1][3] = gm1 / aa2;
-    L[2][0] = (vy - un * ny) / nx;
-    L[2][1] = ny;
-    L[2][2] = (ny * ny - 1.0) / nx;
-    L[2][3] = 0.0;
-  } else {
-    const double un = vy, nx = 0.0, ny = 1.0;
-    L[0][0] = (gm1 * ek + a * un) / aa2;
-    L[0][1] = ((1.0 - g) * vx - a * nx) / aa2;
-    L[0][2] = ((1.0 - g) * vy - a * ny) / aa2;
-    L[0][3] = gm1 / aa2;
-    L[3][0] = (aa - gm1 * ek) / aa;
-    L[3][1] = gm1 * vx / aa;
-    L[3][2] = gm1 * vy / aa;
-    L[3][3] = (1.0 - g) / aa;
-    L[2][0] = (gm1 * ek - a * un) / aa2;
-    L[2][1] = ((1.0 - g) * vx + a * nx) / aa2;
-    L[2][2] = ((1.0 - g) * vy + a * ny) / aa2;
-    L[2][3] = gm1 / aa2;
-    L[1][0] = (un * nx - vx) / ny;
-    L[1][1] = (1.0 - nx * nx) / ny;
-    L[1][2] = -nx;
-    L[1][3] = 0;
-  }
-  const double h0 = a * a / gm1 + ek;
-  const double nx = DIR == 0 ? 1.0 : 0.0, ny = DIR == 0 ? 0.0 : 1.0, un = DIR == 0 ? vx : vy;
-  R[0][0] = 1.0; R[1][0] = vx - a * nx; R[2][0] = vy - a * ny; R[3][0] = h0 - a * un;
-  R[0][3] = 1.0; R[1][3] = vx; R[2][3] = vy; R[3][3] = ek;
-  const int cp = DIR == 0 ? 1 : 2, cz = DIR == 0 ? 2 : 1;
-  R[0][cp] = 1.0; R[1][cp] = vx + a * nx; R[2][cp] = vy + a * ny; R[3][cp] = h0 + a * un;
-  R[0][cz] = 0.0; R[1][cz] = ny; R[2][cz] = -nx; R[3][cz] = vx * ny - vy * nx;
-}
-
-// rf-char selection for one characteristic field (Euler1DUpwindRF,
-// Euler1DUpwind.c:160-173; NavierStokes2DUpwindRF, NavierStokes2DUpwind.c:152-166):
-// upwind when the field's eigenvalue has one sign at the left, averaged and
-// right states, else a local Lax-Friedrichs flux with the largest |eigenvalue|.
-// With llf set, the local Lax-Friedrichs flux is taken for every field
-// (Euler1DUpwindLLF, Euler1DUpwind.c:259-261; NavierStokes2DUpwindLLF,
-// NavierStokes2DUpwind.c:248-250).
-__device__ __forceinline__ double rf_pick(double eL, double eC, double eR, double ucL, double ucR, double fcL,
-                                          double fcR, bool llf) {
-  if (!llf && eL > 0 && eC > 0 && eR > 0) return fcL;
-  if (!llf && eL < 0 && eC < 0 && eR < 0) return fcR;
-  const double x1 = fabs(eL), x2 = fabs(eC), x3 = fabs(eR);
-  const double mx1 = x1 > x2 ? x1 : x2, mx2 = x2 > x3 ? x2 : x3;
-  const double alpha = mx1 > mx2 ? mx1 : mx2;
-  return 0.5 * (fcL + fcR + alpha * (ucL - ucR));
-}
-
-// ---------------------------------------------------------------------------
-// Ensemble indexing: block -> case, local work item
-// ---------------------------------------------------------------------------
-#define CASE_ARGS const CaseDev *__restrict__ cases, const int *__restrict__ blockcase, \
-                  const int *__restrict__ firstblock, int stage
-// Workgroups go to the eight XCDs in turn, each XCD with its own L2.  The tile
-// kernels take their tiles in this order: each XCD gets one contiguous band of
-// the case's nb tiles, so that the cache lines two neighbouring tiles share are
-// fetched into one L2.  It is a bijection of 0..nb-1; a case whose blocks do not
-// start on a multiple of eight keeps workgroup order.
-__device__ __forceinline__ int xcd_order(int id, int nb, int first) {
-  if (!PIAFS_XCD_ORDER || (first & 7)) return id;
-  const int q = nb >> 3, r = nb & 7, x = id & 7, k = id >> 3;
-  return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + k;
-}
-
-#define CASE_PREAMBLE                                                      \
-  const int cidx = blockcase[blockIdx.x];                                  \
-  const CaseDev &C = cases[cidx];                                          \
-  const long t = (long)(blockIdx.x - firstblock[cidx]) * blockDim.x + threadIdx.x; \
-  (void)stage;
 
 // ---------------------------------------------------------------------------
 // Stage state + boundary conditions.
@@ -391,17 +51,6 @@ __device__ __forceinline__ double stage_value(const CaseDev &C, int s, long p) {
 // A ghost point no zone sets keeps the value the reference never changes
 // from its zero initialisation.
 // ---------------------------------------------------------------------------
-// _NavierStokes2DGetFlowVar_, navierstokes2d.h:70-79
-__device__ __forceinline__ void ns2d_flowvar(const double u[4], double gam, double &rho, double &vx, double &vy,
-                                             double &e, double &P) {
-  rho = u[0];
-  vx = (rho == 0) ? 0 : u[1] / rho;
-  vy = (rho == 0) ? 0 : u[2] / rho;
-  e = u[3];
-  const double vsq = (vx * vx) + (vy * vy);
-  P = (e - 0.5 * rho * vsq) * (gam - 1.0);
-}
-
 // does zone z set variable v (the flow BCs exist for ndims 2 only, the slip
 // wall also for ndims 1; walls and outflows leave passive scalars alone)
 __device__ __forceinline__ bool zone_sets(const Zone &z, int v, int ndims) {
@@ -598,39 +247,6 @@ __global__ void __launch_bounds__(256) k_ghost(CASE_ARGS) {
 // NavierStokes2DFlux.c:24-52 (navierstokes2d.h:70-110), Euler1DFlux.c:19
 // (euler1d.h:61-85).
 // ---------------------------------------------------------------------------
-// The flux along dir at one point (NavierStokes2DFlux.c:24-52 with
-// navierstokes2d.h:70-110; Euler1DFlux.c:19 with euler1d.h:61-85): q(m) reads
-// variable m of the point, put(m, value) writes component m of the flux.
-template <class Q, class Put>
-__device__ __forceinline__ void point_flux(int model, int dir, double gamma, int nv, Q q, Put put) {
-  if (model == 1) {
-    const double rho = q(0), v = q(1) / rho, e = q(2);
-    const double P_ = (e - 0.5 * rho * v * v) * (gamma - 1.0);
-    put(0, rho * v);
-    put(1, rho * v * v + P_);
-    put(2, (e + P_) * v);
-    for (int m = 3; m < nv; m++) put(m, v * q(m));
-  } else {
-    const double rho = q(0);
-    const double vx = (rho == 0) ? 0 : q(1) / rho;
-    const double vy = (rho == 0) ? 0 : q(2) / rho;
-    const double e = q(3);
-    const double vsq = (vx * vx) + (vy * vy);
-    const double P_ = (e - 0.5 * rho * vsq) * (gamma - 1.0);
-    const double vn = dir == 0 ? vx : vy;
-    put(0, rho * vn);
-    if (dir == 0) {
-      put(1, rho * vx * vx + P_);
-      put(2, rho * vx * vy);
-    } else {
-      put(1, rho * vy * vx);
-      put(2, rho * vy * vy + P_);
-    }
-    put(3, (e + P_) * vn);
-    for (int m = 4; m < nv; m++) put(m, vn * q(m));
-  }
-}
-
 __global__ void __launch_bounds__(256) k_flux(CASE_ARGS) {
   CASE_PREAMBLE
   if (stage >= C.nstages) return;
@@ -1112,7 +728,7 @@ __device__ __forceinline__ void team_solve(double (&A)[MR], double (&B)[MR], dou
 }
 
 // ---------------------------------------------------------------------------
-// Component-wise WENO5 / CRWENO5 reconstruction.  One system per (line,
+// Component-wise CRWENO5 reconstruction.  One system per (line,
 // variable, reconstruction r): r = 0 uL, 1 uR (of the state), 2 fL, 3 fR (of
 // the flux); r even = left-biased.  A team of lanes covers the interfaces of
 // one system: lane j computes rows 1 + j*m .. of the interior rows 1..N-1,
@@ -1121,7 +737,6 @@ __device__ __forceinline__ void team_solve(double (&A)[MR], double (&B)[MR], dou
 //    (WENOFifthOrderCalculateWeights.c:112-237 and the variants);
 //    optimal weights :202-220 (WENO5 values at the two end interfaces of a
 //    CRWENO line).
-//  * WENO5: Interp1PrimFifthOrderWENO.c:124-166.
 //  * CRWENO5: row assembly Interp1PrimFifthOrderCRWENO.c:132-201 (identity
 //    rows with WENO5 right-hand sides at interfaces 0 and N), then the line
 //    solve (team_solve above).
@@ -1135,7 +750,7 @@ __host__ __device__ inline long recon_systems(const SweepGeom &S, int nv, int pa
   return S.longl ? 0 : (long)S.nlines * nv * (paired ? 2 : 4);
 }
 
-template <int CR, int KIND>
+template <int KIND>
 __device__ __forceinline__ void recon_team(const CaseDev &C, int dir, long sys, bool active, int lane, double *red,
                                            double *stash) {
   const SweepGeom &S = dir ? C.Sy : C.Sx;
@@ -1162,8 +777,8 @@ __device__ __forceinline__ void recon_team(const CaseDev &C, int dir, long sys, 
     const bool left = !(r & 1);
     // the end interfaces 0 and N (identity rows carrying WENO5 values, from k_recon_ends)
     double x0 = 0.0, xN = 0.0;
-    if (CR && active && lane == 0) x0 = paired ? ends[2 * side] : io[r][line];
-    if (CR && active && lane == lastlane) xN = paired ? ends[2 * side + 1] : io[r][line + N];
+    if (active && lane == 0) x0 = paired ? ends[2 * side] : io[r][line];
+    if (active && lane == lastlane) xN = paired ? ends[2 * side + 1] : io[r][line + N];
     // stencil window: positions lo-3 .. lo+n+1
     double win[kMaxRows + 5];
 #pragma unroll
@@ -1175,14 +790,13 @@ __device__ __forceinline__ void recon_team(const CaseDev &C, int dir, long sys, 
 #pragma unroll
     for (int i = 0; i < kMaxRows; i++) {
       if (i < n) {
-        row_coeffs<CR, KIND>(lo + i, N, left, C.R, win[i], win[i + 1], win[i + 2], win[i + 3], win[i + 4],
+        row_coeffs<KIND>(lo + i, N, left, C.R, win[i], win[i + 1], win[i + 2], win[i + 3], win[i + 4],
                              win[i + 5], A[i], B[i], Cc[i], X[i]);
       } else {
         A[i] = 0.0; B[i] = 1.0; Cc[i] = 0.0; X[i] = 0.0;
       }
     }
-    if (CR)
-      team_solve<kMaxRows, false, PIAFS_FAST_WDIV>(A, B, Cc, X, n, lane, S.team, lane == lastlane, x0, xN, red, C.status,
+    team_solve<kMaxRows, false, PIAFS_FAST_WDIV>(A, B, Cc, X, n, lane, S.team, lane == lastlane, x0, xN, red, C.status,
                            C.R.plain_start != 0);
   };
   solve(r0, 0);
@@ -1226,14 +840,6 @@ __host__ __device__ inline int line_region(int T, int m) {
 // plus the overrun of the last lane's window when its segment is short
 constexpr int kLineLds = 256 * (16 + 5 + 2) + 32;
 
-// Block barrier that orders LDS accesses only: global loads and stores issued
-// before it stay in flight (a __syncthreads also waits for those).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // all lanes of the team have finished their LDS accesses before any lane goes on
 __device__ __forceinline__ void team_lds_sync(int T) {
   if (T > 64) {
@@ -1245,7 +851,7 @@ __device__ __forceinline__ void team_lds_sync(int T) {
   }
 }
 
-template <int CR, int KIND, bool FULL>
+template <int KIND, bool FULL>
 __device__ __forceinline__ void recon_pair_lds(const CaseDev &C, int dir, long sys, bool active, int lane,
                                                double *red, double *stash, double *lines) {
   const SweepGeom &S = dir ? C.Sy : C.Sx;
@@ -1294,8 +900,8 @@ __device__ __forceinline__ void recon_pair_lds(const CaseDev &C, int dir, long s
     // order and the register count at two waves per SIMD)
     const int nrow = FULL ? m : n;
     double x0 = 0.0, xN = 0.0;
-    if (CR && active && lane == 0) x0 = ends[2 * side];
-    if (CR && active && lane == xn_lane) xN = ends[2 * side + 1];
+    if (active && lane == 0) x0 = ends[2 * side];
+    if (active && lane == xn_lane) xN = ends[2 * side + 1];
     // stencil window: positions lo-3 .. lo+n+1
     double win[kMaxRows + 5];
 #pragma unroll
@@ -1304,7 +910,7 @@ __device__ __forceinline__ void recon_pair_lds(const CaseDev &C, int dir, long s
 #pragma unroll
     for (int i = 0; i < kMaxRows; i++) {
       if (i < nrow) {
-        row_coeffs<CR, KIND>(lo + i, N, LEFT, C.R, win[i], win[i + 1], win[i + 2], win[i + 3], win[i + 4],
+        row_coeffs<KIND>(lo + i, N, LEFT, C.R, win[i], win[i + 1], win[i + 2], win[i + 3], win[i + 4],
                              win[i + 5], A[i], B[i], Cc[i], X[i]);
       } else {
         A[i] = 0.0; B[i] = 1.0; Cc[i] = 0.0; X[i] = 0.0;
@@ -1319,14 +925,12 @@ __device__ __forceinline__ void recon_pair_lds(const CaseDev &C, int dir, long s
         }
       }
     }
-    if (CR) {
-      if (FULL)
-        team_solve<kMaxRows, true, PIAFS_FAST_WDIV>(A, B, Cc, X, kMaxRows, lane, T, lane == T - 1, x0, nlane < T ? 0.0 : xN, red,
-                                   C.status, C.R.plain_start != 0);
-      else
-        team_solve<kMaxRows, false, PIAFS_FAST_WDIV>(A, B, Cc, X, n, lane, T, lane == lastlane, x0, xN, red, C.status,
-                             C.R.plain_start != 0);
-    }
+    if (FULL)
+      team_solve<kMaxRows, true, PIAFS_FAST_WDIV>(A, B, Cc, X, kMaxRows, lane, T, lane == T - 1, x0, nlane < T ? 0.0 : xN, red,
+                                 C.status, C.R.plain_start != 0);
+    else
+      team_solve<kMaxRows, false, PIAFS_FAST_WDIV>(A, B, Cc, X, n, lane, T, lane == lastlane, x0, xN, red, C.status,
+                           C.R.plain_start != 0);
   };
   solve(std::integral_constant<bool, true>(), 0);
 #pragma unroll
@@ -1406,15 +1010,15 @@ __device__ __forceinline__ void recon_pair_lds(const CaseDev &C, int dir, long s
 // the WENO5 weights at the ends; plain WENO5 for the non-compact scheme).  In
 // paired mode a thread does both systems of its pair: the raw values go to
 // the case's `ends` table for the line solves, the combination to the output.
-template <int CR, int KIND>
+template <int KIND>
 __device__ __forceinline__ double end_value(const CaseDev &C, const SweepGeom &S, const double *src, int r, int k) {
   double a_, b_, c_, x_;
-  row_coeffs<CR, KIND>(k, S.N, !(r & 1), C.R, src[k - 3], src[k - 2], src[k - 1], src[k], src[k + 1], src[k + 2],
+  row_coeffs<KIND>(k, S.N, !(r & 1), C.R, src[k - 3], src[k - 2], src[k - 1], src[k], src[k + 1], src[k + 2],
                        a_, b_, c_, x_);
   return x_;
 }
 
-template <int CR, int KIND>
+template <int KIND>
 __device__ __forceinline__ void recon_end(const CaseDev &C, int dir, long sys, int e) {
   const SweepGeom &S = dir ? C.Sy : C.Sx;
   const int nv = C.G.nv, N = S.N, nl = S.nlines;
@@ -1428,182 +1032,14 @@ __device__ __forceinline__ void recon_end(const CaseDev &C, int dir, long sys, i
   double *const *io = dir ? C.iy : C.ix;
   const long at = ((long)v * nl + l) * (N + 1) + k;
   if (!paired) {
-    io[r0][at] = end_value<CR, KIND>(C, S, src, r0, k);
+    io[r0][at] = end_value<KIND>(C, S, src, r0, k);
     return;
   }
-  const double xl = end_value<CR, KIND>(C, S, src, r0, k), xr = end_value<CR, KIND>(C, S, src, r0 + 1, k);
+  const double xl = end_value<KIND>(C, S, src, r0, k), xr = end_value<KIND>(C, S, src, r0 + 1, k);
   double *ends = C.ends + 4 * ((dir ? recon_systems(C.Sx, nv, 1) : 0) + sys);
   ends[e] = xl;
   ends[2 + e] = xr;
   io[q][at] = q ? 0.5 * (xl + xr) : 0.5 * (xr - xl);
-}
-
-// Characteristic WENO5 for euler1d, one thread per (interface, line).
-// WENOFifthOrderCalculateWeightsChar* (WENOFifthOrderCalculateWeights.c:761-930)
-// and Interp1PrimFifthOrderWENOChar.c:127-195: L and R from the Roe average of
-// the two cells adjacent to the interface; species rows are the identity, so
-// species reconstruct component-wise.
-template <int KIND>
-__device__ __forceinline__ void recon_char_e1d(const SweepGeom &S, int nv, const ReconParams &R, double gam, int l,
-                                               int k, const double *__restrict__ q, const double *__restrict__ f,
-                                               double *const *io) {
-  const int nl = S.nlines, N = S.N;
-  const long pl = S.plane;
-  const long base = S.base + (long)l * S.line_stride;
-  auto at = [&](const double *a, int v, int pos) { return a[v * pl + base + pos]; };
-  double a0, a1, a2;
-  euler1d_roeavg(gam, at(q, 0, k - 1), at(q, 1, k - 1), at(q, 2, k - 1), at(q, 0, k), at(q, 1, k), at(q, 2, k),
-                 a0, a1, a2);
-  Eig3 E;
-  euler1d_eig(gam, a0, a1, a2, E);
-  const double s6 = 1.0 / 6.0;
-  for (int r = 0; r < 4; r++) {
-    const double *src = (r < 2) ? q : f;
-    const bool left = !(r & 1);
-    double *out = io[r];
-    int pos[5];
-    if (left) { pos[0] = k - 3; pos[1] = k - 2; pos[2] = k - 1; pos[3] = k; pos[4] = k + 1; }
-    else { pos[0] = k + 2; pos[1] = k + 1; pos[2] = k; pos[3] = k - 1; pos[4] = k - 2; }
-    double s[5][3];
-    for (int p = 0; p < 5; p++) {
-      const double x0 = at(src, 0, pos[p]), x1 = at(src, 1, pos[p]), x2 = at(src, 2, pos[p]);
-      for (int vv = 0; vv < 3; vv++) s[p][vv] = E.L[vv][0] * x0 + E.L[vv][1] * x1 + E.L[vv][2] * x2;
-    }
-    double fch[3];
-    for (int vv = 0; vv < 3; vv++) {
-      if (KIND == 4) {
-        fch[vv] = upw5_value(s[0][vv], s[1][vv], s[2][vv], s[3][vv], s[4][vv]);
-        continue;
-      }
-      double w1, w2, w3;
-      if (R.no_limiting) { w1 = 0.1; w2 = 0.6; w3 = 0.3; }
-      else weno_w<KIND>(0.1, 0.6, 0.3, s[0][vv], s[1][vv], s[2][vv], s[3][vv], s[4][vv], R.eps, w1, w2, w3);
-      const double f1 = (2 * s6) * s[0][vv] - (7.0 * s6) * s[1][vv] + (11.0 * s6) * s[2][vv];
-      const double f2 = (-s6) * s[1][vv] + (5.0 * s6) * s[2][vv] + (2 * s6) * s[3][vv];
-      const double f3 = (2 * s6) * s[2][vv] + (5 * s6) * s[3][vv] - (s6)*s[4][vv];
-      fch[vv] = w1 * f1 + w2 * f2 + w3 * f3;
-    }
-    for (int vv = 0; vv < 3; vv++)
-      out[((long)vv * nl + l) * (N + 1) + k] = E.R[vv][0] * fch[0] + E.R[vv][1] * fch[1] + E.R[vv][2] * fch[2];
-    for (int m = 3; m < nv; m++) {
-      const double m3 = at(src, m, pos[0]), m2 = at(src, m, pos[1]), m1 = at(src, m, pos[2]);
-      const double p1 = at(src, m, pos[3]), p2 = at(src, m, pos[4]);
-      if (KIND == 4) {
-        out[((long)m * nl + l) * (N + 1) + k] = upw5_value(m3, m2, m1, p1, p2);
-        continue;
-      }
-      double w1, w2, w3, f1, f2, f3;
-      if (R.no_limiting) { w1 = 0.1; w2 = 0.6; w3 = 0.3; }
-      else weno_w<KIND>(0.1, 0.6, 0.3, m3, m2, m1, p1, p2, R.eps, w1, w2, w3);
-      weno5_cands(m3, m2, m1, p1, p2, f1, f2, f3);
-      out[((long)m * nl + l) * (N + 1) + k] = w1 * f1 + w2 * f2 + w3 * f3;
-    }
-  }
-}
-
-// Characteristic WENO5 for navierstokes2d along DIR, one thread per
-// (interface, line): Interp1PrimFifthOrderWENOChar.c:89-201 with
-// WENOFifthOrderCalculateWeightsChar* (WENOFifthOrderCalculateWeights.c:761-930).
-// L and R come from the Roe average of the two cells adjacent to the
-// interface (navierstokes2d.h:115-311).  The flow values of the six stencil
-// positions k-3 .. k+2 are projected once and serve both biases; the species
-// rows of L and R are the identity, so species reconstruct component-wise.
-// Products are summed in index order, as MatVecMult does (the reference's
-// zero entries add exact zeros).
-template <int DIR, int KIND>
-__device__ __forceinline__ void recon_char_ns2d(const SweepGeom &S, int nv, const ReconParams &P, double gam, int l,
-                                                int k, const double *__restrict__ q, const double *__restrict__ f,
-                                                double *const *io) {
-  const int nl = S.nlines, N = S.N;
-  const long pl = S.plane;
-  const double *ql = q + S.base + (long)l * S.line_stride, *fl = f + S.base + (long)l * S.line_stride;
-  const double uLc[4] = {ql[k - 1], ql[pl + k - 1], ql[2 * pl + k - 1], ql[3 * pl + k - 1]};
-  const double uRc[4] = {ql[k], ql[pl + k], ql[2 * pl + k], ql[3 * pl + k]};
-  double ua[4], L[4][4], R[4][4];
-  ns2d_roeavg(gam, uLc, uRc, ua);
-  ns2d_eigvecs<DIR>(gam, ua, L, R);
-  const long vs = (long)nl * (N + 1), ii = (long)l * (N + 1) + k;
-  const double s6 = 1.0 / 6.0;
-  auto weno = [&](double m3, double m2, double m1, double p1, double p2) {
-    if (KIND == 4) return upw5_value(m3, m2, m1, p1, p2);
-    double w1, w2, w3;
-    if (P.no_limiting) { w1 = 0.1; w2 = 0.6; w3 = 0.3; }
-    else weno_w<KIND>(0.1, 0.6, 0.3, m3, m2, m1, p1, p2, P.eps, w1, w2, w3);
-    const double f1 = (2 * s6) * m3 - (7.0 * s6) * m2 + (11.0 * s6) * m1;
-    const double f2 = (-s6) * m2 + (5.0 * s6) * m1 + (2 * s6) * p1;
-    const double f3 = (2 * s6) * m1 + (5 * s6) * p1 - (s6)*p2;
-    return w1 * f1 + w2 * f2 + w3 * f3;
-  };
-#pragma unroll
-  for (int src = 0; src < 2; src++) {  // 0: the solution (uL, uR), 1: the flux (fL, fR)
-    const double *a = src ? fl : ql;
-    double c[6][4];  // characteristic values at k-3 .. k+2
-#pragma unroll
-    for (int p = 0; p < 6; p++) {
-      const int pos = k - 3 + p;
-      const double x0 = a[pos], x1 = a[pl + pos], x2 = a[2 * pl + pos], x3 = a[3 * pl + pos];
-#pragma unroll
-      for (int v = 0; v < 4; v++) c[p][v] = L[v][0] * x0 + L[v][1] * x1 + L[v][2] * x2 + L[v][3] * x3;
-    }
-#pragma unroll
-    for (int side = 0; side < 2; side++) {  // 0: left-biased (k-3 .. k+1), 1: right-biased (k+2 .. k-2)
-      double fch[4];
-#pragma unroll
-      for (int v = 0; v < 4; v++)
-        fch[v] = side ? weno(c[5][v], c[4][v], c[3][v], c[2][v], c[1][v])
-                      : weno(c[0][v], c[1][v], c[2][v], c[3][v], c[4][v]);
-      double *out = io[2 * src + side] + ii;
-#pragma unroll
-      for (int i = 0; i < 4; i++) out[i * vs] = R[i][0] * fch[0] + R[i][1] * fch[1] + R[i][2] * fch[2] + R[i][3] * fch[3];
-    }
-    for (int m = 4; m < nv; m++) {
-      const double *am = a + m * pl + k;
-      const double x[6] = {am[-3], am[-2], am[-1], am[0], am[1], am[2]};
-      io[2 * src][m * vs + ii] = weno(x[0], x[1], x[2], x[3], x[4]);
-      io[2 * src + 1][m * vs + ii] = weno(x[5], x[4], x[3], x[2], x[1]);
-    }
-  }
-}
-
-// Characteristic reconstruction: one thread per (interface, line) of each
-// sweep, x sweep first (from the natural layout), then y (from the
-// transposed copy).  Kept apart from the line-solve kernel so that neither's
-// register allocation limits the other's occupancy.
-__global__ void __launch_bounds__(256) k_recon_char(CASE_ARGS) {
-  CASE_PREAMBLE
-  if (stage >= C.nstages) return;
-  const long nX = (long)(C.Sx.N + 1) * C.Sx.nlines;
-  const long nY = (C.G.ndims == 2) ? (long)(C.Sy.N + 1) * C.Sy.nlines : 0;
-  if (t >= nX + nY) return;
-  const int dir = t < nX ? 0 : 1;
-  const SweepGeom &S = dir ? C.Sy : C.Sx;
-  const long u = dir ? t - nX : t;
-  const int k = (int)(u % (S.N + 1)), l = (int)(u / (S.N + 1));
-  const int nv = C.G.nv;
-  const double gam = C.P.gamma;
-  if (C.model == 1) {
-    switch (C.R.kind) {
-      case 1: recon_char_e1d<1>(S, nv, C.R, gam, l, k, C.U, C.flux_x, C.ix); break;
-      case 2: recon_char_e1d<2>(S, nv, C.R, gam, l, k, C.U, C.flux_x, C.ix); break;
-      case 3: recon_char_e1d<3>(S, nv, C.R, gam, l, k, C.U, C.flux_x, C.ix); break;
-      case 4: recon_char_e1d<4>(S, nv, C.R, gam, l, k, C.U, C.flux_x, C.ix); break;
-      default: recon_char_e1d<0>(S, nv, C.R, gam, l, k, C.U, C.flux_x, C.ix); break;
-    }
-    return;
-  }
-  const double *q = dir ? C.UT : C.U, *f = dir ? C.flux_y : C.flux_x;
-  double *const *io = dir ? C.iy : C.ix;
-#define RCHAR(KIND)                                                                  \
-  (dir ? recon_char_ns2d<1, KIND>(S, nv, C.R, gam, l, k, q, f, io)                  \
-       : recon_char_ns2d<0, KIND>(S, nv, C.R, gam, l, k, q, f, io))
-  switch (C.R.kind) {
-    case 1: RCHAR(1); break;
-    case 2: RCHAR(2); break;
-    case 3: RCHAR(3); break;
-    case 4: RCHAR(4); break;
-    default: RCHAR(0); break;
-  }
-#undef RCHAR
 }
 
 // ---------------------------------------------------------------------------
@@ -2337,7 +1773,7 @@ __host__ __device__ inline long long_rows(const SweepGeom &S, int nv) {
   return S.longl ? (long)(S.N + 1) * S.nlines * nv * 4 : 0;
 }
 
-template <int CR, int KIND>
+template <int KIND>
 __device__ __forceinline__ void lrow_at(const CaseDev &C, int dir, long t) {
   const SweepGeom &S = dir ? C.Sy : C.Sx;
   const int nv = C.G.nv, N = S.N;
@@ -2348,7 +1784,7 @@ __device__ __forceinline__ void lrow_at(const CaseDev &C, int dir, long t) {
   const double *src = (r < 2 ? (dir ? C.UT : C.U) : (dir ? C.flux_y : C.flux_x)) + (long)v * S.plane + S.base +
                       (long)l * S.line_stride;
   double a, b, c, x;
-  row_coeffs<CR, KIND>(k, N, !(r & 1), C.R, src[k - 3], src[k - 2], src[k - 1], src[k], src[k + 1], src[k + 2], a,
+  row_coeffs<KIND>(k, N, !(r & 1), C.R, src[k - 3], src[k - 2], src[k - 1], src[k], src[k + 1], src[k + 2], a,
                        b, c, x);
   double *L = C.lrow[dir];
   const long f = (long)(N + 1) * ns4, o = sys * (N + 1) + k;
@@ -2365,13 +1801,11 @@ __global__ void __launch_bounds__(256) k_lrows(CASE_ARGS) {
   if (t >= nX + nY) return;
   const int dir = t < nX ? 0 : 1;
   const long tt = dir ? t - nX : t;
-  const int cr = C.R.crweno;
   switch (C.R.kind) {
-    case 1: cr ? lrow_at<1, 1>(C, dir, tt) : lrow_at<0, 1>(C, dir, tt); break;
-    case 2: cr ? lrow_at<1, 2>(C, dir, tt) : lrow_at<0, 2>(C, dir, tt); break;
-    case 3: cr ? lrow_at<1, 3>(C, dir, tt) : lrow_at<0, 3>(C, dir, tt); break;
-    case 4: lrow_at<0, 4>(C, dir, tt); break;
-    default: cr ? lrow_at<1, 0>(C, dir, tt) : lrow_at<0, 0>(C, dir, tt); break;
+    case 1: lrow_at<1>(C, dir, tt); break;
+    case 2: lrow_at<2>(C, dir, tt); break;
+    case 3: lrow_at<3>(C, dir, tt); break;
+    default: lrow_at<0>(C, dir, tt); break;
   }
 }
 
@@ -2507,13 +1941,11 @@ __global__ void __launch_bounds__(256) k_recon_ends(CASE_ARGS) {
   const long q = dir ? t - 2 * nsx : t;
   const long sys = q >> 1;
   const int e = (int)(q & 1);
-  const int cr = C.R.crweno;
   switch (C.R.kind) {
-    case 1: cr ? recon_end<1, 1>(C, dir, sys, e) : recon_end<0, 1>(C, dir, sys, e); break;
-    case 2: cr ? recon_end<1, 2>(C, dir, sys, e) : recon_end<0, 2>(C, dir, sys, e); break;
-    case 3: cr ? recon_end<1, 3>(C, dir, sys, e) : recon_end<0, 3>(C, dir, sys, e); break;
-    case 4: recon_end<0, 4>(C, dir, sys, e); break;
-    default: cr ? recon_end<1, 0>(C, dir, sys, e) : recon_end<0, 0>(C, dir, sys, e); break;
+    case 1: recon_end<1>(C, dir, sys, e); break;
+    case 2: recon_end<2>(C, dir, sys, e); break;
+    case 3: recon_end<3>(C, dir, sys, e); break;
+    default: recon_end<0>(C, dir, sys, e); break;
   }
 }
 
@@ -2534,27 +1966,24 @@ __device__ __forceinline__ void recon_body(CASE_ARGS) {
   const int lane = threadIdx.x & (T - 1);
   const long sys = (long)lb * (256 / T) + threadIdx.x / T;
   const bool active = sys < recon_systems(S, C.G.nv, C.paired);
-  const int cr = C.R.crweno;
 #if PIAFS_RECON_LDS
   if (FULL || C.paired) {
     __shared__ double lines[kLineLds];
     switch (C.R.kind) {
-      case 1: cr ? recon_pair_lds<1, 1, FULL>(C, dir, sys, active, lane, red, stash, lines) : recon_pair_lds<0, 1, FULL>(C, dir, sys, active, lane, red, stash, lines); break;
-      case 2: cr ? recon_pair_lds<1, 2, FULL>(C, dir, sys, active, lane, red, stash, lines) : recon_pair_lds<0, 2, FULL>(C, dir, sys, active, lane, red, stash, lines); break;
-      case 3: cr ? recon_pair_lds<1, 3, FULL>(C, dir, sys, active, lane, red, stash, lines) : recon_pair_lds<0, 3, FULL>(C, dir, sys, active, lane, red, stash, lines); break;
-      case 4: recon_pair_lds<0, 4, FULL>(C, dir, sys, active, lane, red, stash, lines); break;
-      default: cr ? recon_pair_lds<1, 0, FULL>(C, dir, sys, active, lane, red, stash, lines) : recon_pair_lds<0, 0, FULL>(C, dir, sys, active, lane, red, stash, lines); break;
+      case 1: recon_pair_lds<1, FULL>(C, dir, sys, active, lane, red, stash, lines); break;
+      case 2: recon_pair_lds<2, FULL>(C, dir, sys, active, lane, red, stash, lines); break;
+      case 3: recon_pair_lds<3, FULL>(C, dir, sys, active, lane, red, stash, lines); break;
+      default: recon_pair_lds<0, FULL>(C, dir, sys, active, lane, red, stash, lines); break;
     }
     return;
   }
 #endif
   if (FULL) return;  // not reached: K_RECONF holds paired cases only
   switch (C.R.kind) {
-    case 1: cr ? recon_team<1, 1>(C, dir, sys, active, lane, red, stash) : recon_team<0, 1>(C, dir, sys, active, lane, red, stash); break;
-    case 2: cr ? recon_team<1, 2>(C, dir, sys, active, lane, red, stash) : recon_team<0, 2>(C, dir, sys, active, lane, red, stash); break;
-    case 3: cr ? recon_team<1, 3>(C, dir, sys, active, lane, red, stash) : recon_team<0, 3>(C, dir, sys, active, lane, red, stash); break;
-    case 4: recon_team<0, 4>(C, dir, sys, active, lane, red, stash); break;
-    default: cr ? recon_team<1, 0>(C, dir, sys, active, lane, red, stash) : recon_team<0, 0>(C, dir, sys, active, lane, red, stash); break;
+    case 1: recon_team<1>(C, dir, sys, active, lane, red, stash); break;
+    case 2: recon_team<2>(C, dir, sys, active, lane, red, stash); break;
+    case 3: recon_team<3>(C, dir, sys, active, lane, red, stash); break;
+    default: recon_team<0>(C, dir, sys, active, lane, red, stash); break;
   }
 }
 __global__ void __launch_bounds__(256) k_recon(CASE_ARGS) { recon_body<false>(cases, blockcase, firstblock, stage); }
@@ -2581,117 +2010,57 @@ __device__ __forceinline__ void upwind_ns2d_roe(const SweepGeom &S, int nv, doub
   const int k = (int)(t % (N + 1)), l = (int)(t / (N + 1));
   const long pl = S.plane;
   const long cL = S.base + (long)l * S.line_stride + (k - 1), cR = cL + 1;
-  // Roe average of the cell-centred neighbours, then its eigenstructure
   const double uLc[4] = {q[cL], q[pl + cL], q[2 * pl + cL], q[3 * pl + cL]};
   const double uRc[4] = {q[cR], q[pl + cR], q[2 * pl + cR], q[3 * pl + cR]};
-  double ua[4], D[4], L[4][4], R[4][4];
-  ns2d_roeavg(g, uLc, uRc, ua);
-  ns2d_eigvals<DIR>(g, ua, D);
-  ns2d_eigvecs<DIR>(g, ua, L, R);
-  const double vn = D[3];
-  const double delta = 0.000001, delta2 = delta * delta;
-  const double Dsp = (fabs(vn) < delta ? (vn * vn + delta2) / (2 * delta) : fabs(vn));
-#pragma unroll
-  for (int m = 0; m < 4; m++) D[m] = (fabs(D[m]) < delta ? (D[m] * D[m] + delta2) / (2 * delta) : fabs(D[m]));
   const long ii = (long)l * (N + 1) + k, vstride = (long)nl * (N + 1);
-  double ud[4], fo[4];
+  double ud[4], fs[4], fo[4];
 #pragma unroll
-  for (int m = 0; m < 4; m++) ud[m] = UD(m);
-  // modA = R (D L), row-major sums in index order (matmult_native.h:21-34)
-  double DL[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) DL[i][j] = D[i] * L[i][j];
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    double us = 0.0;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const double mA = R[i][0] * DL[0][j] + R[i][1] * DL[1][j] + R[i][2] * DL[2][j] + R[i][3] * DL[3][j];
-      us += mA * ud[j];
-    }
-    fo[i] = FS(i) - us;
+  for (int m = 0; m < 4; m++) {
+    ud[m] = UD(m);
+    fs[m] = FS(m);
   }
+  const double Dsp = roe_ns2d<DIR>(g, uLc, uRc, ud, fs, fo);
 #pragma unroll
   for (int m = 0; m < 4; m++) fI[m * vstride + ii] = fo[m];
   if (species)  // else the reconstruction has written them
     for (int m = 4; m < nv; m++) fI[m * vstride + ii] = FS(m) - Dsp * UD(m);
 }
 
-// mode: 0 Roe (Euler1DUpwind.c:27-93), 1 rf-char (:107-190), 2 llf-char
-// (:199-266), 3 rusanov (:282-353; its wave speed is gamma P/rho + |u|, with
-// no square root, as the reference computes it)
 template <int PAIR>
 __device__ __forceinline__ void upwind_e1d(const SweepGeom &S, int nv, double g, int mode, long t,
                                            const double *__restrict__ q, double *const *io, double *__restrict__ fI) {
-  const double *uL = io[0], *uR = io[1], *fL = io[2], *fR = io[3];
   const int nl = S.nlines, N = S.N;
   const int k = (int)(t % (N + 1)), l = (int)(t / (N + 1));
   const long pl = S.plane;
   const long cL = S.base + (long)l * S.line_stride + (k - 1), cR = cL + 1;
-  double a0, a1, a2;
-  euler1d_roeavg(g, q[cL], q[pl + cL], q[2 * pl + cL], q[cR], q[pl + cR], q[2 * pl + cR], a0, a1, a2);
   const long ii = (long)l * (N + 1) + k, vs = (long)nl * (N + 1), vstride = vs;
-  if (mode == 3) {
-    auto speed = [&](double rho, double mom, double e) {
-      const double uvel = mom / rho, P = (e - 0.5 * rho * uvel * uvel) * (g - 1.0);
-      return g * P / rho + fabs(uvel);
-    };
-    const double aL = speed(q[cL], q[pl + cL], q[2 * pl + cL]), aR = speed(q[cR], q[pl + cR], q[2 * pl + cR]);
-    const double aA = speed(a0, a1, a2);
-    const double m1 = aL > aR ? aL : aR, m2 = aR > aA ? aR : aA;  // max3, math_ops.h:30
-    const double alpha = m1 > m2 ? m1 : m2;
-    for (int m = 0; m < nv; m++) fI[m * vs + ii] = FS(m) - alpha * UD(m);
-    return;
-  }
-  Eig3 E;
-  euler1d_eig(g, a0, a1, a2, E);
-  if (mode == 0) {
-    double ud[3], DL[3][3];
-    for (int m = 0; m < 3; m++) ud[m] = UD(m);
-    for (int i = 0; i < 3; i++)
-      for (int j = 0; j < 3; j++) DL[i][j] = fabs(E.D[i]) * E.L[i][j];
-    for (int i = 0; i < 3; i++) {
-      double us = 0.0;
-      for (int j = 0; j < 3; j++) {
-        const double mA = E.R[i][0] * DL[0][j] + E.R[i][1] * DL[1][j] + E.R[i][2] * DL[2][j];
-        us += mA * ud[j];
-      }
-      fI[i * vs + ii] = FS(i) - us;
+  const double uLc[3] = {q[cL], q[pl + cL], q[2 * pl + cL]}, uRc[3] = {q[cR], q[pl + cR], q[2 * pl + cR]};
+  if (mode == 0 || mode == 3) {
+    double ud[3], fs[3], fo[3];
+    for (int m = 0; m < 3; m++) {
+      ud[m] = UD(m);
+      fs[m] = FS(m);
     }
-    const double Dsp = fabs(E.D[0]);
-    for (int m = 3; m < nv; m++) fI[m * vs + ii] = FS(m) - Dsp * UD(m);
+    const double c = mode == 3 ? rusanov_e1d(g, uLc, uRc) : roe_e1d(g, uLc, uRc, ud, fs, fo);
+    for (int m = 0; m < 3; m++) fI[m * vs + ii] = mode == 3 ? fs[m] - c * ud[m] : fo[m];
+    for (int m = 3; m < nv; m++) fI[m * vs + ii] = FS(m) - c * UD(m);
     return;
   }
-  // cell eigenvalues (euler1d.h:131-147) of the two neighbours
-  Eig3 EL, ER;
-  euler1d_eig(g, q[cL], q[pl + cL], q[2 * pl + cL], EL);
-  euler1d_eig(g, q[cR], q[pl + cR], q[2 * pl + cR], ER);
-  double fc[3];
+  const double *uL = io[0] + ii, *uR = io[1] + ii, *fL = io[2] + ii, *fR = io[3] + ii;
+  double a[4][3], fo[3], es[3];
   for (int m = 0; m < 3; m++) {
-    double ucL = 0, ucR = 0, fcL = 0, fcR = 0;
-    for (int j = 0; j < 3; j++) {
-      ucL += E.L[m][j] * uL[j * vs + ii];
-      ucR += E.L[m][j] * uR[j * vs + ii];
-      fcL += E.L[m][j] * fL[j * vs + ii];
-      fcR += E.L[m][j] * fR[j * vs + ii];
-    }
-    fc[m] = rf_pick(EL.D[m], E.D[m], ER.D[m], ucL, ucR, fcL, fcR, mode == 2);
+    a[0][m] = uL[m * vs];
+    a[1][m] = uR[m * vs];
+    a[2][m] = fL[m * vs];
+    a[3][m] = fR[m * vs];
   }
-  for (int i = 0; i < 3; i++) fI[i * vs + ii] = E.R[i][0] * fc[0] + E.R[i][1] * fc[1] + E.R[i][2] * fc[2];
-  // species rows: identity eigenvectors, eigenvalue v
-  const double eLs = EL.D[0], eCs = E.D[0], eRs = ER.D[0];
+  rf_e1d(g, mode == 2, uLc, uRc, a[0], a[1], a[2], a[3], fo, es);
+  for (int m = 0; m < 3; m++) fI[m * vs + ii] = fo[m];
   for (int m = 3; m < nv; m++)
-    fI[m * vs + ii] =
-        rf_pick(eLs, eCs, eRs, uL[m * vs + ii], uR[m * vs + ii], fL[m * vs + ii], fR[m * vs + ii], mode == 2);
+    fI[m * vs + ii] = rf_pick(es[0], es[1], es[2], uL[m * vs], uR[m * vs], fL[m * vs], fR[m * vs], mode == 2);
 }
 
-// NavierStokes2DUpwindRF (NavierStokes2DUpwind.c:106-187): L and R from the
-// Roe average of the two reconstructed interface states uL, uR (not of the
-// neighbouring cells); a field is upwinded by the signs of its eigenvalue at
-// uL, uR and the average.  Species fields have eigenvalue vn and identity
-// eigenvectors.  Split mode only: uL, uR, fL, fR in io[0..3].
+// Split mode only: uL, uR, fL, fR in io[0..3].
 template <int DIR, bool LLF>
 __device__ __forceinline__ void upwind_ns2d_rf(const SweepGeom &S, int nv, double g, long t, double *const *io,
                                                double *__restrict__ fI) {
@@ -2703,30 +2072,14 @@ __device__ __forceinline__ void upwind_ns2d_rf(const SweepGeom &S, int nv, doubl
   const double uRk[4] = {uR[0], uR[vs], uR[2 * vs], uR[3 * vs]};
   const double fLk[4] = {fL[0], fL[vs], fL[2 * vs], fL[3 * vs]};
   const double fRk[4] = {fR[0], fR[vs], fR[2 * vs], fR[3 * vs]};
-  double ua[4], L[4][4], R[4][4], eL[4], eC[4], eR[4];
-  ns2d_roeavg(g, uLk, uRk, ua);
-  ns2d_eigvecs<DIR>(g, ua, L, R);
-  ns2d_eigvals<DIR>(g, uLk, eL);
-  ns2d_eigvals<DIR>(g, uRk, eR);
-  ns2d_eigvals<DIR>(g, ua, eC);
-  double fc[4];
+  double fo[4], es[3];
+  rf_ns2d<DIR>(g, LLF, uLk, uRk, fLk, fRk, fo, es);
 #pragma unroll
-  for (int m = 0; m < 4; m++) {
-    // MatVecMult (matmult_native.h:119-130): row sums in index order
-    const double ucL = L[m][0] * uLk[0] + L[m][1] * uLk[1] + L[m][2] * uLk[2] + L[m][3] * uLk[3];
-    const double ucR = L[m][0] * uRk[0] + L[m][1] * uRk[1] + L[m][2] * uRk[2] + L[m][3] * uRk[3];
-    const double fcL = L[m][0] * fLk[0] + L[m][1] * fLk[1] + L[m][2] * fLk[2] + L[m][3] * fLk[3];
-    const double fcR = L[m][0] * fRk[0] + L[m][1] * fRk[1] + L[m][2] * fRk[2] + L[m][3] * fRk[3];
-    fc[m] = rf_pick(eL[m], eC[m], eR[m], ucL, ucR, fcL, fcR, LLF);
-  }
-#pragma unroll
-  for (int i = 0; i < 4; i++) fI[i * vs + ii] = R[i][0] * fc[0] + R[i][1] * fc[1] + R[i][2] * fc[2] + R[i][3] * fc[3];
+  for (int i = 0; i < 4; i++) fI[i * vs + ii] = fo[i];
   for (int m = 4; m < nv; m++)
-    fI[m * vs + ii] = rf_pick(eL[3], eC[3], eR[3], uL[m * vs], uR[m * vs], fL[m * vs], fR[m * vs], LLF);
+    fI[m * vs + ii] = rf_pick(es[0], es[1], es[2], uL[m * vs], uR[m * vs], fL[m * vs], fR[m * vs], LLF);
 }
 
-// NavierStokes2DUpwindRusanov (NavierStokes2DUpwind.c:271-332): the largest of
-// c + |v_n| at the two neighbouring cells and their Roe average.
 template <int DIR, int PAIR>
 __device__ __forceinline__ void upwind_ns2d_rusanov(const SweepGeom &S, int nv, double g, long t,
                                                     const double *__restrict__ q, double *const *io,
@@ -2737,16 +2090,7 @@ __device__ __forceinline__ void upwind_ns2d_rusanov(const SweepGeom &S, int nv, 
   const long cL = S.base + (long)l * S.line_stride + (k - 1), cR = cL + 1;
   const double uLc[4] = {q[cL], q[pl + cL], q[2 * pl + cL], q[3 * pl + cL]};
   const double uRc[4] = {q[cR], q[pl + cR], q[2 * pl + cR], q[3 * pl + cR]};
-  double ua[4];
-  ns2d_roeavg(g, uLc, uRc, ua);
-  auto speed = [&](const double u[4]) {
-    double rho, vx, vy, e, P;
-    ns2d_flowvar(u, g, rho, vx, vy, e, P);
-    return sqrt(g * P / rho) + fabs(DIR == 0 ? vx : vy);
-  };
-  const double aL = speed(uLc), aR = speed(uRc), aA = speed(ua);
-  const double m1 = aL > aR ? aL : aR, m2 = aR > aA ? aR : aA;  // max3, math_ops.h:30
-  const double alpha = m1 > m2 ? m1 : m2;
+  const double alpha = rusanov_ns2d<DIR>(g, uLc, uRc);
   const long ii = (long)l * (N + 1) + k, vstride = (long)nl * (N + 1);
   for (int m = 0; m < nv; m++) fI[m * vstride + ii] = FS(m) - alpha * UD(m);
 }
@@ -3540,8 +2884,8 @@ __global__ void __launch_bounds__(TB) k_dev_iface(int ndims, int dir, int nx, in
 
 static const char *kKNames[K_NCLASS] = {"stage_bc", "ghost",  "flux",    "recon_ends", "recon", "recon_full",
                                         "long_rows", "long_solve",
-                                        "recon_char", "cw_rows", "cw_solve", "upwind", "bflux",
-                                        "qderiv",   "viscflux", "assemble", "update"};
+                                        "cw_rows", "cw_solve", "weno", "upwind", "bflux",
+                                        "qderiv",   "viscflux", "assemble", "update", "flux_all"};
 const char *kclass_name(int k) { return kKNames[k]; }
 
 int cw_row_fields(int nflow, int nv) { return nflow * nflow + 16 * nv; }
@@ -3566,7 +2910,7 @@ bool stage_tile_64(const CaseDev &c) { return c.G.ndims == 2 && (long)c.G.nx * c
 #endif
 bool species_in_recon(const CaseDev &c) {
   const bool two = (c.G.ndims == 2);
-  return PIAFS_RECON_SPECIES && PIAFS_RECON_LDS && two && c.model == 2 && c.paired && c.upwind == 0 &&
+  return PIAFS_RECON_SPECIES && PIAFS_RECON_LDS && two && c.model == 2 && c.paired && c.R.crweno && c.upwind == 0 &&
          !c.R.characteristic && c.G.nv > 4 && c.dsp[0] && c.dsp[1] && c.Sx.team <= PIAFS_SP_TEAM_MAX &&
          c.Sy.team <= PIAFS_SP_TEAM_MAX && c.Sx.team >= PIAFS_SP_TEAM_MIN && c.Sy.team >= PIAFS_SP_TEAM_MIN &&
          long_rows(c.Sx, c.G.nv) == 0 && long_rows(c.Sy, c.G.nv) == 0;
@@ -3582,19 +2926,21 @@ void case_blocks(const CaseDev &c, int blocks[K_NCLASS]) {
   auto pad8 = [](int n) { return (n + 7) & ~7; };
   blocks[K_STAGE] = pad8(two ? ((G.nx + st - 1) / st) * ((G.ny + st - 1) / st) * G.nv : nb((long)G.nx * G.nv));
   blocks[K_GHOST] = nb(ghost_points(G) * G.nv);
-  blocks[K_FLUX] = nb((long)(c.Sx.N + 2 * c.Sx.g) * c.Sx.nlines + (two ? (long)(c.Sy.N + 2 * c.Sy.g) * c.Sy.nlines : 0));
+  auto faces = [&](long per) {  // blocks of `per` interfaces, the sweeps apart
+    const long x = (long)(c.Sx.N + 1) * c.Sx.nlines, y = two ? (long)(c.Sy.N + 1) * c.Sy.nlines : 0;
+    return (int)((x + per - 1) / per + (y + per - 1) / per);
+  };
+  const int nf = c.model == 1 ? 3 : 4;
+  const bool weno = !c.R.crweno && !c.unit;
+  blocks[K_FLUXALL] = nb((long)(c.Sx.N + 2 * c.Sx.g) * c.Sx.nlines + (two ? (long)(c.Sy.N + 2 * c.Sy.g) * c.Sy.nlines : 0));
+  blocks[K_FLUX] = weno ? 0 : blocks[K_FLUXALL];
+  blocks[K_WENO] = weno ? faces(kWenoTile) : 0;
   blocks[K_CWROWS] = blocks[K_CWSOLVE] = blocks[K_LROWS] = blocks[K_LSOLVE] = 0;
-  if (c.R.characteristic && c.R.crweno) {
-    const int nf = c.model == 1 ? 3 : 4;
-    blocks[K_ENDS] = blocks[K_RECON] = blocks[K_RECONF] = blocks[K_RCHAR] = 0;
+  blocks[K_ENDS] = blocks[K_RECON] = blocks[K_RECONF] = 0;
+  if (c.R.crweno && c.R.characteristic) {
     blocks[K_CWROWS] = nb((long)(c.Sx.N + 1) * c.Sx.nlines + (two ? (long)(c.Sy.N + 1) * c.Sy.nlines : 0));
     blocks[K_CWSOLVE] = nb(cw_x_span(c, nf) + (two ? cw_items(c.Sy, G.nv, nf) : 0));
-  } else if (c.R.characteristic) {
-    blocks[K_ENDS] = 0;
-    blocks[K_RECON] = blocks[K_RECONF] = 0;
-    blocks[K_RCHAR] = nb((long)(c.Sx.N + 1) * c.Sx.nlines + (two ? (long)(c.Sy.N + 1) * c.Sy.nlines : 0));
-  } else {
-    blocks[K_RCHAR] = 0;
+  } else if (c.R.crweno) {
     blocks[K_ENDS] = nb(2 * (recon_systems(c.Sx, G.nv, c.paired) + (two ? recon_systems(c.Sy, G.nv, c.paired) : 0)));
     const int nrec = recon_sweep_blocks(c.Sx, G.nv, c.paired) + (two ? recon_sweep_blocks(c.Sy, G.nv, c.paired) : 0);
     // full segments: both sweeps' lanes hold kMaxRows rows each
@@ -3605,7 +2951,7 @@ void case_blocks(const CaseDev &c, int blocks[K_NCLASS]) {
     blocks[K_LROWS] = nb(long_rows(c.Sx, G.nv) + (two ? long_rows(c.Sy, G.nv) : 0));
     blocks[K_LSOLVE] = (int)(long_pairs(c.Sx, G.nv) + (two ? long_pairs(c.Sy, G.nv) : 0));  // a block per pair
   }
-  blocks[K_UPWIND] = nb((long)(c.Sx.N + 1) * c.Sx.nlines + (two ? (long)(c.Sy.N + 1) * c.Sy.nlines : 0));
+  blocks[K_UPWIND] = weno ? 0 : nb((long)(c.Sx.N + 1) * c.Sx.nlines + (two ? (long)(c.Sy.N + 1) * c.Sy.nlines : 0));
   blocks[K_BFLUX] = c.cons ? 1 : 0;
   const bool visc = two && c.P.viscous;
   blocks[K_QDERIV] = visc ? nb((long)G.nxg * G.nyg) : 0;
@@ -3613,8 +2959,6 @@ void case_blocks(const CaseDev &c, int blocks[K_NCLASS]) {
   blocks[K_ASSEMBLE] = pad8(two ? ((G.nx + 31) / 32) * ((G.ny + 31) / 32) * G.nv : nb((long)G.nx * G.nv));
   blocks[K_UPDATE] = nb((long)G.nx * G.ny * G.nv);
 }
-
-typedef void (*KernFn)(const CaseDev *, const int *, const int *, int);
 
 static void run(KernFn k, int cls, const CaseDev *d, const Plan &pl, int s, hipStream_t st, MarkFn mark,
                 void *ctx) {
@@ -3630,11 +2974,11 @@ static void run(KernFn k, int cls, const CaseDev *d, const Plan &pl, int s, hipS
 void launch_stage(const CaseDev *d, const Plan &pl, int s, hipStream_t st, MarkFn mark, void *ctx,
                   const StageFork *fk, int last) {
   auto R = [&](KernFn k, int cls, hipStream_t on) {
-    if (cls <= last) run(k, cls, d, pl, s, on, mark, ctx);
+    if (cls <= last || cls == K_FLUXALL) run(k, cls, d, pl, s, on, mark, ctx);
   };
   R(pl.stage64 ? k_stage64 : k_stage, K_STAGE, st);
   R(k_ghost, K_GHOST, st);
-  R(k_flux, K_FLUX, st);
+  R(k_flux, last == K_FLUX ? K_FLUXALL : K_FLUX, st);
   R(k_recon_ends, K_ENDS, st);
   const bool fork = fk && fk->side && last >= K_ASSEMBLE &&
                     (pl.nblocks[K_QDERIV] > 0 || pl.nblocks[K_VISCFLUX] > 0);
@@ -3649,9 +2993,9 @@ void launch_stage(const CaseDev *d, const Plan &pl, int s, hipStream_t st, MarkF
   R(k_recon_full, K_RECONF, st);
   R(k_lrows, K_LROWS, st);
   R(k_lsolve, K_LSOLVE, st);
-  R(k_recon_char, K_RCHAR, st);
   R(k_cw_rows, K_CWROWS, st);
   R(k_cw_solve, K_CWSOLVE, st);
+  R(weno_kernel(), K_WENO, st);
   R(k_upwind, K_UPWIND, st);
   R(k_bflux, K_BFLUX, st);
   if (fork) {
@@ -3736,9 +3080,8 @@ void launch_dev_iface(int ndims, int dir, int nx, int N, int nl, int nv, const d
 
 void launch_class(const CaseDev *d, const Plan &pl, int cls, int s, hipStream_t st) {
   static const KernFn table[K_NCLASS] = {k_stage, k_ghost, k_flux, k_recon_ends, k_recon, k_recon_full, k_lrows,
-                                         k_lsolve, k_recon_char,
-                                         k_cw_rows, k_cw_solve, k_upwind, k_bflux, k_qderiv, k_viscflux,
-                                         k_assemble, k_update};
+                                         k_lsolve, k_cw_rows, k_cw_solve, weno_kernel(),
+                                         k_upwind, k_bflux, k_qderiv, k_viscflux, k_assemble, k_update, k_flux};
   run(cls == K_STAGE && pl.stage64 ? k_stage64 : table[cls], cls, d, pl, s, st, nullptr, nullptr);
 }
 

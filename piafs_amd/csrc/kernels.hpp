@@ -145,6 +145,7 @@ struct CaseDev {
   int fuse_sp;   // species interface fluxes written by the reconstruction (set by the plan; see species_in_recon)
   double *dsp[2];  // per sweep and interface: Roe-average |v_n| with the entropy fix (k_flux, when fuse_sp)
   int stage_tile; // side of k_stage's transpose tiles, 32 or 64 (set by the plan)
+  int unit;      // descriptor of the device-buffer operators: the interface flux in separate passes
   int terms;     // terms k_assemble adds: bit 0 hyperbolic, bit 1 parabolic, bit 2 source (7 in a step)
   double dt, A[16], b[4], c[4];
   double *u, *U, *UT, *Udot[4];
@@ -170,10 +171,12 @@ struct CaseDev {
   int *status;   // bit 0: a zero pivot met in a line solve (tridiagLU.c:139-142 returns -1)
 };
 
-// Kernel classes launched per RK stage (plus the final update).
+// Kernel classes launched per RK stage (plus the final update).  K_FLUXALL is
+// K_FLUX for every case, those of K_WENO (which form their own fluxes) among
+// them, and runs only when the fluxes themselves are asked for.
 enum KClass {
-  K_STAGE = 0, K_GHOST, K_FLUX, K_ENDS, K_RECON, K_RECONF, K_LROWS, K_LSOLVE, K_RCHAR, K_CWROWS, K_CWSOLVE, K_UPWIND,
-  K_BFLUX, K_QDERIV, K_VISCFLUX, K_ASSEMBLE, K_UPDATE,
+  K_STAGE = 0, K_GHOST, K_FLUX, K_ENDS, K_RECON, K_RECONF, K_LROWS, K_LSOLVE, K_CWROWS, K_CWSOLVE, K_WENO, K_UPWIND,
+  K_BFLUX, K_QDERIV, K_VISCFLUX, K_ASSEMBLE, K_UPDATE, K_FLUXALL,
   K_NCLASS
 };
 const char *kclass_name(int k);
@@ -186,6 +189,10 @@ struct Plan {
   int *blockcase[K_NCLASS] = {nullptr};   // device arrays, one int per block
   int *firstblock[K_NCLASS] = {nullptr};  // device arrays, one int per case
 };
+
+typedef void (*KernFn)(const CaseDev *, const int *, const int *, int);
+KernFn weno_kernel();        // k_weno (weno.hip)
+constexpr int kWenoTile = 64;  // interfaces of a block
 
 // Host side: blocks each case needs for each kernel class (0 = class unused).
 void case_blocks(const CaseDev &c, int blocks[K_NCLASS]);
@@ -242,6 +249,10 @@ void launch_dev_fd(const AosGrid &A, int dir, int par4, int bias, const double *
 void launch_dev_weights(const AosGrid &A, int model, double gamma, int dir, int kind, int crweno,
                         int characteristic, int no_limiting, double eps, const double *fC, const double *u,
                         double *w1, double *w2, double *w3, long size, hipStream_t s);
+// interface values of the schemes without line systems, straight between the
+// reference-layout arrays (weno.hip)
+void launch_dev_weno(const AosGrid &A, int model, double gamma, const ReconParams &R, int dir, bool left,
+                     const double *a, const double *u, double *fI, hipStream_t s);
 // ghosted reference-layout array <-> planar natural / transposed copies
 void launch_dev_planar(const Grid &G, const double *a, double *nat, double *tr, int to_planar, int ghosts_only,
                        double *out, hipStream_t s);

@@ -90,7 +90,7 @@ size_t Case::plan_bytes(const Config &c) {
     n += (size_t)(cw_row_fields(nf, (int)nv) + 4 * cw_back_fields(nf, (int)nv)) * (ix + iy) / nv;
   }
   if (c.model_id == MODEL_NS2D) n += 12 * (size_t)g.nxg * g.nyg;
-  if (!c.characteristic) {  // long-line scratch of sweeps longer than one team
+  if (c.crweno && !c.characteristic) {  // long-line scratch of sweeps longer than one team
     int T, m;
     for (int d = 0; d < c.ndims; d++)
       if (!team_shape(c.dim[d], kMaxRows, T, m))
@@ -300,7 +300,7 @@ int Case::setup(int dev, hipStream_t st) {
 
 int Case::set_team_rows(int max_rows) {
   CaseDev &D = h;
-  if (cfg.characteristic) {  // characteristic WENO5 runs one thread per interface: no line teams
+  if (cfg.characteristic || !cfg.crweno) {  // no line teams
     D.Sx.team = D.Sy.team = 1;
     D.Sx.rows = D.Sy.rows = 1;
     return 0;
@@ -534,30 +534,29 @@ int Engine::step(int n) {
   return 0;
 }
 
-// Device time (ms) per stage of the kernel classes `cls` and `cls2` (-1:
-// none) -- the sum of their average launch times -- over `reps` evaluations
+// Device time (ms) per stage of the kernel classes `cls` -- the sum of their average launch times -- over `reps` evaluations
 // of stage 0 of every member.  A stage leaves the solution and the time alone
 // (it writes the stage state, the interface arrays and Udot[0] only).
-double Engine::time_class(int cls, int reps, int cls2) {
+double Engine::time_classes(const std::vector<int> &cls, int reps) {
   if (!built || cases.empty()) return 0.0;
   const bool was = profiling;
   profiling = true;
   ev_used = 0;
   for (int r = 0; r < reps; r++) launch_stage(d_cases, plan, 0, stream, mark_cb, this);
   hipStreamSynchronize(stream);
-  double tot[2] = {0.0, 0.0};
-  int cnt[2] = {0, 0};
+  double tot[K_NCLASS] = {0.0}, sum = 0.0;
+  int cnt[K_NCLASS] = {0};
   for (size_t k = 0; k < ev_used; k++) {
-    const int which = ev_cls[k] == cls ? 0 : (ev_cls[k] == cls2 ? 1 : -1);
-    if (which < 0) continue;
     float m = 0.f;
     hipEventElapsedTime(&m, ev[k].first, ev[k].second);
-    tot[which] += m;
-    cnt[which]++;
+    tot[ev_cls[k]] += m;
+    cnt[ev_cls[k]]++;
   }
   ev_used = 0;
   profiling = was;
-  return (cnt[0] ? tot[0] / cnt[0] : 0.0) + (cnt[1] ? tot[1] / cnt[1] : 0.0);
+  for (int c : cls)
+    if (cnt[c]) sum += tot[c] / cnt[c];
+  return sum;
 }
 
 // Segment length of the line solves (rows per lane, which sets each case's
@@ -566,6 +565,7 @@ double Engine::time_class(int cls, int reps, int cls2) {
 int Engine::autotune(const int *cands, int ncand, int reps, int *best_rows, double *best_ms) {
   HIPCHK(hipSetDevice(device));
   if (cases.empty()) return 0;
+  const std::vector<int> recon = {K_RECON, K_RECONF, K_WENO};
   int best = -1;
   double bms = 0.0;
   for (int k = 0; k < ncand; k++) {
@@ -574,8 +574,8 @@ int Engine::autotune(const int *cands, int ncand, int reps, int *best_rows, doub
     if (!ok) continue;
     int rc = build();
     if (rc) return rc;
-    time_class(K_RECON, 1, K_RECONF);  // warm
-    const double ms = time_class(K_RECON, reps, K_RECONF);
+    time_classes(recon, 1);  // warm
+    const double ms = time_classes(recon, reps);
     if (best < 0 || ms < bms) {
       best = cands[k];
       bms = ms;
