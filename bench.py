@@ -56,7 +56,7 @@ def kernel_algorithmic_bytes(name, nx, ny, nv, g, nstages, crweno, paired=True):
     sweeps = 2
     nio = 2 if paired else 4
     fused = species_fused(nx, ny, nv, paired)
-    if name in ("recon", "recon_full"):  # u and f at every position of every line; the interface arrays
+    if name.startswith("recon_") and name != "recon_ends":  # u and f at every position of every line; the interface arrays
         if fused:  # flow: the two combinations; species: their flux, from |v_n| (one value per interface)
             return sweeps * 8 * (2 * nv * pos * lines + (2 * 4 + (nv - 4) + 1) * (N + 1) * lines)
         return sweeps * 8 * (2 * nv * pos * lines + nio * nv * (N + 1) * lines)

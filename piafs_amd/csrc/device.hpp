@@ -25,11 +25,7 @@ namespace {
 // interpolated value is still NaN as the reference's is, and a tiny weight's
 // term lies far below the last bit of a sum led by the large weights.
 // ---------------------------------------------------------------------------
-#ifndef PIAFS_FAST_WDIV
-#define PIAFS_FAST_WDIV 1
-#endif
 __device__ __forceinline__ double wdiv(double n, double d) {
-#if PIAFS_FAST_WDIV
   const double r0 = __builtin_amdgcn_rcp(d);
   const double e0 = __builtin_fma(-d, r0, 1.0);
   const double r1 = __builtin_fma(r0, e0, r0);
@@ -38,34 +34,19 @@ __device__ __forceinline__ double wdiv(double n, double d) {
   const double q = n * r2;
   const double t = __builtin_fma(-d, q, n);
   return __builtin_fma(t, r2, q);
-#else
-  return n / d;
-#endif
 }
 
 // ---------------------------------------------------------------------------
 // WENO5 nonlinear weights, include/interpolation.h:255-490
 // (JS :255-281, mapped :309-341, Z (Borges) :420-450, YC :478-508)
 // ---------------------------------------------------------------------------
+// from the smoothness indicators b1..b3; t: YC's fourth difference
 template <int KIND>
-__device__ __forceinline__ void weno_w(double c1, double c2, double c3, double m3, double m2, double m1,
-                                       double p1, double p2, double eps, double &w1, double &w2, double &w3) {
-  const double t1312 = 13.0 / 12.0, q14 = 1.0 / 4.0;
-  const double d1 = m3 - 2 * m2 + m1, e1 = m3 - 4 * m2 + 3 * m1;
-  const double d2 = m2 - 2 * m1 + p1, e2 = m2 - p1;
-  const double d3 = m1 - 2 * p1 + p2, e3 = 3 * m1 - 4 * p1 + p2;
-  const double b1 = t1312 * d1 * d1 + q14 * e1 * e1;
-  const double b2 = t1312 * d2 * d2 + q14 * e2 * e2;
-  const double b3 = t1312 * d3 * d3 + q14 * e3 * e3;
+__device__ __forceinline__ void weno_of(double c1, double c2, double c3, double b1, double b2, double b3, double t,
+                                        double eps, double &w1, double &w2, double &w3) {
   double a1, a2, a3;
   if (KIND == 2 || KIND == 3) {
-    double tau;
-    if (KIND == 2) {
-      tau = fabs(b3 - b1);
-    } else {
-      const double t = m3 - 4 * m2 + 6 * m1 - 4 * p1 + p2;
-      tau = t * t;
-    }
+    const double tau = KIND == 2 ? fabs(b3 - b1) : t * t;
     const double r1 = wdiv(tau, b1 + eps), r2 = wdiv(tau, b2 + eps), r3 = wdiv(tau, b3 + eps);
     a1 = c1 * (1.0 + r1 * r1);
     a2 = c2 * (1.0 + r2 * r2);
@@ -88,6 +69,20 @@ __device__ __forceinline__ void weno_w(double c1, double c2, double c3, double m
     w2 = a2 * s;
     w3 = a3 * s;
   }
+}
+
+template <int KIND>
+__device__ __forceinline__ void weno_w(double c1, double c2, double c3, double m3, double m2, double m1,
+                                       double p1, double p2, double eps, double &w1, double &w2, double &w3) {
+  const double t1312 = 13.0 / 12.0, q14 = 1.0 / 4.0;
+  const double d1 = m3 - 2 * m2 + m1, e1 = m3 - 4 * m2 + 3 * m1;
+  const double d2 = m2 - 2 * m1 + p1, e2 = m2 - p1;
+  const double d3 = m1 - 2 * p1 + p2, e3 = 3 * m1 - 4 * p1 + p2;
+  const double b1 = t1312 * d1 * d1 + q14 * e1 * e1;
+  const double b2 = t1312 * d2 * d2 + q14 * e2 * e2;
+  const double b3 = t1312 * d3 * d3 + q14 * e3 * e3;
+  const double t = KIND == 3 ? m3 - 4 * m2 + 6 * m1 - 4 * p1 + p2 : 0.0;
+  weno_of<KIND>(c1, c2, c3, b1, b2, b3, t, eps, w1, w2, w3);
 }
 
 __device__ __forceinline__ void weno_w_rt(int kind, double c1, double c2, double c3, double m3, double m2,

@@ -139,17 +139,24 @@ int piafs_dev_interp_interfaces(piafs_case *pc, double *fI, const double *fC, co
   UnitOps &un = *pc->unit;
   const CaseDev &d = un.desc;
   const Grid &G = c->h.G;
-  // the solution systems read the stage state, the flux systems the flux
-  // buffers; the systems of the other biases and of the other sweep are
-  // solved too, on the state's own flux, and discarded
-  stage_state(pc, uflag ? fC : u_ghosted, st);
-  launch_class(un.eng.d_cases, un.eng.plan, K_FLUX, 0, st);
-  if (!uflag)
-    launch_dev_planar(G, fC, dir ? nullptr : d.flux_x, dir ? d.flux_y : nullptr, 1, 0, nullptr, st);
-  for (int cls : {K_ENDS, K_RECON, K_RECONF, K_LROWS, K_LSOLVE, K_CWROWS, K_CWSOLVE})
-    launch_class(un.eng.d_cases, un.eng.plan, cls, 0, st);
   const int r = (uflag ? 0 : 2) + (upw > 0 ? 0 : 1);
   const SweepGeom &S = dir ? d.Sy : d.Sx;
+  if (!d.R.characteristic && !S.longl) {
+    // component-wise systems read one array, the state's or the flux's, along
+    // one sweep; only the systems of this bias are solved
+    double *nat = dir ? nullptr : (uflag ? d.U : d.flux_x), *tr = dir ? (uflag ? d.UT : d.flux_y) : nullptr;
+    launch_dev_planar(G, fC, nat, tr, 1, 0, nullptr, st);
+    launch_recon_only(un.eng.d_cases, un.eng.plan, d, dir, r, st);
+  } else {
+    // the solution systems read the stage state, the flux systems the flux
+    // buffers; the systems of the other biases and of the other sweep are
+    // solved too, on the state's own flux, and discarded
+    stage_state(pc, uflag ? fC : u_ghosted, st);
+    launch_class(un.eng.d_cases, un.eng.plan, K_FLUX, 0, st);
+    if (!uflag)
+      launch_dev_planar(G, fC, dir ? nullptr : d.flux_x, dir ? d.flux_y : nullptr, 1, 0, nullptr, st);
+    for (int cls = K_ENDS; cls <= K_CWSOLVE; cls++) launch_class(un.eng.d_cases, un.eng.plan, cls, 0, st);
+  }
   launch_dev_iface(G.ndims, dir, G.nx, S.N, S.nlines, G.nv, dir ? d.iy[r] : d.ix[r], fI, 0, st);
   return launched(pc);
 }

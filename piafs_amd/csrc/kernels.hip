@@ -6,6 +6,7 @@
 // and the library is compiled without floating-point contraction so that the
 // rounding of every +, -, *, / and sqrt matches the reference build.
 #include "device.hpp"
+#include "teams.hpp"
 
 #include <cstdio>
 #include <type_traits>
@@ -272,774 +273,39 @@ __global__ void __launch_bounds__(256) k_flux(CASE_ARGS) {
   }
 }
 
-// ---------------------------------------------------------------------------
-// Tridiagonal line systems solved by teams of lanes, with the reference's
-// arithmetic.
-//
-// A team of T lanes (a power of two; teams of more than 64 lanes span whole
-// waves of one block) owns one system, and each lane keeps a segment of at
-// most kMaxRows consecutive rows in registers.  The result is the one of the
-// sequential Thomas sweep of tridiagLU.c:133-150 (fac = a_k/b'_{k-1},
-// b'_k = b_k - fac c_{k-1}, x'_k = x_k - fac x'_{k-1}) and :243-255
-// (x_k = (x'_k - c_k x_{k+1}) / b'_k), bit for bit:
-//  1. each segment gets an estimate of the state entering it -- the pivot
-//     b' from a scan of the segments' Moebius maps b'_{k-1} -> b'_k (2x2
-//     matrices), x' from a scan of their affine maps;
-//  2. every lane runs the sweep over its rows from its entry state, and each
-//     lane's entry becomes the state its predecessor ended with; this repeats
-//     until no entry changes.  Lane 0 starts from the exact state, so the
-//     fixed point is reached after at most T passes and is exactly the
-//     sequential sweep; with the estimates (and the sweep's contraction) the
-//     ends are usually exact after the first pass, so two passes are typical;
-//  3. the back substitution is treated the same way from the top.
-// The systems are never written to memory; only the solution is.
-// ---------------------------------------------------------------------------
-struct Mob {
-  double a, b, c, d;  // [[a, b], [c, d]]
-};
-struct Aff {
-  double a, b;  // x -> a*x + b
-};
-
-// Rescale by a power of two (exact) so that products of many segment maps
-// neither overflow nor underflow; a Moebius map is unchanged by scaling.
-__device__ __forceinline__ Mob mob_norm(Mob r) {
-  const double mx = fmax(fmax(fabs(r.a), fabs(r.b)), fmax(fabs(r.c), fabs(r.d)));
-  if (mx > 0.0 && mx < INFINITY) {
-    const int e = ilogb(mx);
-    r.a = ldexp(r.a, -e);
-    r.b = ldexp(r.b, -e);
-    r.c = ldexp(r.c, -e);
-    r.d = ldexp(r.d, -e);
-  }
-  return r;
-}
-__device__ __forceinline__ Mob mob_mul(const Mob &x, const Mob &y) {
-  Mob r;
-  r.a = x.a * y.a + x.b * y.c;
-  r.b = x.a * y.b + x.b * y.d;
-  r.c = x.c * y.a + x.d * y.c;
-  r.d = x.c * y.b + x.d * y.d;
-  return mob_norm(r);
-}
-// outer o inner
-__device__ __forceinline__ Aff aff_cmp(const Aff &o, const Aff &i) { return Aff{o.a * i.a, o.a * i.b + o.b}; }
-
-// Lane moves of a double by DPP (a VALU operand modifier, no LDS round trip):
-// lanes without a source (or outside ROWMASK) keep their own value.  CTRL:
-// row_shr:d 0x110+d and row_shl:d 0x100+d move within rows of 16 lanes,
-// wave_shr:1 0x138 and wave_shl:1 0x130 across the wave, row_bcast:15 0x142
-// and row_bcast:31 0x143 broadcast a row's last lane to the following rows.
-template <int CTRL, int ROWMASK = 0xF>
-__device__ __forceinline__ double dpp_move(double v) {
-  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-  const int l0 = (int)(unsigned)b, h0 = (int)(unsigned)(b >> 32);
-  const int lo = __builtin_amdgcn_update_dpp(l0, l0, CTRL, ROWMASK, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(h0, h0, CTRL, ROWMASK, 0xF, false);
-  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
-}
-template <int CTRL, int ROWMASK = 0xF>
-__device__ __forceinline__ Mob dpp_mob(const Mob &x) {
-  return Mob{dpp_move<CTRL, ROWMASK>(x.a), dpp_move<CTRL, ROWMASK>(x.b), dpp_move<CTRL, ROWMASK>(x.c),
-             dpp_move<CTRL, ROWMASK>(x.d)};
-}
-template <int CTRL, int ROWMASK = 0xF>
-__device__ __forceinline__ Aff dpp_aff(const Aff &x) {
-  return Aff{dpp_move<CTRL, ROWMASK>(x.a), dpp_move<CTRL, ROWMASK>(x.b)};
-}
-// value of lane i-1 (UP) or i+1 of the wave
-template <bool UP>
-__device__ __forceinline__ double lane_step(double v) {
-  return UP ? dpp_move<0x138>(v) : dpp_move<0x130>(v);
-}
-
-// Exclusive scans over the lanes of a team.  `lane` is the lane within the
-// team; `red` is LDS for one Mob per wave of the block.
-__device__ Mob team_scan_mob(Mob x, int lane, int T, double *red) {
-  const int W = T < 64 ? T : 64;
-  const int wl = lane & (W - 1);
-#if PIAFS_SCAN_DPP
-  // within rows of 16 lanes (a team of fewer lanes lies inside one row), then
-  // across the rows of the wave from each row's last lane
-  const int rl = wl & 15;
-  if (W > 1) { const Mob o = dpp_mob<0x111>(x); if (rl >= 1) x = mob_mul(x, o); }
-  if (W > 2) { const Mob o = dpp_mob<0x112>(x); if (rl >= 2) x = mob_mul(x, o); }
-  if (W > 4) { const Mob o = dpp_mob<0x114>(x); if (rl >= 4) x = mob_mul(x, o); }
-  if (W > 8) { const Mob o = dpp_mob<0x118>(x); if (rl >= 8) x = mob_mul(x, o); }
-  if (W > 16) { const Mob o = dpp_mob<0x142, 0xA>(x); if (wl & 16) x = mob_mul(x, o); }
-  if (W > 32) { const Mob o = dpp_mob<0x143, 0xC>(x); if (wl & 32) x = mob_mul(x, o); }
-#else
-  for (int d = 1; d < W; d <<= 1) {
-    Mob o;
-    o.a = __shfl_up(x.a, d, W);
-    o.b = __shfl_up(x.b, d, W);
-    o.c = __shfl_up(x.c, d, W);
-    o.d = __shfl_up(x.d, d, W);
-    if (wl >= d) x = mob_mul(x, o);
-  }
-#endif
-  Mob pre = {1.0, 0.0, 0.0, 1.0};
-  if (T > 64) {
-    const int w = lane >> 6, wave = threadIdx.x >> 6;
-    if (wl == 63) {
-      double *s = red + 4 * wave;
-      s[0] = x.a; s[1] = x.b; s[2] = x.c; s[3] = x.d;
-    }
-    __syncthreads();
-    for (int k = 0; k < w; k++) {
-      const double *s = red + 4 * (wave - w + k);
-      pre = mob_mul(Mob{s[0], s[1], s[2], s[3]}, pre);
-    }
-    __syncthreads();
-  }
-  Mob e;
-#if PIAFS_SCAN_DPP
-  e = Mob{lane_step<true>(x.a), lane_step<true>(x.b), lane_step<true>(x.c), lane_step<true>(x.d)};
-#else
-  e.a = __shfl_up(x.a, 1, W);
-  e.b = __shfl_up(x.b, 1, W);
-  e.c = __shfl_up(x.c, 1, W);
-  e.d = __shfl_up(x.d, 1, W);
-#endif
-  if (wl == 0) e = pre;
-  else if (T > 64) e = mob_mul(e, pre);
-  return e;
-}
-
-__device__ Aff team_scan_aff_fwd(Aff x, int lane, int T, double *red) {
-  const int W = T < 64 ? T : 64;
-  const int wl = lane & (W - 1);
-#if PIAFS_SCAN_DPP
-  const int rl = wl & 15;
-  if (W > 1) { const Aff o = dpp_aff<0x111>(x); if (rl >= 1) x = aff_cmp(x, o); }
-  if (W > 2) { const Aff o = dpp_aff<0x112>(x); if (rl >= 2) x = aff_cmp(x, o); }
-  if (W > 4) { const Aff o = dpp_aff<0x114>(x); if (rl >= 4) x = aff_cmp(x, o); }
-  if (W > 8) { const Aff o = dpp_aff<0x118>(x); if (rl >= 8) x = aff_cmp(x, o); }
-  if (W > 16) { const Aff o = dpp_aff<0x142, 0xA>(x); if (wl & 16) x = aff_cmp(x, o); }
-  if (W > 32) { const Aff o = dpp_aff<0x143, 0xC>(x); if (wl & 32) x = aff_cmp(x, o); }
-#else
-  for (int d = 1; d < W; d <<= 1) {
-    const Aff o = {__shfl_up(x.a, d, W), __shfl_up(x.b, d, W)};
-    if (wl >= d) x = aff_cmp(x, o);
-  }
-#endif
-  Aff pre = {1.0, 0.0};
-  if (T > 64) {
-    const int w = lane >> 6, wave = threadIdx.x >> 6;
-    if (wl == 63) {
-      red[2 * wave] = x.a;
-      red[2 * wave + 1] = x.b;
-    }
-    __syncthreads();
-    for (int k = 0; k < w; k++) pre = aff_cmp(Aff{red[2 * (wave - w + k)], red[2 * (wave - w + k) + 1]}, pre);
-    __syncthreads();
-  }
-#if PIAFS_SCAN_DPP
-  Aff e = {lane_step<true>(x.a), lane_step<true>(x.b)};
-#else
-  Aff e = {__shfl_up(x.a, 1, W), __shfl_up(x.b, 1, W)};
-#endif
-  if (wl == 0) e = pre;
-  else if (T > 64) e = aff_cmp(e, pre);
-  return e;
-}
-
-__device__ Aff team_scan_aff_bwd(Aff x, int lane, int T, double *red) {
-  const int W = T < 64 ? T : 64;
-  const int wl = lane & (W - 1);
-#if PIAFS_SCAN_DPP
-  // within rows of 16 lanes, then from the first lane of the following rows
-  // (no DPP broadcast runs backwards: two LDS permutes)
-  const int rl = wl & 15, rw = W < 16 ? W : 16;
-  if (W > 1) { const Aff o = dpp_aff<0x101>(x); if (rl + 1 < rw) x = aff_cmp(x, o); }
-  if (W > 2) { const Aff o = dpp_aff<0x102>(x); if (rl + 2 < rw) x = aff_cmp(x, o); }
-  if (W > 4) { const Aff o = dpp_aff<0x104>(x); if (rl + 4 < rw) x = aff_cmp(x, o); }
-  if (W > 8) { const Aff o = dpp_aff<0x108>(x); if (rl + 8 < rw) x = aff_cmp(x, o); }
-  if (W > 16) {
-    const int src = ((int)(threadIdx.x & 63) | 15) + 1;  // first lane of the next row
-    const Aff o = {__shfl(x.a, src & 63, 64), __shfl(x.b, src & 63, 64)};
-    if (!(wl & 16)) x = aff_cmp(x, o);
-  }
-  if (W > 32) {
-    const Aff o = {__shfl(x.a, 32, 64), __shfl(x.b, 32, 64)};
-    if (!(wl & 32)) x = aff_cmp(x, o);
-  }
-#else
-  for (int d = 1; d < W; d <<= 1) {
-    const Aff o = {__shfl_down(x.a, d, W), __shfl_down(x.b, d, W)};
-    if (wl + d < W) x = aff_cmp(x, o);
-  }
-#endif
-  Aff suf = {1.0, 0.0};
-  if (T > 64) {
-    const int w = lane >> 6, nw = T >> 6, wave = threadIdx.x >> 6;
-    if (wl == 0) {
-      red[2 * wave] = x.a;
-      red[2 * wave + 1] = x.b;
-    }
-    __syncthreads();
-    for (int k = nw - 1; k > w; k--) suf = aff_cmp(Aff{red[2 * (wave - w + k)], red[2 * (wave - w + k) + 1]}, suf);
-    __syncthreads();
-  }
-#if PIAFS_SCAN_DPP
-  Aff e = {lane_step<false>(x.a), lane_step<false>(x.b)};
-#else
-  Aff e = {__shfl_down(x.a, 1, W), __shfl_down(x.b, 1, W)};
-#endif
-  if (wl == W - 1) e = suf;
-  else if (T > 64) e = aff_cmp(e, suf);
-  return e;
-}
-
-// (a, b) of the previous lane of the team (dir = +1) or of the next one
-// (dir = -1); the first (last) lane of the team keeps its own values.
-__device__ __forceinline__ void team_shift2(double &a, double &b, int lane, int T, int dir, double *red) {
-  const int W = T < 64 ? T : 64;
-  const int wl = lane & (W - 1);
-  double pa, pb;
-#if PIAFS_SCAN_DPP
-  // across team boundaries too: a team's first (last) lane receives another
-  // team's value, which it does not use
-  if (dir > 0) {
-    pa = lane_step<true>(a);
-    pb = lane_step<true>(b);
-  } else {
-    pa = lane_step<false>(a);
-    pb = lane_step<false>(b);
-  }
-#else
-  if (dir > 0) {
-    pa = __shfl_up(a, 1, W);
-    pb = __shfl_up(b, 1, W);
-  } else {
-    pa = __shfl_down(a, 1, W);
-    pb = __shfl_down(b, 1, W);
-  }
-#endif
-  if (T > 64) {
-    const int wave = threadIdx.x >> 6;
-    const bool edge_out = dir > 0 ? (wl == 63) : (wl == 0);
-    if (edge_out) {
-      red[2 * wave] = a;
-      red[2 * wave + 1] = b;
-    }
-    __syncthreads();
-    const bool edge_in = dir > 0 ? (wl == 0 && lane != 0) : (wl == 63 && lane != T - 1);
-    if (edge_in) {
-      pa = red[2 * (wave - dir)];
-      pb = red[2 * (wave - dir) + 1];
-    }
-    __syncthreads();
-  }
-  a = pa;
-  b = pb;
-}
-
-// true on every lane of the wave (T <= 64) or block (T > 64) when `p` holds
-// on any of them
-__device__ __forceinline__ bool team_any(bool p, int T) {
-  if (T > 64) return __syncthreads_or(p) != 0;
-  return __any(p) != 0;
-}
-
-// v_rcp_f64 refined by two Newton steps: a reciprocal good to the last bits,
-// used only for the estimates that start the exact passes
-__device__ __forceinline__ double rcp_est(double b) {
-  double r = __builtin_amdgcn_rcp(b);
-  r = fma(r, fma(-b, r, 1.0), r);
-  r = fma(r, fma(-b, r, 1.0), r);
-  return r;
-}
-
-// Forward elimination of team_solve: on exit B holds b' and X holds x' of
-// every row, Fk the multipliers.  The row before the team's first row has
-// pivot bfirst, super-diagonal cfirst and x' xfirst (an identity row: 1, 0,
-// its value).  zp is set when a pivot is zero.  QD: the system is a CRWENO5
-// coefficient system (a_k >= +0, true pivots positive and of order one), whose
-// multipliers a_k / b'_{k-1} divide with wdiv; the relay ends on the true
-// pivots, where wdiv gives the IEEE quotient's bits within its envelope (the
-// weights in a_k not tiny).
-template <int MR, bool FULL = false, bool QD = false>
-__device__ __forceinline__ void team_forward(double (&A)[MR], double (&B)[MR], double (&Cc)[MR], double (&X)[MR],
-                                             double (&Fk)[MR], int n, int lane, int T, double bfirst, double cfirst,
-                                             double xfirst, double *red, bool plain_start, bool &zp) {
-  const bool has = FULL || n > 0;
-  double cin = 0.0, unused = 0.0;
-#pragma unroll
-  for (int i = 0; i < MR; i++)
-    if (FULL ? i == MR - 1 : i == n - 1) cin = Cc[i];
-  team_shift2(cin, unused, lane, T, +1, red);
-  if (lane == 0) cin = cfirst;
-  // pivot entering the segment: scan of M_k = [[b_k, -a_k c_{k-1}], [1, 0]] on (b'_{k-1}, 1)
-  Mob P = {1.0, 0.0, 0.0, 1.0};
-#pragma unroll
-  for (int i = 0; i < MR; i++) {
-    if (FULL || i < n) {
-      const double ac = A[i] * (i == 0 ? cin : Cc[i > 0 ? i - 1 : 0]);
-      const Mob R = {B[i] * P.a - ac * P.c, B[i] * P.b - ac * P.d, P.a, P.b};
-      P = R;
-    }
-  }
-  P = mob_norm(P);
-  const Mob E = team_scan_mob(P, lane, T, red);
-  double bin = lane == 0 ? bfirst : (plain_start ? 1.0 : (E.a + E.b) / (E.c + E.d));
-  // multipliers along the estimated pivots; affine maps of x'
-  double bend = bin;
-  Aff F = {lane == 0 ? 0.0 : 1.0, lane == 0 ? xfirst : 0.0};
-  {
-    double c = cin;
-#pragma unroll
-    for (int i = 0; i < MR; i++) {
-      if (FULL || i < n) {
-        const double fac = QD ? wdiv(A[i], bend) : A[i] / bend;
-        bend = B[i] - fac * c;
-        c = Cc[i];
-        Fk[i] = fac;
-        F = Aff{-(fac * F.a), X[i] - fac * F.b};
-      } else {
-        Fk[i] = 0.0;
-      }
-    }
-  }
-  const Aff Ef = team_scan_aff_fwd(F, lane, T, red);
-  double xin = lane == 0 ? xfirst : (plain_start ? 0.0 : Ef.a * xfirst + Ef.b);
-  // relay of segment ends until every entry equals its predecessor's end
-  for (int it = 0;; it++) {
-    double xend = xin;
-#pragma unroll
-    for (int i = 0; i < MR; i++)
-      if (FULL || i < n) xend = X[i] - Fk[i] * xend;
-    double nb = bend;
-    team_shift2(nb, xend, lane, T, +1, red);
-    const bool bchg = lane != 0 && !(nb == bin);
-    const bool changed = has && lane != 0 && (bchg || !(xend == xin));
-    if (lane != 0) {
-      bin = nb;
-      xin = xend;
-    }
-    if (!team_any(changed, T) || it > T) break;
-    if (bchg) {  // pivots of this segment derived again from the new entry, until they repeat
-      const double bend_old = bend;
-      double c = cin, bb = bin;
-      bool live = true;
-#pragma unroll
-      for (int i = 0; i < MR; i++) {
-        if ((FULL || i < n) && live) {
-          const double fac = QD ? wdiv(A[i], bb) : A[i] / bb;
-          if (__double_as_longlong(fac) == __double_as_longlong(Fk[i])) {
-            live = false;  // same multiplier, so the same pivot here and in every later row
-          } else {
-            bb = B[i] - fac * c;
-            c = Cc[i];
-            Fk[i] = fac;
-          }
-        }
-      }
-      bend = live ? bb : bend_old;
-    }
-  }
-  // b' and x' of every row, in the reference's arithmetic
-  zp = zp || ((bin == 0.0) && has);
-  {
-    double b = bin, x = xin, c = cin;
-#pragma unroll
-    for (int i = 0; i < MR; i++) {
-      if (FULL || i < n) {
-        b = B[i] - Fk[i] * c;
-        x = X[i] - Fk[i] * x;
-        c = Cc[i];
-        zp = zp || (b == 0.0);
-        B[i] = b;
-        X[i] = x;
-      }
-    }
-  }
-}
-
-// Back substitution of team_solve: B holds b', X holds x' of every row; on
-// exit X holds the solution.  The row after the team's last row (held by the
-// lane with is_last) has solution xlast.  W is scratch.
-template <int MR, bool FULL = false>
-__device__ __forceinline__ void team_backward(double (&B)[MR], double (&Cc)[MR], double (&X)[MR], double (&W)[MR],
-                                              int n, int lane, int T, bool is_last, double xlast, double *red,
-                                              bool plain_start) {
-  const bool has = FULL || n > 0;
-  // estimate of x entering from above, then the relay
-  Aff Gm = {is_last ? 0.0 : 1.0, is_last ? xlast : 0.0};
-#pragma unroll
-  for (int i = MR - 1; i >= 0; i--) {
-    if (FULL || i < n) {
-      const double rb = rcp_est(B[i]);
-      Gm = Aff{-(Cc[i] * rb) * Gm.a, (X[i] - Cc[i] * Gm.b) * rb};
-    }
-  }
-  const Aff Eb = team_scan_aff_bwd(Gm, lane, T, red);
-  double yin = is_last ? xlast : (plain_start ? 0.0 : Eb.a * xlast + Eb.b);
-  for (int it = 0;; it++) {
-    double xv = yin, dummy = 0.0;
-    bool live = true;
-#pragma unroll
-    for (int i = MR - 1; i >= 0; i--) {
-      if ((FULL || i < n) && live) {
-        const double nx = (X[i] - Cc[i] * xv) / B[i];
-        // from the second pass on: a row that repeats its value leaves every row above unchanged
-        if (it > 0 && __double_as_longlong(nx) == __double_as_longlong(W[i])) live = false;
-        W[i] = nx;
-        xv = nx;
-      }
-    }
-    if (FULL || n > 0) xv = W[0];
-    team_shift2(xv, dummy, lane, T, -1, red);
-    const bool changed = has && !is_last && !(xv == yin);
-    if (!is_last) yin = xv;
-    if (!team_any(changed, T) || it > T) break;
-  }
-#pragma unroll
-  for (int i = 0; i < MR; i++)
-    if (FULL || i < n) X[i] = W[i];
-}
-
-// Solve one team's system.  On entry the n rows of this lane hold
-// (A, B, Cc, X) = (sub-, main, super-diagonal, right-hand side); on exit X
-// holds the solution and B the pivots.  The row before the team's first row
-// is an identity row carrying xfirst; the row after the team's last row (held
-// by the lane with is_last) is one carrying xlast.  Every lane of every team
-// of the block must call this (it may synchronise the block).
-// The multipliers of the
-// pivot chain (fac = a_k / b'_{k-1}, one division each) are kept per row, so
-// the x' chain of a pass costs no division: every pass takes the segments'
-// entry states, runs the x' chain along the kept multipliers, and relays the
-// segment ends; only when an entry pivot changes are the multipliers derived
-// again.  Once no entry changes, one pass without divisions writes b' and x'
-// (fac * c and fac * x' exactly as the reference computes them).  The back
-// substitution iterates the same way from the top.  If `plain_start` is set
-// the scanned estimates are replaced by the trivial ones (b' = 1, x' = 0), so
-// that the relay runs through many passes (testing).  FULL: every lane holds
-// MR rows (n is not read), rows past the system's end being identity rows.
-template <int MR, bool FULL = false, bool QD = false>
-__device__ __forceinline__ void team_solve(double (&A)[MR], double (&B)[MR], double (&Cc)[MR], double (&X)[MR],
-                                                int n, int lane, int T, bool is_last, double xfirst, double xlast,
-                                                double *red, int *status, bool plain_start) {
-  double Fk[MR];
-  bool zp = false;
-  team_forward<MR, FULL, QD>(A, B, Cc, X, Fk, n, lane, T, 1.0, 0.0, xfirst, red, plain_start, zp);
-  team_backward<MR, FULL>(B, Cc, X, Fk, n, lane, T, is_last, xlast, red, plain_start);
-  if (zp) atomicOr(status, 1);
-}
-
-// ---------------------------------------------------------------------------
-// Component-wise CRWENO5 reconstruction.  One system per (line,
-// variable, reconstruction r): r = 0 uL, 1 uR (of the state), 2 fL, 3 fR (of
-// the flux); r even = left-biased.  A team of lanes covers the interfaces of
-// one system: lane j computes rows 1 + j*m .. of the interior rows 1..N-1,
-// lane 0 also interface 0 and the lane holding row N-1 also interface N.
-//  * weights: WENOFifthOrderCalculateWeights{JS,M,Z,YC}
-//    (WENOFifthOrderCalculateWeights.c:112-237 and the variants);
-//    optimal weights :202-220 (WENO5 values at the two end interfaces of a
-//    CRWENO line).
-//  * CRWENO5: row assembly Interp1PrimFifthOrderCRWENO.c:132-201 (identity
-//    rows with WENO5 right-hand sides at interfaces 0 and N), then the line
-//    solve (team_solve above).
-// ---------------------------------------------------------------------------
-// Systems of a sweep: split mode, one per (line, var, r); paired mode, one
-// team per (line, var, pair) solving the left- and right-biased systems of
-// the pair in turn (pair 0: uL, uR; pair 1: fL, fR) and writing the two
-// combinations the Roe upwinding uses, 0.5*(uR - uL) and 0.5*(fL + fR)
-// (NavierStokes2DUpwind.c:58-60, Euler1DUpwind.c:45-52).
-__host__ __device__ inline long recon_systems(const SweepGeom &S, int nv, int paired) {
-  return S.longl ? 0 : (long)S.nlines * nv * (paired ? 2 : 4);
-}
-
+// The two end interfaces (0 and N) of the line systems, a thread per pair of
+// systems and end: WENO5 values on identity rows
+// (Interp1PrimFifthOrderCRWENO.c:132-201 with the WENO5 weights at the ends).
+// The raw values go to the case's `ends` table for the line solves, and, in
+// paired mode their combination, to the interface arrays.
 template <int KIND>
-__device__ __forceinline__ void recon_team(const CaseDev &C, int dir, long sys, bool active, int lane, double *red,
-                                           double *stash) {
-  const SweepGeom &S = dir ? C.Sy : C.Sx;
-  const int nv = C.G.nv, N = S.N, nl = S.nlines, m = S.rows, g = S.g;
-  const bool paired = C.paired != 0;
-  const long sy = active ? sys : 0;
-  const int per = paired ? 2 : 4;
-  const int q = (int)(sy % per), v = (int)((sy / per) % nv), l = (int)((sy / per) / nv);
-  const int r0 = paired ? 2 * q : q;
-  const double *src = ((r0 < 2) ? (dir ? C.UT : C.U) : (dir ? C.flux_y : C.flux_x)) + (long)v * S.plane + S.base +
-                      (long)l * S.line_stride;
-  double *const *io = dir ? C.iy : C.ix;
-  const long line = ((long)v * nl + l) * (N + 1);
-  const int lo = 1 + lane * m;
-  int n = N - lo;
-  n = n < 0 ? 0 : (n > m ? m : n);
-  if (!active) n = 0;
-  const int lastlane = (N - 2) / m;
-  const int hi_pos = N + g - 1;
-  const double *ends = C.ends + 4 * ((dir ? recon_systems(C.Sx, nv, 1) : 0) + sy);
-  double X[kMaxRows];
-  // solve the system of reconstruction r into X
-  auto solve = [&](int r, int side) {
-    const bool left = !(r & 1);
-    // the end interfaces 0 and N (identity rows carrying WENO5 values, from k_recon_ends)
-    double x0 = 0.0, xN = 0.0;
-    if (active && lane == 0) x0 = paired ? ends[2 * side] : io[r][line];
-    if (active && lane == lastlane) xN = paired ? ends[2 * side + 1] : io[r][line + N];
-    // stencil window: positions lo-3 .. lo+n+1
-    double win[kMaxRows + 5];
-#pragma unroll
-    for (int j = 0; j < kMaxRows + 5; j++) {
-      const int pos = lo - 3 + j;
-      win[j] = (n > 0 && j < n + 5 && pos <= hi_pos) ? src[pos] : 0.0;
-    }
-    double A[kMaxRows], B[kMaxRows], Cc[kMaxRows];
-#pragma unroll
-    for (int i = 0; i < kMaxRows; i++) {
-      if (i < n) {
-        row_coeffs<KIND>(lo + i, N, left, C.R, win[i], win[i + 1], win[i + 2], win[i + 3], win[i + 4],
-                             win[i + 5], A[i], B[i], Cc[i], X[i]);
-      } else {
-        A[i] = 0.0; B[i] = 1.0; Cc[i] = 0.0; X[i] = 0.0;
-      }
-    }
-    team_solve<kMaxRows, false, PIAFS_FAST_WDIV>(A, B, Cc, X, n, lane, S.team, lane == lastlane, x0, xN, red, C.status,
-                           C.R.plain_start != 0);
-  };
-  solve(r0, 0);
-  if (paired) {
-#pragma unroll
-    for (int i = 0; i < kMaxRows; i++) stash[i * 256 + threadIdx.x] = X[i];  // this lane's own rows
-    solve(r0 + 1, 1);
-  }
-  if (!paired) {
-#pragma unroll
-    for (int i = 0; i < kMaxRows; i++)
-      if (i < n) io[r0][line + lo + i] = X[i];
-  } else {
-    double *out = io[q] + line;  // io[0]: 0.5*(uR - uL), io[1]: 0.5*(fL + fR)
-#pragma unroll
-    for (int i = 0; i < kMaxRows; i++) {
-      if (i < n) {
-        const double xl = stash[i * 256 + threadIdx.x];
-        out[lo + i] = q ? 0.5 * (xl + X[i]) : 0.5 * (X[i] - xl);
-      }
-    }
-  }
-}
-
-// Paired mode with the team's line staged in LDS.  The two systems of a pair
-// read the same line (the state for pair 0, the flux for pair 1), so the team
-// loads it once, with consecutive lanes reading consecutive positions, into a
-// region of its own; each lane then reads its stencil window from there for
-// both systems.  The combinations are written back through the same region so
-// that the global stores are consecutive too.  The bias of each system is a
-// compile-time constant.  Arithmetic and results are those of recon_team.
-// Region layout: line position p (-2 .. T*m+2) at lds_slot(p + 2), one unused
-// slot after every 16 so that lanes reading 16 apart hit different banks.
-__device__ __forceinline__ int lds_slot(int i) { return i + (i >> 4); }
-__host__ __device__ inline int line_region(int T, int m) {
-  const int n = T * m + 5;
-  return n + (n >> 4) + 1;
-}
-// LDS doubles of the staged lines of one 256-thread block: the largest
-// (256 / T) * line_region(T, m) over teams T = 1 .. 256 and m <= 16 (T = 1),
-// plus the overrun of the last lane's window when its segment is short
-constexpr int kLineLds = 256 * (16 + 5 + 2) + 32;
-
-// all lanes of the team have finished their LDS accesses before any lane goes on
-__device__ __forceinline__ void team_lds_sync(int T) {
-  if (T > 64) {
-    __syncthreads();
-  } else {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  }
-}
-
-template <int KIND, bool FULL>
-__device__ __forceinline__ void recon_pair_lds(const CaseDev &C, int dir, long sys, bool active, int lane,
-                                               double *red, double *stash, double *lines) {
-  const SweepGeom &S = dir ? C.Sy : C.Sx;
-  const int nv = C.G.nv, N = S.N, nl = S.nlines, m = S.rows, g = S.g, T = S.team;
-  const long sy = active ? sys : 0;
-  const int q = (int)(sy % 2), v = (int)((sy / 2) % nv), l = (int)((sy / 2) / nv);
-  const double *src = (q == 0 ? (dir ? C.UT : C.U) : (dir ? C.flux_y : C.flux_x)) + (long)v * S.plane + S.base +
-                      (long)l * S.line_stride;
-  const long line = ((long)v * nl + l) * (N + 1);
-  const int lo = 1 + lane * m;
-  int n = N - lo;
-  n = n < 0 ? 0 : (n > m ? m : n);
-  if (!active) n = 0;
-  const int lastlane = (N - 2) / m;
-  const int hi_pos = N + g - 1;
-  const double *ends = C.ends + 4 * ((dir ? recon_systems(C.Sx, nv, 1) : 0) + sy);
-  double *L = lines + (threadIdx.x / T) * line_region(T, m);
-  // species pairs whose two teams are different waves (T = 64) meet through
-  // an arrival counter per pair, cleared before any wave can reach it
-  __shared__ unsigned pair_arrived[2];
-  if (C.fuse_sp && T == 64) {
-    if (threadIdx.x < 2) pair_arrived[threadIdx.x] = 0u;
-    __syncthreads();
-  }
-  // the line, positions -2 .. T*m+2 (zero past its last ghost)
-  const int tot = T * m + 5;
-  for (int b = 0; b < tot; b += T) {
-    const int idx = b + lane;
-    if (idx < tot) {
-      const int pos = idx - 2;
-      L[lds_slot(idx)] = (active && pos <= hi_pos) ? src[pos] : 0.0;
-    }
-  }
-  team_lds_sync(T);
-  double X[kMaxRows];
-  // FULL (every lane holds kMaxRows rows): the rows past row N-1 are identity
-  // rows, the first of them -- interface N -- carrying xN, so that no row
-  // needs a bound check; the identity row at interface N lies in the team
-  // unless T*kMaxRows == N-1, when it follows the team as in the general case
-  const int nlane = (N - 1) / kMaxRows;  // the lane holding row N in FULL mode
-  auto solve = [&](auto left_c, int side) {
-    constexpr bool LEFT = decltype(left_c)::value;
-    const int xn_lane = FULL ? (nlane < T ? nlane : T - 1) : lastlane;
-    // rows assembled: all kMaxRows in FULL mode (m == kMaxRows there; the
-    // row bound stays a run-time value, which keeps the row assembly in
-    // order and the register count at two waves per SIMD)
-    const int nrow = FULL ? m : n;
-    double x0 = 0.0, xN = 0.0;
-    if (active && lane == 0) x0 = ends[2 * side];
-    if (active && lane == xn_lane) xN = ends[2 * side + 1];
-    // stencil window: positions lo-3 .. lo+n+1
-    double win[kMaxRows + 5];
-#pragma unroll
-    for (int j = 0; j < kMaxRows + 5; j++) win[j] = (j < nrow + 5) ? L[lds_slot(lo - 1 + j)] : 0.0;
-    double A[kMaxRows], B[kMaxRows], Cc[kMaxRows];
-#pragma unroll
-    for (int i = 0; i < kMaxRows; i++) {
-      if (i < nrow) {
-        row_coeffs<KIND>(lo + i, N, LEFT, C.R, win[i], win[i + 1], win[i + 2], win[i + 3], win[i + 4],
-                             win[i + 5], A[i], B[i], Cc[i], X[i]);
-      } else {
-        A[i] = 0.0; B[i] = 1.0; Cc[i] = 0.0; X[i] = 0.0;
-      }
-    }
-    if (FULL && lo + kMaxRows > N) {
-#pragma unroll
-      for (int i = 0; i < kMaxRows; i++) {
-        if (lo + i >= N) {
-          A[i] = 0.0; B[i] = 1.0; Cc[i] = 0.0;
-          X[i] = (lo + i == N) ? xN : 0.0;
-        }
-      }
-    }
-    if (FULL)
-      team_solve<kMaxRows, true, PIAFS_FAST_WDIV>(A, B, Cc, X, kMaxRows, lane, T, lane == T - 1, x0, nlane < T ? 0.0 : xN, red,
-                                 C.status, C.R.plain_start != 0);
-    else
-      team_solve<kMaxRows, false, PIAFS_FAST_WDIV>(A, B, Cc, X, n, lane, T, lane == lastlane, x0, xN, red, C.status,
-                           C.R.plain_start != 0);
-  };
-  solve(std::integral_constant<bool, true>(), 0);
-#pragma unroll
-  for (int i = 0; i < kMaxRows; i++) stash[i * 256 + threadIdx.x] = X[i];  // this lane's own rows
-  solve(std::integral_constant<bool, false>(), 1);
-  // a species of a case whose reconstruction writes the species fluxes: the
-  // |v_n| of this lane's interfaces, loaded now so that the combination step
-  // below hides their latency (the line's N + 1 <= T kMaxRows + 2 interfaces
-  // take at most kMaxRows + 2 per lane)
-  constexpr int KO = kMaxRows + 2;
-  const bool fsp = C.fuse_sp && v >= 4;
-  double dvv[KO];
-#pragma unroll
-  for (int it = 0; it < KO; it++) dvv[it] = 0.0;
-  if (fsp && (T == 64 || q == 1)) {  // a team of at most 32 lanes writes when it is the flux team
-    const double *dv = C.dsp[dir] + (long)l * (N + 1);
-#pragma unroll
-    for (int it = 0; it < KO; it++) {
-      const int k = it * T + lane;
-      if (active && k <= N) dvv[it] = dv[k];
-    }
-  }
-  team_lds_sync(T);  // every window of the team is read
-#pragma unroll
-  for (int i = 0; i < kMaxRows; i++) {
-    if (i < n) {
-      const double xl = stash[i * 256 + threadIdx.x];
-      L[lds_slot(lo + i)] = q ? 0.5 * (xl + X[i]) : 0.5 * (X[i] - xl);
-    }
-  }
-  team_lds_sync(T);
-  if (fsp) {
-    // A species: its Roe flux f_I = 0.5 (fL + fR) - |v_n| 0.5 (uR - uL), the
-    // upwinder's arithmetic, is written here from the combinations of the
-    // pair's two teams (u and f sources of one line and species), which sit
-    // side by side in the block.  A team of at most 32 lanes shares its wave
-    // with its partner, so the wave's own LDS sync has made both visible and
-    // the flux team writes.  Teams of 64 lanes are two waves: each publishes
-    // its combination with a release increment of the pair's counter, and the
-    // one that arrives second (acquire) writes, so neither waits.  The two end
-    // interfaces take the combinations k_recon_ends wrote.
-    bool writer = q == 1;
-    if (T == 64) {
-      unsigned prev = 0u;
-      if (lane == 0)
-        prev = __hip_atomic_fetch_add(&pair_arrived[(threadIdx.x >> 6) >> 1], 1u, __ATOMIC_ACQ_REL,
-                                      __HIP_MEMORY_SCOPE_WORKGROUP);
-      writer = __shfl(prev, 0, 64) == 1u;
-    }
-    if (writer && active) {
-      const double *Lp = lines + ((threadIdx.x / T) ^ 1) * line_region(T, m);
-      const double *Lf = q ? L : Lp, *Lu = q ? Lp : L;
-      double *const *io = dir ? C.iy : C.ix;
-      double *fo = (dir ? C.fIy : C.fIx) + line;
-#pragma unroll
-      for (int it = 0; it < KO; it++) {
-        const int k = it * T + lane;
-        if (k <= N) {
-          const bool end = k == 0 || k == N;
-          const double fs = end ? io[1][line + k] : Lf[lds_slot(k)];
-          const double ud = end ? io[0][line + k] : Lu[lds_slot(k)];
-          fo[k] = fs - dvv[it] * ud;
-        }
-      }
-    }
-    return;
-  }
-  double *out = (dir ? C.iy : C.ix)[q] + line;  // [0]: 0.5*(uR - uL), [1]: 0.5*(fL + fR)
-  for (int b = 1; b < N; b += T) {
-    const int k = b + lane;
-    if (active && k < N) out[k] = L[lds_slot(k)];
-  }
-}
-
-// The two end interfaces (0 and N) of every line system, one thread each:
-// WENO5 values on identity rows (Interp1PrimFifthOrderCRWENO.c:132-201 with
-// the WENO5 weights at the ends; plain WENO5 for the non-compact scheme).  In
-// paired mode a thread does both systems of its pair: the raw values go to
-// the case's `ends` table for the line solves, the combination to the output.
-template <int KIND>
-__device__ __forceinline__ double end_value(const CaseDev &C, const SweepGeom &S, const double *src, int r, int k) {
+__device__ __forceinline__ double end_value(const CaseDev &C, const SweepGeom &S, const double *src, bool left, int k) {
   double a_, b_, c_, x_;
-  row_coeffs<KIND>(k, S.N, !(r & 1), C.R, src[k - 3], src[k - 2], src[k - 1], src[k], src[k + 1], src[k + 2],
-                       a_, b_, c_, x_);
+  row_coeffs<KIND>(k, S.N, left, C.R, src[k - 3], src[k - 2], src[k - 1], src[k], src[k + 1], src[k + 2], a_, b_, c_,
+                   x_);
   return x_;
 }
 
 template <int KIND>
-__device__ __forceinline__ void recon_end(const CaseDev &C, int dir, long sys, int e) {
+__device__ __forceinline__ void recon_end(const CaseDev &C, int dir, long pair, int e) {
   const SweepGeom &S = dir ? C.Sy : C.Sx;
   const int nv = C.G.nv, N = S.N, nl = S.nlines;
-  const bool paired = C.paired != 0;
-  const int per = paired ? 2 : 4;
-  const int q = (int)(sys % per), v = (int)((sys / per) % nv), l = (int)((sys / per) / nv);
-  const int r0 = paired ? 2 * q : q;
-  const double *src = ((r0 < 2) ? (dir ? C.UT : C.U) : (dir ? C.flux_y : C.flux_x)) + (long)v * S.plane + S.base +
+  const int q = (int)(pair % 2), v = (int)((pair / 2) % nv), l = (int)((pair / 2) / nv);
+  const double *src = (q == 0 ? (dir ? C.UT : C.U) : (dir ? C.flux_y : C.flux_x)) + (long)v * S.plane + S.base +
                       (long)l * S.line_stride;
   const int k = e ? N : 0;
   double *const *io = dir ? C.iy : C.ix;
   const long at = ((long)v * nl + l) * (N + 1) + k;
-  if (!paired) {
-    io[r0][at] = end_value<KIND>(C, S, src, r0, k);
-    return;
-  }
-  const double xl = end_value<KIND>(C, S, src, r0, k), xr = end_value<KIND>(C, S, src, r0 + 1, k);
-  double *ends = C.ends + 4 * ((dir ? recon_systems(C.Sx, nv, 1) : 0) + sys);
+  const double xl = end_value<KIND>(C, S, src, true, k), xr = end_value<KIND>(C, S, src, false, k);
+  double *ends = C.ends + 4 * ((dir ? recon_pairs(C.Sx, nv) : 0) + pair);
   ends[e] = xl;
   ends[2 + e] = xr;
-  io[q][at] = q ? 0.5 * (xl + xr) : 0.5 * (xr - xl);
+  if (C.paired) {
+    io[q][at] = q ? 0.5 * (xl + xr) : 0.5 * (xr - xl);
+  } else {
+    io[2 * q][at] = xl;
+    io[2 * q + 1][at] = xr;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1745,14 +1011,6 @@ __global__ void __launch_bounds__(256, PIAFS_CWSOLVE_MINB) k_cw_solve(CASE_ARGS)
   cwc_species(C, S, dir, l, sys, chain, nf, seg, segs);
 }
 
-// Blocks of a sweep for the team-based reconstruction (each block holds
-// 256/team whole teams; a block never mixes sweeps).
-__host__ __device__ inline int recon_sweep_blocks(const SweepGeom &S, int nv, int paired) {
-  const long teams_per_block = 256 / S.team;
-  const long nsys = recon_systems(S, nv, paired);
-  return (int)((nsys + teams_per_block - 1) / teams_per_block);
-}
-
 // ---------------------------------------------------------------------------
 // Component-wise reconstruction of lines longer than one team covers
 // (SweepGeom::longl).  k_lrows assembles every row of every system, end rows
@@ -1933,61 +1191,23 @@ __global__ void __launch_bounds__(kLongTeam) k_lsolve(CASE_ARGS) {
 
 __global__ void __launch_bounds__(256) k_recon_ends(CASE_ARGS) {
   CASE_PREAMBLE
-  if (stage >= C.nstages) return;
-  const long nsx = recon_systems(C.Sx, C.G.nv, C.paired);
-  const long nsy = (C.G.ndims == 2) ? recon_systems(C.Sy, C.G.nv, C.paired) : 0;
-  if (t >= 2 * (nsx + nsy)) return;
-  const int dir = t < 2 * nsx ? 0 : 1;
-  const long q = dir ? t - 2 * nsx : t;
-  const long sys = q >> 1;
+  if ((stage & 0xFF) >= C.nstages) return;
+  const int nv = C.G.nv;
+  const long npx = recon_pairs(C.Sx, nv), npy = C.G.ndims == 2 ? recon_pairs(C.Sy, nv) : 0;
+  if (t >= 2 * (npx + npy)) return;
+  const int dir = t < 2 * npx ? 0 : 1;
+  const long q = dir ? t - 2 * npx : t;
+  const long pair = q >> 1;
   const int e = (int)(q & 1);
+  const int only = stage >> 8;
+  if (only && (dir != ((only >> 3) & 1) || (pair & 1) != ((only >> 2) & 1))) return;
   switch (C.R.kind) {
-    case 1: recon_end<1>(C, dir, sys, e); break;
-    case 2: recon_end<2>(C, dir, sys, e); break;
-    case 3: recon_end<3>(C, dir, sys, e); break;
-    default: recon_end<0>(C, dir, sys, e); break;
+    case 1: recon_end<1>(C, dir, pair, e); break;
+    case 2: recon_end<2>(C, dir, pair, e); break;
+    case 3: recon_end<3>(C, dir, pair, e); break;
+    default: recon_end<0>(C, dir, pair, e); break;
   }
 }
-
-// FULL: the kernel of class K_RECONF, for paired cases whose lanes all hold
-// kMaxRows rows (recon_pair_lds<..., true>); the other cases run in K_RECON.
-template <bool FULL>
-__device__ __forceinline__ void recon_body(CASE_ARGS) {
-  CASE_PREAMBLE
-  if (stage >= C.nstages) return;
-  __shared__ double red[16];
-  __shared__ double stash[kMaxRows * 256];
-  const int bid = (int)(blockIdx.x - firstblock[cidx]);
-  const int nbx = recon_sweep_blocks(C.Sx, C.G.nv, C.paired);
-  const int dir = bid < nbx ? 0 : 1;
-  const int lb = dir ? bid - nbx : bid;
-  const SweepGeom &S = dir ? C.Sy : C.Sx;
-  const int T = S.team;
-  const int lane = threadIdx.x & (T - 1);
-  const long sys = (long)lb * (256 / T) + threadIdx.x / T;
-  const bool active = sys < recon_systems(S, C.G.nv, C.paired);
-#if PIAFS_RECON_LDS
-  if (FULL || C.paired) {
-    __shared__ double lines[kLineLds];
-    switch (C.R.kind) {
-      case 1: recon_pair_lds<1, FULL>(C, dir, sys, active, lane, red, stash, lines); break;
-      case 2: recon_pair_lds<2, FULL>(C, dir, sys, active, lane, red, stash, lines); break;
-      case 3: recon_pair_lds<3, FULL>(C, dir, sys, active, lane, red, stash, lines); break;
-      default: recon_pair_lds<0, FULL>(C, dir, sys, active, lane, red, stash, lines); break;
-    }
-    return;
-  }
-#endif
-  if (FULL) return;  // not reached: K_RECONF holds paired cases only
-  switch (C.R.kind) {
-    case 1: recon_team<1>(C, dir, sys, active, lane, red, stash); break;
-    case 2: recon_team<2>(C, dir, sys, active, lane, red, stash); break;
-    case 3: recon_team<3>(C, dir, sys, active, lane, red, stash); break;
-    default: recon_team<0>(C, dir, sys, active, lane, red, stash); break;
-  }
-}
-__global__ void __launch_bounds__(256) k_recon(CASE_ARGS) { recon_body<false>(cases, blockcase, firstblock, stage); }
-__global__ void __launch_bounds__(256, PIAFS_RECONF_MINB) k_recon_full(CASE_ARGS) { recon_body<true>(cases, blockcase, firstblock, stage); }
 
 // ---------------------------------------------------------------------------
 // Upwinding.
@@ -2882,8 +2102,9 @@ __global__ void __launch_bounds__(TB) k_dev_iface(int ndims, int dir, int nx, in
 // host side: work decomposition and launchers
 // ===========================================================================
 
-static const char *kKNames[K_NCLASS] = {"stage_bc", "ghost",  "flux",    "recon_ends", "recon", "recon_full",
-                                        "long_rows", "long_solve",
+static const char *kKNames[K_NCLASS] = {"stage_bc", "ghost",  "flux",    "recon_ends",
+                                        "recon_4",  "recon_6", "recon_8", "recon_10", "recon_12", "recon_14", "recon_16",
+                                        "recon_w10", "recon_w12", "recon_w16", "long_rows", "long_solve",
                                         "cw_rows", "cw_solve", "weno", "upwind", "bflux",
                                         "qderiv",   "viscflux", "assemble", "update", "flux_all"};
 const char *kclass_name(int k) { return kKNames[k]; }
@@ -2900,20 +2121,84 @@ bool team_shape(int N, int max_rows, int &team, int &rows) {
   return team <= 256;
 }
 
+bool line_shape(int N, int rows, int &team) {
+  team = 1;
+  while ((long)team * rows < N - 1) team <<= 1;
+  if (team > 256) return false;
+  for (const ReconVariant &v : kRecon)
+    if (v.rows == rows && v.wide == (team > 64)) return true;
+  return false;
+}
+
+// A launch of a variant costs its latency once and its lanes' rows; the choice
+// minimises the sum over the variants used, of all sets of variants.  Both terms
+// are fitted to launches of nv 11 grids of side N (us; rows 4 6 8 10 12 14 16):
+//   N  33: 14.4 16.7 17.2 19.1 21.0 22.2 23.9     N 257: 65.3 78.6 57.5 74.9 83.1 93.8 68.6
+//   N 129: 28.8 32.7 25.7 27.9 31.1 33.7 36.4     N 385:   -   114  142  178  122  138  149
+//   N 193: 51.8 42.7 48.7 57.5 46.9 51.9 53.5     N 513:   -    -   186  239  271  299  202
+// (teams are powers of two, so a row count serves some lengths better than
+// others; short segments have more waves to hide their chains, long ones less
+// overhead per row).  Rows 16 only, the choice before, is the last column.
+void choose_rows(const std::vector<SweepGeom *> &sweeps, const std::vector<int> &nvars) {
+  static const double per_row[kNRecon] = {1.25, 1.10, 1.00, 1.06, 1.11, 1.10, 1.06, 1.44, 1.28, 1.13};
+  auto latency = [](int v) { return 10.0 + 0.75 * kRecon[v].rows; };
+  const int ns = (int)sweeps.size();
+  for (int wide = 0; wide < 2; wide++) {  // lines of up to 64 * kMaxRows rows take narrow teams
+    const int v0 = wide ? 7 : 0, n = wide ? kNRecon - 7 : 7;
+    std::vector<int> idx;
+    for (int s = 0; s < ns; s++)
+      if ((sweeps[s]->N - 1 > 64 * kMaxRows) == (wide == 1)) idx.push_back(s);
+    if (idx.empty()) continue;
+    std::vector<double> work(idx.size() * n);
+    std::vector<int> team(idx.size() * n);
+    for (size_t k = 0; k < idx.size(); k++)
+      for (int v = 0; v < n; v++) {
+        const SweepGeom &S = *sweeps[idx[k]];
+        const int rows = kRecon[v0 + v].rows;
+        int T;
+        const bool fits = line_shape(S.N, rows, T) && (T > 64) == kRecon[v0 + v].wide;
+        team[k * n + v] = fits ? T : 0;
+        work[k * n + v] = fits ? 1.57e-5 * per_row[v0 + v] * T * rows * (2.0 * S.nlines * nvars[idx[k]]) : 1e30;
+      }
+    auto total = [&](int set, std::vector<int> *pick) {
+      double sum = 0.0;
+      int used = 0;
+      for (size_t k = 0; k < idx.size(); k++) {
+        int best = -1;
+        for (int v = 0; v < n; v++)
+          if ((set >> v & 1) && (best < 0 || work[k * n + v] < work[k * n + best])) best = v;
+        sum += work[k * n + best];
+        used |= 1 << best;
+        if (pick) (*pick)[k] = best;
+      }
+      for (int v = 0; v < n; v++)
+        if (used >> v & 1) sum += latency(v0 + v);
+      return sum;
+    };
+    int set = 1 << (n - 1);  // the longest segments fit every line
+    double best = total(set, nullptr);
+    for (int c = 1; c < 1 << n; c++) {
+      const double t = total(c, nullptr);
+      if (t < best) {
+        best = t;
+        set = c;
+      }
+    }
+    std::vector<int> pick(idx.size());
+    total(set, &pick);
+    for (size_t k = 0; k < idx.size(); k++) {
+      sweeps[idx[k]]->rows = kRecon[v0 + pick[k]].rows;
+      sweeps[idx[k]]->team = team[k * n + pick[k]];
+    }
+  }
+}
+
 bool stage_tile_64(const CaseDev &c) { return c.G.ndims == 2 && (long)c.G.nx * c.G.ny >= 2048L * 2048L; }
 
-#ifndef PIAFS_SP_TEAM_MIN
-#define PIAFS_SP_TEAM_MIN 32
-#endif
-#ifndef PIAFS_SP_TEAM_MAX
-#define PIAFS_SP_TEAM_MAX 64
-#endif
 bool species_in_recon(const CaseDev &c) {
-  const bool two = (c.G.ndims == 2);
-  return PIAFS_RECON_SPECIES && PIAFS_RECON_LDS && two && c.model == 2 && c.paired && c.R.crweno && c.upwind == 0 &&
-         !c.R.characteristic && c.G.nv > 4 && c.dsp[0] && c.dsp[1] && c.Sx.team <= PIAFS_SP_TEAM_MAX &&
-         c.Sy.team <= PIAFS_SP_TEAM_MAX && c.Sx.team >= PIAFS_SP_TEAM_MIN && c.Sy.team >= PIAFS_SP_TEAM_MIN &&
-         long_rows(c.Sx, c.G.nv) == 0 && long_rows(c.Sy, c.G.nv) == 0;
+  auto fits = [](const SweepGeom &S) { return !S.longl && (S.team == 32 || S.team == 64); };
+  return c.G.ndims == 2 && c.model == 2 && c.paired && c.R.crweno && c.upwind == 0 && !c.R.characteristic &&
+         c.G.nv > 4 && c.dsp[0] && c.dsp[1] && fits(c.Sx) && fits(c.Sy);
 }
 
 void case_blocks(const CaseDev &c, int blocks[K_NCLASS]) {
@@ -2936,18 +2221,17 @@ void case_blocks(const CaseDev &c, int blocks[K_NCLASS]) {
   blocks[K_FLUX] = weno ? 0 : blocks[K_FLUXALL];
   blocks[K_WENO] = weno ? faces(kWenoTile) : 0;
   blocks[K_CWROWS] = blocks[K_CWSOLVE] = blocks[K_LROWS] = blocks[K_LSOLVE] = 0;
-  blocks[K_ENDS] = blocks[K_RECON] = blocks[K_RECONF] = 0;
+  blocks[K_ENDS] = 0;
+  for (int v = 0; v < kNRecon; v++) blocks[K_RECON + v] = 0;
   if (c.R.crweno && c.R.characteristic) {
     blocks[K_CWROWS] = nb((long)(c.Sx.N + 1) * c.Sx.nlines + (two ? (long)(c.Sy.N + 1) * c.Sy.nlines : 0));
     blocks[K_CWSOLVE] = nb(cw_x_span(c, nf) + (two ? cw_items(c.Sy, G.nv, nf) : 0));
   } else if (c.R.crweno) {
-    blocks[K_ENDS] = nb(2 * (recon_systems(c.Sx, G.nv, c.paired) + (two ? recon_systems(c.Sy, G.nv, c.paired) : 0)));
-    const int nrec = recon_sweep_blocks(c.Sx, G.nv, c.paired) + (two ? recon_sweep_blocks(c.Sy, G.nv, c.paired) : 0);
-    // full segments: both sweeps' lanes hold kMaxRows rows each
-    const bool full = PIAFS_RECON_LDS && PIAFS_RECON_FULL && c.paired && c.Sx.rows == kMaxRows &&
-                      (!two || c.Sy.rows == kMaxRows);
-    blocks[K_RECON] = full ? 0 : nrec;
-    blocks[K_RECONF] = full ? nrec : 0;
+    blocks[K_ENDS] = nb(2 * (recon_pairs(c.Sx, G.nv) + (two ? recon_pairs(c.Sy, G.nv) : 0)));
+    for (int v = 0; v < kNRecon; v++) {
+      if (recon_in(c.Sx, kRecon[v].rows, kRecon[v].wide)) blocks[K_RECON + v] += recon_sweep_blocks(c.Sx, G.nv);
+      if (two && recon_in(c.Sy, kRecon[v].rows, kRecon[v].wide)) blocks[K_RECON + v] += recon_sweep_blocks(c.Sy, G.nv);
+    }
     blocks[K_LROWS] = nb(long_rows(c.Sx, G.nv) + (two ? long_rows(c.Sy, G.nv) : 0));
     blocks[K_LSOLVE] = (int)(long_pairs(c.Sx, G.nv) + (two ? long_pairs(c.Sy, G.nv) : 0));  // a block per pair
   }
@@ -2960,11 +2244,39 @@ void case_blocks(const CaseDev &c, int blocks[K_NCLASS]) {
   blocks[K_UPDATE] = nb((long)G.nx * G.ny * G.nv);
 }
 
-static void run(KernFn k, int cls, const CaseDev *d, const Plan &pl, int s, hipStream_t st, MarkFn mark,
-                void *ctx) {
+static KernFn class_kernel(const Plan &pl, int cls) {
+  static const KernFn recon[] = {recon_kernel<4, false>(),  recon_kernel<6, false>(),  recon_kernel<8, false>(),
+                                 recon_kernel<10, false>(), recon_kernel<12, false>(), recon_kernel<14, false>(),
+                                 recon_kernel<16, false>(), recon_kernel<10, true>(),  recon_kernel<12, true>(),
+                                 recon_kernel<16, true>()};
+  static_assert(sizeof recon / sizeof recon[0] == kNRecon, "a kernel per variant");
+  if (cls >= K_RECON && cls < K_RECON + kNRecon) return recon[cls - K_RECON];
+  switch (cls) {
+    case K_STAGE: return pl.stage64 ? k_stage64 : k_stage;
+    case K_GHOST: return k_ghost;
+    case K_FLUX: case K_FLUXALL: return k_flux;
+    case K_ENDS: return k_recon_ends;
+    case K_LROWS: return k_lrows;
+    case K_LSOLVE: return k_lsolve;
+    case K_CWROWS: return k_cw_rows;
+    case K_CWSOLVE: return k_cw_solve;
+    case K_WENO: return weno_kernel();
+    case K_UPWIND: return k_upwind;
+    case K_BFLUX: return k_bflux;
+    case K_QDERIV: return k_qderiv;
+    case K_VISCFLUX: return k_viscflux;
+    case K_ASSEMBLE: return k_assemble;
+    default: return k_update;
+  }
+}
+
+static void run(int cls, const CaseDev *d, const Plan &pl, int s, hipStream_t st, MarkFn mark, void *ctx) {
   if (pl.nblocks[cls] <= 0) return;
+  const bool recon = cls >= K_RECON && cls < K_RECON + kNRecon;
+  const int threads = recon ? recon_threads(kRecon[cls - K_RECON].wide) : TB;
   if (mark) mark(ctx, cls, true, st);
-  hipLaunchKernelGGL(k, dim3(pl.nblocks[cls]), dim3(TB), 0, st, d, pl.blockcase[cls], pl.firstblock[cls], s);
+  hipLaunchKernelGGL(class_kernel(pl, cls), dim3(pl.nblocks[cls]), dim3(threads), 0, st, d, pl.blockcase[cls],
+                     pl.firstblock[cls], s);
   if (mark) mark(ctx, cls, false, st);
 }
 
@@ -2973,41 +2285,33 @@ static void run(KernFn k, int cls, const CaseDev *d, const Plan &pl, int s, hipS
 // reconstruction / upwinding chain neither reads nor writes Qd or FV.
 void launch_stage(const CaseDev *d, const Plan &pl, int s, hipStream_t st, MarkFn mark, void *ctx,
                   const StageFork *fk, int last) {
-  auto R = [&](KernFn k, int cls, hipStream_t on) {
-    if (cls <= last || cls == K_FLUXALL) run(k, cls, d, pl, s, on, mark, ctx);
+  auto R = [&](int cls, hipStream_t on) {
+    if (cls <= last || cls == K_FLUXALL) run(cls, d, pl, s, on, mark, ctx);
   };
-  R(pl.stage64 ? k_stage64 : k_stage, K_STAGE, st);
-  R(k_ghost, K_GHOST, st);
-  R(k_flux, last == K_FLUX ? K_FLUXALL : K_FLUX, st);
-  R(k_recon_ends, K_ENDS, st);
+  R(K_STAGE, st);
+  R(K_GHOST, st);
+  R(last == K_FLUX ? K_FLUXALL : K_FLUX, st);
+  R(K_ENDS, st);
   const bool fork = fk && fk->side && last >= K_ASSEMBLE &&
                     (pl.nblocks[K_QDERIV] > 0 || pl.nblocks[K_VISCFLUX] > 0);
   if (fork) {
     hipEventRecord(fk->fork, st);
     hipStreamWaitEvent(fk->side, fk->fork, 0);
-    R(k_qderiv, K_QDERIV, fk->side);
-    R(k_viscflux, K_VISCFLUX, fk->side);
+    R(K_QDERIV, fk->side);
+    R(K_VISCFLUX, fk->side);
     hipEventRecord(fk->join, fk->side);
   }
-  R(k_recon, K_RECON, st);
-  R(k_recon_full, K_RECONF, st);
-  R(k_lrows, K_LROWS, st);
-  R(k_lsolve, K_LSOLVE, st);
-  R(k_cw_rows, K_CWROWS, st);
-  R(k_cw_solve, K_CWSOLVE, st);
-  R(weno_kernel(), K_WENO, st);
-  R(k_upwind, K_UPWIND, st);
-  R(k_bflux, K_BFLUX, st);
+  for (int cls = K_RECON; cls <= K_BFLUX; cls++) R(cls, st);
   if (fork) {
     hipStreamWaitEvent(st, fk->join, 0);
   } else {
-    R(k_qderiv, K_QDERIV, st);
-    R(k_viscflux, K_VISCFLUX, st);
+    R(K_QDERIV, st);
+    R(K_VISCFLUX, st);
   }
-  R(k_assemble, K_ASSEMBLE, st);
+  R(K_ASSEMBLE, st);
 }
 
-void launch_update(const CaseDev *d, const Plan &pl, hipStream_t st) { run(k_update, K_UPDATE, d, pl, 0, st, nullptr, nullptr); }
+void launch_update(const CaseDev *d, const Plan &pl, hipStream_t st) { run(K_UPDATE, d, pl, 0, st, nullptr, nullptr); }
 
 int cfl_norm_blocks(const Grid &G) {
   const long n = (long)G.nx * G.ny;
@@ -3078,11 +2382,22 @@ void launch_dev_iface(int ndims, int dir, int nx, int N, int nl, int nv, const d
   hipLaunchKernelGGL(k_dev_iface, dim3(nblk(n)), dim3(TB), 0, s, ndims, dir, nx, N, nl, nv, src, dst, to_lines);
 }
 
+void launch_recon_only(const CaseDev *d, const Plan &pl, const CaseDev &c, int dir, int r, hipStream_t st) {
+  const SweepGeom &S = dir ? c.Sy : c.Sx;
+  const int what = recon_only(dir, r);
+  run(K_ENDS, d, pl, what, st, nullptr, nullptr);
+  for (int v = 0; v < kNRecon; v++) {
+    const int cls = K_RECON + v, threads = recon_threads(kRecon[v].wide);
+    if (!recon_in(S, kRecon[v].rows, kRecon[v].wide)) continue;
+    // half the sweep's pairs, in blocks that all belong to the plan's only case
+    const long per = threads / S.team, n = (recon_pairs(S, c.G.nv) / 2 + per - 1) / per;
+    hipLaunchKernelGGL(class_kernel(pl, cls), dim3((unsigned)n), dim3(threads), 0, st, d, pl.blockcase[cls],
+                       pl.firstblock[cls], what);
+  }
+}
+
 void launch_class(const CaseDev *d, const Plan &pl, int cls, int s, hipStream_t st) {
-  static const KernFn table[K_NCLASS] = {k_stage, k_ghost, k_flux, k_recon_ends, k_recon, k_recon_full, k_lrows,
-                                         k_lsolve, k_cw_rows, k_cw_solve, weno_kernel(),
-                                         k_upwind, k_bflux, k_qderiv, k_viscflux, k_assemble, k_update, k_flux};
-  run(cls == K_STAGE && pl.stage64 ? k_stage64 : table[cls], cls, d, pl, s, st, nullptr, nullptr);
+  run(cls, d, pl, s, st, nullptr, nullptr);
 }
 
 void launch_weno_weights(int kind, const double *copt, const double *st, int count, double eps, double *w,

@@ -42,8 +42,7 @@ struct SweepGeom {
                      // component-wise systems go through k_lrows / k_lsolve instead
 };
 
-// Longest segment of a line system one lane keeps in registers (the
-// register arrays of the reconstruction kernel are sized by it).
+// Longest segment of a line system one lane keeps in registers.
 #ifndef PIAFS_MAX_ROWS
 #define PIAFS_MAX_ROWS 16
 #endif
@@ -52,24 +51,6 @@ constexpr int kMaxRows = PIAFS_MAX_ROWS;
 // piafs_tridiag_host_noalloc takes n*ns <= (capacity - 1) / 4.
 #ifndef PIAFS_NOALLOC_SCRATCH_DOUBLES
 #define PIAFS_NOALLOC_SCRATCH_DOUBLES ((size_t)1 << 22)
-#endif
-// Paired reconstruction with each team's line staged in LDS (1) or read by
-// every lane from global memory (0).
-#ifndef PIAFS_RECON_LDS
-#define PIAFS_RECON_LDS 1
-#endif
-// Paired reconstruction of cases whose lanes all hold kMaxRows rows in a
-// kernel of its own (class K_RECONF), whose line solves need no per-row
-// bounds (rows past the system's end made identity rows).
-#ifndef PIAFS_RECON_FULL
-#define PIAFS_RECON_FULL 1
-#endif
-// NS2D paired Roe: the reconstruction writes the species' interface fluxes
-// f_I = 0.5 (fL + fR) - |v_n| 0.5 (uR - uL) itself, with |v_n| per interface
-// from k_flux, and k_upwind does the four flow variables only (1); or every
-// variable goes through k_upwind (0).
-#ifndef PIAFS_RECON_SPECIES
-#define PIAFS_RECON_SPECIES 1
 #endif
 // Lane exchanges of the line-solve scans and relays by DPP (1) or by LDS
 // permutes (0).
@@ -81,15 +62,16 @@ constexpr int kMaxRows = PIAFS_MAX_ROWS;
 #ifndef PIAFS_XCD_ORDER
 #define PIAFS_XCD_ORDER 1
 #endif
-// blocks per CU that the register allocation of k_recon_full aims at (2: two
-// waves per SIMD, which the DPP exchanges need a few registers' spill for)
-#ifndef PIAFS_RECONF_MINB
-#define PIAFS_RECONF_MINB 2
-#endif
 // Team shape for lines of N points: the fewest lanes (a power of two) whose
 // segments of at most max_rows rows cover interior rows 1..N-1.  Returns
 // false when a line is too long for one block.
 bool team_shape(int N, int max_rows, int &team, int &rows);
+// Lanes of the reconstruction's teams for lines of N points with `rows` rows
+// per lane; false when no kernel has that shape.
+bool line_shape(int N, int rows, int &team);
+// Rows and team of each sweep (none longl) of one step's line systems, for its
+// case's number of variables.
+void choose_rows(const std::vector<SweepGeom *> &sweeps, const std::vector<int> &nvars);
 
 // Boundary zones of boundary.inp, applied in list order: a later zone
 // overwrites an earlier one where both set a variable at a ghost point.
@@ -175,7 +157,7 @@ struct CaseDev {
 // K_FLUX for every case, those of K_WENO (which form their own fluxes) among
 // them, and runs only when the fluxes themselves are asked for.
 enum KClass {
-  K_STAGE = 0, K_GHOST, K_FLUX, K_ENDS, K_RECON, K_RECONF, K_LROWS, K_LSOLVE, K_CWROWS, K_CWSOLVE, K_WENO, K_UPWIND,
+  K_STAGE = 0, K_GHOST, K_FLUX, K_ENDS, K_RECON, K_LROWS = K_RECON + 10, K_LSOLVE, K_CWROWS, K_CWSOLVE, K_WENO, K_UPWIND,
   K_BFLUX, K_QDERIV, K_VISCFLUX, K_ASSEMBLE, K_UPDATE, K_FLUXALL,
   K_NCLASS
 };
@@ -191,14 +173,45 @@ struct Plan {
 };
 
 typedef void (*KernFn)(const CaseDev *, const int *, const int *, int);
+
+// The line systems of the component-wise CRWENO5 reconstruction (recon.hip):
+// one kernel, and one class K_RECON + index, per segment length and team
+// width.  Narrow teams (at most 64 lanes) lie inside a wave.
+struct ReconVariant {
+  int rows;
+  bool wide;
+};
+constexpr ReconVariant kRecon[] = {{4, false},  {6, false},  {8, false}, {10, false}, {12, false},
+                                   {14, false}, {16, false}, {10, true}, {12, true},  {16, true}};
+constexpr int kNRecon = sizeof kRecon / sizeof kRecon[0];
+static_assert(K_LROWS == K_RECON + kNRecon, "a kernel class per variant");
+template <int ROWS, bool WIDE>
+KernFn recon_kernel();
+// threads of a block: narrow teams need no more than the two that share their
+// results, and small blocks leave the CU as they finish
+__host__ __device__ constexpr int recon_threads(bool wide) { return wide ? 256 : 128; }
+// LDS doubles of a team's line, positions -2 .. T*rows+2 with a slot unused after every `rows`
+__host__ __device__ constexpr int recon_region(int T, int rows) { return T * rows + 5 + (T * rows + 5) / rows + 1; }
+// of a block's: most for T = 1
+__host__ __device__ constexpr int recon_line_doubles(int rows, int threads) { return threads * recon_region(1, rows); }
+__host__ __device__ inline bool recon_in(const SweepGeom &S, int rows, bool wide) {
+  return !S.longl && S.rows == rows && (S.team > 64) == wide;
+}
+__host__ __device__ inline long recon_pairs(const SweepGeom &S, int nv) { return S.longl ? 0 : (long)S.nlines * nv * 2; }
+__host__ __device__ inline int recon_sweep_blocks(const SweepGeom &S, int nv) {
+  const long per = recon_threads(S.team > 64) / S.team;
+  return (int)((recon_pairs(S, nv) + per - 1) / per);
+}
+// `stage` argument that restricts a launch to reconstruction r (0 uL, 1 uR, 2
+// fL, 3 fR) of one sweep
+__host__ __device__ constexpr int recon_only(int dir, int r) { return (1 | (r & 1) << 1 | (r >> 1) << 2 | dir << 3) << 8; }
 KernFn weno_kernel();        // k_weno (weno.hip)
 constexpr int kWenoTile = 64;  // interfaces of a block
 
 // Host side: blocks each case needs for each kernel class (0 = class unused).
 void case_blocks(const CaseDev &c, int blocks[K_NCLASS]);
 // Whether the reconstruction can write the species' Roe interface fluxes
-// itself (NS2D, paired Roe, teams of 32 or 64 lanes -- lines of 258 to 1025
-// rows -- no line longer than a team, |v_n| buffers present).
+// itself (NS2D, paired Roe, teams of 32 or 64 lanes, |v_n| buffers present).
 bool species_in_recon(const CaseDev &c);
 // Whether the case is large enough for k_stage's 64 x 64 tiles.
 bool stage_tile_64(const CaseDev &c);
@@ -264,6 +277,9 @@ void launch_set_time(double *time, double t, hipStream_t s);
 // one sweep's interface array: reference layout <-> line-major
 void launch_dev_iface(int ndims, int dir, int nx, int N, int nl, int nv, const double *src, double *dst,
                       int to_lines, hipStream_t s);
+// reconstruction r of the systems of one sweep (not longl), end values included,
+// of a plan's only case, whose descriptor is c
+void launch_recon_only(const CaseDev *d_cases, const Plan &plan, const CaseDev &c, int dir, int r, hipStream_t st);
 // one kernel class of stage s over the plan's cases
 void launch_class(const CaseDev *d_cases, const Plan &plan, int cls, int s, hipStream_t st);
 

@@ -73,7 +73,7 @@ static bool paired_mode(const Config &c) {
 // Cases whose species Roe fluxes the reconstruction can write (NS2D with
 // species, paired Roe, component-wise): they keep |v_n| per interface.
 static bool species_dsp(const Config &c) {
-  return PIAFS_RECON_SPECIES && c.model_id == MODEL_NS2D && c.ndims == 2 && c.nvars > 4 && paired_mode(c) &&
+  return c.crweno && c.model_id == MODEL_NS2D && c.ndims == 2 && c.nvars > 4 && paired_mode(c) &&
          c.upwind == UPW_ROE;
 }
 
@@ -123,7 +123,7 @@ int Case::setup(int dev, hipStream_t st) {
     D.Sy.N = G.ny; D.Sy.g = G.g; D.Sy.plane = G.plane;
     D.Sy.nlines = G.nx; D.Sy.base = (long)G.g * G.nyg + G.gy; D.Sy.line_stride = G.nyg;
   }
-  if (set_team_rows(kMaxRows)) return 1;
+  if (set_team_rows(0)) return 1;
   // boundary zones, in list order (ApplyBoundaryConditions.c:20-40)
   std::vector<double> zvals;
   D.nzones = 0;
@@ -265,7 +265,7 @@ int Case::setup(int dev, hipStream_t st) {
     D.tbi = dalloc(nv, st);
     if (!D.bflux || !D.tbi) return fail(-2, "device allocation failed");
   }
-  if (D.paired) {
+  if (cfg.crweno && !cfg.characteristic) {
     D.ends = dalloc(4 * 2 * (size_t)nv * (D.Sx.nlines + (two ? D.Sy.nlines : 0)), st);
     if (!D.ends) return fail(-2, "device allocation failed");
   }
@@ -298,26 +298,28 @@ int Case::setup(int dev, hipStream_t st) {
   return 0;
 }
 
-int Case::set_team_rows(int max_rows) {
+int Case::set_team_rows(int want) {
   CaseDev &D = h;
   if (cfg.characteristic || !cfg.crweno) {  // no line teams
     D.Sx.team = D.Sy.team = 1;
     D.Sx.rows = D.Sy.rows = 1;
     return 0;
   }
+  std::vector<SweepGeom *> sweeps;
   for (int d = 0; d < cfg.ndims; d++) {
     SweepGeom &S = d ? D.Sy : D.Sx;
-    int T, m;
-    if (!team_shape(S.N, kMaxRows, T, m)) {  // longer than a 256-lane team covers: the sequential solver
-      S.longl = 1;
-      S.team = S.rows = 1;
-      continue;
-    }
-    S.longl = 0;
-    if (!team_shape(S.N, max_rows, S.team, S.rows))
-      return fail(1, "lines of " + std::to_string(S.N) + " points need more than 256 lanes at " +
-                         std::to_string(max_rows) + " rows per lane");
+    S.longl = S.N - 1 > 256 * kMaxRows ? 1 : 0;  // longer than a 256-lane team covers
+    S.team = S.rows = 1;
+    if (S.longl) continue;
+    sweeps.push_back(&S);
+    if (want <= 0) continue;
+    S.rows = want;
+    if (!line_shape(S.N, want, S.team))
+      return fail(1, "lines of " + std::to_string(S.N) + " points have no team shape with " + std::to_string(want) +
+                         " rows per lane");
   }
+  if (want <= 0) choose_rows(sweeps, std::vector<int>(sweeps.size(), cfg.nvars));
+  rows_set = want > 0;
   return 0;
 }
 
@@ -430,8 +432,20 @@ int Engine::build() {
       hd[k] = cases[k]->h;
       hd[k].status = d_status + k;
     }
-    hd[k].fuse_sp = species_in_recon(hd[k]) ? 1 : 0;
   }
+  if (nc > 1) {  // members whose lanes' rows were not set share the choice
+    std::vector<SweepGeom *> sweeps;
+    std::vector<int> nvars;
+    for (int k = 0; k < nc; k++)
+      for (int d = 0; d < hd[k].G.ndims; d++) {
+        SweepGeom &S = d ? hd[k].Sy : hd[k].Sx;
+        if (cases[k]->rows_set || S.longl || !hd[k].R.crweno || hd[k].R.characteristic) continue;
+        sweeps.push_back(&S);
+        nvars.push_back(hd[k].G.nv);
+      }
+    choose_rows(sweeps, nvars);
+  }
+  for (int k = 0; k < nc; k++) hd[k].fuse_sp = species_in_recon(hd[k]) ? 1 : 0;
   plan.stage64 = true;
   for (int k = 0; k < nc; k++) plan.stage64 = plan.stage64 && stage_tile_64(hd[k]);
   for (int k = 0; k < nc; k++) hd[k].stage_tile = plan.stage64 ? 64 : 32;
@@ -565,7 +579,8 @@ double Engine::time_classes(const std::vector<int> &cls, int reps) {
 int Engine::autotune(const int *cands, int ncand, int reps, int *best_rows, double *best_ms) {
   HIPCHK(hipSetDevice(device));
   if (cases.empty()) return 0;
-  const std::vector<int> recon = {K_RECON, K_RECONF, K_WENO};
+  std::vector<int> recon = {K_WENO};
+  for (int v = 0; v < kNRecon; v++) recon.push_back(K_RECON + v);
   int best = -1;
   double bms = 0.0;
   for (int k = 0; k < ncand; k++) {

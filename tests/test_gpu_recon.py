@@ -1,0 +1,71 @@
+"""The CRWENO5 line systems over segment lengths and team widths: right-hand
+sides against the oracle on lines that fill a team exactly, by one row less and
+one more, in both sweeps, paired (Roe) and split (llf-char), and every
+reconstruction alone through the device-buffer operator.  Tolerance as for the
+other pieces of a right-hand side: 1e-12 of each variable's largest magnitude."""
+import numpy as np
+import pytest
+
+import _oracle as orc
+import piafs_amd
+from piafs_amd import decks
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+
+
+def _close(got, want):
+    got, want = got.reshape(-1, got.shape[-1]), want.reshape(-1, want.shape[-1])
+    scale = np.abs(want).max(axis=0)
+    assert np.all(np.abs(got - want).max(axis=0) <= TOL * np.where(scale > 0, scale, 1.0))
+
+
+def _deck(nx, ny, **kw):
+    periodic = [("periodic", 0, 1, 0, 0, -1e99, 1e99), ("periodic", 0, -1, 0, 0, -1e99, 1e99),
+                ("periodic", 1, 1, -1e99, 1e99, 0, 0), ("periodic", 1, -1, -1e99, 1e99, 0, 0)]
+    return decks.ns2d_open_box(nx=nx, ny=ny, flow=(1.0, 0.3, -0.2, None), scheme="crweno5", include_chemistry=True,
+                               Re=500.0, boundary=periodic, **kw)
+
+
+# interior rows N - 1 at, below and above 4, 6, .. 16 rows on 1 .. 256 lanes
+SIZES = [(5, 8), (9, 17), (33, 34), (64, 66), (97, 98), (129, 130), (161, 12), (193, 194), (225, 14), (257, 256),
+         (321, 10), (449, 9), (577, 8), (641, 7), (769, 8), (898, 7), (1024, 8), (1025, 6), (1026, 6), (1281, 7),
+         (1537, 6), (2049, 5), (4097, 5), (6, 1500)]
+
+
+@pytest.mark.parametrize("nx,ny", SIZES)
+@pytest.mark.parametrize("upwinding", ["roe", "llf-char"])
+def test_segment_lengths(tmp_path, nx, ny, upwinding):
+    dk = _deck(nx, ny, upwinding=upwinding)
+    u = dk.u * (1.0 + 1e-2 * np.random.default_rng(nx + ny).uniform(-1, 1, dk.u.shape))
+    d = dk.write(str(tmp_path))
+    want = orc.OCase(d).rhs(u, 0.45)
+    with piafs_amd.Case(d) as c:
+        _close(c.rhs(u, 0.45), want)
+
+
+@pytest.mark.parametrize("rows", [4, 6, 8, 10, 12, 14, 16])
+@pytest.mark.parametrize("weights", ["js", "mapped", "z", "yc", "none"])
+def test_rows_and_weights(tmp_path, rows, weights):
+    """Lines of 8 lanes of each segment length, the last one a row short."""
+    dk = _deck(8 * rows, 8 * rows, weights=weights)
+    u = dk.u * (1.0 + 1e-2 * np.random.default_rng(rows).uniform(-1, 1, dk.u.shape))
+    d = dk.write(str(tmp_path))
+    want = orc.OCase(d).rhs(u, 0.45)
+    with piafs_amd.Case(d) as c:
+        _close(c.rhs(u, 0.45), want)
+
+
+def test_members_of_many_shapes(tmp_path):
+    """Members share the choice of segment lengths; each equals its solo run."""
+    dirs = []
+    for k, (nx, ny) in enumerate([(33, 97), (129, 65), (200, 40), (1100, 9), (50, 300), (257, 31)]):
+        dirs.append(_deck(nx, ny, n_iter=2, dt=1e-4).write(str(tmp_path / str(k))))
+    with piafs_amd.Batch(dirs) as b:
+        b.step(2)
+        got = [b.solution(k) for k in b.slots]
+    for k, d in enumerate(dirs):
+        with piafs_amd.Case(d) as c:
+            c.step(2)
+            assert np.array_equal(got[k], c.solution()), k
