@@ -1415,129 +1415,128 @@ __device__ __forceinline__ Prim prim_at(long plane, double gam, const double *U,
   return r;
 }
 
-// FirstDerivativeFourthOrder.c:39-132 (PAR4) / FirstDerivativeFirstOrder.c (bias +1)
-// of the three primitives at position i of a line of N interior points.
-template <int PAR4>
-__device__ __forceinline__ void deriv_prim(long plane, int g, double gam, const double *U, long p0, long st, int i,
-                                           int N, double out[3]) {
-  auto P = [&](int k) { return prim_at(plane, gam, U, p0 + (long)k * st); };
-  if (PAR4) {
-    const double t12 = 1.0 / 12.0;
-    if (i == -g) {
-      Prim a = P(i), b = P(i + 1), c = P(i + 2), d = P(i + 3), e = P(i + 4);
-      out[0] = (-25 * a.vx + 48 * b.vx - 36 * c.vx + 16 * d.vx - 3 * e.vx) * t12;
-      out[1] = (-25 * a.vy + 48 * b.vy - 36 * c.vy + 16 * d.vy - 3 * e.vy) * t12;
-      out[2] = (-25 * a.T + 48 * b.T - 36 * c.T + 16 * d.T - 3 * e.T) * t12;
-    } else if (i == -g + 1) {
-      Prim a = P(i - 1), b = P(i), c = P(i + 1), d = P(i + 2), e = P(i + 3);
-      out[0] = (-3 * a.vx - 10 * b.vx + 18 * c.vx - 6 * d.vx + e.vx) * t12;
-      out[1] = (-3 * a.vy - 10 * b.vy + 18 * c.vy - 6 * d.vy + e.vy) * t12;
-      out[2] = (-3 * a.T - 10 * b.T + 18 * c.T - 6 * d.T + e.T) * t12;
-    } else if (i == N + g - 2) {
-      Prim a = P(i - 3), b = P(i - 2), c = P(i - 1), d = P(i), e = P(i + 1);
-      out[0] = (-a.vx + 6 * b.vx - 18 * c.vx + 10 * d.vx + 3 * e.vx) * t12;
-      out[1] = (-a.vy + 6 * b.vy - 18 * c.vy + 10 * d.vy + 3 * e.vy) * t12;
-      out[2] = (-a.T + 6 * b.T - 18 * c.T + 10 * d.T + 3 * e.T) * t12;
+// FirstDerivativeFourthOrder.c:39-132 (par4) / FirstDerivativeFirstOrder.c (bias +1)
+// of the three primitives at position i of a line of N interior points, P(k)
+// the primitives at position k (component c: P(k, c)).
+template <class F>
+__device__ __forceinline__ void deriv_prim(int g, bool par4, int i, int N, F P, double out[3]) {
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    if (par4) {
+      const double t12 = 1.0 / 12.0;
+      if (i == -g)
+        out[c] = (-25 * P(i, c) + 48 * P(i + 1, c) - 36 * P(i + 2, c) + 16 * P(i + 3, c) - 3 * P(i + 4, c)) * t12;
+      else if (i == -g + 1)
+        out[c] = (-3 * P(i - 1, c) - 10 * P(i, c) + 18 * P(i + 1, c) - 6 * P(i + 2, c) + P(i + 3, c)) * t12;
+      else if (i == N + g - 2)
+        out[c] = (-P(i - 3, c) + 6 * P(i - 2, c) - 18 * P(i - 1, c) + 10 * P(i, c) + 3 * P(i + 1, c)) * t12;
+      else if (i == N + g - 1)
+        out[c] = (3 * P(i - 4, c) - 16 * P(i - 3, c) + 36 * P(i - 2, c) - 48 * P(i - 1, c) + 25 * P(i, c)) * t12;
+      else
+        out[c] = (P(i - 2, c) - 8 * P(i - 1, c) + 8 * P(i + 1, c) - P(i + 2, c)) * t12;
+    } else if (i == -g) {
+      out[c] = P(i + 1, c) - P(i, c);
     } else if (i == N + g - 1) {
-      Prim a = P(i - 4), b = P(i - 3), c = P(i - 2), d = P(i - 1), e = P(i);
-      out[0] = (3 * a.vx - 16 * b.vx + 36 * c.vx - 48 * d.vx + 25 * e.vx) * t12;
-      out[1] = (3 * a.vy - 16 * b.vy + 36 * c.vy - 48 * d.vy + 25 * e.vy) * t12;
-      out[2] = (3 * a.T - 16 * b.T + 36 * c.T - 48 * d.T + 25 * e.T) * t12;
+      out[c] = P(i, c) - P(i - 1, c);
     } else {
-      Prim a = P(i - 2), b = P(i - 1), d = P(i + 1), e = P(i + 2);
-      out[0] = (a.vx - 8 * b.vx + 8 * d.vx - e.vx) * t12;
-      out[1] = (a.vy - 8 * b.vy + 8 * d.vy - e.vy) * t12;
-      out[2] = (a.T - 8 * b.T + 8 * d.T - e.T) * t12;
-    }
-  } else {
-    if (i == -g) {
-      Prim a = P(i), b = P(i + 1);
-      out[0] = b.vx - a.vx; out[1] = b.vy - a.vy; out[2] = b.T - a.T;
-    } else if (i == N + g - 1) {
-      Prim a = P(i - 1), b = P(i);
-      out[0] = b.vx - a.vx; out[1] = b.vy - a.vy; out[2] = b.T - a.T;
-    } else {
-      Prim a = P(i - 1), b = P(i), c = P(i + 1);
-      out[0] = 1.0 * c.vx - 1.0 * b.vx + 0.0 * a.vx;
-      out[1] = 1.0 * c.vy - 1.0 * b.vy + 0.0 * a.vy;
-      out[2] = 1.0 * c.T - 1.0 * b.T + 0.0 * a.T;
+      out[c] = 1.0 * P(i + 1, c) - 1.0 * P(i, c) + 0.0 * P(i - 1, c);
     }
   }
-}
-
-// Qd planes: 0 ux, 1 vx, 2 Tx (d/dx), 3 uy, 4 vy, 5 Ty (d/dy), each scaled by
-// dxinv (NavierStokes2DParabolicFunction.c:96-106).  With the derivative
-// exchange along a periodic dimension (xchg, MPIExchangeBoundariesnD.c:
-// 109-167 as called at NavierStokes2DParabolicFunction.c:91-94), a ghost point
-// of an interior line across that dimension takes the unscaled derivatives of
-// its periodic image, scaled by its own dxinv; corners are not exchanged.
-__global__ void __launch_bounds__(256) k_qderiv(CASE_ARGS) {
-  CASE_PREAMBLE
-  if (stage >= C.nstages) return;
-  const Grid &G = C.G;
-  if (t >= (long)G.nxg * G.nyg) return;
-  const int i = (int)(t % G.nxg) - G.g, j = (int)(t / G.nxg) - G.g;
-  const long pl = (long)G.nxg * G.nyg;
-  const double gam = C.P.gamma;
-  double dx[3] = {0, 0, 0}, dy[3] = {0, 0, 0};
-  const bool iin = i >= 0 && i < G.nx, jin = j >= 0 && j < G.ny;
-  int si = i, sj = j;  // the point whose derivatives this point holds
-  if (C.P.xchg[0] && jin && !iin) si = i < 0 ? i + G.nx : i - G.nx;
-  if (C.P.xchg[1] && iin && !jin) sj = j < 0 ? j + G.ny : j - G.ny;
-  if (sj >= 0 && sj < G.ny) {
-    const long p0 = (long)(sj + G.g) * G.nxg + G.g;  // (0, sj)
-    if (C.P.par4) deriv_prim<1>(G.plane, G.g, gam, C.U, p0, 1, si, G.nx, dx);
-    else deriv_prim<0>(G.plane, G.g, gam, C.U, p0, 1, si, G.nx, dx);
-    const double s = C.dxinv[G.g + i];
-    dx[0] *= s; dx[1] *= s; dx[2] *= s;
-  }
-  if (si >= 0 && si < G.nx) {
-    const long p0 = (long)G.g * G.nxg + (si + G.g);  // (si, 0)
-    if (C.P.par4) deriv_prim<1>(G.plane, G.g, gam, C.U, p0, G.nxg, sj, G.ny, dy);
-    else deriv_prim<0>(G.plane, G.g, gam, C.U, p0, G.nxg, sj, G.ny, dy);
-    const double s = C.dxinv[(G.nx + 2 * G.g) + G.g + j];
-    dy[0] *= s; dy[1] *= s; dy[2] *= s;
-  }
-  double *Qd = C.Qd;
-  Qd[t] = dx[0]; Qd[pl + t] = dx[1]; Qd[2 * pl + t] = dx[2];
-  Qd[3 * pl + t] = dy[0]; Qd[4 * pl + t] = dy[1]; Qd[5 * pl + t] = dy[2];
 }
 
 // Viscous fluxes (NavierStokes2DParabolicFunction.c:112-143 and :155-186),
 // Sutherland viscosity and the conductivity law of navierstokes2d.h:315-331
-// (raiseto(x,1.5) = exp(1.5 log x), include/math_ops.h:40).
+// (raiseto(x,1.5) = exp(1.5 log x), include/math_ops.h:40), from the derivatives
+// of velocity and temperature, each scaled by dxinv
+// (NavierStokes2DParabolicFunction.c:96-106).  With the derivative exchange
+// along a periodic dimension (xchg, MPIExchangeBoundariesnD.c:109-167 as called
+// at NavierStokes2DParabolicFunction.c:91-94), a ghost point of an interior
+// line across that dimension takes the unscaled derivatives of its periodic
+// image, scaled by its own dxinv; corners are not exchanged, and never read.
 // FV planes: 0..2 = x-flux components 1..3, 3..5 = y-flux components 1..3.
-__global__ void __launch_bounds__(256) k_viscflux(CASE_ARGS) {
+//
+// A 32 x 8 tile of ghosted points per block.  Bound by latency on small grids
+// and by HBM on large ones: the primitives of the tile and of the four points
+// beside it (one-sided stencils reach that far) are formed once into LDS, 2.25
+// divisions chains a thread instead of 21 in two passes with the derivatives
+// in memory between them.
+constexpr int kVisX = 32, kVisY = 8, kVisH = 4;
+__global__ void __launch_bounds__(256) k_viscous(CASE_ARGS) {
   CASE_PREAMBLE
+  (void)t;
   if (stage >= C.nstages) return;
   const Grid &G = C.G;
   const PhysParams &P = C.P;
-  if (t >= (long)G.nxg * G.nyg) return;
-  const int i = (int)(t % G.nxg) - G.g, j = (int)(t / G.nxg) - G.g;
-  const bool ix = (i >= 0 && i < G.nx), jy = (j >= 0 && j < G.ny);
-  if (!ix && !jy) return;  // corners are never read
-  const long pl = (long)G.nxg * G.nyg;
-  const double *Qd = C.Qd;
-  double *FV = C.FV;
-  const Prim q = prim_at(G.plane, P.gamma, C.U, t);
-  const double ux = Qd[t], vx = Qd[pl + t], Tx = Qd[2 * pl + t];
-  const double uy = Qd[3 * pl + t], vy = Qd[4 * pl + t], Ty = Qd[5 * pl + t];
-  const double Td = q.T * P.Tref;
+  __shared__ double pr[3][kVisY + 2 * kVisH][kVisX + 2 * kVisH];
+  const int tiles = (G.nxg + kVisX - 1) / kVisX;
+  const int b = (int)(blockIdx.x - firstblock[cidx]);
+  const int I0 = (b % tiles) * kVisX, J0 = (b / tiles) * kVisY;  // ghosted indices
+  const double gam = P.gamma;
+  auto fill = [&](int a, int c) {  // LDS position (row a, column c)
+    const int I = I0 + c - kVisH, J = J0 + a - kVisH;
+    if (I < 0 || I >= G.nxg || J < 0 || J >= G.nyg) return;
+    const Prim q = prim_at(G.plane, gam, C.U, (long)J * G.nxg + I);
+    pr[0][a][c] = q.vx;
+    pr[1][a][c] = q.vy;
+    pr[2][a][c] = q.T;
+  };
+  const int tx = threadIdx.x & (kVisX - 1), ty = threadIdx.x / kVisX;
+  fill(ty + kVisH, tx + kVisH);
+  // four rows below and four above, then the columns beside the tile
+  fill(ty < kVisH ? ty : ty + kVisY, tx + kVisH);
+  if (threadIdx.x < 2 * kVisH * kVisY) {
+    const int c = threadIdx.x & (2 * kVisH - 1), r = threadIdx.x / (2 * kVisH);
+    fill(r + kVisH, c < kVisH ? c : c + kVisX);
+  }
+  lds_barrier();
+  const int I = I0 + tx, J = J0 + ty;
+  if (I >= G.nxg || J >= G.nyg) return;
+  const int i = I - G.g, j = J - G.g;
+  const bool iin = i >= 0 && i < G.nx, jin = j >= 0 && j < G.ny;
+  if (!iin && !jin) return;  // corners are never read
+  double dx[3] = {0, 0, 0}, dy[3] = {0, 0, 0};
+  // derivatives along x on interior rows, along y on interior columns
+  const bool ex = P.xchg[0] && jin && !iin, ey = P.xchg[1] && iin && !jin;
+  auto far = [&](int x, int y, int c) {  // a point outside the tile's reach
+    const Prim q = prim_at(G.plane, gam, C.U, (long)(y + G.g) * G.nxg + (x + G.g));
+    return c == 0 ? q.vx : c == 1 ? q.vy : q.T;
+  };
+  if (ex) {  // both derivatives of the image in x
+    const int si = i < 0 ? i + G.nx : i - G.nx;
+    deriv_prim(G.g, P.par4, si, G.nx, [&](int k, int c) { return far(k, j, c); }, dx);
+    deriv_prim(G.g, P.par4, j, G.ny, [&](int k, int c) { return far(si, k, c); }, dy);
+  } else if (ey) {
+    const int sj = j < 0 ? j + G.ny : j - G.ny;
+    deriv_prim(G.g, P.par4, i, G.nx, [&](int k, int c) { return far(k, sj, c); }, dx);
+    deriv_prim(G.g, P.par4, sj, G.ny, [&](int k, int c) { return far(i, k, c); }, dy);
+  } else {
+    if (jin)
+      deriv_prim(G.g, P.par4, i, G.nx, [&](int k, int c) { return pr[c][ty + kVisH][tx + kVisH + k - i]; }, dx);
+    if (iin)
+      deriv_prim(G.g, P.par4, j, G.ny, [&](int k, int c) { return pr[c][ty + kVisH + k - j][tx + kVisH]; }, dy);
+  }
+  const double sx = C.dxinv[G.g + i], sy = C.dxinv[(G.nx + 2 * G.g) + G.g + j];
+  const double ux = dx[0] * sx, vx = dx[1] * sx, Tx = dx[2] * sx;
+  const double uy = dy[0] * sy, vy = dy[1] * sy, Ty = dy[2] * sy;
+  const double qx = pr[0][ty + kVisH][tx + kVisH], qy = pr[1][ty + kVisH][tx + kVisH];
+  const double Td = pr[2][ty + kVisH][tx + kVisH] * P.Tref;
   const double r15 = exp(1.5 * log(Td / P.T0));
   const double mu = r15 * (P.T0 + P.TS) / (Td + P.TS);
   const double kap = r15 * P.kappa_num / (Td + P.TA * exp(-P.TB / Td));
   const double muRe = mu * P.inv_Re;
   const double kc = kap * P.inv_Re * P.inv_gm1 * P.inv_Pr;
+  const long pl = (long)G.nxg * G.nyg, p = (long)J * G.nxg + I;
+  double *FV = C.FV;
   const double txx = P.two_third * muRe * (2 * ux - vy);
   const double txy = muRe * (uy + vx);
-  FV[t] = txx;
-  FV[pl + t] = txy;
-  FV[2 * pl + t] = q.vx * txx + q.vy * txy + kc * Tx;
+  FV[p] = txx;
+  FV[pl + p] = txy;
+  FV[2 * pl + p] = qx * txx + qy * txy + kc * Tx;
   const double tyx = muRe * (uy + vx);
   const double tyy = P.two_third * muRe * (-ux + 2 * vy);
-  FV[3 * pl + t] = tyx;
-  FV[4 * pl + t] = tyy;
-  FV[5 * pl + t] = q.vx * tyx + q.vy * tyy + kc * Ty;
+  FV[3 * pl + p] = tyx;
+  FV[4 * pl + p] = tyy;
+  FV[5 * pl + p] = qx * tyx + qy * tyy + kc * Ty;
 }
 
 // ---------------------------------------------------------------------------
@@ -2106,7 +2105,7 @@ static const char *kKNames[K_NCLASS] = {"stage_bc", "ghost",  "flux",    "recon_
                                         "recon_4",  "recon_6", "recon_8", "recon_10", "recon_12", "recon_14", "recon_16",
                                         "recon_w10", "recon_w12", "recon_w16", "long_rows", "long_solve",
                                         "cw_rows", "cw_solve", "weno", "upwind", "bflux",
-                                        "qderiv",   "viscflux", "assemble", "update", "flux_all"};
+                                        "viscous", "assemble", "update", "flux_all"};
 const char *kclass_name(int k) { return kKNames[k]; }
 
 int cw_row_fields(int nflow, int nv) { return nflow * nflow + 16 * nv; }
@@ -2238,8 +2237,7 @@ void case_blocks(const CaseDev &c, int blocks[K_NCLASS]) {
   blocks[K_UPWIND] = weno ? 0 : nb((long)(c.Sx.N + 1) * c.Sx.nlines + (two ? (long)(c.Sy.N + 1) * c.Sy.nlines : 0));
   blocks[K_BFLUX] = c.cons ? 1 : 0;
   const bool visc = two && c.P.viscous;
-  blocks[K_QDERIV] = visc ? nb((long)G.nxg * G.nyg) : 0;
-  blocks[K_VISCFLUX] = visc ? nb((long)G.nxg * G.nyg) : 0;
+  blocks[K_VISCOUS] = visc ? ((G.nxg + kVisX - 1) / kVisX) * ((G.nyg + kVisY - 1) / kVisY) : 0;
   blocks[K_ASSEMBLE] = pad8(two ? ((G.nx + 31) / 32) * ((G.ny + 31) / 32) * G.nv : nb((long)G.nx * G.nv));
   blocks[K_UPDATE] = nb((long)G.nx * G.ny * G.nv);
 }
@@ -2263,8 +2261,7 @@ static KernFn class_kernel(const Plan &pl, int cls) {
     case K_WENO: return weno_kernel();
     case K_UPWIND: return k_upwind;
     case K_BFLUX: return k_bflux;
-    case K_QDERIV: return k_qderiv;
-    case K_VISCFLUX: return k_viscflux;
+    case K_VISCOUS: return k_viscous;
     case K_ASSEMBLE: return k_assemble;
     default: return k_update;
   }
@@ -2280,9 +2277,9 @@ static void run(int cls, const CaseDev *d, const Plan &pl, int s, hipStream_t st
   if (mark) mark(ctx, cls, false, st);
 }
 
-// k_qderiv and k_viscflux read only the stage state (after k_ghost) and
-// write only Qd and FV, which nothing before k_assemble reads; the
-// reconstruction / upwinding chain neither reads nor writes Qd or FV.
+// k_viscous reads only the stage state (after k_ghost) and writes only FV, which
+// nothing before k_assemble reads; the reconstruction / upwinding chain neither
+// reads nor writes FV.
 void launch_stage(const CaseDev *d, const Plan &pl, int s, hipStream_t st, MarkFn mark, void *ctx,
                   const StageFork *fk, int last) {
   auto R = [&](int cls, hipStream_t on) {
@@ -2292,21 +2289,18 @@ void launch_stage(const CaseDev *d, const Plan &pl, int s, hipStream_t st, MarkF
   R(K_GHOST, st);
   R(last == K_FLUX ? K_FLUXALL : K_FLUX, st);
   R(K_ENDS, st);
-  const bool fork = fk && fk->side && last >= K_ASSEMBLE &&
-                    (pl.nblocks[K_QDERIV] > 0 || pl.nblocks[K_VISCFLUX] > 0);
+  const bool fork = fk && fk->side && last >= K_ASSEMBLE && pl.nblocks[K_VISCOUS] > 0;
   if (fork) {
     hipEventRecord(fk->fork, st);
     hipStreamWaitEvent(fk->side, fk->fork, 0);
-    R(K_QDERIV, fk->side);
-    R(K_VISCFLUX, fk->side);
+    R(K_VISCOUS, fk->side);
     hipEventRecord(fk->join, fk->side);
   }
   for (int cls = K_RECON; cls <= K_BFLUX; cls++) R(cls, st);
   if (fork) {
     hipStreamWaitEvent(st, fk->join, 0);
   } else {
-    R(K_QDERIV, st);
-    R(K_VISCFLUX, st);
+    R(K_VISCOUS, st);
   }
   R(K_ASSEMBLE, st);
 }

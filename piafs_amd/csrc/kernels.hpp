@@ -132,7 +132,7 @@ struct CaseDev {
   double dt, A[16], b[4], c[4];
   double *u, *U, *UT, *Udot[4];
   double *flux_x, *flux_y, *ix[4], *iy[4], *fIx, *fIy;
-  double *Qd, *FV, *dxinv, *imap;
+  double *FV, *dxinv, *imap;
   double *xc;      // grid coordinates with ghosts, one dimension after the other
   double *bcvals;  // the zones' values (Zone::vals)
   double *ends;  // paired mode: raw end-interface values of both systems of every pair [dir][pair][side][0|N]
@@ -158,7 +158,7 @@ struct CaseDev {
 // them, and runs only when the fluxes themselves are asked for.
 enum KClass {
   K_STAGE = 0, K_GHOST, K_FLUX, K_ENDS, K_RECON, K_LROWS = K_RECON + 10, K_LSOLVE, K_CWROWS, K_CWSOLVE, K_WENO, K_UPWIND,
-  K_BFLUX, K_QDERIV, K_VISCFLUX, K_ASSEMBLE, K_UPDATE, K_FLUXALL,
+  K_BFLUX, K_VISCOUS, K_ASSEMBLE, K_UPDATE, K_FLUXALL,
   K_NCLASS
 };
 const char *kclass_name(int k);

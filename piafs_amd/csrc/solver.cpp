@@ -89,7 +89,7 @@ size_t Case::plan_bytes(const Config &c) {
     const int nf = c.model_id == MODEL_EULER1D ? 3 : 4;
     n += (size_t)(cw_row_fields(nf, (int)nv) + 4 * cw_back_fields(nf, (int)nv)) * (ix + iy) / nv;
   }
-  if (c.model_id == MODEL_NS2D) n += 12 * (size_t)g.nxg * g.nyg;
+  if (c.model_id == MODEL_NS2D) n += 6 * (size_t)g.nxg * g.nyg;
   if (c.crweno && !c.characteristic) {  // long-line scratch of sweeps longer than one team
     int T, m;
     for (int d = 0; d < c.ndims; d++)
@@ -227,7 +227,6 @@ int Case::setup(int dev, hipStream_t st) {
     if (!D.dsp[0] || !D.dsp[1]) return fail(-2, "device allocation failed");
   }
   if (P.viscous) {
-    D.Qd = dalloc(6 * (size_t)G.nxg * G.nyg, st);
     D.FV = dalloc(6 * (size_t)G.nxg * G.nyg, st);
   }
   D.dxinv = dalloc(cfg.dxinv.size(), st);
