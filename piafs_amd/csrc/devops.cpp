@@ -152,7 +152,7 @@ int piafs_dev_interp_interfaces(piafs_case *pc, double *fI, const double *fC, co
     // buffers; the systems of the other biases and of the other sweep are
     // solved too, on the state's own flux, and discarded
     stage_state(pc, uflag ? fC : u_ghosted, st);
-    launch_class(un.eng.d_cases, un.eng.plan, K_FLUX, 0, st);
+    launch_class(un.eng.d_cases, un.eng.plan, K_FLUXALL, 0, st);
     if (!uflag)
       launch_dev_planar(G, fC, dir ? nullptr : d.flux_x, dir ? d.flux_y : nullptr, 1, 0, nullptr, st);
     for (int cls = K_ENDS; cls <= K_CWSOLVE; cls++) launch_class(un.eng.d_cases, un.eng.plan, cls, 0, st);

@@ -7,6 +7,7 @@
 // rounding of every +, -, *, / and sqrt matches the reference build.
 #include "device.hpp"
 #include "teams.hpp"
+#include "viscous.hpp"
 
 #include <cstdio>
 #include <type_traits>
@@ -156,12 +157,58 @@ __device__ double ghost_value(const CaseDev &C, int s, int v, int i, int j) {
   return igm1 * pg + 0.5 * rg * (ug * ug + vg * vg);
 }
 
+// Ghost points of the stage state, one thread per (variable, ghost point):
+// the g rows below and above the interior (full ghosted width), then the g
+// columns left and right of it (interior height).  Written to both layouts.
+
+__host__ __device__ inline long ghost_points(const Grid &G) {
+  return G.ndims == 1 ? 2L * G.g : 2L * G.gy * G.nxg + 2L * G.g * G.ny;
+}
+
+__device__ __forceinline__ void ghost_body(const CaseDev &C, int stage, long t) {
+  const Grid &G = C.G;
+  const long ng = ghost_points(G);
+  if (t >= ng * G.nv) return;
+  const int v = (int)(t / ng);
+  long q = t % ng;
+  int i, j = 0;
+  if (G.ndims == 1) {
+    i = (q < G.g) ? (int)q - G.g : G.nx + (int)(q - G.g);
+  } else if (q < 2L * G.gy * G.nxg) {
+    const int row = (int)(q / G.nxg);
+    i = (int)(q % G.nxg) - G.g;
+    j = row < G.gy ? row - G.gy : G.ny + (row - G.gy);
+  } else {
+    q -= 2L * G.gy * G.nxg;
+    const int col = (int)(q / G.ny);
+    j = (int)(q % G.ny);
+    i = col < G.g ? col - G.g : G.nx + (col - G.g);
+  }
+  const double val = ghost_value(C, stage, v, i, j);
+  const long pl = (long)v * G.plane;
+  C.U[pl + (long)(j + G.gy) * G.nxg + (i + G.g)] = val;
+  if (G.ndims == 2) C.UT[pl + (long)(i + G.g) * G.nyg + (j + G.gy)] = val;
+}
+
+// blocks of the interior points, padded to a multiple of eight for xcd_order;
+// the blocks of the ghost points follow (they read the solution, not the stage
+// state, so neither waits for the other)
+__host__ __device__ inline int stage_blocks(const Grid &G, int st) {
+  const long n = G.ndims == 1 ? ((long)G.nx * G.nv + TB - 1) / TB
+                              : (long)((G.nx + st - 1) / st) * ((G.ny + st - 1) / st) * G.nv;
+  return (int)((n + 7) & ~7L);
+}
+
 template <int ST>
 __device__ __forceinline__ void stage_body(CASE_ARGS) {
   CASE_PREAMBLE
   if (stage >= C.nstages) return;
   const Grid &G = C.G;
-  const int s = stage;
+  const int s = stage, bid = (int)(blockIdx.x - firstblock[cidx]), ns = stage_blocks(G, ST);
+  if (bid >= ns) {
+    ghost_body(C, s, t - (long)ns * TB);
+    return;
+  }
   if (G.ndims == 1) {
     if (t >= (long)G.nx * G.nv) return;
     const int v = (int)(t / G.nx), i = (int)(t % G.nx);
@@ -170,15 +217,14 @@ __device__ __forceinline__ void stage_body(CASE_ARGS) {
     return;
   }
   // 2D interior: ST x ST tiles, 256 threads; natural write, then transposed
-  // write via LDS.  The ghost layer is k_ghost's.
+  // write via LDS.
   constexpr int SR = 256 / ST;
   __shared__ double tile[ST][ST + 1];
   const int ntx = (G.nx + ST - 1) / ST, nty = (G.ny + ST - 1) / ST;
   // (64-point tiles: workgroup order, which timed faster for them at 4096^2);
   // the case's block count is padded to a multiple of eight
   const int nb = G.nv * ntx * nty;
-  const int lid = (int)(blockIdx.x - firstblock[cidx]);
-  const int id = ST == 32 ? xcd_order(lid, (nb + 7) & ~7, firstblock[cidx]) : lid;
+  const int id = ST == 32 ? xcd_order(bid, ns, firstblock[cidx]) : bid;
   if (id >= nb) return;
   const int v = id / (ntx * nty), rem = id % (ntx * nty);
   const int i0 = (rem % ntx) * ST, j0 = (rem / ntx) * ST;
@@ -207,40 +253,11 @@ __device__ __forceinline__ void stage_body(CASE_ARGS) {
 __global__ void __launch_bounds__(256) k_stage(CASE_ARGS) { stage_body<32>(cases, blockcase, firstblock, stage); }
 __global__ void __launch_bounds__(256) k_stage64(CASE_ARGS) { stage_body<64>(cases, blockcase, firstblock, stage); }
 
-// Ghost points of the stage state, one thread per (variable, ghost point):
-// the g rows below and above the interior (full ghosted width), then the g
-// columns left and right of it (interior height).  Written to both layouts.
-__host__ __device__ inline long ghost_points(const Grid &G) {
-  return G.ndims == 1 ? 2L * G.g : 2L * G.gy * G.nxg + 2L * G.g * G.ny;
-}
-
+// the ghost points alone, for the boundary-fill operator
 __global__ void __launch_bounds__(256) k_ghost(CASE_ARGS) {
   CASE_PREAMBLE
-  if (stage >= C.nstages) return;
-  const Grid &G = C.G;
-  const long ng = ghost_points(G);
-  if (t >= ng * G.nv) return;
-  const int v = (int)(t / ng);
-  long q = t % ng;
-  int i, j = 0;
-  if (G.ndims == 1) {
-    i = (q < G.g) ? (int)q - G.g : G.nx + (int)(q - G.g);
-  } else if (q < 2L * G.gy * G.nxg) {
-    const int row = (int)(q / G.nxg);
-    i = (int)(q % G.nxg) - G.g;
-    j = row < G.gy ? row - G.gy : G.ny + (row - G.gy);
-  } else {
-    q -= 2L * G.gy * G.nxg;
-    const int col = (int)(q / G.ny);
-    j = (int)(q % G.ny);
-    i = col < G.g ? col - G.g : G.nx + (col - G.g);
-  }
-  const double val = ghost_value(C, stage, v, i, j);
-  const long pl = (long)v * G.plane;
-  C.U[pl + (long)(j + G.gy) * G.nxg + (i + G.g)] = val;
-  if (G.ndims == 2) C.UT[pl + (long)(i + G.g) * G.nyg + (j + G.gy)] = val;
+  if (stage < C.nstages) ghost_body(C, stage, t);
 }
-
 
 // ---------------------------------------------------------------------------
 // Cell-centred flux at every position of every interior line, both sweeps:
@@ -248,9 +265,90 @@ __global__ void __launch_bounds__(256) k_ghost(CASE_ARGS) {
 // NavierStokes2DFlux.c:24-52 (navierstokes2d.h:70-110), Euler1DFlux.c:19
 // (euler1d.h:61-85).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_flux(CASE_ARGS) {
+// The two end interfaces (0 and N) of the line systems, a thread per pair of
+// systems and end: WENO5 values on identity rows
+// (Interp1PrimFifthOrderCRWENO.c:132-201 with the WENO5 weights at the ends).
+// The raw values go to the case's `ends` table for the line solves, and, in
+// paired mode their combination, to the interface arrays.  w: the six values at
+// positions k-3 .. k+2.
+template <int KIND>
+__device__ __forceinline__ void recon_end(const CaseDev &C, int dir, long pair, int e, const double w[6]) {
+  const SweepGeom &S = dir ? C.Sy : C.Sx;
+  const int nv = C.G.nv, N = S.N, nl = S.nlines;
+  const int q = (int)(pair % 2), v = (int)((pair / 2) % nv), l = (int)((pair / 2) / nv);
+  const int k = e ? N : 0;
+  double *const *io = dir ? C.iy : C.ix;
+  const long at = ((long)v * nl + l) * (N + 1) + k;
+  double a, b, c, xl, xr;
+  row_coeffs<KIND>(k, N, true, C.R, w[0], w[1], w[2], w[3], w[4], w[5], a, b, c, xl);
+  row_coeffs<KIND>(k, N, false, C.R, w[0], w[1], w[2], w[3], w[4], w[5], a, b, c, xr);
+  double *ends = C.ends + 4 * ((dir ? recon_pairs(C.Sx, nv) : 0) + pair);
+  ends[e] = xl;
+  ends[2 + e] = xr;
+  if (C.paired) {
+    io[q][at] = q ? 0.5 * (xl + xr) : 0.5 * (xr - xl);
+  } else {
+    io[2 * q][at] = xl;
+    io[2 * q + 1][at] = xr;
+  }
+}
+
+__host__ __device__ inline long end_items(const CaseDev &C) {
+  return C.R.crweno && !C.R.characteristic
+             ? 2 * (recon_pairs(C.Sx, C.G.nv) + (C.G.ndims == 2 ? recon_pairs(C.Sy, C.G.nv) : 0))
+             : 0;
+}
+
+// item t of the ends; from_flux: the flux at the six positions is in memory,
+// else it is formed here
+__device__ __forceinline__ void recon_ends_item(const CaseDev &C, long t, int only, bool from_flux) {
+  if (t >= end_items(C)) return;
+  const int nv = C.G.nv;
+  const long nx = 2 * recon_pairs(C.Sx, nv);
+  const int dir = t < nx ? 0 : 1;
+  const long pair = (dir ? t - nx : t) >> 1;
+  const int e = (int)(t & 1), q = (int)(pair % 2), v = (int)((pair / 2) % nv), l = (int)((pair / 2) / nv);
+  if (only && (dir != ((only >> 3) & 1) || q != ((only >> 2) & 1))) return;
+  const SweepGeom &S = dir ? C.Sy : C.Sx;
+  const long pl = S.plane, at = S.base + (long)l * S.line_stride + (e ? S.N : 0) - 3;
+  const double *u = (dir ? C.UT : C.U) + at, *f = (dir ? C.flux_y : C.flux_x) + at;
+  double w[6];
+#pragma unroll
+  for (int p = 0; p < 6; p++) {
+    if (q == 0) {
+      w[p] = u[v * pl + p];
+    } else if (from_flux) {
+      w[p] = f[v * pl + p];
+    } else {
+      double y = 0.0;
+      const int nf = C.model == 1 ? 3 : 4;
+      point_flux(C.model, dir, C.P.gamma, nf + 1, [&](int m) { return u[(m < nf ? m : v) * pl + p]; },
+                 [&](int m, double x) {
+                   if (m == (v < nf ? v : nf)) y = x;
+                 });
+      w[p] = y;
+    }
+  }
+  switch (C.R.kind) {
+    case 1: recon_end<1>(C, dir, pair, e, w); break;
+    case 2: recon_end<2>(C, dir, pair, e, w); break;
+    case 3: recon_end<3>(C, dir, pair, e, w); break;
+    default: recon_end<0>(C, dir, pair, e, w); break;
+  }
+}
+
+// the end interfaces alone, from given arrays (the operators)
+__global__ void __launch_bounds__(256) k_recon_ends(CASE_ARGS) {
   CASE_PREAMBLE
-  if (stage >= C.nstages) return;
+  if ((stage & 0xFF) < C.nstages) recon_ends_item(C, t, stage >> 8, true);
+}
+
+__host__ __device__ inline long flux_items(const CaseDev &C) {
+  return (long)(C.Sx.N + 2 * C.Sx.g) * C.Sx.nlines +
+         (C.G.ndims == 2 ? (long)(C.Sy.N + 2 * C.Sy.g) * C.Sy.nlines : 0);
+}
+
+__device__ __forceinline__ void flux_item(const CaseDev &C, long t) {
   const long nX = (long)(C.Sx.N + 2 * C.Sx.g) * C.Sx.nlines;
   const long nY = (C.G.ndims == 2) ? (long)(C.Sy.N + 2 * C.Sy.g) * C.Sy.nlines : 0;
   if (t >= nX + nY) return;
@@ -273,39 +371,27 @@ __global__ void __launch_bounds__(256) k_flux(CASE_ARGS) {
   }
 }
 
-// The two end interfaces (0 and N) of the line systems, a thread per pair of
-// systems and end: WENO5 values on identity rows
-// (Interp1PrimFifthOrderCRWENO.c:132-201 with the WENO5 weights at the ends).
-// The raw values go to the case's `ends` table for the line solves, and, in
-// paired mode their combination, to the interface arrays.
-template <int KIND>
-__device__ __forceinline__ double end_value(const CaseDev &C, const SweepGeom &S, const double *src, bool left, int k) {
-  double a_, b_, c_, x_;
-  row_coeffs<KIND>(k, S.N, left, C.R, src[k - 3], src[k - 2], src[k - 1], src[k], src[k + 1], src[k + 2], a_, b_, c_,
-                   x_);
-  return x_;
+// What the line-system schemes need of the stage state before their solves:
+// the viscous fluxes, the systems' end values and the cell fluxes, each in
+// blocks of its own (the first two take longest).  One launch of a few
+// microseconds' work costs as much again; with three, and the viscous fluxes on
+// a second stream (whose fork and join cost 10 us a stage), 128 x 97 took 6.26 ms
+// where it takes 4.77, cavity 128 x 128 (k_weno's launch) 4.15 -> 2.54.
+__global__ void __launch_bounds__(256) k_flux(CASE_ARGS) {
+  CASE_PREAMBLE
+  if (stage >= C.nstages) return;
+  __shared__ Prims prims;
+  const int bid = (int)(blockIdx.x - firstblock[cidx]);
+  const int nvis = viscous_blocks(C), nends = (int)((end_items(C) + TB - 1) / TB);
+  if (bid < nvis) viscous_tile(C, bid, prims);
+  else if (bid < nvis + nends) recon_ends_item(C, t - (long)nvis * TB, 0, false);
+  else flux_item(C, t - (long)(nvis + nends) * TB);
 }
 
-template <int KIND>
-__device__ __forceinline__ void recon_end(const CaseDev &C, int dir, long pair, int e) {
-  const SweepGeom &S = dir ? C.Sy : C.Sx;
-  const int nv = C.G.nv, N = S.N, nl = S.nlines;
-  const int q = (int)(pair % 2), v = (int)((pair / 2) % nv), l = (int)((pair / 2) / nv);
-  const double *src = (q == 0 ? (dir ? C.UT : C.U) : (dir ? C.flux_y : C.flux_x)) + (long)v * S.plane + S.base +
-                      (long)l * S.line_stride;
-  const int k = e ? N : 0;
-  double *const *io = dir ? C.iy : C.ix;
-  const long at = ((long)v * nl + l) * (N + 1) + k;
-  const double xl = end_value<KIND>(C, S, src, true, k), xr = end_value<KIND>(C, S, src, false, k);
-  double *ends = C.ends + 4 * ((dir ? recon_pairs(C.Sx, nv) : 0) + pair);
-  ends[e] = xl;
-  ends[2 + e] = xr;
-  if (C.paired) {
-    io[q][at] = q ? 0.5 * (xl + xr) : 0.5 * (xr - xl);
-  } else {
-    io[2 * q][at] = xl;
-    io[2 * q + 1][at] = xr;
-  }
+// the cell fluxes alone, of any case (the operators)
+__global__ void __launch_bounds__(256) k_flux_all(CASE_ARGS) {
+  CASE_PREAMBLE
+  if (stage < C.nstages) flux_item(C, t);
 }
 
 // ---------------------------------------------------------------------------
@@ -1189,26 +1275,6 @@ __global__ void __launch_bounds__(kLongTeam) k_lsolve(CASE_ARGS) {
   }
 }
 
-__global__ void __launch_bounds__(256) k_recon_ends(CASE_ARGS) {
-  CASE_PREAMBLE
-  if ((stage & 0xFF) >= C.nstages) return;
-  const int nv = C.G.nv;
-  const long npx = recon_pairs(C.Sx, nv), npy = C.G.ndims == 2 ? recon_pairs(C.Sy, nv) : 0;
-  if (t >= 2 * (npx + npy)) return;
-  const int dir = t < 2 * npx ? 0 : 1;
-  const long q = dir ? t - 2 * npx : t;
-  const long pair = q >> 1;
-  const int e = (int)(q & 1);
-  const int only = stage >> 8;
-  if (only && (dir != ((only >> 3) & 1) || (pair & 1) != ((only >> 2) & 1))) return;
-  switch (C.R.kind) {
-    case 1: recon_end<1>(C, dir, pair, e); break;
-    case 2: recon_end<2>(C, dir, pair, e); break;
-    case 3: recon_end<3>(C, dir, pair, e); break;
-    default: recon_end<0>(C, dir, pair, e); break;
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Upwinding.
 //  NS2D Roe: NavierStokes2DUpwind.c:26-92 with navierstokes2d.h:115-311 --
@@ -1391,152 +1457,6 @@ __global__ void __launch_bounds__(256) k_bflux(CASE_ARGS) {
     local += step[1] * C.dS[d];
   }
   C.tbi[v] += 1.0 * local;
-}
-
-// ---------------------------------------------------------------------------
-// Parabolic term (navierstokes2d): NavierStokes2DParabolicFunction.c:41-204.
-// Serial-run semantics: d/dx of Q is evaluated on interior rows only and d/dy
-// on interior columns only (FirstDerivativeFourthOrder.c:66-71 loops over the
-// interior lines of the other dimension); elsewhere the derivative is zero.
-// ---------------------------------------------------------------------------
-struct Prim {
-  double vx, vy, T;
-};
-__device__ __forceinline__ Prim prim_at(long plane, double gam, const double *U, long p) {
-  const double rho = U[p];
-  const double vx = (rho == 0) ? 0 : U[plane + p] / rho, vy = (rho == 0) ? 0 : U[2 * plane + p] / rho;
-  const double e = U[3 * plane + p];
-  const double vsq = (vx * vx) + (vy * vy);
-  const double P = (e - 0.5 * rho * vsq) * (gam - 1.0);
-  Prim r;
-  r.vx = vx;
-  r.vy = vy;
-  r.T = gam * P / rho;
-  return r;
-}
-
-// FirstDerivativeFourthOrder.c:39-132 (par4) / FirstDerivativeFirstOrder.c (bias +1)
-// of the three primitives at position i of a line of N interior points, P(k)
-// the primitives at position k (component c: P(k, c)).
-template <class F>
-__device__ __forceinline__ void deriv_prim(int g, bool par4, int i, int N, F P, double out[3]) {
-#pragma unroll
-  for (int c = 0; c < 3; c++) {
-    if (par4) {
-      const double t12 = 1.0 / 12.0;
-      if (i == -g)
-        out[c] = (-25 * P(i, c) + 48 * P(i + 1, c) - 36 * P(i + 2, c) + 16 * P(i + 3, c) - 3 * P(i + 4, c)) * t12;
-      else if (i == -g + 1)
-        out[c] = (-3 * P(i - 1, c) - 10 * P(i, c) + 18 * P(i + 1, c) - 6 * P(i + 2, c) + P(i + 3, c)) * t12;
-      else if (i == N + g - 2)
-        out[c] = (-P(i - 3, c) + 6 * P(i - 2, c) - 18 * P(i - 1, c) + 10 * P(i, c) + 3 * P(i + 1, c)) * t12;
-      else if (i == N + g - 1)
-        out[c] = (3 * P(i - 4, c) - 16 * P(i - 3, c) + 36 * P(i - 2, c) - 48 * P(i - 1, c) + 25 * P(i, c)) * t12;
-      else
-        out[c] = (P(i - 2, c) - 8 * P(i - 1, c) + 8 * P(i + 1, c) - P(i + 2, c)) * t12;
-    } else if (i == -g) {
-      out[c] = P(i + 1, c) - P(i, c);
-    } else if (i == N + g - 1) {
-      out[c] = P(i, c) - P(i - 1, c);
-    } else {
-      out[c] = 1.0 * P(i + 1, c) - 1.0 * P(i, c) + 0.0 * P(i - 1, c);
-    }
-  }
-}
-
-// Viscous fluxes (NavierStokes2DParabolicFunction.c:112-143 and :155-186),
-// Sutherland viscosity and the conductivity law of navierstokes2d.h:315-331
-// (raiseto(x,1.5) = exp(1.5 log x), include/math_ops.h:40), from the derivatives
-// of velocity and temperature, each scaled by dxinv
-// (NavierStokes2DParabolicFunction.c:96-106).  With the derivative exchange
-// along a periodic dimension (xchg, MPIExchangeBoundariesnD.c:109-167 as called
-// at NavierStokes2DParabolicFunction.c:91-94), a ghost point of an interior
-// line across that dimension takes the unscaled derivatives of its periodic
-// image, scaled by its own dxinv; corners are not exchanged, and never read.
-// FV planes: 0..2 = x-flux components 1..3, 3..5 = y-flux components 1..3.
-//
-// A 32 x 8 tile of ghosted points per block.  Bound by latency on small grids
-// and by HBM on large ones: the primitives of the tile and of the four points
-// beside it (one-sided stencils reach that far) are formed once into LDS, 2.25
-// divisions chains a thread instead of 21 in two passes with the derivatives
-// in memory between them.
-constexpr int kVisX = 32, kVisY = 8, kVisH = 4;
-__global__ void __launch_bounds__(256) k_viscous(CASE_ARGS) {
-  CASE_PREAMBLE
-  (void)t;
-  if (stage >= C.nstages) return;
-  const Grid &G = C.G;
-  const PhysParams &P = C.P;
-  __shared__ double pr[3][kVisY + 2 * kVisH][kVisX + 2 * kVisH];
-  const int tiles = (G.nxg + kVisX - 1) / kVisX;
-  const int b = (int)(blockIdx.x - firstblock[cidx]);
-  const int I0 = (b % tiles) * kVisX, J0 = (b / tiles) * kVisY;  // ghosted indices
-  const double gam = P.gamma;
-  auto fill = [&](int a, int c) {  // LDS position (row a, column c)
-    const int I = I0 + c - kVisH, J = J0 + a - kVisH;
-    if (I < 0 || I >= G.nxg || J < 0 || J >= G.nyg) return;
-    const Prim q = prim_at(G.plane, gam, C.U, (long)J * G.nxg + I);
-    pr[0][a][c] = q.vx;
-    pr[1][a][c] = q.vy;
-    pr[2][a][c] = q.T;
-  };
-  const int tx = threadIdx.x & (kVisX - 1), ty = threadIdx.x / kVisX;
-  fill(ty + kVisH, tx + kVisH);
-  // four rows below and four above, then the columns beside the tile
-  fill(ty < kVisH ? ty : ty + kVisY, tx + kVisH);
-  if (threadIdx.x < 2 * kVisH * kVisY) {
-    const int c = threadIdx.x & (2 * kVisH - 1), r = threadIdx.x / (2 * kVisH);
-    fill(r + kVisH, c < kVisH ? c : c + kVisX);
-  }
-  lds_barrier();
-  const int I = I0 + tx, J = J0 + ty;
-  if (I >= G.nxg || J >= G.nyg) return;
-  const int i = I - G.g, j = J - G.g;
-  const bool iin = i >= 0 && i < G.nx, jin = j >= 0 && j < G.ny;
-  if (!iin && !jin) return;  // corners are never read
-  double dx[3] = {0, 0, 0}, dy[3] = {0, 0, 0};
-  // derivatives along x on interior rows, along y on interior columns
-  const bool ex = P.xchg[0] && jin && !iin, ey = P.xchg[1] && iin && !jin;
-  auto far = [&](int x, int y, int c) {  // a point outside the tile's reach
-    const Prim q = prim_at(G.plane, gam, C.U, (long)(y + G.g) * G.nxg + (x + G.g));
-    return c == 0 ? q.vx : c == 1 ? q.vy : q.T;
-  };
-  if (ex) {  // both derivatives of the image in x
-    const int si = i < 0 ? i + G.nx : i - G.nx;
-    deriv_prim(G.g, P.par4, si, G.nx, [&](int k, int c) { return far(k, j, c); }, dx);
-    deriv_prim(G.g, P.par4, j, G.ny, [&](int k, int c) { return far(si, k, c); }, dy);
-  } else if (ey) {
-    const int sj = j < 0 ? j + G.ny : j - G.ny;
-    deriv_prim(G.g, P.par4, i, G.nx, [&](int k, int c) { return far(k, sj, c); }, dx);
-    deriv_prim(G.g, P.par4, sj, G.ny, [&](int k, int c) { return far(i, k, c); }, dy);
-  } else {
-    if (jin)
-      deriv_prim(G.g, P.par4, i, G.nx, [&](int k, int c) { return pr[c][ty + kVisH][tx + kVisH + k - i]; }, dx);
-    if (iin)
-      deriv_prim(G.g, P.par4, j, G.ny, [&](int k, int c) { return pr[c][ty + kVisH + k - j][tx + kVisH]; }, dy);
-  }
-  const double sx = C.dxinv[G.g + i], sy = C.dxinv[(G.nx + 2 * G.g) + G.g + j];
-  const double ux = dx[0] * sx, vx = dx[1] * sx, Tx = dx[2] * sx;
-  const double uy = dy[0] * sy, vy = dy[1] * sy, Ty = dy[2] * sy;
-  const double qx = pr[0][ty + kVisH][tx + kVisH], qy = pr[1][ty + kVisH][tx + kVisH];
-  const double Td = pr[2][ty + kVisH][tx + kVisH] * P.Tref;
-  const double r15 = exp(1.5 * log(Td / P.T0));
-  const double mu = r15 * (P.T0 + P.TS) / (Td + P.TS);
-  const double kap = r15 * P.kappa_num / (Td + P.TA * exp(-P.TB / Td));
-  const double muRe = mu * P.inv_Re;
-  const double kc = kap * P.inv_Re * P.inv_gm1 * P.inv_Pr;
-  const long pl = (long)G.nxg * G.nyg, p = (long)J * G.nxg + I;
-  double *FV = C.FV;
-  const double txx = P.two_third * muRe * (2 * ux - vy);
-  const double txy = muRe * (uy + vx);
-  FV[p] = txx;
-  FV[pl + p] = txy;
-  FV[2 * pl + p] = qx * txx + qy * txy + kc * Tx;
-  const double tyx = muRe * (uy + vx);
-  const double tyy = P.two_third * muRe * (-ux + 2 * vy);
-  FV[3 * pl + p] = tyx;
-  FV[4 * pl + p] = tyy;
-  FV[5 * pl + p] = qx * tyx + qy * tyy + kc * Ty;
 }
 
 // ---------------------------------------------------------------------------
@@ -2105,7 +2025,7 @@ static const char *kKNames[K_NCLASS] = {"stage_bc", "ghost",  "flux",    "recon_
                                         "recon_4",  "recon_6", "recon_8", "recon_10", "recon_12", "recon_14", "recon_16",
                                         "recon_w10", "recon_w12", "recon_w16", "long_rows", "long_solve",
                                         "cw_rows", "cw_solve", "weno", "upwind", "bflux",
-                                        "viscous", "assemble", "update", "flux_all"};
+                                        "assemble", "update", "flux_all"};
 const char *kclass_name(int k) { return kKNames[k]; }
 
 int cw_row_fields(int nflow, int nv) { return nflow * nflow + 16 * nv; }
@@ -2208,25 +2128,24 @@ void case_blocks(const CaseDev &c, int blocks[K_NCLASS]) {
   // the tile kernels' counts are padded to a multiple of eight, so that every
   // case's tiles start on one and can be taken in xcd_order
   auto pad8 = [](int n) { return (n + 7) & ~7; };
-  blocks[K_STAGE] = pad8(two ? ((G.nx + st - 1) / st) * ((G.ny + st - 1) / st) * G.nv : nb((long)G.nx * G.nv));
   blocks[K_GHOST] = nb(ghost_points(G) * G.nv);
+  blocks[K_STAGE] = stage_blocks(G, st) + blocks[K_GHOST];
   auto faces = [&](long per) {  // blocks of `per` interfaces, the sweeps apart
     const long x = (long)(c.Sx.N + 1) * c.Sx.nlines, y = two ? (long)(c.Sy.N + 1) * c.Sy.nlines : 0;
     return (int)((x + per - 1) / per + (y + per - 1) / per);
   };
   const int nf = c.model == 1 ? 3 : 4;
   const bool weno = !c.R.crweno && !c.unit;
-  blocks[K_FLUXALL] = nb((long)(c.Sx.N + 2 * c.Sx.g) * c.Sx.nlines + (two ? (long)(c.Sy.N + 2 * c.Sy.g) * c.Sy.nlines : 0));
-  blocks[K_FLUX] = weno ? 0 : blocks[K_FLUXALL];
-  blocks[K_WENO] = weno ? faces(kWenoTile) : 0;
+  blocks[K_FLUXALL] = nb(flux_items(c));
+  blocks[K_ENDS] = nb(end_items(c));
+  blocks[K_FLUX] = weno ? 0 : viscous_blocks(c) + blocks[K_ENDS] + blocks[K_FLUXALL];
+  blocks[K_WENO] = weno ? viscous_blocks(c) + faces(kWenoTile) : 0;
   blocks[K_CWROWS] = blocks[K_CWSOLVE] = blocks[K_LROWS] = blocks[K_LSOLVE] = 0;
-  blocks[K_ENDS] = 0;
   for (int v = 0; v < kNRecon; v++) blocks[K_RECON + v] = 0;
   if (c.R.crweno && c.R.characteristic) {
     blocks[K_CWROWS] = nb((long)(c.Sx.N + 1) * c.Sx.nlines + (two ? (long)(c.Sy.N + 1) * c.Sy.nlines : 0));
     blocks[K_CWSOLVE] = nb(cw_x_span(c, nf) + (two ? cw_items(c.Sy, G.nv, nf) : 0));
   } else if (c.R.crweno) {
-    blocks[K_ENDS] = nb(2 * (recon_pairs(c.Sx, G.nv) + (two ? recon_pairs(c.Sy, G.nv) : 0)));
     for (int v = 0; v < kNRecon; v++) {
       if (recon_in(c.Sx, kRecon[v].rows, kRecon[v].wide)) blocks[K_RECON + v] += recon_sweep_blocks(c.Sx, G.nv);
       if (two && recon_in(c.Sy, kRecon[v].rows, kRecon[v].wide)) blocks[K_RECON + v] += recon_sweep_blocks(c.Sy, G.nv);
@@ -2236,8 +2155,6 @@ void case_blocks(const CaseDev &c, int blocks[K_NCLASS]) {
   }
   blocks[K_UPWIND] = weno ? 0 : nb((long)(c.Sx.N + 1) * c.Sx.nlines + (two ? (long)(c.Sy.N + 1) * c.Sy.nlines : 0));
   blocks[K_BFLUX] = c.cons ? 1 : 0;
-  const bool visc = two && c.P.viscous;
-  blocks[K_VISCOUS] = visc ? ((G.nxg + kVisX - 1) / kVisX) * ((G.nyg + kVisY - 1) / kVisY) : 0;
   blocks[K_ASSEMBLE] = pad8(two ? ((G.nx + 31) / 32) * ((G.ny + 31) / 32) * G.nv : nb((long)G.nx * G.nv));
   blocks[K_UPDATE] = nb((long)G.nx * G.ny * G.nv);
 }
@@ -2252,7 +2169,8 @@ static KernFn class_kernel(const Plan &pl, int cls) {
   switch (cls) {
     case K_STAGE: return pl.stage64 ? k_stage64 : k_stage;
     case K_GHOST: return k_ghost;
-    case K_FLUX: case K_FLUXALL: return k_flux;
+    case K_FLUX: return k_flux;
+    case K_FLUXALL: return k_flux_all;
     case K_ENDS: return k_recon_ends;
     case K_LROWS: return k_lrows;
     case K_LSOLVE: return k_lsolve;
@@ -2261,7 +2179,6 @@ static KernFn class_kernel(const Plan &pl, int cls) {
     case K_WENO: return weno_kernel();
     case K_UPWIND: return k_upwind;
     case K_BFLUX: return k_bflux;
-    case K_VISCOUS: return k_viscous;
     case K_ASSEMBLE: return k_assemble;
     default: return k_update;
   }
@@ -2277,32 +2194,16 @@ static void run(int cls, const CaseDev *d, const Plan &pl, int s, hipStream_t st
   if (mark) mark(ctx, cls, false, st);
 }
 
-// k_viscous reads only the stage state (after k_ghost) and writes only FV, which
-// nothing before k_assemble reads; the reconstruction / upwinding chain neither
-// reads nor writes FV.
-void launch_stage(const CaseDev *d, const Plan &pl, int s, hipStream_t st, MarkFn mark, void *ctx,
-                  const StageFork *fk, int last) {
-  auto R = [&](int cls, hipStream_t on) {
-    if (cls <= last || cls == K_FLUXALL) run(cls, d, pl, s, on, mark, ctx);
-  };
-  R(K_STAGE, st);
-  R(K_GHOST, st);
-  R(last == K_FLUX ? K_FLUXALL : K_FLUX, st);
-  R(K_ENDS, st);
-  const bool fork = fk && fk->side && last >= K_ASSEMBLE && pl.nblocks[K_VISCOUS] > 0;
-  if (fork) {
-    hipEventRecord(fk->fork, st);
-    hipStreamWaitEvent(fk->side, fk->fork, 0);
-    R(K_VISCOUS, fk->side);
-    hipEventRecord(fk->join, fk->side);
+void launch_stage(const CaseDev *d, const Plan &pl, int s, hipStream_t st, MarkFn mark, void *ctx, int last) {
+  run(K_STAGE, d, pl, s, st, mark, ctx);
+  if (last <= K_GHOST) return;
+  if (last == K_FLUX) {
+    run(K_FLUXALL, d, pl, s, st, mark, ctx);
+    return;
   }
-  for (int cls = K_RECON; cls <= K_BFLUX; cls++) R(cls, st);
-  if (fork) {
-    hipStreamWaitEvent(st, fk->join, 0);
-  } else {
-    R(K_VISCOUS, st);
-  }
-  R(K_ASSEMBLE, st);
+  run(K_FLUX, d, pl, s, st, mark, ctx);
+  for (int cls = K_RECON; cls <= K_ASSEMBLE; cls++)
+    if (cls <= last) run(cls, d, pl, s, st, mark, ctx);
 }
 
 void launch_update(const CaseDev *d, const Plan &pl, hipStream_t st) { run(K_UPDATE, d, pl, 0, st, nullptr, nullptr); }

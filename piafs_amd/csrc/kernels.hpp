@@ -153,12 +153,13 @@ struct CaseDev {
   int *status;   // bit 0: a zero pivot met in a line solve (tridiagLU.c:139-142 returns -1)
 };
 
-// Kernel classes launched per RK stage (plus the final update).  K_FLUXALL is
-// K_FLUX for every case, those of K_WENO (which form their own fluxes) among
-// them, and runs only when the fluxes themselves are asked for.
+// Kernel classes launched per RK stage (plus the final update).  K_STAGE fills
+// the ghost points too and K_FLUX the line systems' end values and the viscous
+// fluxes; K_GHOST, K_ENDS and K_FLUXALL (the cell fluxes of every case, those
+// of K_WENO among them, which forms its own) do one thing for the operators.
 enum KClass {
   K_STAGE = 0, K_GHOST, K_FLUX, K_ENDS, K_RECON, K_LROWS = K_RECON + 10, K_LSOLVE, K_CWROWS, K_CWSOLVE, K_WENO, K_UPWIND,
-  K_BFLUX, K_VISCOUS, K_ASSEMBLE, K_UPDATE, K_FLUXALL,
+  K_BFLUX, K_ASSEMBLE, K_UPDATE, K_FLUXALL,
   K_NCLASS
 };
 const char *kclass_name(int k);
@@ -223,25 +224,16 @@ bool stage_tile_64(const CaseDev &c);
 int cw_row_fields(int nflow, int nv);
 int cw_back_fields(int nflow, int nv);
 
-// A second stream for the branch of a stage that does not depend on the
-// reconstruction: the viscous derivatives and fluxes (HBM-bound) run beside
-// the reconstruction (FP64-VALU-bound).  The branch forks from the main
-// stream before the reconstruction and joins it before the assembly.
-struct StageFork {
-  hipStream_t side = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr;
-};
-
 // Stage s of the RK step for every case in the plan: stage state + BCs,
-// fluxes, reconstruction, upwinding, divergence, viscous terms, assembly of
-// Udot[s].  Times: stage time = *time + c[s]*dt of each case.  With `fk`
-// the viscous branch runs on fk->side.  `mark` (per-class timing) is called
-// before and after each launch with the stream the launch goes to.
+// fluxes and viscous terms, reconstruction, upwinding, assembly of Udot[s].
+// Times: stage time = *time + c[s]*dt of each case.  `mark` (per-class timing)
+// is called before and after each launch with the stream the launch goes to.
 typedef void (*MarkFn)(void *ctx, int cls, bool begin, hipStream_t st);
-// With `last` < K_NCLASS only the classes up to `last` run (in launch order,
-// which is the order of KClass), for the per-operator entry points.
+// With `last` < K_NCLASS only the work up to that class is done (in launch
+// order, which is the order of KClass), for the per-operator entry points:
+// K_GHOST ends with the stage state, K_FLUX with the cell fluxes.
 void launch_stage(const CaseDev *d_cases, const Plan &plan, int s, hipStream_t st, MarkFn mark, void *mark_ctx,
-                  const StageFork *fk = nullptr, int last = K_NCLASS);
+                  int last = K_NCLASS);
 // u += dt*b_s*Udot_s for every stage, time += dt.
 void launch_update(const CaseDev *d_cases, const Plan &plan, hipStream_t st);
 

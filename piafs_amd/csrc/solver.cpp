@@ -380,13 +380,6 @@ int Engine::init(int dev) {
   device = dev;
   HIPCHK(hipSetDevice(device));
   HIPCHK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-  // PIAFS_AMD_ONE_STREAM=1 keeps every launch of a step on one stream
-  const char *one = getenv("PIAFS_AMD_ONE_STREAM");
-  if (!(one && one[0] == '1')) {
-    HIPCHK(hipStreamCreateWithFlags(&fork.side, hipStreamNonBlocking));
-    HIPCHK(hipEventCreateWithFlags(&fork.fork, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&fork.join, hipEventDisableTiming));
-  }
   return 0;
 }
 
@@ -481,7 +474,7 @@ int Engine::build() {
 static void mark_cb(void *ctx, int cls, bool begin, hipStream_t st) { ((Engine *)ctx)->mark(cls, begin, st); }
 
 // Events bracketing one launch of class cls, recorded on the stream the launch
-// goes to (the viscous branch runs on the side stream beside the main one).
+// goes to.
 void Engine::mark(int cls, bool begin, hipStream_t st) {
   if (!profiling) return;
   if (begin) {
@@ -504,7 +497,7 @@ void Engine::enqueue_step() {
   int ns = 0;
   for (Case *c : cases) ns = std::max(ns, c->cfg.nstages);
   for (int s = 0; s < ns; s++)
-    launch_stage(d_cases, plan, s, stream, profiling ? mark_cb : nullptr, this, fork.side ? &fork : nullptr);
+    launch_stage(d_cases, plan, s, stream, profiling ? mark_cb : nullptr, this);
   if (profiling) mark(K_UPDATE, true, stream);
   launch_update(d_cases, plan, stream);
   if (profiling) mark(K_UPDATE, false, stream);
@@ -607,7 +600,7 @@ int Engine::autotune(const int *cands, int ncand, int reps, int *best_rows, doub
 int Engine::stage_only(int s, int last) {
   HIPCHK(hipSetDevice(device));
   if (!built) return fail(-1, "the ensemble plan is not built");
-  launch_stage(d_cases, plan, s, stream, nullptr, nullptr, nullptr, last);
+  launch_stage(d_cases, plan, s, stream, nullptr, nullptr, last);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -637,12 +630,8 @@ Engine::~Engine() {
     hipEventDestroy(e.first);
     hipEventDestroy(e.second);
   }
-  if (fork.side) hipStreamSynchronize(fork.side);
   if (owns_cases)
     for (Case *c : cases) delete c;
-  if (fork.side) hipStreamDestroy(fork.side);
-  if (fork.fork) hipEventDestroy(fork.fork);
-  if (fork.join) hipEventDestroy(fork.join);
   if (stream) hipStreamDestroy(stream);
 }
 

@@ -1,6 +1,6 @@
 // The hyperbolic interface flux of the schemes without line systems (WENO5 and
 // upw5, component-wise or characteristic) in one pass over the stage state.
-#include "device.hpp"
+#include "viscous.hpp"
 
 namespace piafs {
 
@@ -212,7 +212,8 @@ __device__ __forceinline__ void weno_tile(const CaseDev &C, long item, int uw, R
 // Reconstruction of the state and of its flux, and the upwinding, at every
 // interface of both sweeps, from the stage state alone: cell fluxes are formed
 // at the six stencil positions, so neither they nor the reconstructed values
-// exist in memory.  Bound by FP64 issue on large grids and by the latency of
+// exist in memory.  The viscous fluxes, which need the stage state alone too,
+// have the launch's first blocks.  Bound by FP64 issue on large grids and by the latency of
 // the FP64 chains on small ones.  A block of four waves takes 64 interfaces, a
 // wave a variable at a time: with a thread taking an interface through every
 // variable the kernel needs 236 registers (characteristic 318), which leaves
@@ -225,10 +226,19 @@ __device__ __forceinline__ void weno_tile(const CaseDev &C, long item, int uw, R
 __global__ void __launch_bounds__(256) k_weno(CASE_ARGS) {
   CASE_PREAMBLE
   if (stage >= C.nstages) return;
-  __shared__ Rows sh;
+  __shared__ union Lds {
+    Rows rows;
+    Prims prims;
+  } lds;
+  const int nvis = viscous_blocks(C);
+  if ((int)(blockIdx.x - firstblock[cidx]) < nvis) {
+    viscous_tile(C, (int)(blockIdx.x - firstblock[cidx]), lds.prims);
+    return;
+  }
+  Rows &sh = lds.rows;
   const long nX = (long)(C.Sx.N + 1) * C.Sx.nlines;
   const int nbx = (int)((nX + 63) / 64);
-  const int bid = (int)(blockIdx.x - firstblock[cidx]);
+  const int bid = (int)(blockIdx.x - firstblock[cidx]) - nvis;
   const int dir = bid < nbx ? 0 : 1;
   const long item = (long)(dir ? bid - nbx : bid) * 64 + (threadIdx.x & 63);
   const int uw = bid & 3;  // in turn, since a block's waves sit on the SIMDs in order
