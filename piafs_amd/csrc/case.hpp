@@ -85,6 +85,7 @@ struct Engine {
   ~Engine();
   int init(int dev);
   int add(Case *c);
+  std::vector<CaseDev> lines;  // descriptors of the members when all are 1D cases that take whole-step launches
   bool built = false;          // plan and descriptor table valid for the member set
   const CaseDev *override_desc = nullptr;  // one-member engine: descriptor to use instead of the case's
   int build();                 // descriptor table and plans for the current member set

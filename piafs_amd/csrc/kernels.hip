@@ -6,6 +6,7 @@
 // and the library is compiled without floating-point contraction so that the
 // rounding of every +, -, *, / and sqrt matches the reference build.
 #include "device.hpp"
+#include "boundary.hpp"
 #include "teams.hpp"
 #include "viscous.hpp"
 
@@ -40,123 +41,6 @@ __device__ __forceinline__ double stage_value(const CaseDev &C, int s, long p) {
   return val;
 }
 
-// ---------------------------------------------------------------------------
-// Boundary conditions as a gather: each ghost point finds the last zone (in
-// list order) that sets its variable and evaluates that zone's rule on the
-// stage values of the interior points it reads.  The zones read interior
-// points only, so list order matters only where zones overlap.
-//  periodic BCPeriodic.c:22-62, extrapolate BCExtrapolate.c:16-51,
-//  dirichlet BCDirichlet.c:16-45, reflect BCReflect.c:17-50, walls
-//  BCSlipWall.c:24-135 / BCNoslipWall.c:22-80, BCSubsonicInflow.c:22-90,
-//  BCSubsonicOutflow.c:21-78, BCSubsonicAmbivalent.c:30-125,
-//  BCSupersonicInflow.c:26-80, BCSupersonicOutflow.c:25-80.
-// A ghost point no zone sets keeps the value the reference never changes
-// from its zero initialisation.
-// ---------------------------------------------------------------------------
-// does zone z set variable v (the flow BCs exist for ndims 2 only, the slip
-// wall also for ndims 1; walls and outflows leave passive scalars alone)
-__device__ __forceinline__ bool zone_sets(const Zone &z, int v, int ndims) {
-  switch (z.kind) {
-    case Z_PERIODIC: case Z_EXTRAPOLATE: case Z_DIRICHLET: case Z_REFLECT: return true;
-    case Z_SPONGE: return false;
-    case Z_SLIP_WALL: return ndims == 1 ? v < 3 : v < 4;
-    case Z_SUBSONIC_INFLOW: case Z_SUPERSONIC_INFLOW: return ndims == 2;
-    default: return ndims == 2 && v < 4;
-  }
-}
-
-
-// stage values of the four flow variables at point p
-__device__ __forceinline__ void stage_flow(const CaseDev &C, int s, long p, double u[4]) {
-#pragma unroll
-  for (int m = 0; m < 4; m++) u[m] = stage_value(C, s, (long)m * C.G.plane + p);
-}
-
-// value of variable v at ghost point (i, j) for stage s
-__device__ double ghost_value(const CaseDev &C, int s, int v, int i, int j) {
-  const Grid &G = C.G;
-  const int nd = G.ndims;
-  int d, face, gd, o;
-  if (i < 0 || i >= G.nx) {
-    d = 0; face = (i < 0) ? 1 : -1; gd = i; o = j;
-    if (nd == 2 && (j < 0 || j >= G.ny)) return 0.0;  // corner: no zone reaches it
-  } else {
-    d = 1; face = (j < 0) ? 1 : -1; gd = j; o = i;
-  }
-  const int N = d ? G.ny : G.nx, od = 1 - d;
-  int z = C.nzones - 1;
-  for (; z >= 0; z--) {
-    const Zone &Z = C.zones[z];
-    if (Z.kind == Z_SPONGE || Z.dim != d || Z.face != face || !zone_sets(Z, v, nd)) continue;
-    if (nd == 2 && (o < Z.is[od] || o >= Z.ie[od])) continue;
-    break;
-  }
-  if (z < 0) return 0.0;
-  const Zone &Z = C.zones[z];
-  auto at = [&](int a, int b) -> long {  // ghosted offset of (index along d, index across d)
-    const int ii = d ? b : a, jj = d ? a : b;
-    return (long)(jj + G.gy) * G.nxg + (ii + G.g);
-  };
-  if (Z.kind == Z_DIRICHLET) return C.bcvals[Z.vals + v];
-  if (Z.kind == Z_PERIODIC) {
-    // the source index across d is taken without the zone offset (BCPeriodic.c:44-52)
-    const int src = (face == 1) ? gd + N : gd - N;
-    return stage_value(C, s, (long)v * G.plane + at(src, nd == 2 ? o - Z.is[od] : 0));
-  }
-  const int mir = (face == 1) ? -gd - 1 : 2 * N - gd - 1;
-  const long pm = at(mir, nd == 2 ? o : 0);
-  if (Z.kind == Z_EXTRAPOLATE) return stage_value(C, s, (long)v * G.plane + pm);
-  if (Z.kind == Z_REFLECT) return (-1.0) * stage_value(C, s, (long)v * G.plane + pm);
-  const double gam = Z.gamma, igm1 = 1.0 / (gam - 1.0);
-  if (nd == 1) {  // slip wall, euler1d
-    const double rho = stage_value(C, s, pm), uvel = stage_value(C, s, G.plane + pm) / rho;
-    const double energy = stage_value(C, s, 2 * G.plane + pm);
-    const double pressure = (energy - 0.5 * rho * uvel * uvel) * (gam - 1.0);
-    const double rg = rho, pg = pressure, ug = 2.0 * Z.vel[0] - uvel;
-    if (v == 0) return rg;
-    if (v == 1) return rg * ug;
-    return igm1 * pg + 0.5 * rg * ug * ug;
-  }
-  if (v >= 4) return C.bcvals[Z.vals + v - 4];  // inflow passive scalars
-  double um[4], rho, uvel, vvel, energy, pressure, rg, ug, vg, pg;
-  if (Z.kind == Z_SUBSONIC_AMBIVALENT) {
-    const double nx = (d == 0 ? 1.0 : 0.0) * (double)face, ny = (d == 1 ? 1.0 : 0.0) * (double)face;
-    const int i1 = (face == 1) ? 0 : N - 1, i2 = (face == 1) ? 1 : N - 2;
-    double u1, v1, u2, v2;
-    stage_flow(C, s, at(i1, o), um);
-    ns2d_flowvar(um, gam, rho, u1, v1, energy, pressure);
-    stage_flow(C, s, at(i2, o), um);
-    ns2d_flowvar(um, gam, rho, u2, v2, energy, pressure);
-    const double vn = (1.5 * u1 - 0.5 * u2) * nx + (1.5 * v1 - 0.5 * v2) * ny;
-    stage_flow(C, s, pm, um);
-    ns2d_flowvar(um, gam, rho, uvel, vvel, energy, pressure);
-    if (vn > 0) { rg = Z.rho; pg = pressure; ug = Z.vel[0]; vg = Z.vel[1]; }
-    else { rg = rho; pg = Z.p; ug = uvel; vg = vvel; }
-  } else {
-    stage_flow(C, s, pm, um);
-    ns2d_flowvar(um, gam, rho, uvel, vvel, energy, pressure);
-    rg = rho; pg = pressure; ug = uvel; vg = vvel;  // supersonic outflow
-    switch (Z.kind) {
-      case Z_SLIP_WALL:
-        if (d == 0) ug = 2.0 * Z.vel[0] - uvel;
-        else vg = 2.0 * Z.vel[1] - vvel;
-        break;
-      case Z_NOSLIP_WALL:
-        ug = 2.0 * Z.vel[0] - uvel;
-        vg = 2.0 * Z.vel[1] - vvel;
-        break;
-      case Z_SUBSONIC_INFLOW: rg = Z.rho; ug = Z.vel[0]; vg = Z.vel[1]; break;
-      case Z_SUBSONIC_OUTFLOW: pg = Z.p; break;
-      case Z_SUPERSONIC_INFLOW: rg = Z.rho; pg = Z.p; ug = Z.vel[0]; vg = Z.vel[1]; break;
-      default: break;
-    }
-  }
-  if (v == 0) return rg;
-  if (v == 1) return rg * ug;
-  if (v == 2) return rg * vg;
-  return igm1 * pg + 0.5 * rg * (ug * ug + vg * vg);
-}
-
 // Ghost points of the stage state, one thread per (variable, ghost point):
 // the g rows below and above the interior (full ghosted width), then the g
 // columns left and right of it (interior height).  Written to both layouts.
@@ -184,7 +68,9 @@ __device__ __forceinline__ void ghost_body(const CaseDev &C, int stage, long t) 
     j = (int)(q % G.ny);
     i = col < G.g ? col - G.g : G.nx + (col - G.g);
   }
-  const double val = ghost_value(C, stage, v, i, j);
+  const double val = ghost_value(C, v, i, j, [&](int m, int a, int b) {
+    return stage_value(C, stage, (long)m * G.plane + (long)(b + G.gy) * G.nxg + (a + G.g));
+  });
   const long pl = (long)v * G.plane;
   C.U[pl + (long)(j + G.gy) * G.nxg + (i + G.g)] = val;
   if (G.ndims == 2) C.UT[pl + (long)(i + G.g) * G.nyg + (j + G.gy)] = val;
@@ -2025,7 +1911,8 @@ static const char *kKNames[K_NCLASS] = {"stage_bc", "ghost",  "flux",    "recon_
                                         "recon_4",  "recon_6", "recon_8", "recon_10", "recon_12", "recon_14", "recon_16",
                                         "recon_w10", "recon_w12", "recon_w16", "long_rows", "long_solve",
                                         "cw_rows", "cw_solve", "weno", "upwind", "bflux",
-                                        "assemble", "update", "flux_all"};
+                                        "assemble", "update", "flux_all",
+                                        "line_4", "line_8", "tube", "tube_back"};
 const char *kclass_name(int k) { return kKNames[k]; }
 
 int cw_row_fields(int nflow, int nv) { return nflow * nflow + 16 * nv; }
@@ -2157,6 +2044,11 @@ void case_blocks(const CaseDev &c, int blocks[K_NCLASS]) {
   blocks[K_BFLUX] = c.cons ? 1 : 0;
   blocks[K_ASSEMBLE] = pad8(two ? ((G.nx + 31) / 32) * ((G.ny + 31) / 32) * G.nv : nb((long)G.nx * G.nv));
   blocks[K_UPDATE] = nb((long)G.nx * G.ny * G.nv);
+  const int line = line_class(c);
+  blocks[K_LINE4] = line == K_LINE4;
+  blocks[K_LINE8] = line == K_LINE8;
+  blocks[K_TUBE] = line == K_TUBE ? (G.nx + tube_core(c.nstages) - 1) / tube_core(c.nstages) : 0;
+  blocks[K_TUBEBACK] = line == K_TUBE ? nb((long)G.nx * G.nv) : 0;
 }
 
 static KernFn class_kernel(const Plan &pl, int cls) {

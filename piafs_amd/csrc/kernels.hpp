@@ -157,9 +157,11 @@ struct CaseDev {
 // the ghost points too and K_FLUX the line systems' end values and the viscous
 // fluxes; K_GHOST, K_ENDS and K_FLUXALL (the cell fluxes of every case, those
 // of K_WENO among them, which forms its own) do one thing for the operators.
+// K_LINE* and K_TUBE advance 1D cases by whole steps (line.hip).
 enum KClass {
   K_STAGE = 0, K_GHOST, K_FLUX, K_ENDS, K_RECON, K_LROWS = K_RECON + 10, K_LSOLVE, K_CWROWS, K_CWSOLVE, K_WENO, K_UPWIND,
   K_BFLUX, K_ASSEMBLE, K_UPDATE, K_FLUXALL,
+  K_LINE4, K_LINE8, K_TUBE, K_TUBEBACK,
   K_NCLASS
 };
 const char *kclass_name(int k);
@@ -208,6 +210,17 @@ __host__ __device__ inline int recon_sweep_blocks(const SweepGeom &S, int nv) {
 __host__ __device__ constexpr int recon_only(int dir, int r) { return (1 | (r & 1) << 1 | (r >> 1) << 2 | dir << 3) << 8; }
 KernFn weno_kernel();        // k_weno (weno.hip)
 constexpr int kWenoTile = 64;  // interfaces of a block
+
+// 1D cases advanced by whole steps: the class that can take a case (-1: none;
+// such a case takes the kernels of a stage), and n steps of a plan whose members
+// all have one.
+constexpr int kTubeVars = 8;
+constexpr size_t kLineLdsMax = 150 * 1024;
+// points of its window a k_tube block keeps
+__host__ __device__ constexpr int tube_core(int nstages) { return 63 - 6 * (nstages - 1); }
+int line_class(const CaseDev &c);
+hipError_t launch_lines(const CaseDev *d_cases, const Plan &plan, const std::vector<CaseDev> &cases, int n,
+                        hipStream_t st);
 
 // Host side: blocks each case needs for each kernel class (0 = class unused).
 void case_blocks(const CaseDev &c, int blocks[K_NCLASS]);

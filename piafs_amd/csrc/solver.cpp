@@ -398,6 +398,7 @@ void Engine::release_plan() {
   d_cases = nullptr;
   d_status = nullptr;
   plan = Plan();
+  lines.clear();
   built = false;
 }
 
@@ -467,6 +468,9 @@ int Engine::build() {
     HIPCHK(hipStreamSynchronize(stream));
   }
   HIPCHK(hipStreamSynchronize(stream));  // hd is a host temporary
+  bool all = true;
+  for (const CaseDev &c : hd) all = all && line_class(c) >= 0;
+  if (all) lines = std::move(hd);
   built = true;
   return 0;
 }
@@ -507,7 +511,7 @@ void Engine::enqueue_step() {
 int Engine::prepare() {
   HIPCHK(hipSetDevice(device));
   if (!built) return fail(-1, "the ensemble plan is not built");
-  if (!use_graph || profiling || gexec || cases.empty()) return 0;
+  if (!use_graph || profiling || gexec || cases.empty() || !lines.empty()) return 0;
   HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
   enqueue_step();
   hipGraph_t g = nullptr;
@@ -525,7 +529,9 @@ int Engine::step(int n) {
   HIPCHK(hipSetDevice(device));
   if (!built) return fail(-1, "the ensemble plan is not built");
   if (cases.empty()) return 0;
-  if (use_graph && !profiling) {
+  if (!lines.empty() && !profiling) {
+    HIPCHK(launch_lines(d_cases, plan, lines, n, stream));
+  } else if (use_graph && !profiling) {
     if (!gexec) {
       int rc = prepare();
       if (rc) return rc;

@@ -1,0 +1,79 @@
+"""1D cases advanced by whole steps (one launch for many steps, or one a step)
+against the kernels of a stage, which a profiled case runs: the same bits."""
+import numpy as np
+import pytest
+
+import piafs_amd
+from piafs_amd import decks
+
+pytestmark = pytest.mark.gpu
+
+# the reflect rule negates every variable, density too: those runs turn to NaN,
+# and have to do so at the same points
+ENDS = {
+    "mirror": None,
+    "periodic": [("periodic", 0, 1, 0, 0), ("periodic", 0, -1, 0, 0)],
+    "walls": [("slip-wall", 0, 1, 0, 0, 0.1), ("slip-wall", 0, -1, 0, 0, -0.2)],
+    "reflect": [("reflect", 0, 1, 0, 0), ("extrapolate", 0, -1, 0, 0)],
+}
+
+
+def _same(tmp_path, dk, steps, finite=True):
+    d = dk.write(str(tmp_path))
+    with piafs_amd.Case(d) as a, piafs_amd.Case(d) as b:
+        b.profile(True)
+        for n in steps:
+            a.step(n)
+            b.step(n)
+            a.sync()
+            b.sync()
+            got, want = a.solution(), b.solution()
+            assert np.all(np.isfinite(want)) or not finite
+            assert np.array_equal(got, want, equal_nan=True)
+
+
+def _deck(N, ends, scheme, interp, upwinding, rk, weights=0):
+    dk = decks.sod_1d(N=N, scheme=scheme, interp=interp, upwinding=upwinding, rk=rk, boundary=ENDS[ends], mapped=weights)
+    r = np.random.default_rng(N)
+    dk.u[:, 0] *= 1.0 + 0.02 * r.uniform(-1, 1, N)
+    dk.u[:, 1] = 0.1 * dk.u[:, 0]
+    return dk
+
+
+# windows that keep 51 (RK3), 45 (RK4) points: less than one, exactly, one more, many
+@pytest.mark.parametrize("N", [8, 45, 51, 52, 90, 300])
+@pytest.mark.parametrize("ends", sorted(ENDS))
+@pytest.mark.parametrize("interp,upwinding,rk", [("characteristic", "roe", "ssprk3"), ("components", "rf-char", "44"),
+                                                 ("characteristic", "llf-char", "44"), ("components", "rusanov", "1fe")])
+def test_windows(tmp_path, N, ends, interp, upwinding, rk):
+    _same(tmp_path, _deck(N, ends, "weno5", interp, upwinding, rk), (1, 4, 3), ends != "reflect")
+
+
+# teams of 4 and 8 rows a lane, full and not, the last and first size of each;
+# 514 goes the general way on both sides
+@pytest.mark.parametrize("N", [8, 33, 128, 257, 258, 513, 514])
+@pytest.mark.parametrize("ends,upwinding", [("mirror", "roe"), ("periodic", "rf-char"), ("walls", "llf-char"),
+                                            ("reflect", "rusanov")])
+def test_line_systems(tmp_path, N, ends, upwinding):
+    _same(tmp_path, _deck(N, ends, "crweno5", "components", upwinding, "44", weights=N & 1), (1, 6), ends != "reflect")
+
+
+def test_members_together(tmp_path):
+    """Lines of both kinds in a batch, and with a 2D member, equal their solo runs."""
+    mem = [_deck(70, "mirror", "weno5", "characteristic", "roe", "ssprk3"),
+           _deck(129, "periodic", "crweno5", "components", "roe", "44"),
+           _deck(300, "walls", "crweno5", "components", "roe", "44"),
+           _deck(111, "periodic", "weno5", "components", "roe", "44")]
+    two = decks.ns2d_photochem(nx=20, ny=12, n_iter=5)
+    dirs = [dk.write(str(tmp_path / str(k))) for k, dk in enumerate(mem + [two])]
+    solo = []
+    for d in dirs:
+        with piafs_amd.Case(d) as c:
+            c.step(5)
+            solo.append(c.solution())
+    for some in (dirs[:4], dirs):
+        with piafs_amd.Batch(some) as b:
+            b.step(2)
+            b.step(3)
+            for k in b.slots:
+                assert np.array_equal(b.solution(k), solo[k]), k
