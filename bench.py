@@ -436,7 +436,9 @@ def main():
         if ktimes:
             # per-class average launch time (ms) x launches per step -> share of the step
             ns = inf.nstages
-            share = {k: v * (1 if k == "update" else ns) for k, v in ktimes.items()}
+            # (the stage state is formed apart from the assembly once per call only)
+            per_step = {"update": 1, "stage_bc": 1 / args.profile_steps if "next" in ktimes else ns}
+            share = {k: v * per_step.get(k, ns) for k, v in ktimes.items()}
             dom = max(share.items(), key=lambda kv: kv[1])[0]
             paired = (not inf.characteristic) and dk.physics["upwinding"] in ("roe", "rusanov")
             io_byts = kernel_algorithmic_bytes(dom, nx, nx, nv, g, inf.nstages, True, paired)

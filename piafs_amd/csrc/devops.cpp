@@ -69,6 +69,7 @@ int unit_prepare(piafs_case *pc, hipStream_t st) {
   CaseDev d = c->h;
   d.paired = 0;
   d.unit = 1;
+  d.fused = 0;
   d.terms = 7;
   d.u = un.u;
   d.status = pc->eng.d_status;  // zero pivots reach the case's own status word (piafs_sync)
@@ -175,7 +176,7 @@ int piafs_dev_upwind(piafs_case *pc, double *fI, const double *fL, const double 
   const CaseDev &d = un.desc;
   const Grid &G = c->h.G;
   const SweepGeom &S = dir ? d.Sy : d.Sx;
-  double *const *io = dir ? d.iy : d.ix;
+  const Global<double> *io = dir ? d.iy : d.ix;
   stage_state(pc, u_ghosted, st);
   const double *in[4] = {uL, uR, fL, fR};
   for (int r = 0; r < 4; r++) launch_dev_iface(G.ndims, dir, G.nx, S.N, S.nlines, G.nv, in[r], io[r], 1, st);

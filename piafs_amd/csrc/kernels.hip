@@ -11,6 +11,7 @@
 #include "viscous.hpp"
 
 #include <cstdio>
+#include <cstring>
 #include <type_traits>
 
 namespace piafs {
@@ -31,6 +32,10 @@ inline unsigned nblk(long n, int tb = TB) { return (unsigned)((n + tb - 1) / tb)
 // boundary zone (the corners) are zero, as in the reference where they are
 // never written.
 // ---------------------------------------------------------------------------
+// `stage` arguments with this bit leave the fused cases out
+constexpr int kUnfused = 1 << 8;
+__device__ __forceinline__ bool skipped(const CaseDev &C, int stage) { return (stage & kUnfused) && C.fused; }
+
 __device__ __forceinline__ double stage_value(const CaseDev &C, int s, long p) {
   double val = C.u[p];
   const int ns = C.nstages;
@@ -49,7 +54,9 @@ __host__ __device__ inline long ghost_points(const Grid &G) {
   return G.ndims == 1 ? 2L * G.g : 2L * G.gy * G.nxg + 2L * G.g * G.ny;
 }
 
-__device__ __forceinline__ void ghost_body(const CaseDev &C, int stage, long t) {
+// state(p): the state at offset p; U: where the ghost points go, in the natural layout
+template <class V>
+__device__ __forceinline__ void ghost_body(const CaseDev &C, long t, V state, double *U) {
   const Grid &G = C.G;
   const long ng = ghost_points(G);
   if (t >= ng * G.nv) return;
@@ -69,10 +76,10 @@ __device__ __forceinline__ void ghost_body(const CaseDev &C, int stage, long t) 
     i = col < G.g ? col - G.g : G.nx + (col - G.g);
   }
   const double val = ghost_value(C, v, i, j, [&](int m, int a, int b) {
-    return stage_value(C, stage, (long)m * G.plane + (long)(b + G.gy) * G.nxg + (a + G.g));
+    return state((long)m * G.plane + (long)(b + G.gy) * G.nxg + (a + G.g));
   });
   const long pl = (long)v * G.plane;
-  C.U[pl + (long)(j + G.gy) * G.nxg + (i + G.g)] = val;
+  U[pl + (long)(j + G.gy) * G.nxg + (i + G.g)] = val;
   if (G.ndims == 2) C.UT[pl + (long)(i + G.g) * G.nyg + (j + G.gy)] = val;
 }
 
@@ -88,11 +95,12 @@ __host__ __device__ inline int stage_blocks(const Grid &G, int st) {
 template <int ST>
 __device__ __forceinline__ void stage_body(CASE_ARGS) {
   CASE_PREAMBLE
-  if (stage >= C.nstages) return;
+  const int s = stage & 0xFF;
+  if (s >= C.nstages || skipped(C, stage)) return;
   const Grid &G = C.G;
-  const int s = stage, bid = (int)(blockIdx.x - firstblock[cidx]), ns = stage_blocks(G, ST);
+  const int bid = (int)(blockIdx.x - firstblock[cidx]), ns = stage_blocks(G, ST);
   if (bid >= ns) {
-    ghost_body(C, s, t - (long)ns * TB);
+    ghost_body(C, t - (long)ns * TB, [&](long p) { return stage_value(C, s, p); }, C.U);
     return;
   }
   if (G.ndims == 1) {
@@ -142,7 +150,12 @@ __global__ void __launch_bounds__(256) k_stage64(CASE_ARGS) { stage_body<64>(cas
 // the ghost points alone, for the boundary-fill operator
 __global__ void __launch_bounds__(256) k_ghost(CASE_ARGS) {
   CASE_PREAMBLE
-  if (stage < C.nstages) ghost_body(C, stage, t);
+  if (stage < C.nstages) ghost_body(C, t, [&](long p) { return stage_value(C, stage, p); }, C.U);
+}
+// those of the state k_next wrote, of the cases with faces it does not fill
+__global__ void __launch_bounds__(256) k_ghost_next(CASE_ARGS) {
+  CASE_PREAMBLE
+  if (stage < C.nstages) ghost_body(C, t, [&](long p) { return C.Un[p]; }, C.Un);
 }
 
 // ---------------------------------------------------------------------------
@@ -163,7 +176,7 @@ __device__ __forceinline__ void recon_end(const CaseDev &C, int dir, long pair, 
   const int nv = C.G.nv, N = S.N, nl = S.nlines;
   const int q = (int)(pair % 2), v = (int)((pair / 2) % nv), l = (int)((pair / 2) / nv);
   const int k = e ? N : 0;
-  double *const *io = dir ? C.iy : C.ix;
+  const Global<double> *io = dir ? C.iy : C.ix;
   const long at = ((long)v * nl + l) * (N + 1) + k;
   double a, b, c, xl, xr;
   row_coeffs<KIND>(k, N, true, C.R, w[0], w[1], w[2], w[3], w[4], w[5], a, b, c, xl);
@@ -1149,7 +1162,7 @@ __global__ void __launch_bounds__(kLongTeam) k_lsolve(CASE_ARGS) {
   }
   // interface arrays: split mode uL, uR (q 0) or fL, fR (q 1); paired mode
   // 0.5*(uR - uL) or 0.5*(fL + fR)
-  double *const *io = dir ? C.iy : C.ix;
+  const Global<double> *io = dir ? C.iy : C.ix;
   const long line = ((long)v * S.nlines + l) * (N + 1);
   const double *xl = L + 3 * f + s0 * (N + 1), *xr = xl + (N + 1);
   for (int k = threadIdx.x; k <= N; k += kLongTeam) {
@@ -1176,7 +1189,7 @@ __global__ void __launch_bounds__(kLongTeam) k_lsolve(CASE_ARGS) {
 
 template <int DIR, int PAIR>
 __device__ __forceinline__ void upwind_ns2d_roe(const SweepGeom &S, int nv, double g, long t,
-                                                const double *__restrict__ q, double *const *io,
+                                                const double *__restrict__ q, const Global<double> *io,
                                                 double *__restrict__ fI, bool species = true) {
   const int nl = S.nlines, N = S.N;
   const int k = (int)(t % (N + 1)), l = (int)(t / (N + 1));
@@ -1200,7 +1213,7 @@ __device__ __forceinline__ void upwind_ns2d_roe(const SweepGeom &S, int nv, doub
 
 template <int PAIR>
 __device__ __forceinline__ void upwind_e1d(const SweepGeom &S, int nv, double g, int mode, long t,
-                                           const double *__restrict__ q, double *const *io, double *__restrict__ fI) {
+                                           const double *__restrict__ q, const Global<double> *io, double *__restrict__ fI) {
   const int nl = S.nlines, N = S.N;
   const int k = (int)(t % (N + 1)), l = (int)(t / (N + 1));
   const long pl = S.plane;
@@ -1234,7 +1247,7 @@ __device__ __forceinline__ void upwind_e1d(const SweepGeom &S, int nv, double g,
 
 // Split mode only: uL, uR, fL, fR in io[0..3].
 template <int DIR, bool LLF>
-__device__ __forceinline__ void upwind_ns2d_rf(const SweepGeom &S, int nv, double g, long t, double *const *io,
+__device__ __forceinline__ void upwind_ns2d_rf(const SweepGeom &S, int nv, double g, long t, const Global<double> *io,
                                                double *__restrict__ fI) {
   const int nl = S.nlines, N = S.N;
   const int k = (int)(t % (N + 1)), l = (int)(t / (N + 1));
@@ -1254,7 +1267,7 @@ __device__ __forceinline__ void upwind_ns2d_rf(const SweepGeom &S, int nv, doubl
 
 template <int DIR, int PAIR>
 __device__ __forceinline__ void upwind_ns2d_rusanov(const SweepGeom &S, int nv, double g, long t,
-                                                    const double *__restrict__ q, double *const *io,
+                                                    const double *__restrict__ q, const Global<double> *io,
                                                     double *__restrict__ fI) {
   const int nl = S.nlines, N = S.N;
   const int k = (int)(t % (N + 1)), l = (int)(t / (N + 1));
@@ -1356,20 +1369,22 @@ __global__ void __launch_bounds__(256) k_bflux(CASE_ARGS) {
 // the Gaussian pulse at the stage time.
 // ---------------------------------------------------------------------------
 // component c (variable c + 1) of the parabolic term
-__device__ __forceinline__ double viscous_par(const CaseDev &C, int c, int i, int j, long p) {
+// at point (i, j), byte offset o of the ghosted planes
+__device__ __forceinline__ double viscous_par(const CaseDev &C, int c, int i, int j, unsigned o) {
   const Grid &G = C.G;
   const PhysParams &P = C.P;
   const long pl = (long)G.nxg * G.nyg;
   const double dxi = C.dxinv[G.g + i], dyi = C.dxinv[(G.nx + 2 * G.g) + G.g + j];
   const double *Fx = C.FV + c * pl, *Fy = C.FV + (3 + c) * pl;
+  const unsigned row = 8u * G.nxg;
   double dfx, dfy;
   if (P.par4) {
     const double t12 = 1.0 / 12.0;
-    dfx = (Fx[p - 2] - 8 * Fx[p - 1] + 8 * Fx[p + 1] - Fx[p + 2]) * t12;
-    dfy = (Fy[p - 2 * G.nxg] - 8 * Fy[p - G.nxg] + 8 * Fy[p + G.nxg] - Fy[p + 2 * G.nxg]) * t12;
+    dfx = (elem(Fx, o - 16) - 8 * elem(Fx, o - 8) + 8 * elem(Fx, o + 8) - elem(Fx, o + 16)) * t12;
+    dfy = (elem(Fy, o - 2 * row) - 8 * elem(Fy, o - row) + 8 * elem(Fy, o + row) - elem(Fy, o + 2 * row)) * t12;
   } else {
-    dfx = 0.0 * Fx[p + 1] - (-1.0) * Fx[p] + (-1.0) * Fx[p - 1];
-    dfy = 0.0 * Fy[p + G.nxg] - (-1.0) * Fy[p] + (-1.0) * Fy[p - G.nxg];
+    dfx = 0.0 * elem(Fx, o + 8) - (-1.0) * elem(Fx, o) + (-1.0) * elem(Fx, o - 8);
+    dfy = 0.0 * elem(Fy, o + row) - (-1.0) * elem(Fy, o) + (-1.0) * elem(Fy, o - row);
   }
   const double px = dxi * dfx;
   return px + dyi * dfy;
@@ -1400,155 +1415,287 @@ __device__ __forceinline__ double sponge(const CaseDev &C, int i, int j, int v, 
 
 // the Gaussian pulse at the stage time (ChemistrySolve.c:36-43); the photon
 // density reaching layer 0 is its product with the beam map
-__device__ __forceinline__ double chem_pulse(const CaseDev &C, int stage) {
+__device__ __forceinline__ double chem_pulse(const CaseDev &C, int stage, double t0) {
   const PhysParams &P = C.P;
-  const double time = *C.time + C.c[stage] * C.dt;
+  const double time = t0 + C.c[stage] * C.dt;
   if (!(time > P.t_start_norm)) return 0.0;
   const double sigma = P.t_pulse_norm / 2.35482;
   const double tp = time - (P.t_start_norm + P.t_pulse_norm);
   return P.I0 * exp(-(tp * tp) / (2 * sigma * sigma));
 }
 
-// Photochemistry source of variable v at point p (chemistry.h:30-127,
-// ChemistrySolve.c:45-110): a species' own term, or the energy's, which is the
-// last layer's heating.  The other variables have none.  hs: the pulse at the
-// stage time (chem_pulse).
-__device__ __forceinline__ double chem_var(const CaseDev &C, int v, long p, double hs) {
-  const PhysParams &P = C.P;
-  const double *U = C.U;
-  const long pl = C.G.plane;
-  const bool energy = v == P.nflow - 1;
-  const int iz = energy ? P.nlayers - 1 : (v - P.nflow) / P.z_stride, m = v - P.nflow - P.z_stride * iz;
-  if (!energy && (m == 0 || m == 6)) return 0.0;
-  auto n = [&](int q) { return U[(long)(P.nflow + P.z_stride * iz + q) * pl + p]; };
-  // photon density reaching layer iz
-  auto photons = [&]() {
-    double nh = (hs * C.imap[p]) / P.hnu_den;
-    for (int z = 0; z < iz; z++) nh = nh * (1.0 - P.damp_coef * U[(long)(P.nflow + P.z_stride * z + 1) * pl + p]);
-    return nh;
-  };
-  const double nO3 = n(1);
-  if (m == 4 && !energy) return P.k2a * nO3 * n(2) - P.k5 * nO3 * n(4);
-  if (m == 5 && !energy) return P.k1a * n(2) * n(0) - (P.k3a + P.k3b) * nO3 * n(5);
-  const double nh = photons();
-  if (energy) {
-    const double nO2 = n(0), n1D = n(2), n1Dg = n(3), n3Su = n(4), n1Sg = n(5), nCO2 = n(6);
+// Photochemistry source of variable v (chemistry.h:30-127, ChemistrySolve.c:
+// 45-110): a species' own term, or the energy's, which is the last layer's
+// heating.  The other variables have none.  n(q): species q of the layer; nh:
+// the photon density reaching it.
+struct ChemVar {
+  int layer, m;   // m: species of the layer, -1 the energy
+  unsigned need;  // what the source reads, bits 0..6 the species of the layer, bit 7 the photons
+};
+__device__ __forceinline__ ChemVar chem_of(const PhysParams &P, int v) {
+  ChemVar c = {P.nlayers - 1, -1, 0xFF};
+  if (v >= P.nflow) {
+    c.layer = P.nlayers > 1 ? (v - P.nflow) / P.z_stride : 0;
+    c.m = v - P.nflow - P.z_stride * c.layer;
+    c.need = c.m == 1 ? 0xBE : c.m == 2 ? 0xC7 : c.m == 3 ? 0x9A : c.m == 4 ? 0x16 : c.m == 5 ? 0x27 : 0;
+  }
+  return c;
+}
+template <class F>
+__device__ __forceinline__ double chem_term(const PhysParams &P, int m, F n, double nh) {
+  if (m < 0) {
+    const double nO3 = n(1), nO2 = n(0), n1D = n(2), n1Dg = n(3), n3Su = n(4), n1Sg = n(5), nCO2 = n(6);
     return ((P.q0a * P.k0a + P.q0b * P.k0b) * nh * nO3 + (P.q1a * P.k1a + P.q1b * P.k1b) * nO2 * n1D +
             (P.q2a * P.k2a + P.q2b * P.k2b) * nO3 * n1D + (P.q3a * P.k3a + P.q3b * P.k3b) * nO3 * n1Sg +
             P.q4 * P.k4 * n1D * nCO2 + P.q5 * P.k5 * nO3 * n3Su + P.q6 * P.k6 * n1Dg * nO3) /
            P.ch_gm1;
   }
-  if (m == 1)
-    return -(P.k0a + P.k0b) * nh * nO3 - (P.k2a + P.k2b) * nO3 * n(2) - (P.k3a + P.k3b) * nO3 * n(5) -
-           P.k5 * nO3 * n(4) - P.k6 * n(3) * nO3;
-  if (m == 2) {
-    const double n1D = n(2);
-    return P.k0a * nh * nO3 - (P.k1a + P.k1b) * n1D * n(0) - (P.k2a + P.k2b) * n1D * nO3 - P.k4 * n1D * n(6);
+  switch (m) {
+    case 1: {
+      const double nO3 = n(1);
+      return -(P.k0a + P.k0b) * nh * nO3 - (P.k2a + P.k2b) * nO3 * n(2) - (P.k3a + P.k3b) * nO3 * n(5) -
+             P.k5 * nO3 * n(4) - P.k6 * n(3) * nO3;
+    }
+    case 2: {
+      const double nO3 = n(1), n1D = n(2);
+      return P.k0a * nh * nO3 - (P.k1a + P.k1b) * n1D * n(0) - (P.k2a + P.k2b) * n1D * nO3 - P.k4 * n1D * n(6);
+    }
+    case 3: return P.k0a * nh * n(1) + P.k5 * n(1) * n(4) - P.k6 * n(3) * n(1);
+    case 4: return P.k2a * n(1) * n(2) - P.k5 * n(1) * n(4);
+    case 5: return P.k1a * n(2) * n(0) - (P.k3a + P.k3b) * n(1) * n(5);
+    default: return 0.0;
   }
-  return P.k0a * nh * nO3 + P.k5 * nO3 * n(4) - P.k6 * n(3) * nO3;  // m == 3
+}
+// photon density reaching layer iz at byte offset o, from the pulse at the stage
+// time (chem_pulse) and the beam map
+__device__ __forceinline__ double chem_photons(const CaseDev &C, int iz, unsigned o, double hs, double imap) {
+  const PhysParams &P = C.P;
+  double nh = (hs * imap) / P.hnu_den;
+  for (int z = 0; z < iz; z++)
+    nh = nh * (1.0 - P.damp_coef * elem(C.U + (long)(P.nflow + P.z_stride * z + 1) * C.G.plane, o));
+  return nh;
+}
+// the species of a layer
+__device__ __forceinline__ const double *chem_planes(const CaseDev &C, int layer) {
+  return C.U + (long)(C.P.nflow + C.P.z_stride * layer) * C.G.plane;
 }
 
 // rhs of variable v at interior point (i, j), ghosted offset p, with its
 // source added (SourceFunction.c:21-60): chemistry, then the sponge zones
 __device__ __forceinline__ double with_source(const CaseDev &C, int v, int i, int j, long p, double hs, double r) {
   const bool chem = C.P.chem && v >= C.P.nflow - 1;
-  const double s = chem ? chem_var(C, v, p, hs) : 0.0;
+  double s = 0.0;
+  if (chem) {
+    const unsigned o = 8u * (unsigned)p;
+    const ChemVar cv = chem_of(C.P, v);
+    const double *n = chem_planes(C, cv.layer);
+    const double nh = cv.need >> 7 ? chem_photons(C, cv.layer, o, hs, elem(C.imap, o)) : 0.0;
+    s = chem_term(C.P, cv.m, [&](int q) { return elem(n + q * C.G.plane, o); }, nh);
+  }
   if (C.sponge && in_sponge(C, i, j)) return r + sponge(C, i, j, v, p, s);
   return chem ? r + s : r;
 }
 
-// One variable of one 32 x 32 tile per block, the tile's variables in
-// neighbouring blocks of one XCD (the species a source reads are shared in its
-// L2).  Bound by memory latency on small grids and by HBM on large ones.  A
-// block has one exchange through LDS (the y-sweep interfaces, which are
-// contiguous along y) and no serial walk over the variables: a tile's latency
-// is paid once, not once per variable, a grid of few tiles has nv times as many
-// blocks, and the source is added before the one store of a value.  With a tile
-// per block walking all variables (a load round and two barriers each, the
-// source a second pass over the stored values) a launch took, nv 11: 128 x 97
-// 53.3 -> 10.5 us, 600 x 343 59.4 -> 26, 1024^2 119 -> 115, 2048 x 1531 368 ->
-// 336 us.
-__global__ void __launch_bounds__(256) k_assemble(CASE_ARGS) {
-  CASE_PREAMBLE
-  if (stage >= C.nstages) return;
+// One variable of one 32 x 32 tile per block, a row of tiles variable by variable
+// in neighbouring blocks of one XCD.  Bound by memory latency on small grids and
+// by HBM on large ones.  A block has one exchange through LDS (the y-sweep
+// interfaces, which are contiguous along y) and no serial walk over the variables:
+// a tile's latency is paid once, not once per variable, a grid of few tiles has
+// nv times as many blocks, and the source is added before the one store of a
+// value.  Every load, the species of the source among them, is issued before the
+// first is needed; the pulse is formed by one wave.  512 threads with two points
+// each: with four the kernel takes 152 registers and the grids of few tiles have
+// half the waves (k_next, 128 x 97: 11.9 -> 9.2 us, 201 x 201: 6.4 -> 5.7; large
+// grids alike, and so are they with 16, 20 or 24 waves a CU).  With a tile per
+// block walking all variables k_assemble took, nv 11: 128 x 97 53.3 -> 10.5 us,
+// 600 x 343 59.4 -> 26, 1024^2 119 -> 115, 2048 x 1531 368 -> 336 us.
+constexpr int kTileThreads = 512;
+struct Tile {
+  double y[32][33];     // y-sweep interfaces
+  double pulse;         // chem_pulse of the stage
+  double next[32][33];  // the state k_next writes, for the transposed copy and the ghost points
+};
+
+// NEXT: the values of the next stage's state (or the new solution) follow from
+// the right-hand side at once (k_next)
+template <bool NEXT>
+__device__ __forceinline__ void assemble_tile(const CaseDev &C, int stage, int block, int first, Tile &sh) {
   const Grid &G = C.G;
   const int nv = G.nv;
-  double *udot = C.Udot[stage];
-  const bool src = (C.P.chem || C.sponge) && (C.terms & 4);
-  if (G.ndims == 1) {
-    if (t >= (long)G.nx * nv) return;
-    const int v = (int)(t / G.nx), i = (int)(t % G.nx);
-    const long p = i + G.g;
-    const long a = (long)v * (G.nx + 1) + i;
-    const double hyp = C.dxinv[G.g + i] * (C.fIx[a + 1] - C.fIx[a]);
-    double r = (C.terms & 1) ? -hyp : 0.0;
-    if (src) r = with_source(C, v, i, 0, p, C.P.chem ? chem_pulse(C, stage) : 0.0, r);
-    udot[(long)v * G.plane + p] = r;
-    return;
-  }
-  __shared__ double tl[32][33];
+  constexpr int R = kTileThreads / 32, Q = 32 / R;  // rows of the tile at a time, and of a thread
+  auto &tl = sh.y;
   const int ntx = (G.nx + 31) / 32;
   const int nb = ntx * ((G.ny + 31) / 32) * nv;  // the case's blocks are padded to a multiple of eight
-  const int id = xcd_order((int)(blockIdx.x - firstblock[cidx]), (nb + 7) & ~7, firstblock[cidx]);
+  const int id = xcd_order(block, (nb + 7) & ~7, first);
   if (id >= nb) return;
-  const int v = id % nv, tile = id / nv;
-  const int i0 = (tile % ntx) * 32, j0 = (tile / ntx) * 32;
+  const int strip = (unsigned)id / (unsigned)ntx, row = (unsigned)strip / (unsigned)nv, v = strip - row * nv;
+  const int i0 = (id - strip * ntx) * 32, j0 = row * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int i = i0 + tx;
+  const long pl = (long)v * G.plane;
   // Points outside the grid read the nearest one inside and are not stored, so
   // that every load is issued without a branch (a branch would wait for the
   // loads before it).
   const int ic = min(i, G.nx - 1);
-  auto jq = [&](int q) { return min(j0 + ty + 8 * q, G.ny - 1); };
+  auto jq = [&](int q) { return min(j0 + ty + R * q, G.ny - 1); };
+  unsigned o[Q];  // byte offset of the thread's points in a plane
+#pragma unroll
+  for (int q = 0; q < Q; q++) o[q] = 8u * ((unsigned)(jq(q) + G.gy) * G.nxg + (ic + G.g));
   // y-sweep interfaces of lines i0..i0+31, interfaces j0..j0+32
-  double fy[4], fy32 = 0.0;
+  const double *fIx = C.fIx + (long)v * G.ny * (G.nx + 1), *fIy = C.fIy + (long)v * G.nx * (G.ny + 1);
+  double fy[Q], fy32 = 0.0;
 #pragma unroll
-  for (int q = 0; q < 4; q++)
-    fy[q] = C.fIy[((long)v * G.nx + min(i0 + ty + 8 * q, G.nx - 1)) * (G.ny + 1) + min(j0 + tx, G.ny)];
+  for (int q = 0; q < Q; q++)
+    fy[q] = elem(fIy, 8u * ((unsigned)min(i0 + ty + R * q, G.nx - 1) * (G.ny + 1) + min(j0 + tx, G.ny)));
   // interface j0 + 32 of line i0 + the thread's index, by the first 32 threads
-  if (threadIdx.x < 32) fy32 = C.fIy[((long)v * G.nx + ic) * (G.ny + 1) + min(j0 + 32, G.ny)];
+  if (threadIdx.x < 32) fy32 = elem(fIy, 8u * ((unsigned)ic * (G.ny + 1) + min(j0 + 32, G.ny)));
   const bool visc = C.P.viscous && (C.terms & 2) && v >= 1 && v <= 3;
-  double hx[4], add[4];
+  double hx[Q], add[Q];
   {
-    double x0[4], x1[4];
+    double x0[Q], x1[Q];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const long a = ((long)v * G.ny + jq(q)) * (G.nx + 1) + ic;
-      x0[q] = C.fIx[a];
-      x1[q] = C.fIx[a + 1];
+    for (int q = 0; q < Q; q++) {
+      const unsigned a = 8u * ((unsigned)jq(q) * (G.nx + 1) + ic);
+      x0[q] = elem(fIx, a);
+      x1[q] = elem(fIx, a + 8);
     }
     const double dxi = C.dxinv[G.g + ic];
 #pragma unroll
-    for (int q = 0; q < 4; q++) hx[q] = dxi * (x1[q] - x0[q]);
+    for (int q = 0; q < Q; q++) hx[q] = dxi * (x1[q] - x0[q]);
+  }
+  // the solution and the stages before, with their coefficients in what follows
+  const int ns = C.nstages;
+  const bool last = stage == ns - 1;
+  double un[Q], prev[3][Q], cf[4];
+  if (NEXT) {
+#pragma unroll
+    for (int q = 0; q < Q; q++) un[q] = elem(C.u + pl, o[q]);
+#pragma unroll
+    for (int j = 0; j < 4; j++) cf[j] = j <= stage ? C.dt * (last ? C.b[j] : C.A[(stage + 1) * ns + j]) : 0.0;
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+      if (j < stage && (last || cf[j] != 0.0))
+#pragma unroll
+        for (int q = 0; q < Q; q++) prev[j][q] = elem(C.Udot[j] + pl, o[q]);
   }
 #pragma unroll
-  for (int q = 0; q < 4; q++)
-    add[q] = visc ? viscous_par(C, v - 1, ic, jq(q), (long)(jq(q) + G.gy) * G.nxg + (ic + G.g)) : 0.0;
-  double sv[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int q = 0; q < Q; q++) add[q] = visc ? viscous_par(C, v - 1, ic, jq(q), o[q]) : 0.0;
+  // what the variable's source reads
   const bool chem = C.P.chem && (C.terms & 4) && v >= C.P.nflow - 1;
-  if (chem) {
-    const double hs = chem_pulse(C, stage);
+  const ChemVar cv = chem ? chem_of(C.P, v) : ChemVar{0, 0, 0};
+  const unsigned need = cv.need;
+  const double *species = chem_planes(C, cv.layer);
+  double sp[8][Q];
 #pragma unroll
-    for (int q = 0; q < 4; q++) sv[q] = chem_var(C, v, (long)(jq(q) + G.gy) * G.nxg + (ic + G.g), hs);
+  for (int k = 0; k < 7; k++)
+    if (need >> k & 1)
+#pragma unroll
+      for (int q = 0; q < Q; q++) sp[k][q] = elem(species + k * G.plane, o[q]);
+  if (need >> 7)
+#pragma unroll
+    for (int q = 0; q < Q; q++) sp[7][q] = elem(C.imap, o[q]);
+  const double t0 = C.time[NEXT && stage ? 1 : 0];
+  if (NEXT && block == 0 && threadIdx.x == 0) {  // the blocks read the other of the two
+    if (stage == 0) C.time[1] = t0;
+    else if (last) C.time[0] = t0 + C.dt;
   }
 #pragma unroll
-  for (int q = 0; q < 4; q++) tl[ty + 8 * q][tx] = fy[q];
+  for (int q = 0; q < Q; q++) tl[ty + R * q][tx] = fy[q];
   if (threadIdx.x < 32) tl[threadIdx.x][32] = fy32;
+  if (need >> 7 && threadIdx.x < 64) sh.pulse = chem_pulse(C, stage, t0);
   lds_barrier();
+  double sv[Q] = {};
+  if (need) {
+    const double hs = sh.pulse;
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const int jl = ty + 8 * q, j = j0 + jl;
-    const long p = (long)(j + G.gy) * G.nxg + (i + G.g);
+    for (int q = 0; q < Q; q++) {
+      const double nh = need >> 7 ? chem_photons(C, cv.layer, o[q], hs, sp[7][q]) : 0.0;
+      sv[q] = chem_term(C.P, cv.m, [&](int k) { return sp[k][q]; }, nh);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const int jl = ty + R * q, j = j0 + jl;
     const double hyp = hx[q] + C.dxinv[(G.nx + 2 * G.g) + G.g + jq(q)] * (tl[tx][jl + 1] - tl[tx][jl]);
     double r = (C.terms & 1) ? -hyp : 0.0;
     if (visc) r = r + add[q];
     if (i < G.nx && j < G.ny) {
       // chemistry, then the sponge zones (SourceFunction.c:21-60)
-      if (C.sponge && (C.terms & 4) && in_sponge(C, i, j)) r = r + sponge(C, i, j, v, p, sv[q]);
+      if (C.sponge && (C.terms & 4) && in_sponge(C, i, j)) r = r + sponge(C, i, j, v, o[q] / 8, sv[q]);
       else if (chem) r = r + sv[q];
-      udot[(long)v * G.plane + p] = r;
+      if (!NEXT || !last) elem(C.Udot[stage] + pl, o[q]) = r;
+      if (NEXT) {
+        double x = un[q];
+#pragma unroll
+        for (int m = 0; m < 3; m++)
+          if (m < stage && (last || cf[m] != 0.0)) x += cf[m] * prev[m][q];
+        if (last || cf[stage] != 0.0) x += cf[stage] * r;
+        if (last) elem(C.u + pl, o[q]) = x;
+        elem(C.Un + pl, o[q]) = x;
+        sh.next[jl][tx] = x;
+      }
     }
   }
+  if (!NEXT) return;
+  lds_barrier();
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const int il = ty + R * q;
+    if (i0 + il < G.nx && j0 + tx < G.ny)
+      elem(C.UT + pl, 8u * ((unsigned)(i0 + il + G.g) * G.nyg + (j0 + tx + G.gy))) = sh.next[tx][il];
+  }
+  // ghost points whose source lies in the tile, of the faces that copy
+  if (!C.push[0] || (i0 >= G.g && i0 + 32 <= G.nx - G.g && j0 >= G.g && j0 + 32 <= G.ny - G.g)) return;
+#pragma unroll
+  for (int f = 0; f < 4; f++) {
+    const int kind = C.push[f], d = f >> 1, hi = f & 1;
+    const int N = d ? G.ny : G.nx, No = d ? G.nx : G.ny, b0 = d ? j0 : i0, o0 = d ? i0 : j0;
+    for (int e = threadIdx.x; e < 32 * G.g; e += kTileThreads) {
+      const int m = e >> 5, o = e & 31, k = hi ? N + m : -1 - m;  // ghost position m along d
+      const int src = (kind == 1 ? (hi ? m : N - 1 - m) : (hi ? N - 1 - m : m)) - b0;
+      if (src < 0 || src >= 32 || o0 + o >= No) continue;
+      const double x = d ? sh.next[src][o] : sh.next[o][src];
+      const int gi = d ? o0 + o : k, gj = d ? k : o0 + o;
+      C.Un[pl + (long)(gj + G.gy) * G.nxg + (gi + G.g)] = x;
+      C.UT[pl + (long)(gi + G.g) * G.nyg + (gj + G.gy)] = x;
+    }
+  }
+}
+
+__global__ void __launch_bounds__(kTileThreads) k_assemble(CASE_ARGS) {
+  CASE_PREAMBLE
+  const int s = stage & 0xFF;
+  if (s >= C.nstages || skipped(C, stage)) return;
+  const Grid &G = C.G;
+  if (G.ndims == 1) {
+    const bool src = (C.P.chem || C.sponge) && (C.terms & 4);
+    if (t >= (long)G.nx * G.nv) return;
+    const int v = (int)(t / G.nx), i = (int)(t % G.nx);
+    const long p = i + G.g;
+    const long a = (long)v * (G.nx + 1) + i;
+    const double hyp = C.dxinv[G.g + i] * (C.fIx[a + 1] - C.fIx[a]);
+    double r = (C.terms & 1) ? -hyp : 0.0;
+    if (src) r = with_source(C, v, i, 0, p, C.P.chem ? chem_pulse(C, s, *C.time) : 0.0, r);
+    C.Udot[s][(long)v * G.plane + p] = r;
+    return;
+  }
+  __shared__ Tile sh;
+  assemble_tile<false>(C, s, (int)(blockIdx.x - firstblock[cidx]), firstblock[cidx], sh);
+}
+
+// The assembly with what follows from it point by point: the next stage's state
+// (TimeRK.c:46-57, as stage_value) in both layouts, after the last stage the new
+// solution (:86-99) and with it the next step's first state, and the ghost points
+// that are copies of interior ones.  With k_stage and k_update apart a step had
+// five launches more and 33 passes over a state's values, now 27.  Per stage, their
+// share of k_update included: 128 x 97 17.4 -> 7.9 us, 201 x 201 12.0 -> 5.7,
+// 600 x 343 46.8 -> 35.7, 1024^2 208 -> 193, 2048 x 1531 629 -> 622.
+__global__ void __launch_bounds__(kTileThreads) k_next(CASE_ARGS) {
+  CASE_PREAMBLE
+  (void)t;
+  if (stage >= C.nstages) return;
+  __shared__ Tile sh;
+  assemble_tile<true>(C, stage, (int)(blockIdx.x - firstblock[cidx]), firstblock[cidx], sh);
 }
 
 // u += (dt*b_s) * Udot_s stage by stage (TimeRK.c:86-99) at interior points;
@@ -1557,7 +1704,7 @@ __global__ void __launch_bounds__(256) k_update(CASE_ARGS) {
   CASE_PREAMBLE
   const Grid &G = C.G;
   const long nint = (long)G.nx * G.ny;
-  if (t >= nint * G.nv) return;
+  if (skipped(C, stage) || t >= nint * G.nv) return;
   if (t == 0) *C.time = *C.time + C.dt;
   const int v = (int)(t / nint);
   const long q = t % nint;
@@ -1911,7 +2058,7 @@ static const char *kKNames[K_NCLASS] = {"stage_bc", "ghost",  "flux",    "recon_
                                         "recon_4",  "recon_6", "recon_8", "recon_10", "recon_12", "recon_14", "recon_16",
                                         "recon_w10", "recon_w12", "recon_w16", "long_rows", "long_solve",
                                         "cw_rows", "cw_solve", "weno", "upwind", "bflux",
-                                        "assemble", "update", "flux_all",
+                                        "assemble", "next", "ghost_next", "update", "flux_all",
                                         "line_4", "line_8", "tube", "tube_back"};
 const char *kclass_name(int k) { return kKNames[k]; }
 
@@ -2042,7 +2189,10 @@ void case_blocks(const CaseDev &c, int blocks[K_NCLASS]) {
   }
   blocks[K_UPWIND] = weno ? 0 : nb((long)(c.Sx.N + 1) * c.Sx.nlines + (two ? (long)(c.Sy.N + 1) * c.Sy.nlines : 0));
   blocks[K_BFLUX] = c.cons ? 1 : 0;
-  blocks[K_ASSEMBLE] = pad8(two ? ((G.nx + 31) / 32) * ((G.ny + 31) / 32) * G.nv : nb((long)G.nx * G.nv));
+  blocks[K_ASSEMBLE] = pad8(two ? ((G.nx + 31) / 32) * ((G.ny + 31) / 32) * G.nv
+                                 : (int)(((long)G.nx * G.nv + kTileThreads - 1) / kTileThreads));
+  blocks[K_NEXT] = c.fused ? blocks[K_ASSEMBLE] : 0;
+  blocks[K_GHOSTNEXT] = c.fused && !c.push[0] ? blocks[K_GHOST] : 0;
   blocks[K_UPDATE] = nb((long)G.nx * G.ny * G.nv);
   const int line = line_class(c);
   blocks[K_LINE4] = line == K_LINE4;
@@ -2072,6 +2222,8 @@ static KernFn class_kernel(const Plan &pl, int cls) {
     case K_UPWIND: return k_upwind;
     case K_BFLUX: return k_bflux;
     case K_ASSEMBLE: return k_assemble;
+    case K_NEXT: return k_next;
+    case K_GHOSTNEXT: return k_ghost_next;
     default: return k_update;
   }
 }
@@ -2079,7 +2231,8 @@ static KernFn class_kernel(const Plan &pl, int cls) {
 static void run(int cls, const CaseDev *d, const Plan &pl, int s, hipStream_t st, MarkFn mark, void *ctx) {
   if (pl.nblocks[cls] <= 0) return;
   const bool recon = cls >= K_RECON && cls < K_RECON + kNRecon;
-  const int threads = recon ? recon_threads(kRecon[cls - K_RECON].wide) : TB;
+  const int threads = recon ? recon_threads(kRecon[cls - K_RECON].wide)
+                            : (cls == K_ASSEMBLE || cls == K_NEXT) ? kTileThreads : TB;
   if (mark) mark(ctx, cls, true, st);
   hipLaunchKernelGGL(class_kernel(pl, cls), dim3(pl.nblocks[cls]), dim3(threads), 0, st, d, pl.blockcase[cls],
                      pl.firstblock[cls], s);
@@ -2098,7 +2251,42 @@ void launch_stage(const CaseDev *d, const Plan &pl, int s, hipStream_t st, MarkF
     if (cls <= last) run(cls, d, pl, s, st, mark, ctx);
 }
 
-void launch_update(const CaseDev *d, const Plan &pl, hipStream_t st) { run(K_UPDATE, d, pl, 0, st, nullptr, nullptr); }
+void launch_begin(const CaseDev *d, const Plan &pl, hipStream_t st, MarkFn mark, void *ctx) {
+  if (pl.nfused) run(K_STAGE, d, pl, 0, st, mark, ctx);
+}
+
+void launch_step_stage(const CaseDev *d, const Plan &pl, int s, hipStream_t st, MarkFn mark, void *ctx) {
+  const bool rest = pl.nfused < pl.ncases;
+  if (pl.nfused) d += (long)s * pl.ncases;
+  if (rest) run(K_STAGE, d, pl, s | kUnfused, st, mark, ctx);
+  run(K_FLUX, d, pl, s, st, mark, ctx);
+  for (int cls = K_RECON; cls <= K_BFLUX; cls++) run(cls, d, pl, s, st, mark, ctx);
+  if (rest) run(K_ASSEMBLE, d, pl, s | kUnfused, st, mark, ctx);
+  run(K_NEXT, d, pl, s, st, mark, ctx);
+  run(K_GHOSTNEXT, d, pl, s, st, mark, ctx);
+}
+
+void launch_update(const CaseDev *d, const Plan &pl, hipStream_t st, MarkFn mark, void *ctx) {
+  if (pl.nfused < pl.ncases) run(K_UPDATE, d, pl, kUnfused, st, mark, ctx);
+}
+
+void choose_push(CaseDev &c) {
+  const int n[2] = {c.G.nx, c.G.ny};
+  for (int f = 0; f < 4; f++) {
+    const int d = f >> 1, face = f & 1 ? -1 : 1, o = 1 - d;
+    c.push[f] = 0;
+    if (c.G.ndims != 2 || n[d] < c.G.g) continue;
+    int z = c.nzones - 1;  // the last zone of the face decides, if it covers the face
+    while (z >= 0 && (c.zones[z].kind == Z_SPONGE || c.zones[z].dim != d || c.zones[z].face != face)) z--;
+    if (z < 0) continue;
+    const Zone &Z = c.zones[z];
+    if (Z.is[o] > 0 || Z.ie[o] < n[o]) continue;
+    // (a periodic zone takes its source without its offset along the face)
+    if (Z.kind == Z_PERIODIC && Z.is[o] == 0) c.push[f] = 1;
+    if (Z.kind == Z_EXTRAPOLATE) c.push[f] = 2;
+  }
+  if (!(c.push[0] && c.push[1] && c.push[2] && c.push[3])) memset(c.push, 0, sizeof c.push);
+}
 
 int cfl_norm_blocks(const Grid &G) {
   const long n = (long)G.nx * G.ny;

@@ -114,6 +114,25 @@ struct ReconParams {
   double eps;
 };
 
+// A pointer to device memory in a table that kernels read.  A pointer read from
+// memory is generic to the compiler: every access through it is a FLAT one, with
+// its address in vector registers, and waits for LDS traffic too.  Read through
+// this it is known to be global (k_next at 1024 x 1024 206 -> 193 us, 600 x 343
+// 40.2 -> 35.7, 128 x 97 9.2 -> 7.9).
+template <class T>
+struct Global {
+#ifdef __HIP_DEVICE_COMPILE__
+  __attribute__((address_space(1))) T *p;
+#else
+  T *p;
+#endif
+  __host__ __device__ __forceinline__ operator T *() const { return (T *)p; }
+  __host__ __device__ Global &operator=(T *q) {
+    p = (decltype(p))q;
+    return *this;
+  }
+};
+
 // Everything a kernel needs to know about one case (device-resident table).
 struct CaseDev {
   Grid G;
@@ -125,42 +144,50 @@ struct CaseDev {
   int model, upwind, nstages;  // upwind: 0 Roe, 1 rf-char, 2 llf-char, 3 rusanov
   int paired;    // reconstruction writes 0.5*(uR-uL), 0.5*(fL+fR) only (Roe with component-wise interpolation)
   int fuse_sp;   // species interface fluxes written by the reconstruction (set by the plan; see species_in_recon)
-  double *dsp[2];  // per sweep and interface: Roe-average |v_n| with the entropy fix (k_flux, when fuse_sp)
+  Global<double> dsp[2];  // per sweep and interface: Roe-average |v_n| with the entropy fix (k_flux, when fuse_sp)
   int stage_tile; // side of k_stage's transpose tiles, 32 or 64 (set by the plan)
   int unit;      // descriptor of the device-buffer operators: the interface flux in separate passes
   int terms;     // terms k_assemble adds: bit 0 hyperbolic, bit 1 parabolic, bit 2 source (7 in a step)
   double dt, A[16], b[4], c[4];
-  double *u, *U, *UT, *Udot[4];
-  double *flux_x, *flux_y, *ix[4], *iy[4], *fIx, *fIy;
-  double *FV, *dxinv, *imap;
-  double *xc;      // grid coordinates with ghosts, one dimension after the other
-  double *bcvals;  // the zones' values (Zone::vals)
-  double *ends;  // paired mode: raw end-interface values of both systems of every pair [dir][pair][side][0|N]
-  double *time;  // current simulation time of the case (one double)
+  Global<double> u, U, UT, Udot[4];
+  // 2D cases of two and more stages (fused): k_next writes the next stage's
+  // state itself, to Un.  The chemistry reads the stage state of other variables
+  // while it does, so stage s of a case with chemistry has a buffer Us[s] apart
+  // from the next one's; the other cases have one.  The descriptor table has an
+  // entry of every case per stage, with U and Un those of the stage.
+  int fused;
+  int push[4];  // per face 2 d + (high end): ghost points that k_next copies, 1 periodic, 2 mirrored; all 0: k_ghost_next's
+  Global<double> Us[4], Un;
+  Global<double> flux_x, flux_y, ix[4], iy[4], fIx, fIy;
+  Global<double> FV, dxinv, imap;
+  Global<double> xc;      // grid coordinates with ghosts, one dimension after the other
+  Global<double> bcvals;  // the zones' values (Zone::vals)
+  Global<double> ends;  // paired mode: raw end-interface values of both systems of every pair [dir][pair][side][0|N]
+  Global<double> time;  // current simulation time of the case; second double: the time at the start of a fused case's step
   // conservation check (conservation_check yes): boundary flux sums of each
   // stage [stage][(2 d + face) nv + v], the total boundary integral [nv], and
   // dS[d], the face element of dimension d (BoundaryIntegral.c:37-44)
   int cons;
   double dS[2];
-  double *bflux, *tbi;
+  Global<double> bflux, tbi;
   // characteristic CRWENO5: block rows of each sweep [field][line][k] and the
   // back-substitution data of its four systems [field][system][line][k]
-  double *cwr[2], *cwb[2];
+  Global<double> cwr[2], cwb[2];
   // sweeps of long lines: rows A, B, C and right-hand side of every system
   // [field][interface k][system], system = (line*nvars + var)*4 + r
   // (r: uL, uR, fL, fR), written by k_lrows and solved in place by k_lsolve
-  double *lrow[2];
-  int *status;   // bit 0: a zero pivot met in a line solve (tridiagLU.c:139-142 returns -1)
+  Global<double> lrow[2];
+  Global<int> status;   // bit 0: a zero pivot met in a line solve (tridiagLU.c:139-142 returns -1)
 };
 
-// Kernel classes launched per RK stage (plus the final update).  K_STAGE fills
-// the ghost points too and K_FLUX the line systems' end values and the viscous
+// Kernel classes launched per RK stage.  K_STAGE fills the ghost points too
+// (fused cases need it at the start of a call only) and K_FLUX the line systems' end values and the viscous
 // fluxes; K_GHOST, K_ENDS and K_FLUXALL (the cell fluxes of every case, those
 // of K_WENO among them, which forms its own) do one thing for the operators.
 // K_LINE* and K_TUBE advance 1D cases by whole steps (line.hip).
 enum KClass {
   K_STAGE = 0, K_GHOST, K_FLUX, K_ENDS, K_RECON, K_LROWS = K_RECON + 10, K_LSOLVE, K_CWROWS, K_CWSOLVE, K_WENO, K_UPWIND,
-  K_BFLUX, K_ASSEMBLE, K_UPDATE, K_FLUXALL,
+  K_BFLUX, K_ASSEMBLE, K_NEXT, K_GHOSTNEXT, K_UPDATE, K_FLUXALL,
   K_LINE4, K_LINE8, K_TUBE, K_TUBEBACK,
   K_NCLASS
 };
@@ -168,7 +195,7 @@ const char *kclass_name(int k);
 
 // Block -> case tables of every kernel class for one ensemble.
 struct Plan {
-  int ncases = 0;
+  int ncases = 0, nfused = 0;
   bool stage64 = false;  // k_stage with 64 x 64 tiles (every case at least 2048 x 2048)
   int nblocks[K_NCLASS] = {0};
   int *blockcase[K_NCLASS] = {nullptr};   // device arrays, one int per block
@@ -247,8 +274,15 @@ typedef void (*MarkFn)(void *ctx, int cls, bool begin, hipStream_t st);
 // K_GHOST ends with the stage state, K_FLUX with the cell fluxes.
 void launch_stage(const CaseDev *d_cases, const Plan &plan, int s, hipStream_t st, MarkFn mark, void *mark_ctx,
                   int last = K_NCLASS);
-// u += dt*b_s*Udot_s for every stage, time += dt.
-void launch_update(const CaseDev *d_cases, const Plan &plan, hipStream_t st);
+// A step: launch_begin once before the first of a call's steps, then every stage
+// of each step with launch_step_stage (d_cases: the table of all stages) and
+// launch_update.  Fused cases go through k_next, the others through the stage
+// state, the assembly and the update u += dt*b_s*Udot_s, time += dt.
+void launch_begin(const CaseDev *d_cases, const Plan &plan, hipStream_t st, MarkFn mark, void *mark_ctx);
+void launch_step_stage(const CaseDev *d_cases, const Plan &plan, int s, hipStream_t st, MarkFn mark, void *mark_ctx);
+void launch_update(const CaseDev *d_cases, const Plan &plan, hipStream_t st, MarkFn mark, void *mark_ctx);
+// How the ghost points of each face of a case are filled (CaseDev::push).
+void choose_push(CaseDev &c);
 
 // diagnostics (single case): per-block partial max CFL and sum of squared
 // step differences of the interior state

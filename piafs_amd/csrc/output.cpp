@@ -110,7 +110,7 @@ int Case::write_species(const std::string &dir, const std::string &suffix, doubl
   if (rc) return rc;
   if (stage_time >= 0.0 && nz > 1) {
     Us.resize((size_t)np * nv);
-    if ((rc = download(Us.data(), st, h.U))) return rc;
+    if ((rc = download(Us.data(), st, h.Us[cfg.nstages - 1]))) return rc;
   }
   // ChemistrySetPhotonDensity (ChemistrySolve.c:33-60) at the interior points
   std::vector<double> hnu((size_t)np * nz, 0.0);

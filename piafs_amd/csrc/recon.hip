@@ -120,7 +120,7 @@ __device__ __forceinline__ void recon_pair(const CaseDev &C, int dir, long sys, 
       for (int i = 0; i < MR; i++) stash[i * BT + threadIdx.x] = X[i];  // this lane's own rows
   }
   if (sides & 2) solve(std::integral_constant<bool, false>(), 1);
-  double *const *io = dir ? C.iy : C.ix;
+  const Global<double> *io = dir ? C.iy : C.ix;
   if (!C.paired) {  // interior interfaces of uL, uR / fL, fR apart
     for (int side = sides == 2 ? 1 : 0; side < (sides == 1 ? 1 : 2); side++) {
       sync();  // the windows, or the side before, are read
@@ -185,12 +185,11 @@ __device__ __forceinline__ void recon_pair(const CaseDev &C, int dir, long sys, 
 #pragma unroll
       for (int it = 0; it < KO; it++) {
         const int k = it * T + lane;
-        if (k <= N) {
-          const bool end = k == 0 || k == N;
-          const double fs = end ? io[1][line + k] : Lf[slot(k)];
-          const double ud = end ? io[0][line + k] : Lu[slot(k)];
-          fo[k] = fs - dvv[it] * ud;
-        }
+        if (k > 0 && k < N) fo[k] = Lf[slot(k)] - dvv[it] * Lu[slot(k)];
+      }
+      if (lane < 2) {  // apart: one load for either would be a FLAT one of LDS or memory
+        const int k = lane ? N : 0;
+        fo[k] = io[1][line + k] - C.dsp[dir][(long)l * (N + 1) + k] * io[0][line + k];
       }
     }
     return;

@@ -77,6 +77,13 @@ static bool species_dsp(const Config &c) {
          c.upwind == UPW_ROE;
 }
 
+// Stage states a case keeps apart (CaseDev::Us): with chemistry two, in turn, or
+// one per stage where two would give a step's last and first stage the same
+static int stage_buffers(const Config &c) {
+  if (c.ndims != 2 || c.nstages < 2 || !c.include_chem) return 1;
+  return c.nstages % 2 ? c.nstages : 2;
+}
+
 size_t Case::plan_bytes(const Config &c) {
   Grid g = make_grid(c);
   size_t plane = g.plane, nv = c.nvars;
@@ -90,6 +97,7 @@ size_t Case::plan_bytes(const Config &c) {
     n += (size_t)(cw_row_fields(nf, (int)nv) + 4 * cw_back_fields(nf, (int)nv)) * (ix + iy) / nv;
   }
   if (c.model_id == MODEL_NS2D) n += 6 * (size_t)g.nxg * g.nyg;
+  n += (stage_buffers(c) - 1) * nv * plane;
   if (c.crweno && !c.characteristic) {  // long-line scratch of sweeps longer than one team
     int T, m;
     for (int d = 0; d < c.ndims; d++)
@@ -203,7 +211,12 @@ int Case::setup(int dev, hipStream_t st) {
   const size_t st_sz = (size_t)nv * G.plane;
   const bool two = (cfg.ndims == 2);
   D.u = dalloc(st_sz, st);
-  D.U = dalloc(st_sz, st);
+  D.fused = two && cfg.nstages >= 2;
+  choose_push(D);
+  for (int k = 0; k < stage_buffers(cfg); k++)
+    if (!(D.Us[k] = dalloc(st_sz, st))) return fail(-2, "device allocation failed");
+  for (int s = stage_buffers(cfg); s < cfg.nstages; s++) D.Us[s] = D.Us[s % stage_buffers(cfg)];
+  D.U = D.Us[0];
   if (two) D.UT = dalloc(st_sz, st);
   for (int s = 0; s < cfg.nstages; s++) D.Udot[s] = dalloc(st_sz, st);
   D.flux_x = dalloc(st_sz, st);
@@ -233,7 +246,7 @@ int Case::setup(int dev, hipStream_t st) {
   D.xc = dalloc(cfg.x.size(), st);
   D.bcvals = dalloc(zvals.size() + 1, st);
   D.imap = dalloc(G.plane, st);
-  D.time = dalloc(1, st);
+  D.time = dalloc(2, st);
   // characteristic CRWENO5 scratch (block rows and back-substitution data per sweep)
   if (cfg.characteristic && cfg.crweno) {
     const int nf = cfg.model_id == MODEL_EULER1D ? 3 : 4;
@@ -442,10 +455,21 @@ int Engine::build() {
   plan.stage64 = true;
   for (int k = 0; k < nc; k++) plan.stage64 = plan.stage64 && stage_tile_64(hd[k]);
   for (int k = 0; k < nc; k++) hd[k].stage_tile = plan.stage64 ? 64 : 32;
-  HIPCHK(hipMalloc(&p, nc * sizeof(CaseDev)));
+  plan.nfused = 0;
+  for (const CaseDev &c : hd) plan.nfused += c.fused;
+  std::vector<CaseDev> table;  // an entry of every case per stage
+  for (int s = 0; s < (plan.nfused ? 4 : 1); s++)
+    for (CaseDev c : hd) {
+      if (c.fused && s < c.nstages) {
+        c.U = c.Us[s];
+        c.Un = c.Us[(s + 1) % c.nstages];
+      }
+      table.push_back(c);
+    }
+  HIPCHK(hipMalloc(&p, table.size() * sizeof(CaseDev)));
   plan_allocs.push_back(p);
   d_cases = (CaseDev *)p;
-  HIPCHK(hipMemcpyAsync(d_cases, hd.data(), nc * sizeof(CaseDev), hipMemcpyHostToDevice, stream));
+  HIPCHK(hipMemcpyAsync(d_cases, table.data(), table.size() * sizeof(CaseDev), hipMemcpyHostToDevice, stream));
   for (int cls = 0; cls < K_NCLASS; cls++) {
     std::vector<int> bc, first(nc);
     for (int k = 0; k < nc; k++) {
@@ -467,7 +491,7 @@ int Engine::build() {
     HIPCHK(hipMemcpyAsync(p, first.data(), nc * sizeof(int), hipMemcpyHostToDevice, stream));
     HIPCHK(hipStreamSynchronize(stream));
   }
-  HIPCHK(hipStreamSynchronize(stream));  // hd is a host temporary
+  HIPCHK(hipStreamSynchronize(stream));  // table is a host temporary
   bool all = true;
   for (const CaseDev &c : hd) all = all && line_class(c) >= 0;
   if (all) lines = std::move(hd);
@@ -501,10 +525,8 @@ void Engine::enqueue_step() {
   int ns = 0;
   for (Case *c : cases) ns = std::max(ns, c->cfg.nstages);
   for (int s = 0; s < ns; s++)
-    launch_stage(d_cases, plan, s, stream, profiling ? mark_cb : nullptr, this);
-  if (profiling) mark(K_UPDATE, true, stream);
-  launch_update(d_cases, plan, stream);
-  if (profiling) mark(K_UPDATE, false, stream);
+    launch_step_stage(d_cases, plan, s, stream, profiling ? mark_cb : nullptr, this);
+  launch_update(d_cases, plan, stream, profiling ? mark_cb : nullptr, this);
 }
 
 // Capture one step of the current member set into a graph (once per member set).
@@ -536,8 +558,10 @@ int Engine::step(int n) {
       int rc = prepare();
       if (rc) return rc;
     }
+    if (n > 0) launch_begin(d_cases, plan, stream, nullptr, nullptr);
     for (int i = 0; i < n; i++) HIPCHK(hipGraphLaunch(gexec, stream));
   } else {
+    if (n > 0) launch_begin(d_cases, plan, stream, profiling ? mark_cb : nullptr, this);
     for (int i = 0; i < n; i++) enqueue_step();
   }
   HIPCHK(hipGetLastError());
