@@ -74,13 +74,15 @@ __device__ __forceinline__ void weno_of(double c1, double c2, double c3, double 
 template <int KIND>
 __device__ __forceinline__ void weno_w(double c1, double c2, double c3, double m3, double m2, double m1,
                                        double p1, double p2, double eps, double &w1, double &w2, double &w3) {
+  // 2, 4 and 1/4 scale exactly, so each of those products joins its sum in one
+  // fma with the same bits
   const double t1312 = 13.0 / 12.0, q14 = 1.0 / 4.0;
-  const double d1 = m3 - 2 * m2 + m1, e1 = m3 - 4 * m2 + 3 * m1;
-  const double d2 = m2 - 2 * m1 + p1, e2 = m2 - p1;
-  const double d3 = m1 - 2 * p1 + p2, e3 = 3 * m1 - 4 * p1 + p2;
-  const double b1 = t1312 * d1 * d1 + q14 * e1 * e1;
-  const double b2 = t1312 * d2 * d2 + q14 * e2 * e2;
-  const double b3 = t1312 * d3 * d3 + q14 * e3 * e3;
+  const double d1 = __builtin_fma(-2.0, m2, m3) + m1, e1 = __builtin_fma(-4.0, m2, m3) + 3 * m1;
+  const double d2 = __builtin_fma(-2.0, m1, m2) + p1, e2 = m2 - p1;
+  const double d3 = __builtin_fma(-2.0, p1, m1) + p2, e3 = __builtin_fma(-4.0, p1, 3 * m1) + p2;
+  const double b1 = __builtin_fma(q14, e1 * e1, t1312 * d1 * d1);
+  const double b2 = __builtin_fma(q14, e2 * e2, t1312 * d2 * d2);
+  const double b3 = __builtin_fma(q14, e3 * e3, t1312 * d3 * d3);
   const double t = KIND == 3 ? m3 - 4 * m2 + 6 * m1 - 4 * p1 + p2 : 0.0;
   weno_of<KIND>(c1, c2, c3, b1, b2, b3, t, eps, w1, w2, w3);
 }
@@ -569,10 +571,13 @@ __device__ __forceinline__ int xcd_order(int id, int nb, int first) {
   return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + k;
 }
 
+// A plan of one case has no tables: a launch's first loads are then of the case
+// itself, a memory round trip earlier.
 #define CASE_PREAMBLE                                                      \
-  const int cidx = blockcase[blockIdx.x];                                  \
+  const int cidx = blockcase ? blockcase[blockIdx.x] : 0;                  \
+  const int first = blockcase ? firstblock[cidx] : 0;                      \
   const CaseDev &C = cases[cidx];                                          \
-  const long t = (long)(blockIdx.x - firstblock[cidx]) * blockDim.x + threadIdx.x; \
+  const long t = (long)((int)blockIdx.x - first) * blockDim.x + threadIdx.x; \
   (void)stage;
 
 }  // namespace

@@ -98,7 +98,7 @@ __device__ __forceinline__ void stage_body(CASE_ARGS) {
   const int s = stage & 0xFF;
   if (s >= C.nstages || skipped(C, stage)) return;
   const Grid &G = C.G;
-  const int bid = (int)(blockIdx.x - firstblock[cidx]), ns = stage_blocks(G, ST);
+  const int bid = (int)blockIdx.x - first, ns = stage_blocks(G, ST);
   if (bid >= ns) {
     ghost_body(C, t - (long)ns * TB, [&](long p) { return stage_value(C, s, p); }, C.U);
     return;
@@ -118,7 +118,7 @@ __device__ __forceinline__ void stage_body(CASE_ARGS) {
   // (64-point tiles: workgroup order, which timed faster for them at 4096^2);
   // the case's block count is padded to a multiple of eight
   const int nb = G.nv * ntx * nty;
-  const int id = ST == 32 ? xcd_order(bid, ns, firstblock[cidx]) : bid;
+  const int id = ST == 32 ? xcd_order(bid, ns, first) : bid;
   if (id >= nb) return;
   const int v = id / (ntx * nty), rem = id % (ntx * nty);
   const int i0 = (rem % ntx) * ST, j0 = (rem / ntx) * ST;
@@ -280,7 +280,7 @@ __global__ void __launch_bounds__(256) k_flux(CASE_ARGS) {
   CASE_PREAMBLE
   if (stage >= C.nstages) return;
   __shared__ Prims prims;
-  const int bid = (int)(blockIdx.x - firstblock[cidx]);
+  const int bid = (int)blockIdx.x - first;
   const int nvis = viscous_blocks(C), nends = (int)((end_items(C) + TB - 1) / TB);
   if (bid < nvis) viscous_tile(C, bid, prims);
   else if (bid < nvis + nends) recon_ends_item(C, t - (long)nvis * TB, 0, false);
@@ -1141,7 +1141,7 @@ __global__ void __launch_bounds__(kLongTeam) k_lsolve(CASE_ARGS) {
   const int nv = C.G.nv;
   const long nX = long_pairs(C.Sx, nv);
   const long nY = C.G.ndims == 2 ? long_pairs(C.Sy, nv) : 0;
-  const long pair = blockIdx.x - firstblock[cidx];
+  const long pair = (int)blockIdx.x - first;
   if (pair >= nX + nY) return;  // uniform over the block
   const int dir = pair < nX ? 0 : 1;
   const long p = dir ? pair - nX : pair;  // (line*nv + var)*2 + q
@@ -1680,7 +1680,7 @@ __global__ void __launch_bounds__(kTileThreads) k_assemble(CASE_ARGS) {
     return;
   }
   __shared__ Tile sh;
-  assemble_tile<false>(C, s, (int)(blockIdx.x - firstblock[cidx]), firstblock[cidx], sh);
+  assemble_tile<false>(C, s, (int)blockIdx.x - first, first, sh);
 }
 
 // The assembly with what follows from it point by point: the next stage's state
@@ -1695,7 +1695,7 @@ __global__ void __launch_bounds__(kTileThreads) k_next(CASE_ARGS) {
   (void)t;
   if (stage >= C.nstages) return;
   __shared__ Tile sh;
-  assemble_tile<true>(C, stage, (int)(blockIdx.x - firstblock[cidx]), firstblock[cidx], sh);
+  assemble_tile<true>(C, stage, (int)blockIdx.x - first, first, sh);
 }
 
 // u += (dt*b_s) * Udot_s stage by stage (TimeRK.c:86-99) at interior points;

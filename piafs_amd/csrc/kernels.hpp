@@ -198,7 +198,7 @@ struct Plan {
   int ncases = 0, nfused = 0;
   bool stage64 = false;  // k_stage with 64 x 64 tiles (every case at least 2048 x 2048)
   int nblocks[K_NCLASS] = {0};
-  int *blockcase[K_NCLASS] = {nullptr};   // device arrays, one int per block
+  int *blockcase[K_NCLASS] = {nullptr};   // device arrays, one int per block (null: one case has all blocks)
   int *firstblock[K_NCLASS] = {nullptr};  // device arrays, one int per case
 };
 

@@ -66,7 +66,7 @@ __device__ __forceinline__ void line_system(const CaseDev &C, const double *src,
 template <int MR>
 __global__ void __launch_bounds__(kLineThreads) k_line(CASE_ARGS) {
   extern __shared__ double lds[];
-  const CaseDev &C = cases[blockcase[blockIdx.x]];
+  const CaseDev &C = cases[blockcase ? blockcase[blockIdx.x] : 0];
   const int N = C.Sx.N, nv = C.G.nv, ns = C.nstages, g = C.G.g, P = N + 6, tid = threadIdx.x;
   const double gam = C.P.gamma;
   double *u = lds, *U = u + nv * N + 3, *F = U + nv * P, *Ud = F + nv * P - 3, *io = Ud + ns * nv * N;
@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(256) k_tube(CASE_ARGS) {
   __shared__ Rows rows;
   __shared__ double u0[kTubeVars][kWin], U[kTubeVars][kWin + 6], Ud[4][kTubeVars][kWin], f[kTubeVars][64];
   const int N = C.Sx.N, nv = C.G.nv, ns = C.nstages, g = C.G.g, tid = threadIdx.x;
-  const int lost = 3 * (ns - 1), core = tube_core(ns), bid = (int)blockIdx.x - firstblock[cidx];
+  const int lost = 3 * (ns - 1), core = tube_core(ns), bid = (int)(int)blockIdx.x - first;
   const int c0 = bid * core - lost;  // the window's first point
   const bool wraps = C.nzones > 0 && C.zones[0].kind == Z_PERIODIC;
   const double *src = stage ? C.Udot[0] : C.u;

@@ -213,7 +213,7 @@ k_recon(CASE_ARGS) {
   __shared__ double stash[MR * BT];
   __shared__ double lines[recon_line_doubles(MR, BT)];
   __shared__ unsigned arrived[2];
-  int bid = (int)(blockIdx.x - firstblock[cidx]);
+  int bid = (int)blockIdx.x - first;
   int dir = 0, sides = 3;
   if (only) {
     dir = (only >> 3) & 1;

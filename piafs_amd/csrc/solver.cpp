@@ -470,28 +470,31 @@ int Engine::build() {
   plan_allocs.push_back(p);
   d_cases = (CaseDev *)p;
   HIPCHK(hipMemcpyAsync(d_cases, table.data(), table.size() * sizeof(CaseDev), hipMemcpyHostToDevice, stream));
+  // block tables of every class, one after the other; one case needs none
+  std::vector<std::array<int, K_NCLASS>> blocks(nc);
+  for (int k = 0; k < nc; k++) case_blocks(hd[k], blocks[k].data());
+  std::vector<int> tab;
+  size_t at[K_NCLASS] = {0};
   for (int cls = 0; cls < K_NCLASS; cls++) {
-    std::vector<int> bc, first(nc);
-    for (int k = 0; k < nc; k++) {
-      int b[K_NCLASS];
-      case_blocks(hd[k], b);
-      first[k] = (int)bc.size();
-      for (int j = 0; j < b[cls]; j++) bc.push_back(k);
-    }
-    plan.nblocks[cls] = (int)bc.size();
-    if (bc.empty()) continue;
-    HIPCHK(hipMalloc(&p, bc.size() * sizeof(int)));
-    plan_allocs.push_back(p);
-    plan.blockcase[cls] = (int *)p;
-    HIPCHK(hipMemcpyAsync(p, bc.data(), bc.size() * sizeof(int), hipMemcpyHostToDevice, stream));
-    HIPCHK(hipStreamSynchronize(stream));  // bc and first are host temporaries
-    HIPCHK(hipMalloc(&p, nc * sizeof(int)));
-    plan_allocs.push_back(p);
-    plan.firstblock[cls] = (int *)p;
-    HIPCHK(hipMemcpyAsync(p, first.data(), nc * sizeof(int), hipMemcpyHostToDevice, stream));
-    HIPCHK(hipStreamSynchronize(stream));
+    int n = 0;
+    for (int k = 0; k < nc; k++) n += blocks[k][cls];
+    plan.nblocks[cls] = n;
+    if (nc == 1 || n == 0) continue;
+    at[cls] = tab.size();
+    for (int k = 0; k < nc; k++) tab.insert(tab.end(), blocks[k][cls], k);
+    for (int k = 0, first = 0; k < nc; first += blocks[k++][cls]) tab.push_back(first);
   }
-  HIPCHK(hipStreamSynchronize(stream));  // table is a host temporary
+  if (!tab.empty()) {
+    HIPCHK(hipMalloc(&p, tab.size() * sizeof(int)));
+    plan_allocs.push_back(p);
+    HIPCHK(hipMemcpyAsync(p, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice, stream));
+    for (int cls = 0; cls < K_NCLASS; cls++) {
+      if (plan.nblocks[cls] == 0) continue;
+      plan.blockcase[cls] = (int *)p + at[cls];
+      plan.firstblock[cls] = plan.blockcase[cls] + plan.nblocks[cls];
+    }
+  }
+  HIPCHK(hipStreamSynchronize(stream));  // table and tab are host temporaries
   bool all = true;
   for (const CaseDev &c : hd) all = all && line_class(c) >= 0;
   if (all) lines = std::move(hd);

@@ -18,7 +18,7 @@ namespace {
 // one or two waves per SIMD waiting on their own chains.  Per stage, cell
 // fluxes, end interfaces, reconstruction and upwinding as separate passes ->
 // one thread per interface -> this: 600 x 343, 11 variables, components 186 ->
-// 146 -> 100 us; 500 x 100, 11 variables, characteristic 63 -> 48 -> 35;
+// 146 -> 95 us; 500 x 100, 11 variables, characteristic 63 -> 48 -> 35;
 // 201 x 201, 4 variables, characteristic 36 -> 28 -> 21; 1024-point line,
 // characteristic 17 -> 8.2 -> 7.9.
 __global__ void __launch_bounds__(256) k_weno(CASE_ARGS) {
@@ -29,14 +29,14 @@ __global__ void __launch_bounds__(256) k_weno(CASE_ARGS) {
     Prims prims;
   } lds;
   const int nvis = viscous_blocks(C);
-  if ((int)(blockIdx.x - firstblock[cidx]) < nvis) {
-    viscous_tile(C, (int)(blockIdx.x - firstblock[cidx]), lds.prims);
+  if ((int)blockIdx.x - first < nvis) {
+    viscous_tile(C, (int)blockIdx.x - first, lds.prims);
     return;
   }
   Rows &sh = lds.rows;
   const long nX = (long)(C.Sx.N + 1) * C.Sx.nlines;
   const int nbx = (int)((nX + 63) / 64);
-  const int bid = (int)(blockIdx.x - firstblock[cidx]) - nvis;
+  const int bid = (int)blockIdx.x - first - nvis;
   const int dir = bid < nbx ? 0 : 1;
   const long item = (long)(dir ? bid - nbx : bid) * 64 + (threadIdx.x & 63);
   const int uw = bid & 3;  // in turn, since a block's waves sit on the SIMDs in order
