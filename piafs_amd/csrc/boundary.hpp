@@ -120,6 +120,24 @@ __device__ __forceinline__ double ghost_value(const CaseDev &C, int v, int i, in
   return igm1 * pg + 0.5 * rg * (ug * ug + vg * vg);
 }
 
+// Position i outside a line: whether its ghost values are copies of one interior
+// point's in every variable; then that point, and 1 or -1 to multiply with.
+// (The zone is found once; ghost_value looks for it, through dependent loads, at
+// every call.)
+__device__ __forceinline__ bool ghost_copy_1d(const CaseDev &C, int i, int &src, double &fac) {
+  const int N = C.G.nx, face = i < 0 ? 1 : -1;
+  int z = C.nzones - 1;
+  for (; z >= 0; z--) {
+    const Zone &Z = C.zones[z];
+    if (Z.kind != Z_SPONGE && Z.dim == 0 && Z.face == face && zone_sets(Z, 0, 1)) break;
+  }
+  if (z < 0) return false;
+  const int kind = C.zones[z].kind;
+  src = kind == Z_PERIODIC ? i + face * N : face == 1 ? -i - 1 : 2 * N - i - 1;
+  fac = kind == Z_REFLECT ? -1.0 : 1.0;
+  return kind == Z_PERIODIC || kind == Z_EXTRAPOLATE || kind == Z_REFLECT;
+}
+
 }  // namespace
 
 }  // namespace piafs

@@ -465,29 +465,39 @@ __device__ __forceinline__ void rf_ns2d(double g, bool llf, const double uLk[4],
   es[2] = eR[3];
 }
 
-// Euler1DUpwindRoe (Euler1DUpwind.c:27-93): returns the species' coefficient
-__device__ __forceinline__ double roe_e1d(double g, const double uLc[3], const double uRc[3], const double ud[3],
-                                          const double fs[3], double fo[3]) {
-  double a0, a1, a2;
-  euler1d_roeavg(g, uLc[0], uLc[1], uLc[2], uRc[0], uRc[1], uRc[2], a0, a1, a2);
-  Eig3 E;
-  euler1d_eig(g, a0, a1, a2, E);
+// Euler1DUpwindRoe (Euler1DUpwind.c:27-93): |A| = R |D| L of the average's
+// eigenstructure, with the species' coefficient returned, and the flux from it
+__device__ __forceinline__ double roe_matrix_e1d(const Eig3 &E, double A[3][3]) {
   double DL[3][3];
 #pragma unroll
   for (int i = 0; i < 3; i++)
 #pragma unroll
     for (int j = 0; j < 3; j++) DL[i][j] = fabs(E.D[i]) * E.L[i][j];
 #pragma unroll
+  for (int i = 0; i < 3; i++)
+#pragma unroll
+    for (int j = 0; j < 3; j++) A[i][j] = E.R[i][0] * DL[0][j] + E.R[i][1] * DL[1][j] + E.R[i][2] * DL[2][j];
+  return fabs(E.D[0]);
+}
+__device__ __forceinline__ void roe_apply_e1d(const double A[3][3], const double ud[3], const double fs[3],
+                                              double fo[3]) {
+#pragma unroll
   for (int i = 0; i < 3; i++) {
     double us = 0.0;
 #pragma unroll
-    for (int j = 0; j < 3; j++) {
-      const double mA = E.R[i][0] * DL[0][j] + E.R[i][1] * DL[1][j] + E.R[i][2] * DL[2][j];
-      us += mA * ud[j];
-    }
+    for (int j = 0; j < 3; j++) us += A[i][j] * ud[j];
     fo[i] = fs[i] - us;
   }
-  return fabs(E.D[0]);
+}
+__device__ __forceinline__ double roe_e1d(double g, const double uLc[3], const double uRc[3], const double ud[3],
+                                          const double fs[3], double fo[3]) {
+  double a0, a1, a2, A[3][3];
+  euler1d_roeavg(g, uLc[0], uLc[1], uLc[2], uRc[0], uRc[1], uRc[2], a0, a1, a2);
+  Eig3 E;
+  euler1d_eig(g, a0, a1, a2, E);
+  const double c = roe_matrix_e1d(E, A);
+  roe_apply_e1d(A, ud, fs, fo);
+  return c;
 }
 
 // Euler1DUpwindRusanov (Euler1DUpwind.c:282-353); its wave speed is gamma P/rho

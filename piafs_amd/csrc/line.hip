@@ -40,8 +40,11 @@ __device__ __forceinline__ void line_system(const CaseDev &C, const double *src,
 #pragma unroll
   for (int j = 0; j < MR + 5; j++) w[j] = lo - 3 + j <= N + 2 ? src[lo - 3 + j] : 0.0;
   assemble_rows<MR, KIND, LEFT>(C.R, w, A, B, Cc, X);
-  row_coeffs<KIND>(0, N, LEFT, C.R, src[-3], src[-2], src[-1], src[0], src[1], src[2], a, b, c, x0);
-  row_coeffs<KIND>(N, N, LEFT, C.R, src[N - 3], src[N - 2], src[N - 1], src[N], src[N + 1], src[N + 2], a, b, c, xN);
+  // the end values, one on each half of the team (of two lanes or more)
+  const double *e = lane < T / 2 ? src : src + N;
+  row_coeffs<KIND>(0, N, LEFT, C.R, e[-3], e[-2], e[-1], e[0], e[1], e[2], a, b, c, x0);
+  xN = __shfl(x0, T - 1, T);
+  x0 = __shfl(x0, 0, T);
   if (lo + MR > N) {
 #pragma unroll
     for (int i = 0; i < MR; i++) {
@@ -82,12 +85,18 @@ __global__ void __launch_bounds__(kLineThreads) k_line(CASE_ARGS) {
   while (T * MR < N - 1) T <<= 1;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), per = 64 / T, groups = (2 * nv + per - 1) / per;
   const int lane = tid & (T - 1), sub = (tid & 63) / T;
+  static_assert(2 * 256 + 1 + 6 <= kLineThreads, "a thread has one position at most");
+  int gsrc = 0;
+  double gfac = 0.0;
+  const bool ghost = tid < P && (tid < 3 || tid >= N + 3), copies = ghost && ghost_copy_1d(C, tid - 3, gsrc, gfac);
   for (int step = 0; step < stage; step++)
     for (int s = 0; s < ns; s++) {
       // ghost values and the cell flux, a thread per position
-      for (int p = tid; p < P; p += kLineThreads) {
-        const int i = p - 3;
-        if (i < 0 || i >= N)
+      if (tid < P) {
+        const int i = tid - 3;
+        if (copies)
+          for (int v = 0; v < nv; v++) U[v * P + i] = gfac * U[v * P + gsrc];
+        else if (ghost)
           for (int v = 0; v < nv; v++)
             U[v * P + i] = ghost_value(C, v, i, 0, [&](int m, int a, int) { return U[m * P + a]; });
         point_flux(1, 0, gam, nv, [&](int m) { return U[m * P + i]; }, [&](int m, double x) { F[m * P + i] = x; });
@@ -190,12 +199,19 @@ __global__ void __launch_bounds__(256) k_tube(CASE_ARGS) {
     U[v][p] = x;
     if (p >= 3 && p < kWin + 3) u0[v][p - 3] = x;
   }
+  // this thread's ghost value, if it has one in the window
+  const int gv = tid / 6, gi = tid % 6 < 3 ? tid % 6 - 3 : N + tid % 6 - 3, gp = gi - c0 + 3;
+  const bool ghost = !wraps && tid < 6 * nv && gp >= 0 && gp < kWin + 6;
+  int gsrc = 0;
+  double gfac = 0.0;
+  const bool copies = ghost && ghost_copy_1d(C, gi, gsrc, gfac);
   for (int s = 0; s < ns; s++) {
     __syncthreads();
-    if (!wraps && tid < 6 * nv) {
-      const int v = tid / 6, o = tid % 6, i = o < 3 ? o - 3 : N + o - 3, p = i - c0 + 3;
-      if (p >= 0 && p < kWin + 6)
-        U[v][p] = ghost_value(C, v, i, 0, [&](int m, int a, int) { return U[m][a - c0 + 3]; });
+    if (copies) {
+      U[gv][gp] = gfac * U[gv][gsrc - c0 + 3];
+    } else if (ghost) {
+      const int v = gv, i = gi, p = gp;
+      U[v][p] = ghost_value(C, v, i, 0, [&](int m, int a, int) { return U[m][a - c0 + 3]; });
     }
     __syncthreads();
     const int x = tid & 63;

@@ -52,6 +52,13 @@ __device__ __forceinline__ void weno_tile(const CaseDev &C, const double *__rest
   const int nv = C.G.nv, x = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const double g = C.P.gamma;
+  const int mode = C.upwind;
+  // Roe in 1D: the last wave has no variable to reconstruct, so it forms |A| of
+  // the two cells' average then and upwinds
+  const bool early = MODEL == 1 && mode == 0;
+  if (early) uw = 3;
+  Eig3 E;
+  double A[3][3], es1 = 0.0;
   auto cells = [&](double uLc[4], double uRc[4]) {  // the two cells beside the interface
 #pragma unroll
     for (int m = 0; m < NF; m++) {
@@ -76,7 +83,6 @@ __device__ __forceinline__ void weno_tile(const CaseDev &C, const double *__rest
     if constexpr (MODEL == 1) {
       double a0, a1, a2;
       euler1d_roeavg(g, uLc[0], uLc[1], uLc[2], uRc[0], uRc[1], uRc[2], a0, a1, a2);
-      Eig3 E;
       euler1d_eig(g, a0, a1, a2, E);
 #pragma unroll
       for (int i = 0; i < 3; i++)
@@ -119,6 +125,16 @@ __device__ __forceinline__ void weno_tile(const CaseDev &C, const double *__rest
       sh.o[4 * (2 * src) + v][x] = vl;
       sh.o[4 * (2 * src + 1) + v][x] = vr;
     }
+  } else if (early) {
+    if constexpr (MODEL == 1) {
+      if (!CH) {
+        double uLc[4], uRc[4], a0, a1, a2;
+        cells(uLc, uRc);
+        euler1d_roeavg(g, uLc[0], uLc[1], uLc[2], uRc[0], uRc[1], uRc[2], a0, a1, a2);
+        euler1d_eig(g, a0, a1, a2, E);
+      }
+      es1 = roe_matrix_e1d(E, A);
+    }
   }
   lds_barrier();
   // 3. characteristic: back to the flow variables, wave s array s of uL, uR, fL, fR
@@ -141,10 +157,9 @@ __device__ __forceinline__ void weno_tile(const CaseDev &C, const double *__rest
     lds_barrier();
   }
   // 4. wave uw: the flow's interface flux, while the other waves begin the species
-  const int mode = C.upwind;
   if (wave == uw) {
     double uLc[4], uRc[4], fo[4];
-    if (MODEL == 1 || mode == 0 || mode == 3) cells(uLc, uRc);
+    if (!early && (MODEL == 1 || mode == 0 || mode == 3)) cells(uLc, uRc);
     auto o = [&](int a, int m) { return sh.o[4 * a + m][x]; };
     if (mode == 0 || mode == 3) {
       double ud[4], fs[4], c;
@@ -154,8 +169,10 @@ __device__ __forceinline__ void weno_tile(const CaseDev &C, const double *__rest
         fs[m] = 0.5 * (o(2, m) + o(3, m));
       }
       if (mode == 0) {
-        if constexpr (MODEL == 1) c = roe_e1d(g, uLc, uRc, ud, fs, fo);
-        else c = roe_ns2d<DIR>(g, uLc, uRc, ud, fs, fo);
+        if constexpr (MODEL == 1) {
+          roe_apply_e1d(A, ud, fs, fo);
+          c = es1;
+        } else c = roe_ns2d<DIR>(g, uLc, uRc, ud, fs, fo);
       } else {
         if constexpr (MODEL == 1) c = rusanov_e1d(g, uLc, uRc);
         else c = rusanov_ns2d<DIR>(g, uLc, uRc);
