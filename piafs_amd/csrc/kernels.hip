@@ -211,21 +211,28 @@ __device__ __forceinline__ void recon_ends_item(const CaseDev &C, long t, int on
   const SweepGeom &S = dir ? C.Sy : C.Sx;
   const long pl = S.plane, at = S.base + (long)l * S.line_stride + (e ? S.N : 0) - 3;
   const double *u = (dir ? C.UT : C.U) + at, *f = (dir ? C.flux_y : C.flux_x) + at;
+  const int nf = C.model == 1 ? 3 : 4;
   double w[6];
+  // three positions at a time, every load before the first is needed (with a branch
+  // per position a wave took 17000 cycles, six round trips one after the other)
 #pragma unroll
-  for (int p = 0; p < 6; p++) {
-    if (q == 0) {
-      w[p] = u[v * pl + p];
-    } else if (from_flux) {
-      w[p] = f[v * pl + p];
-    } else {
+  for (int h = 0; h < 6; h += 3) {
+    double c[3][4], x[3];
+    const double *own = (from_flux && q ? f : u) + v * pl + h;
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+      x[p] = own[p];
+#pragma unroll
+      for (int m = 0; m < 4; m++) c[p][m] = from_flux ? 0.0 : u[min(m, nf - 1) * pl + h + p];
+    }
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+      w[h + p] = x[p];
+      if (from_flux) continue;
       double y = 0.0;
-      const int nf = C.model == 1 ? 3 : 4;
-      point_flux(C.model, dir, C.P.gamma, nf + 1, [&](int m) { return u[(m < nf ? m : v) * pl + p]; },
-                 [&](int m, double x) {
-                   if (m == (v < nf ? v : nf)) y = x;
-                 });
-      w[p] = y;
+      point_flux(C.model, dir, C.P.gamma, nf + 1, [&](int m) { return m < nf ? c[p][m] : x[p]; },
+                 [&](int m, double z) { y = m == (v < nf ? v : nf) ? z : y; });
+      w[h + p] = q ? y : x[p];
     }
   }
   switch (C.R.kind) {
@@ -247,7 +254,9 @@ __host__ __device__ inline long flux_items(const CaseDev &C) {
          (C.G.ndims == 2 ? (long)(C.Sy.N + 2 * C.Sy.g) * C.Sy.nlines : 0);
 }
 
-__device__ __forceinline__ void flux_item(const CaseDev &C, long t) {
+// all: every component in its own plane, also where the reconstruction needs the
+// velocity only
+__device__ __forceinline__ void flux_item(const CaseDev &C, long t, bool all) {
   const long nX = (long)(C.Sx.N + 2 * C.Sx.g) * C.Sx.nlines;
   const long nY = (C.G.ndims == 2) ? (long)(C.Sy.N + 2 * C.Sy.g) * C.Sy.nlines : 0;
   if (t >= nX + nY) return;
@@ -260,8 +269,14 @@ __device__ __forceinline__ void flux_item(const CaseDev &C, long t) {
   const int pos = (int)(tt % P) - S.g, l = (int)(tt / P);
   const long b = S.base + (long)l * S.line_stride + pos;
   const long pl = S.plane;
-  point_flux(C.model, dir, C.P.gamma, C.G.nv, [&](int m) { return q[m * pl + b]; },
+  const bool vn = C.vn_flux && !all;
+  const int nf = C.model == 1 ? 3 : 4;
+  point_flux(C.model, dir, C.P.gamma, vn ? nf : C.G.nv, [&](int m) { return q[m * pl + b]; },
              [&](int m, double x) { f[m * pl + b] = x; });
+  if (vn) {
+    const double rho = q[b], mom = q[(1 + dir) * pl + b];
+    f[nf * pl + b] = C.model == 2 && rho == 0 ? 0 : mom / rho;
+  }
   if (C.fuse_sp && pos >= 0 && pos <= S.N) {  // |v_n| at interface pos, between cells pos-1 and pos
     const double uLc[4] = {q[b - 1], q[pl + b - 1], q[2 * pl + b - 1], q[3 * pl + b - 1]};
     const double uRc[4] = {q[b], q[pl + b], q[2 * pl + b], q[3 * pl + b]};
@@ -275,8 +290,12 @@ __device__ __forceinline__ void flux_item(const CaseDev &C, long t) {
 // blocks of its own (the first two take longest).  One launch of a few
 // microseconds' work costs as much again; with three, and the viscous fluxes on
 // a second stream (whose fork and join cost 10 us a stage), 128 x 97 took 6.26 ms
-// where it takes 4.77, cavity 128 x 128 (k_weno's launch) 4.15 -> 2.54.
-__global__ void __launch_bounds__(256) k_flux(CASE_ARGS) {
+// where it took 4.77, cavity 128 x 128 (k_weno's launch) 4.15 -> 2.54.  Small grids
+// wait for the longest block's chain: with the loads of the viscous tiles and of
+// the ends issued together a launch takes 11.4 -> 7.7 us (128 x 97).  Large ones
+// are bound by HBM: seven waves a SIMD, which the viscous blocks' registers would
+// not allow by themselves, 78 us at 1024 x 1024, six 81, five 85.
+__global__ void __launch_bounds__(256, 7) k_flux(CASE_ARGS) {
   CASE_PREAMBLE
   if (stage >= C.nstages) return;
   __shared__ Prims prims;
@@ -284,13 +303,13 @@ __global__ void __launch_bounds__(256) k_flux(CASE_ARGS) {
   const int nvis = viscous_blocks(C), nends = (int)((end_items(C) + TB - 1) / TB);
   if (bid < nvis) viscous_tile(C, bid, prims);
   else if (bid < nvis + nends) recon_ends_item(C, t - (long)nvis * TB, 0, false);
-  else flux_item(C, t - (long)(nvis + nends) * TB);
+  else flux_item(C, t - (long)(nvis + nends) * TB, false);
 }
 
 // the cell fluxes alone, of any case (the operators)
 __global__ void __launch_bounds__(256) k_flux_all(CASE_ARGS) {
   CASE_PREAMBLE
-  if (stage < C.nstages) flux_item(C, t);
+  if (stage < C.nstages) flux_item(C, t, true);
 }
 
 // ---------------------------------------------------------------------------
@@ -2144,6 +2163,11 @@ void choose_rows(const std::vector<SweepGeom *> &sweeps, const std::vector<int> 
       sweeps[idx[k]]->team = team[k * n + pick[k]];
     }
   }
+}
+
+bool velocity_for_flux(const CaseDev &c) {
+  return c.R.crweno && !c.R.characteristic && !c.unit && !c.Sx.longl && !c.Sy.longl &&
+         c.G.nv > (c.model == 1 ? 3 : 4);
 }
 
 bool stage_tile_64(const CaseDev &c) { return c.G.ndims == 2 && (long)c.G.nx * c.G.ny >= 2048L * 2048L; }

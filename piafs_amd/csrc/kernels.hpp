@@ -144,6 +144,8 @@ struct CaseDev {
   int model, upwind, nstages;  // upwind: 0 Roe, 1 rf-char, 2 llf-char, 3 rusanov
   int paired;    // reconstruction writes 0.5*(uR-uL), 0.5*(fL+fR) only (Roe with component-wise interpolation)
   int fuse_sp;   // species interface fluxes written by the reconstruction (set by the plan; see species_in_recon)
+  int vn_flux;   // the fluxes' first species plane holds the velocity along the sweep, the reconstruction forms the
+                 // species' fluxes from it (set by the plan; see velocity_for_flux)
   Global<double> dsp[2];  // per sweep and interface: Roe-average |v_n| with the entropy fix (k_flux, when fuse_sp)
   int stage_tile; // side of k_stage's transpose tiles, 32 or 64 (set by the plan)
   int unit;      // descriptor of the device-buffer operators: the interface flux in separate passes
@@ -254,6 +256,12 @@ void case_blocks(const CaseDev &c, int blocks[K_NCLASS]);
 // Whether the reconstruction can write the species' Roe interface fluxes
 // itself (NS2D, paired Roe, teams of 32 or 64 lanes, |v_n| buffers present).
 bool species_in_recon(const CaseDev &c);
+// Whether the reconstruction can form the species' cell fluxes itself, and from how
+// many cells of a plan on it does: it saves k_flux traffic (1024 x 1024 133 -> 77
+// us, 20 members of 96 .. 320 points a side 56 -> 45) and costs the line teams a
+// load and a product a point (128 x 97: a launch of 20.8 us 0.5 us more).
+constexpr long kVnFluxCells = 1L << 15;
+bool velocity_for_flux(const CaseDev &c);
 // Whether the case is large enough for k_stage's 64 x 64 tiles.
 bool stage_tile_64(const CaseDev &c);
 // doubles per interface of the characteristic CRWENO5 scratch of one sweep:

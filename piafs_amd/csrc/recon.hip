@@ -56,7 +56,12 @@ __device__ __forceinline__ void recon_pair(const CaseDev &C, int dir, long sys, 
   const int nv = C.G.nv, N = S.N, nl = S.nlines, g = S.g, T = S.team;
   const long sy = active ? sys : 0;
   const int q = (int)(sy % 2), v = (int)((sy / 2) % nv), l = (int)((sy / 2) / nv);
-  const double *src = (q == 0 ? (dir ? C.UT : C.U) : (dir ? C.flux_y : C.flux_x)) + (long)v * S.plane + S.base +
+  // a species' flux is formed here from its values and the velocity, which takes one
+  // plane for all of them
+  const int nf = C.model == 1 ? 3 : 4;
+  const bool product = C.vn_flux && q == 1 && v >= nf;
+  const double *vel = (dir ? C.flux_y : C.flux_x) + (long)nf * S.plane + S.base + (long)l * S.line_stride;
+  const double *src = (q == 0 || product ? (dir ? C.UT : C.U) : (dir ? C.flux_y : C.flux_x)) + (long)v * S.plane + S.base +
                       (long)l * S.line_stride;
   const long line = ((long)v * nl + l) * (N + 1);
   const int lo = 1 + lane * MR;
@@ -85,7 +90,12 @@ __device__ __forceinline__ void recon_pair(const CaseDev &C, int dir, long sys, 
     const int idx = b + lane;
     if (idx < tot) {
       const int pos = idx - 2;
-      L[slot(idx)] = (active && pos <= hi_pos) ? src[pos] : 0.0;
+      double x = 0.0;
+      if (active && pos <= hi_pos) {
+        x = src[pos];
+        if (product) x = vel[pos] * x;
+      }
+      L[slot(idx)] = x;
     }
   }
   sync();

@@ -451,7 +451,12 @@ int Engine::build() {
       }
     choose_rows(sweeps, nvars);
   }
-  for (int k = 0; k < nc; k++) hd[k].fuse_sp = species_in_recon(hd[k]) ? 1 : 0;
+  long cells = 0;
+  for (const CaseDev &c : hd) cells += (long)c.G.nx * c.G.ny;
+  for (CaseDev &c : hd) {
+    c.fuse_sp = species_in_recon(c) ? 1 : 0;
+    c.vn_flux = cells >= kVnFluxCells && velocity_for_flux(c) ? 1 : 0;
+  }
   plan.stage64 = true;
   for (int k = 0; k < nc; k++) plan.stage64 = plan.stage64 && stage_tile_64(hd[k]);
   for (int k = 0; k < nc; k++) hd[k].stage_tile = plan.stage64 ? 64 : 32;

@@ -16,10 +16,8 @@ namespace {
 struct Prim {
   double vx, vy, T;
 };
-__device__ __forceinline__ Prim prim_at(long plane, double gam, const double *U, long p) {
-  const double rho = U[p];
-  const double vx = (rho == 0) ? 0 : U[plane + p] / rho, vy = (rho == 0) ? 0 : U[2 * plane + p] / rho;
-  const double e = U[3 * plane + p];
+__device__ __forceinline__ Prim prim_of(double gam, double rho, double mx, double my, double e) {
+  const double vx = (rho == 0) ? 0 : mx / rho, vy = (rho == 0) ? 0 : my / rho;
   const double vsq = (vx * vx) + (vy * vy);
   const double P = (e - 0.5 * rho * vsq) * (gam - 1.0);
   Prim r;
@@ -27,6 +25,9 @@ __device__ __forceinline__ Prim prim_at(long plane, double gam, const double *U,
   r.vy = vy;
   r.T = gam * P / rho;
   return r;
+}
+__device__ __forceinline__ Prim prim_at(long plane, double gam, const double *U, long p) {
+  return prim_of(gam, U[p], U[plane + p], U[2 * plane + p], U[3 * plane + p]);
 }
 
 // FirstDerivativeFourthOrder.c:39-132 (par4) / FirstDerivativeFirstOrder.c (bias +1)
@@ -74,13 +75,42 @@ __device__ __forceinline__ void deriv_prim(int g, bool par4, int i, int N, F P, 
 // waits for the other.  Bound by latency on small grids
 // and by HBM on large ones: the primitives of the tile and of the four points
 // beside it (one-sided stencils reach that far) are formed once into LDS, 2.25
-// divisions chains a thread instead of 21 in two passes with the derivatives
-// in memory between them.
+// division chains a thread instead of 21 in two passes with the derivatives
+// in memory between them.  A block's chain took 17000 cycles with the points
+// formed one after the other and a branch per kind of stencil, now 7500 (cavity
+// 128 x 128, k_weno's launch 9.3 -> 7.9 us).
 constexpr int kVisX = 32, kVisY = 8, kVisH = 4;
 __host__ __device__ inline int viscous_blocks(const CaseDev &C) {
   if (C.G.ndims != 2 || !C.P.viscous) return 0;
   return ((C.G.nxg + kVisX - 1) / kVisX) * ((C.G.nyg + kVisY - 1) / kVisY);
 }
+// FirstDerivativeFourthOrder.c's stencil at position i as deriv_prim has it, for
+// a wave whose lanes have different ones: five coefficients in the order of the
+// sum, from position i + off on (the middle one is zero, and its term left out,
+// away from the ends)
+struct Stencil5 {
+  int off;
+  double c[5];
+};
+__device__ __forceinline__ Stencil5 stencil5(int g, int i, int N) {
+  Stencil5 s = {-2, {1.0, -8.0, 0.0, 8.0, -1.0}};
+  if (i == -g) s = {0, {-25.0, 48.0, -36.0, 16.0, -3.0}};
+  if (i == -g + 1) s = {-1, {-3.0, -10.0, 18.0, -6.0, 1.0}};
+  if (i == N + g - 2) s = {-3, {-1.0, 6.0, -18.0, 10.0, 3.0}};
+  if (i == N + g - 1) s = {-4, {3.0, -16.0, 36.0, -48.0, 25.0}};
+  return s;
+}
+// p: the value at position i, st apart
+__device__ __forceinline__ double derive5(const Stencil5 &s, const double *p, int st) {
+  const double t12 = 1.0 / 12.0, *q = p + s.off * st;
+  double x = s.c[0] * q[0] + s.c[1] * q[st];
+  const double y = x + s.c[2] * q[2 * st];
+  x = s.c[2] == 0.0 ? x : y;
+  x = x + s.c[3] * q[3 * st];
+  x = x + s.c[4] * q[4 * st];
+  return x * t12;
+}
+
 struct Prims {
   double pr[3][kVisY + 2 * kVisH][kVisX + 2 * kVisH];
 };
@@ -92,22 +122,31 @@ __device__ __forceinline__ void viscous_tile(const CaseDev &C, int b, Prims &sh)
   const int tiles = (G.nxg + kVisX - 1) / kVisX;
   const int I0 = (b % tiles) * kVisX, J0 = (b / tiles) * kVisY;  // ghosted indices
   const double gam = P.gamma;
-  auto fill = [&](int a, int c) {  // LDS position (row a, column c)
-    const int I = I0 + c - kVisH, J = J0 + a - kVisH;
-    if (I < 0 || I >= G.nxg || J < 0 || J >= G.nyg) return;
-    const Prim q = prim_at(G.plane, gam, C.U, (long)J * G.nxg + I);
-    pr[0][a][c] = q.vx;
-    pr[1][a][c] = q.vy;
-    pr[2][a][c] = q.T;
-  };
   const int tx = threadIdx.x & (kVisX - 1), ty = threadIdx.x / kVisX;
-  fill(ty + kVisH, tx + kVisH);
-  // four rows below and four above, then the columns beside the tile
-  fill(ty < kVisH ? ty : ty + kVisY, tx + kVisH);
-  if (threadIdx.x < 2 * kVisH * kVisY) {
-    const int c = threadIdx.x & (2 * kVisH - 1), r = threadIdx.x / (2 * kVisH);
-    fill(r + kVisH, c < kVisH ? c : c + kVisX);
-  }
+  // a thread forms its own point's primitives, those of one of the four rows below
+  // and above, and the first 64 threads those of a point in the columns beside;
+  // outside the grid the nearest point's, which no stencil reads, so that all loads
+  // go out before the first is needed
+  const int side = threadIdx.x & (2 * kVisH - 1);
+  const int row[3] = {ty + kVisH, ty < kVisH ? ty : ty + kVisY, (int)threadIdx.x / (2 * kVisH) + kVisH};
+  const int col[3] = {tx + kVisH, tx + kVisH, side < kVisH ? side : side + kVisX};
+  const int nfill = threadIdx.x < 2 * kVisH * kVisY ? 3 : 2;
+  double q[3][4];
+#pragma unroll
+  for (int f = 0; f < 3; f++)
+    if (f < nfill) {
+      const int I = min(max(I0 + col[f] - kVisH, 0), G.nxg - 1), J = min(max(J0 + row[f] - kVisH, 0), G.nyg - 1);
+#pragma unroll
+      for (int m = 0; m < 4; m++) q[f][m] = elem(C.U + m * G.plane, 8u * ((unsigned)J * G.nxg + I));
+    }
+#pragma unroll
+  for (int f = 0; f < 3; f++)
+    if (f < nfill) {
+      const Prim w = prim_of(gam, q[f][0], q[f][1], q[f][2], q[f][3]);
+      pr[0][row[f]][col[f]] = w.vx;
+      pr[1][row[f]][col[f]] = w.vy;
+      pr[2][row[f]][col[f]] = w.T;
+    }
   lds_barrier();
   const int I = I0 + tx, J = J0 + ty;
   if (I >= G.nxg || J >= G.nyg) return;
@@ -129,6 +168,15 @@ __device__ __forceinline__ void viscous_tile(const CaseDev &C, int b, Prims &sh)
     const int sj = j < 0 ? j + G.ny : j - G.ny;
     deriv_prim(G.g, P.par4, i, G.nx, [&](int k, int c) { return far(k, sj, c); }, dx);
     deriv_prim(G.g, P.par4, sj, G.ny, [&](int k, int c) { return far(i, k, c); }, dy);
+  } else if (P.par4) {
+    const Stencil5 sx = stencil5(G.g, i, G.nx), sy = stencil5(G.g, j, G.ny);
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      const double *p = &pr[c][ty + kVisH][tx + kVisH];
+      const double x = derive5(sx, p, 1), y = derive5(sy, p, kVisX + 2 * kVisH);
+      dx[c] = jin ? x : 0.0;
+      dy[c] = iin ? y : 0.0;
+    }
   } else {
     if (jin)
       deriv_prim(G.g, P.par4, i, G.nx, [&](int k, int c) { return pr[c][ty + kVisH][tx + kVisH + k - i]; }, dx);

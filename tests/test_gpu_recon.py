@@ -69,3 +69,18 @@ def test_members_of_many_shapes(tmp_path):
         with piafs_amd.Case(d) as c:
             c.step(2)
             assert np.array_equal(got[k], c.solution()), k
+
+
+# from 2^15 cells on the species' cell fluxes are formed in the line teams: narrow
+# and wide teams, one sweep of each, and the first sizes on either side
+@pytest.mark.parametrize("nx,ny", [(182, 181), (181, 181), (1100, 33), (31, 1100)])
+@pytest.mark.parametrize("upwinding", ["roe", "rf-char"])
+def test_species_fluxes_in_the_teams(tmp_path, nx, ny, upwinding):
+    dk = _deck(nx, ny, upwinding=upwinding)
+    r = np.random.default_rng(nx)
+    u = dk.u * (1.0 + 1e-2 * r.uniform(-1, 1, dk.u.shape))
+    u[:, 6:] = 1e-3 * r.uniform(0.5, 1.0, u[:, 6:].shape)
+    d = dk.write(str(tmp_path))
+    want = orc.OCase(d).rhs(u, 0.45)
+    with piafs_amd.Case(d) as c:
+        _close(c.rhs(u, 0.45), want)
