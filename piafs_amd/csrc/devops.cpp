@@ -158,7 +158,7 @@ int piafs_dev_interp_interfaces(piafs_case *pc, double *fI, const double *fC, co
       launch_dev_planar(G, fC, dir ? nullptr : d.flux_x, dir ? d.flux_y : nullptr, 1, 0, nullptr, st);
     for (int cls = K_ENDS; cls <= K_CWSOLVE; cls++) launch_class(un.eng.d_cases, un.eng.plan, cls, 0, st);
   }
-  launch_dev_iface(G.ndims, dir, G.nx, S.N, S.nlines, G.nv, dir ? d.iy[r] : d.ix[r], fI, 0, st);
+  launch_dev_iface(G.ndims, dir, G.nx, S.N, S.nlines, G.nv, dir ? d.iy[r] : d.ix[r], fI, st);
   return launched(pc);
 }
 
@@ -169,19 +169,8 @@ int piafs_dev_upwind(piafs_case *pc, double *fI, const double *fL, const double 
   if (!fI || !fL || !fR || !uL || !uR || !u_ghosted) return fail(pc, 1, "an array pointer is NULL");
   Case *c = pc->c;
   if (dir < 0 || dir >= c->cfg.ndims) return fail(pc, 1, "dir must be 0 .. ndims-1");
-  const hipStream_t st = stream_of(pc, stream);
-  int rc = unit_prepare(pc, st);
-  if (rc) return rc;
-  UnitOps &un = *pc->unit;
-  const CaseDev &d = un.desc;
-  const Grid &G = c->h.G;
-  const SweepGeom &S = dir ? d.Sy : d.Sx;
-  const Global<double> *io = dir ? d.iy : d.ix;
-  stage_state(pc, u_ghosted, st);
-  const double *in[4] = {uL, uR, fL, fR};
-  for (int r = 0; r < 4; r++) launch_dev_iface(G.ndims, dir, G.nx, S.N, S.nlines, G.nv, in[r], io[r], 1, st);
-  launch_class(un.eng.d_cases, un.eng.plan, K_UPWIND, 0, st);
-  launch_dev_iface(G.ndims, dir, G.nx, S.N, S.nlines, G.nv, dir ? d.fIy : d.fIx, fI, 0, st);
+  launch_dev_upwind(aos_grid(c), c->h.model, c->h.upwind, c->h.P.gamma, dir, uL, uR, fL, fR, u_ghosted, fI,
+                    stream_of(pc, stream));
   return launched(pc);
 }
 

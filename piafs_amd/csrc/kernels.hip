@@ -1201,22 +1201,21 @@ __global__ void __launch_bounds__(kLongTeam) k_lsolve(CASE_ARGS) {
 //   entropy fix delta = 1e-6.
 //  Euler1D Roe: Euler1DUpwind.c:27-93 (no entropy fix); rf-char :107-190.
 // ---------------------------------------------------------------------------
+// An interface: offset of its variable 0 in the interface arrays and of the cells
+// beside it in the state, and how far apart variables are in each.
+struct Iface {
+  long ii, vs, cL, cR, pl;
+};
 // In paired mode io[0] holds 0.5*(uR - uL) and io[1] 0.5*(fL + fR) (the only
 // combinations the Roe flux uses); in split mode io[0..3] hold uL uR fL fR.
-#define UD(m) (PAIR ? io[0][(m) * vstride + ii] : 0.5 * (io[1][(m) * vstride + ii] - io[0][(m) * vstride + ii]))
-#define FS(m) (PAIR ? io[1][(m) * vstride + ii] : 0.5 * (io[2][(m) * vstride + ii] + io[3][(m) * vstride + ii]))
+#define UD(m) (PAIR ? io[0][(m) * a.vs + a.ii] : 0.5 * (io[1][(m) * a.vs + a.ii] - io[0][(m) * a.vs + a.ii]))
+#define FS(m) (PAIR ? io[1][(m) * a.vs + a.ii] : 0.5 * (io[2][(m) * a.vs + a.ii] + io[3][(m) * a.vs + a.ii]))
 
-template <int DIR, int PAIR>
-__device__ __forceinline__ void upwind_ns2d_roe(const SweepGeom &S, int nv, double g, long t,
-                                                const double *__restrict__ q, const Global<double> *io,
-                                                double *__restrict__ fI, bool species = true) {
-  const int nl = S.nlines, N = S.N;
-  const int k = (int)(t % (N + 1)), l = (int)(t / (N + 1));
-  const long pl = S.plane;
-  const long cL = S.base + (long)l * S.line_stride + (k - 1), cR = cL + 1;
-  const double uLc[4] = {q[cL], q[pl + cL], q[2 * pl + cL], q[3 * pl + cL]};
-  const double uRc[4] = {q[cR], q[pl + cR], q[2 * pl + cR], q[3 * pl + cR]};
-  const long ii = (long)l * (N + 1) + k, vstride = (long)nl * (N + 1);
+template <int DIR, int PAIR, class IO>
+__device__ __forceinline__ void upwind_ns2d_roe(const Iface &a, int nv, double g, const double *__restrict__ q, const IO *io,
+                                                double *__restrict__ fI, bool species) {
+  const double uLc[4] = {q[a.cL], q[a.pl + a.cL], q[2 * a.pl + a.cL], q[3 * a.pl + a.cL]};
+  const double uRc[4] = {q[a.cR], q[a.pl + a.cR], q[2 * a.pl + a.cR], q[3 * a.pl + a.cR]};
   double ud[4], fs[4], fo[4];
 #pragma unroll
   for (int m = 0; m < 4; m++) {
@@ -1225,20 +1224,17 @@ __device__ __forceinline__ void upwind_ns2d_roe(const SweepGeom &S, int nv, doub
   }
   const double Dsp = roe_ns2d<DIR>(g, uLc, uRc, ud, fs, fo);
 #pragma unroll
-  for (int m = 0; m < 4; m++) fI[m * vstride + ii] = fo[m];
+  for (int m = 0; m < 4; m++) fI[m * a.vs + a.ii] = fo[m];
   if (species)  // else the reconstruction has written them
-    for (int m = 4; m < nv; m++) fI[m * vstride + ii] = FS(m) - Dsp * UD(m);
+    for (int m = 4; m < nv; m++) fI[m * a.vs + a.ii] = FS(m) - Dsp * UD(m);
 }
 
-template <int PAIR>
-__device__ __forceinline__ void upwind_e1d(const SweepGeom &S, int nv, double g, int mode, long t,
-                                           const double *__restrict__ q, const Global<double> *io, double *__restrict__ fI) {
-  const int nl = S.nlines, N = S.N;
-  const int k = (int)(t % (N + 1)), l = (int)(t / (N + 1));
-  const long pl = S.plane;
-  const long cL = S.base + (long)l * S.line_stride + (k - 1), cR = cL + 1;
-  const long ii = (long)l * (N + 1) + k, vs = (long)nl * (N + 1), vstride = vs;
-  const double uLc[3] = {q[cL], q[pl + cL], q[2 * pl + cL]}, uRc[3] = {q[cR], q[pl + cR], q[2 * pl + cR]};
+template <int PAIR, class IO>
+__device__ __forceinline__ void upwind_e1d(const Iface &a, int nv, double g, int mode, const double *__restrict__ q, const IO *io,
+                                           double *__restrict__ fI) {
+  const double uLc[3] = {q[a.cL], q[a.pl + a.cL], q[2 * a.pl + a.cL]};
+  const double uRc[3] = {q[a.cR], q[a.pl + a.cR], q[2 * a.pl + a.cR]};
+  const long vs = a.vs, ii = a.ii;
   if (mode == 0 || mode == 3) {
     double ud[3], fs[3], fo[3];
     for (int m = 0; m < 3; m++) {
@@ -1251,52 +1247,44 @@ __device__ __forceinline__ void upwind_e1d(const SweepGeom &S, int nv, double g,
     return;
   }
   const double *uL = io[0] + ii, *uR = io[1] + ii, *fL = io[2] + ii, *fR = io[3] + ii;
-  double a[4][3], fo[3], es[3];
+  double b[4][3], fo[3], es[3];
   for (int m = 0; m < 3; m++) {
-    a[0][m] = uL[m * vs];
-    a[1][m] = uR[m * vs];
-    a[2][m] = fL[m * vs];
-    a[3][m] = fR[m * vs];
+    b[0][m] = uL[m * vs];
+    b[1][m] = uR[m * vs];
+    b[2][m] = fL[m * vs];
+    b[3][m] = fR[m * vs];
   }
-  rf_e1d(g, mode == 2, uLc, uRc, a[0], a[1], a[2], a[3], fo, es);
+  rf_e1d(g, mode == 2, uLc, uRc, b[0], b[1], b[2], b[3], fo, es);
   for (int m = 0; m < 3; m++) fI[m * vs + ii] = fo[m];
   for (int m = 3; m < nv; m++)
     fI[m * vs + ii] = rf_pick(es[0], es[1], es[2], uL[m * vs], uR[m * vs], fL[m * vs], fR[m * vs], mode == 2);
 }
 
 // Split mode only: uL, uR, fL, fR in io[0..3].
-template <int DIR, bool LLF>
-__device__ __forceinline__ void upwind_ns2d_rf(const SweepGeom &S, int nv, double g, long t, const Global<double> *io,
+template <int DIR, class IO>
+__device__ __forceinline__ void upwind_ns2d_rf(const Iface &a, int nv, double g, bool llf, const IO *io,
                                                double *__restrict__ fI) {
-  const int nl = S.nlines, N = S.N;
-  const int k = (int)(t % (N + 1)), l = (int)(t / (N + 1));
-  const long ii = (long)l * (N + 1) + k, vs = (long)nl * (N + 1);
+  const long vs = a.vs, ii = a.ii;
   const double *uL = io[0] + ii, *uR = io[1] + ii, *fL = io[2] + ii, *fR = io[3] + ii;
   const double uLk[4] = {uL[0], uL[vs], uL[2 * vs], uL[3 * vs]};
   const double uRk[4] = {uR[0], uR[vs], uR[2 * vs], uR[3 * vs]};
   const double fLk[4] = {fL[0], fL[vs], fL[2 * vs], fL[3 * vs]};
   const double fRk[4] = {fR[0], fR[vs], fR[2 * vs], fR[3 * vs]};
   double fo[4], es[3];
-  rf_ns2d<DIR>(g, LLF, uLk, uRk, fLk, fRk, fo, es);
+  rf_ns2d<DIR>(g, llf, uLk, uRk, fLk, fRk, fo, es);
 #pragma unroll
   for (int i = 0; i < 4; i++) fI[i * vs + ii] = fo[i];
   for (int m = 4; m < nv; m++)
-    fI[m * vs + ii] = rf_pick(es[0], es[1], es[2], uL[m * vs], uR[m * vs], fL[m * vs], fR[m * vs], LLF);
+    fI[m * vs + ii] = rf_pick(es[0], es[1], es[2], uL[m * vs], uR[m * vs], fL[m * vs], fR[m * vs], llf);
 }
 
-template <int DIR, int PAIR>
-__device__ __forceinline__ void upwind_ns2d_rusanov(const SweepGeom &S, int nv, double g, long t,
-                                                    const double *__restrict__ q, const Global<double> *io,
-                                                    double *__restrict__ fI) {
-  const int nl = S.nlines, N = S.N;
-  const int k = (int)(t % (N + 1)), l = (int)(t / (N + 1));
-  const long pl = S.plane;
-  const long cL = S.base + (long)l * S.line_stride + (k - 1), cR = cL + 1;
-  const double uLc[4] = {q[cL], q[pl + cL], q[2 * pl + cL], q[3 * pl + cL]};
-  const double uRc[4] = {q[cR], q[pl + cR], q[2 * pl + cR], q[3 * pl + cR]};
+template <int DIR, int PAIR, class IO>
+__device__ __forceinline__ void upwind_ns2d_rusanov(const Iface &a, int nv, double g, const double *__restrict__ q,
+                                                    const IO *io, double *__restrict__ fI) {
+  const double uLc[4] = {q[a.cL], q[a.pl + a.cL], q[2 * a.pl + a.cL], q[3 * a.pl + a.cL]};
+  const double uRc[4] = {q[a.cR], q[a.pl + a.cR], q[2 * a.pl + a.cR], q[3 * a.pl + a.cR]};
   const double alpha = rusanov_ns2d<DIR>(g, uLc, uRc);
-  const long ii = (long)l * (N + 1) + k, vstride = (long)nl * (N + 1);
-  for (int m = 0; m < nv; m++) fI[m * vstride + ii] = FS(m) - alpha * UD(m);
+  for (int m = 0; m < nv; m++) fI[m * a.vs + a.ii] = FS(m) - alpha * UD(m);
 }
 
 #undef UD
@@ -1308,33 +1296,55 @@ __global__ void __launch_bounds__(256) k_upwind(CASE_ARGS) {
   const long nX = (long)(C.Sx.N + 1) * C.Sx.nlines;
   const long nY = (C.G.ndims == 2) ? (long)(C.Sy.N + 1) * C.Sy.nlines : 0;
   if (t >= nX + nY) return;
+  auto at = [&](const SweepGeom &S, long it) {
+    const int k = (int)(it % (S.N + 1)), l = (int)(it / (S.N + 1));
+    const long c = S.base + (long)l * S.line_stride + k;
+    return Iface{it, (long)S.nlines * (S.N + 1), c - 1, c, S.plane};
+  };
+  const int nv = C.G.nv, mode = C.upwind;
+  const double g = C.P.gamma;
   if (C.model == 1) {
-    if (C.paired) upwind_e1d<1>(C.Sx, C.G.nv, C.P.gamma, C.upwind, t, C.U, C.ix, C.fIx);
-    else upwind_e1d<0>(C.Sx, C.G.nv, C.P.gamma, C.upwind, t, C.U, C.ix, C.fIx);
-  } else if (C.upwind == 1 || C.upwind == 2) {  // rf-char, llf-char
-    const bool llf = C.upwind == 2;
+    if (C.paired) upwind_e1d<1>(at(C.Sx, t), nv, g, mode, C.U, C.ix, C.fIx);
+    else upwind_e1d<0>(at(C.Sx, t), nv, g, mode, C.U, C.ix, C.fIx);
+  } else if (mode == 1 || mode == 2) {  // rf-char, llf-char
+    if (t < nX) upwind_ns2d_rf<0>(at(C.Sx, t), nv, g, mode == 2, C.ix, C.fIx);
+    else upwind_ns2d_rf<1>(at(C.Sy, t - nX), nv, g, mode == 2, C.iy, C.fIy);
+  } else if (mode == 3) {  // rusanov
     if (t < nX) {
-      if (llf) upwind_ns2d_rf<0, true>(C.Sx, C.G.nv, C.P.gamma, t, C.ix, C.fIx);
-      else upwind_ns2d_rf<0, false>(C.Sx, C.G.nv, C.P.gamma, t, C.ix, C.fIx);
+      if (C.paired) upwind_ns2d_rusanov<0, 1>(at(C.Sx, t), nv, g, C.U, C.ix, C.fIx);
+      else upwind_ns2d_rusanov<0, 0>(at(C.Sx, t), nv, g, C.U, C.ix, C.fIx);
     } else {
-      if (llf) upwind_ns2d_rf<1, true>(C.Sy, C.G.nv, C.P.gamma, t - nX, C.iy, C.fIy);
-      else upwind_ns2d_rf<1, false>(C.Sy, C.G.nv, C.P.gamma, t - nX, C.iy, C.fIy);
+      if (C.paired) upwind_ns2d_rusanov<1, 1>(at(C.Sy, t - nX), nv, g, C.UT, C.iy, C.fIy);
+      else upwind_ns2d_rusanov<1, 0>(at(C.Sy, t - nX), nv, g, C.UT, C.iy, C.fIy);
     }
-  } else if (C.upwind == 3) {  // rusanov
-    if (t < nX) {
-      if (C.paired) upwind_ns2d_rusanov<0, 1>(C.Sx, C.G.nv, C.P.gamma, t, C.U, C.ix, C.fIx);
-      else upwind_ns2d_rusanov<0, 0>(C.Sx, C.G.nv, C.P.gamma, t, C.U, C.ix, C.fIx);
-    } else {
-      if (C.paired) upwind_ns2d_rusanov<1, 1>(C.Sy, C.G.nv, C.P.gamma, t - nX, C.UT, C.iy, C.fIy);
-      else upwind_ns2d_rusanov<1, 0>(C.Sy, C.G.nv, C.P.gamma, t - nX, C.UT, C.iy, C.fIy);
-    }
-  } else if (t < nX) {
-    if (C.paired) upwind_ns2d_roe<0, 1>(C.Sx, C.G.nv, C.P.gamma, t, C.U, C.ix, C.fIx, !C.fuse_sp);
-    else upwind_ns2d_roe<0, 0>(C.Sx, C.G.nv, C.P.gamma, t, C.U, C.ix, C.fIx);
+  } else if (t < nX) {  // the species' fluxes may be the reconstruction's
+    if (C.paired) upwind_ns2d_roe<0, 1>(at(C.Sx, t), nv, g, C.U, C.ix, C.fIx, !C.fuse_sp);
+    else upwind_ns2d_roe<0, 0>(at(C.Sx, t), nv, g, C.U, C.ix, C.fIx, true);
   } else {
-    if (C.paired) upwind_ns2d_roe<1, 1>(C.Sy, C.G.nv, C.P.gamma, t - nX, C.UT, C.iy, C.fIy, !C.fuse_sp);
-    else upwind_ns2d_roe<1, 0>(C.Sy, C.G.nv, C.P.gamma, t - nX, C.UT, C.iy, C.fIy);
+    if (C.paired) upwind_ns2d_roe<1, 1>(at(C.Sy, t - nX), nv, g, C.UT, C.iy, C.fIy, !C.fuse_sp);
+    else upwind_ns2d_roe<1, 0>(at(C.Sy, t - nX), nv, g, C.UT, C.iy, C.fIy, true);
   }
+}
+
+// Upwind on the reference's layouts (a point's components contiguous), one thread
+// per interface in memory order: a wave's threads take all of the cache lines
+// they touch.  With the arrays changed to planes and back around k_upwind a call
+// was seven launches of 6 to 20 us; 384 x 250, 11 variables, now one of 27.
+__global__ void __launch_bounds__(256) k_dev_upwind(AosGrid A, int model, int mode, double g, int dir,
+                                                    const double *uL, const double *uR, const double *fL,
+                                                    const double *fR, const double *u, double *fI) {
+  const int N = dir ? A.ny : A.nx, nl = A.ndims == 2 ? (dir ? A.nx : A.ny) : 1;
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= (long)(N + 1) * nl) return;
+  const int k = (int)(dir ? p / A.nx : p % (N + 1)), l = (int)(dir ? p % A.nx : p / (N + 1));
+  const long nxg = A.nx + 2 * A.g;
+  const long row = A.ndims == 2 ? (dir ? k : l) + A.g : 0, cR = (row * nxg + (dir ? l : k) + A.g) * A.nv;
+  const Iface a = {p * A.nv, 1, cR - (dir ? nxg : 1) * A.nv, cR, 1};
+  const double *io[4] = {uL, uR, fL, fR};
+  if (model == 1) upwind_e1d<0>(a, A.nv, g, mode, u, io, fI);
+  else if (mode == 1 || mode == 2) dir ? upwind_ns2d_rf<1>(a, A.nv, g, mode == 2, io, fI) : upwind_ns2d_rf<0>(a, A.nv, g, mode == 2, io, fI);
+  else if (mode == 3) dir ? upwind_ns2d_rusanov<1, 0>(a, A.nv, g, u, io, fI) : upwind_ns2d_rusanov<0, 0>(a, A.nv, g, u, io, fI);
+  else dir ? upwind_ns2d_roe<1, 0>(a, A.nv, g, u, io, fI, true) : upwind_ns2d_roe<0, 0>(a, A.nv, g, u, io, fI, true);
 }
 
 // Conservation check, boundary part: the interface fluxes on the domain
@@ -2053,8 +2063,7 @@ __global__ void k_set_time(double *time, double t) { *time = t; }
 // Interface arrays of one sweep: reference layout <-> line-major
 // a[(v*nlines + l)*(N+1) + k].  One thread per (interface, line, variable).
 __global__ void __launch_bounds__(TB) k_dev_iface(int ndims, int dir, int nx, int N, int nl, int nv,
-                                                  const double *__restrict__ src, double *__restrict__ dst,
-                                                  int to_lines) {
+                                                  const double *__restrict__ src, double *__restrict__ dst) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long)(N + 1) * nl * nv) return;
   const int v = (int)(t % nv);
@@ -2062,8 +2071,7 @@ __global__ void __launch_bounds__(TB) k_dev_iface(int ndims, int dir, int nx, in
   const int k = (int)(r % (N + 1)), l = (int)(r / (N + 1));
   const long p = dir ? (long)k * nx + l : (ndims == 2 ? (long)l * (N + 1) + k : (long)k);
   const long q = ((long)v * nl + l) * (N + 1) + k;
-  if (to_lines) dst[q] = src[p * nv + v];
-  else dst[p * nv + v] = src[q];
+  dst[p * nv + v] = src[q];
 }
 
 
@@ -2341,6 +2349,12 @@ void launch_dev_flux(const AosGrid &A, int model, double gamma, int dir, const d
   hipLaunchKernelGGL(k_dev_flux, dim3(nblk(n)), dim3(TB), 0, s, A, model, gamma, dir, u, f);
 }
 
+void launch_dev_upwind(const AosGrid &A, int model, int mode, double gamma, int dir, const double *uL, const double *uR,
+                       const double *fL, const double *fR, const double *u, double *fI, hipStream_t s) {
+  const long n = (long)((dir ? A.ny : A.nx) + 1) * (A.ndims == 2 ? (dir ? A.nx : A.ny) : 1);
+  hipLaunchKernelGGL(k_dev_upwind, dim3(nblk(n)), dim3(TB), 0, s, A, model, mode, gamma, dir, uL, uR, fL, fR, u, fI);
+}
+
 void launch_dev_fd(const AosGrid &A, int dir, int par4, int bias, const double *f, double *df, hipStream_t s) {
   const int N = dir ? A.ny : A.nx, nl = A.ndims == 2 ? (dir ? A.nx : A.ny) : 1;
   const long n = (long)(N + 2 * A.g) * nl * A.nv;
@@ -2376,9 +2390,9 @@ void launch_set_time(double *time, double t, hipStream_t s) {
 }
 
 void launch_dev_iface(int ndims, int dir, int nx, int N, int nl, int nv, const double *src, double *dst,
-                      int to_lines, hipStream_t s) {
+                      hipStream_t s) {
   const long n = (long)(N + 1) * nl * nv;
-  hipLaunchKernelGGL(k_dev_iface, dim3(nblk(n)), dim3(TB), 0, s, ndims, dir, nx, N, nl, nv, src, dst, to_lines);
+  hipLaunchKernelGGL(k_dev_iface, dim3(nblk(n)), dim3(TB), 0, s, ndims, dir, nx, N, nl, nv, src, dst);
 }
 
 void launch_recon_only(const CaseDev *d, const Plan &pl, const CaseDev &c, int dir, int r, hipStream_t st) {

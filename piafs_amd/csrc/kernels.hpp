@@ -305,6 +305,8 @@ struct AosGrid {
 };
 // device-buffer operators on reference-layout arrays (see kernels.hip)
 void launch_dev_flux(const AosGrid &A, int model, double gamma, int dir, const double *u, double *f, hipStream_t s);
+void launch_dev_upwind(const AosGrid &A, int model, int mode, double gamma, int dir, const double *uL, const double *uR,
+                       const double *fL, const double *fR, const double *u, double *fI, hipStream_t s);
 void launch_dev_fd(const AosGrid &A, int dir, int par4, int bias, const double *f, double *df, hipStream_t s);
 void launch_dev_weights(const AosGrid &A, int model, double gamma, int dir, int kind, int crweno,
                         int characteristic, int no_limiting, double eps, const double *fC, const double *u,
@@ -321,9 +323,9 @@ void launch_dev_planar(const Grid &G, const double *a, double *nat, double *tr, 
 void launch_pack(const Grid &G, const double *host, long q0, long np, double *u, hipStream_t s);
 void launch_unpack(const Grid &G, const double *u, long q0, long np, double *host, hipStream_t s);
 void launch_set_time(double *time, double t, hipStream_t s);
-// one sweep's interface array: reference layout <-> line-major
+// one sweep's interface array: line-major -> reference layout
 void launch_dev_iface(int ndims, int dir, int nx, int N, int nl, int nv, const double *src, double *dst,
-                      int to_lines, hipStream_t s);
+                      hipStream_t s);
 // reconstruction r of the systems of one sweep (not longl), end values included,
 // of a plan's only case, whose descriptor is c
 void launch_recon_only(const CaseDev *d_cases, const Plan &plan, const CaseDev &c, int dir, int r, hipStream_t st);
