@@ -58,14 +58,15 @@ def kernel_algorithmic_bytes(name, nx, ny, nv, g, nstages, crweno, paired=True):
     fused = species_fused(nx, ny, nv, paired)
     if name.startswith("recon_") and name != "recon_ends":  # u and f at every position of every line; the interface arrays
         if fused:  # flow: the two combinations; species: their flux, from |v_n| (one value per interface)
-            return sweeps * 8 * (2 * nv * pos * lines + (2 * 4 + (nv - 4) + 1) * (N + 1) * lines)
+            # (the state, the flow's fluxes and the velocity, from which the species' fluxes are formed)
+            return sweeps * 8 * ((nv + 4 + 1) * pos * lines + (2 * 4 + (nv - 4) + 1) * (N + 1) * lines)
         return sweeps * 8 * (2 * nv * pos * lines + nio * nv * (N + 1) * lines)
     if name == "upwind":  # the interface arrays + 4 flow vars at the two cells; fI
         if fused:  # the flow variables only
             return sweeps * 8 * (nio * 4 * (N + 1) * lines + 2 * 4 * (N + 1) * lines + 4 * (N + 1) * lines)
         return sweeps * 8 * (nio * nv * (N + 1) * lines + 2 * 4 * (N + 1) * lines + nv * (N + 1) * lines)
-    if name == "flux":  # the state and the flux at every position; |v_n| per interface when fused
-        return sweeps * 8 * (2 * nv * pos * lines + ((N + 1) * lines if fused else 0))
+    if name == "flux":  # the flow's variables and fluxes and the velocity at every position; |v_n| per interface when fused
+        return sweeps * 8 * ((4 + 5) * pos * lines + ((N + 1) * lines if fused else 0))
     if name == "stage_bc":  # u + up to one Udot read, U and UT written (ghosted)
         return 8 * nv * (nx + 2 * g) * (ny + 2 * g) * 4
     return None

@@ -2,9 +2,9 @@
 // include/piafs_amd.h.
 //
 // A time step is a fixed sequence of stream-ordered launches with no host
-// synchronisation: per RK stage  stage+BC -> fluxes -> reconstruction (x and
-// y sweeps in one launch) -> upwinding -> x divergence -> transpose ->
-// viscous derivatives -> assembly of Udot; after the last stage the update.
+// synchronisation: per RK stage of a 2D case  fluxes -> reconstruction (x and y
+// sweeps in one launch) -> upwinding -> assembly, which goes on to the next
+// stage's state or the new solution; 1D cases take whole steps in a launch.
 // TimeRK.c:34-102 is the reference control flow this replaces.
 #include <hip/hip_runtime.h>
 
