@@ -2181,7 +2181,7 @@ bool velocity_for_flux(const CaseDev &c) {
 bool stage_tile_64(const CaseDev &c) { return c.G.ndims == 2 && (long)c.G.nx * c.G.ny >= 2048L * 2048L; }
 
 bool species_in_recon(const CaseDev &c) {
-  auto fits = [](const SweepGeom &S) { return !S.longl && (S.team == 32 || S.team == 64); };
+  auto fits = [](const SweepGeom &S) { return !S.longl && (S.team == 32 || S.team == 64 || S.team == 128); };
   return c.G.ndims == 2 && c.model == 2 && c.paired && c.R.crweno && c.upwind == 0 && !c.R.characteristic &&
          c.G.nv > 4 && c.dsp[0] && c.dsp[1] && fits(c.Sx) && fits(c.Sy);
 }

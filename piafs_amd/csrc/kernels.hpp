@@ -254,7 +254,7 @@ hipError_t launch_lines(const CaseDev *d_cases, const Plan &plan, const std::vec
 // Host side: blocks each case needs for each kernel class (0 = class unused).
 void case_blocks(const CaseDev &c, int blocks[K_NCLASS]);
 // Whether the reconstruction can write the species' Roe interface fluxes
-// itself (NS2D, paired Roe, teams of 32 or 64 lanes, |v_n| buffers present).
+// itself (NS2D, paired Roe, teams of 32 to 128 lanes, |v_n| buffers present).
 bool species_in_recon(const CaseDev &c);
 // Whether the reconstruction can form the species' cell fluxes itself, and from how
 // many cells of a plan on it does: it saves k_flux traffic (1024 x 1024 133 -> 77

@@ -258,7 +258,8 @@ size_t line_lds(const CaseDev &c) {
 }  // namespace
 
 int line_class(const CaseDev &c) {
-  if (c.G.ndims != 1 || c.model != 1 || c.G.nv > kTubeVars || c.cons || c.sponge || c.terms != 7 || c.G.nx < 8) return -1;
+  if (c.G.ndims != 1 || c.model != 1 || c.G.nv > kTubeVars || c.cons || c.sponge || c.P.chem || c.terms != 7 || c.G.nx < 8)
+    return -1;
   if (c.R.crweno) {
     if (c.R.characteristic || line_lds(c) > kLineLdsMax) return -1;
     return c.G.nx <= 4 * 64 + 1 ? K_LINE4 : c.G.nx <= 8 * 64 + 1 ? K_LINE8 : -1;

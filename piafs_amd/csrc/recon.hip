@@ -151,7 +151,7 @@ __device__ __forceinline__ void recon_pair(const CaseDev &C, int dir, long sys, 
   // below hides their latency (the line's N + 1 <= T MR + 2 interfaces take at
   // most MR + 2 per lane)
   constexpr int KO = MR + 2;
-  const bool fsp = !WIDE && C.fuse_sp && v >= 4;
+  const bool fsp = C.fuse_sp && v >= 4;
   double dvv[KO];
 #pragma unroll
   for (int it = 0; it < KO; it++) dvv[it] = 0.0;
@@ -180,6 +180,8 @@ __device__ __forceinline__ void recon_pair(const CaseDev &C, int dir, long sys, 
     // its combination with a release increment of the pair's counter, and the
     // one that arrives second (acquire) writes, so neither waits.  The two end
     // interfaces take the combinations k_recon_ends wrote.
+    // A pair of 128-lane teams has a block to itself, whose barrier has made both
+    // visible.
     bool writer = q == 1;
     if (T == 64) {
       unsigned prev = 0u;

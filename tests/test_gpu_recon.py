@@ -72,8 +72,9 @@ def test_members_of_many_shapes(tmp_path):
 
 
 # from 2^15 cells on the species' cell fluxes are formed in the line teams: narrow
-# and wide teams, one sweep of each, and the first sizes on either side
-@pytest.mark.parametrize("nx,ny", [(182, 181), (181, 181), (1100, 33), (31, 1100)])
+# and wide teams, one sweep of each, and the first sizes on either side; the last
+# has teams of 128 lanes whose pairs write the species' interface fluxes
+@pytest.mark.parametrize("nx,ny", [(182, 181), (181, 181), (1100, 33), (31, 1100), (1026, 259)])
 @pytest.mark.parametrize("upwinding", ["roe", "rf-char"])
 def test_species_fluxes_in_the_teams(tmp_path, nx, ny, upwinding):
     dk = _deck(nx, ny, upwinding=upwinding)
