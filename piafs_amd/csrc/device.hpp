@@ -548,14 +548,12 @@ __device__ __forceinline__ void rf_e1d(double g, bool llf, const double uLc[3], 
   es[2] = ER.D[0];
 }
 
-// Element at byte offset o of an array whose base is the same for the block: one
-// address register and no 64-bit arithmetic.  For planes and interface arrays of
-// one variable, which are below 4 GiB (the arrays of a case with larger ones
-// take more than the device has).
-__device__ __forceinline__ const double &elem(const double *base, unsigned o) {
+// Element at byte offset o of an array: the offset of a point is formed once for
+// all planes, whose bases are the same for the block.
+__device__ __forceinline__ const double &elem(const double *base, size_t o) {
   return *(const double *)((const char *)base + o);
 }
-__device__ __forceinline__ double &elem(double *base, unsigned o) { return *(double *)((char *)base + o); }
+__device__ __forceinline__ double &elem(double *base, size_t o) { return *(double *)((char *)base + o); }
 
 // Block barrier that orders LDS accesses only: global loads and stores issued
 // before it stay in flight (a __syncthreads also waits for those).

@@ -1399,13 +1399,13 @@ __global__ void __launch_bounds__(256) k_bflux(CASE_ARGS) {
 // ---------------------------------------------------------------------------
 // component c (variable c + 1) of the parabolic term
 // at point (i, j), byte offset o of the ghosted planes
-__device__ __forceinline__ double viscous_par(const CaseDev &C, int c, int i, int j, unsigned o) {
+__device__ __forceinline__ double viscous_par(const CaseDev &C, int c, int i, int j, size_t o) {
   const Grid &G = C.G;
   const PhysParams &P = C.P;
   const long pl = (long)G.nxg * G.nyg;
   const double dxi = C.dxinv[G.g + i], dyi = C.dxinv[(G.nx + 2 * G.g) + G.g + j];
   const double *Fx = C.FV + c * pl, *Fy = C.FV + (3 + c) * pl;
-  const unsigned row = 8u * G.nxg;
+  const size_t row = 8 * (size_t)G.nxg;
   double dfx, dfy;
   if (P.par4) {
     const double t12 = 1.0 / 12.0;
@@ -1497,7 +1497,7 @@ __device__ __forceinline__ double chem_term(const PhysParams &P, int m, F n, dou
 }
 // photon density reaching layer iz at byte offset o, from the pulse at the stage
 // time (chem_pulse) and the beam map
-__device__ __forceinline__ double chem_photons(const CaseDev &C, int iz, unsigned o, double hs, double imap) {
+__device__ __forceinline__ double chem_photons(const CaseDev &C, int iz, size_t o, double hs, double imap) {
   const PhysParams &P = C.P;
   double nh = (hs * imap) / P.hnu_den;
   for (int z = 0; z < iz; z++)
@@ -1515,7 +1515,7 @@ __device__ __forceinline__ double with_source(const CaseDev &C, int v, int i, in
   const bool chem = C.P.chem && v >= C.P.nflow - 1;
   double s = 0.0;
   if (chem) {
-    const unsigned o = 8u * (unsigned)p;
+    const size_t o = 8 * (size_t)p;
     const ChemVar cv = chem_of(C.P, v);
     const double *n = chem_planes(C, cv.layer);
     const double nh = cv.need >> 7 ? chem_photons(C, cv.layer, o, hs, elem(C.imap, o)) : 0.0;
@@ -1567,24 +1567,24 @@ __device__ __forceinline__ void assemble_tile(const CaseDev &C, int stage, int b
   // loads before it).
   const int ic = min(i, G.nx - 1);
   auto jq = [&](int q) { return min(j0 + ty + R * q, G.ny - 1); };
-  unsigned o[Q];  // byte offset of the thread's points in a plane
+  size_t o[Q];  // byte offset of the thread's points in a plane
 #pragma unroll
-  for (int q = 0; q < Q; q++) o[q] = 8u * ((unsigned)(jq(q) + G.gy) * G.nxg + (ic + G.g));
+  for (int q = 0; q < Q; q++) o[q] = 8 * ((size_t)(jq(q) + G.gy) * G.nxg + (ic + G.g));
   // y-sweep interfaces of lines i0..i0+31, interfaces j0..j0+32
   const double *fIx = C.fIx + (long)v * G.ny * (G.nx + 1), *fIy = C.fIy + (long)v * G.nx * (G.ny + 1);
   double fy[Q], fy32 = 0.0;
 #pragma unroll
   for (int q = 0; q < Q; q++)
-    fy[q] = elem(fIy, 8u * ((unsigned)min(i0 + ty + R * q, G.nx - 1) * (G.ny + 1) + min(j0 + tx, G.ny)));
+    fy[q] = elem(fIy, 8 * ((size_t)min(i0 + ty + R * q, G.nx - 1) * (G.ny + 1) + min(j0 + tx, G.ny)));
   // interface j0 + 32 of line i0 + the thread's index, by the first 32 threads
-  if (threadIdx.x < 32) fy32 = elem(fIy, 8u * ((unsigned)ic * (G.ny + 1) + min(j0 + 32, G.ny)));
+  if (threadIdx.x < 32) fy32 = elem(fIy, 8 * ((size_t)ic * (G.ny + 1) + min(j0 + 32, G.ny)));
   const bool visc = C.P.viscous && (C.terms & 2) && v >= 1 && v <= 3;
   double hx[Q], add[Q];
   {
     double x0[Q], x1[Q];
 #pragma unroll
     for (int q = 0; q < Q; q++) {
-      const unsigned a = 8u * ((unsigned)jq(q) * (G.nx + 1) + ic);
+      const size_t a = 8 * ((size_t)jq(q) * (G.nx + 1) + ic);
       x0[q] = elem(fIx, a);
       x1[q] = elem(fIx, a + 8);
     }
@@ -1671,7 +1671,7 @@ __device__ __forceinline__ void assemble_tile(const CaseDev &C, int stage, int b
   for (int q = 0; q < Q; q++) {
     const int il = ty + R * q;
     if (i0 + il < G.nx && j0 + tx < G.ny)
-      elem(C.UT + pl, 8u * ((unsigned)(i0 + il + G.g) * G.nyg + (j0 + tx + G.gy))) = sh.next[tx][il];
+      elem(C.UT + pl, 8 * ((size_t)(i0 + il + G.g) * G.nyg + (j0 + tx + G.gy))) = sh.next[tx][il];
   }
   // ghost points whose source lies in the tile, of the faces that copy
   if (!C.push[0] || (i0 >= G.g && i0 + 32 <= G.nx - G.g && j0 >= G.g && j0 + 32 <= G.ny - G.g)) return;

@@ -137,7 +137,7 @@ __device__ __forceinline__ void viscous_tile(const CaseDev &C, int b, Prims &sh)
     if (f < nfill) {
       const int I = min(max(I0 + col[f] - kVisH, 0), G.nxg - 1), J = min(max(J0 + row[f] - kVisH, 0), G.nyg - 1);
 #pragma unroll
-      for (int m = 0; m < 4; m++) q[f][m] = elem(C.U + m * G.plane, 8u * ((unsigned)J * G.nxg + I));
+      for (int m = 0; m < 4; m++) q[f][m] = elem(C.U + m * G.plane, 8 * ((size_t)J * G.nxg + I));
     }
 #pragma unroll
   for (int f = 0; f < 3; f++)
