@@ -77,3 +77,18 @@ def test_members_together(tmp_path):
             b.step(3)
             for k in b.slots:
                 assert np.array_equal(b.solution(k), solo[k]), k
+
+
+@pytest.mark.parametrize("scheme,interp", [("weno5", "characteristic"), ("crweno5", "components")])
+def test_no_steps(tmp_path, scheme, interp):
+    """Step counts of zero and less leave the solution and the time as they are,
+    before the first step and after an odd and an even number of them."""
+    d = _deck(90, "mirror", scheme, interp, "roe", "44").write(str(tmp_path))
+    with piafs_amd.Case(d) as c:
+        for n in (0, 1, 1):
+            c.step(n)
+            u, t = c.solution(), c.info.t
+            for none in (0, -1, -2):
+                c.step(none)
+                assert np.array_equal(c.solution(), u), none
+                assert c.info.t == t
