@@ -16,7 +16,7 @@ std::shared_ptr<Staging> Staging::of(int device) {
   return s;
 }
 
-Staging::~Staging() {
+Staging::Set::~Set() {
   {
     std::lock_guard<std::mutex> g(m);
     stop = true;
@@ -27,7 +27,7 @@ Staging::~Staging() {
   release();
 }
 
-void Staging::release() {
+void Staging::Set::release() {
   for (Slot &s : slots) {
     if (s.ev && s.pending) hipEventSynchronize(s.ev);
     if (s.ev) hipEventDestroy(s.ev);
@@ -46,7 +46,7 @@ void Staging::shape(size_t bytes, size_t &chunk, int &n) {
   n = (int)std::min<size_t>(kSlots, std::max<size_t>(1, (bytes + chunk - 1) / chunk));
 }
 
-bool Staging::grow(size_t bytes) {
+bool Staging::Set::grow(size_t bytes) {
   size_t chunk;
   int n;
   shape(bytes, chunk, n);
@@ -79,16 +79,30 @@ bool Staging::grow(size_t bytes) {
   return nslots > 0;
 }
 
+bool Staging::Set::settled(hipStream_t st) {
+  for (Slot &s : slots)
+    if (s.pending && !(st && s.on == st)) {
+      const hipError_t e = hipEventQuery(s.ev);
+      hipGetLastError();  // "not ready" is no error of the caller's
+      if (e != hipSuccess) return false;
+      s.pending = false;
+    }
+  return true;
+}
+
 bool Staging::reserve(size_t bytes) {
-  std::lock_guard<std::mutex> g(use);
+  std::unique_lock<std::mutex> g(ahead.use, std::try_to_lock);
+  const bool first = g.owns_lock() && ahead.settled(nullptr);
+  if (!first) g = std::unique_lock<std::mutex>(after.use);
+  Set &s = first ? ahead : after;
   try {
-    return grow(bytes);
+    return s.grow(bytes);
   } catch (...) {
-    return nslots > 0;
+    return s.nslots > 0;
   }
 }
 
-void Staging::worker(int id) {
+void Staging::Set::worker(int id) {
   hipSetDevice(device);
   uint64_t seen = 0;
   std::unique_lock<std::mutex> g(m);
@@ -107,7 +121,7 @@ void Staging::worker(int id) {
 // body(chunk, slot) for every chunk, on the calling thread and the helpers,
 // each with its own slot.  A thread takes the next chunk when it is done with
 // one.
-hipError_t Staging::each(long nchunks, const std::function<hipError_t(long, Slot &)> &body) {
+hipError_t Staging::Set::each(long nchunks, const std::function<hipError_t(long, Slot &)> &body) {
   std::atomic<long> next{0};
   std::atomic<int> err{(int)hipSuccess};
   const std::function<void(int)> run = [&](int s) {
@@ -136,8 +150,7 @@ hipError_t Staging::each(long nchunks, const std::function<hipError_t(long, Slot
   return (hipError_t)err.load();
 }
 
-hipError_t Staging::upload(const double *src, long npts, int nv, hipStream_t st, const Kern &kernel) {
-  std::lock_guard<std::mutex> g(use);
+hipError_t Staging::Set::upload(const double *src, long npts, int nv, hipStream_t st, const Kern &kernel) {
   const size_t bytes = (size_t)npts * nv * sizeof(double);
   if (!grow(bytes)) return hipErrorOutOfMemory;
   size_t chunk;
@@ -154,12 +167,12 @@ hipError_t Staging::upload(const double *src, long npts, int nv, hipStream_t st,
     memcpy(s.buf, src + q0 * nv, (size_t)np * nv * sizeof(double));
     kernel(q0, np, s.buf);
     s.pending = true;
+    s.on = st;
     return hipEventRecord(s.ev, st);
   });
 }
 
-hipError_t Staging::download(double *dst, long npts, int nv, hipStream_t st, const Kern &kernel) {
-  std::lock_guard<std::mutex> g(use);
+hipError_t Staging::Set::download(double *dst, long npts, int nv, hipStream_t st, const Kern &kernel) {
   const size_t bytes = (size_t)npts * nv * sizeof(double);
   if (!grow(bytes)) return hipErrorOutOfMemory;
   size_t chunk;
@@ -179,6 +192,27 @@ hipError_t Staging::download(double *dst, long npts, int nv, hipStream_t st, con
     if (e == hipSuccess) memcpy(dst + q0 * nv, s.buf, (size_t)np * nv * sizeof(double));
     return e;
   });
+}
+
+// move(set) with a set that this transfer has
+template <class F>
+hipError_t Staging::on_a_set(hipStream_t st, F move) {
+  {
+    std::unique_lock<std::mutex> g(ahead.use, std::try_to_lock);
+    if (g.owns_lock() && ahead.settled(st)) return move(ahead);
+  }
+  const hipError_t e = hipStreamSynchronize(st);
+  if (e != hipSuccess) return e;
+  std::lock_guard<std::mutex> g(after.use);
+  return move(after);
+}
+
+hipError_t Staging::upload(const double *src, long npts, int nv, hipStream_t st, const Kern &kernel) {
+  return on_a_set(st, [&](Set &s) { return s.upload(src, npts, nv, st, kernel); });
+}
+
+hipError_t Staging::download(double *dst, long npts, int nv, hipStream_t st, const Kern &kernel) {
+  return on_a_set(st, [&](Set &s) { return s.download(dst, npts, nv, st, kernel); });
 }
 
 }  // namespace piafs
