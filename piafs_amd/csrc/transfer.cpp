@@ -118,19 +118,23 @@ void Staging::Set::worker(int id) {
   }
 }
 
-// body(chunk, slot) for every chunk, on the calling thread and the helpers,
-// each with its own slot.  A thread takes the next chunk when it is done with
-// one.
+int Staging::Set::threads(long nchunks) const {
+  return (int)std::max(1L, std::min<long>({(long)nslots, (long)pool.size() + 1, nchunks}));
+}
+
+// body(chunk, slot) for every chunk, on the calling thread (slot 0) and the
+// helpers, each with its own slot.  The first chunk of the thread with slot k is
+// chunk k; a thread takes the next chunk when it is done with one.
 hipError_t Staging::Set::each(long nchunks, const std::function<hipError_t(long, Slot &)> &body) {
-  std::atomic<long> next{0};
+  const int n = threads(nchunks) - 1;
+  std::atomic<long> next{n + 1};
   std::atomic<int> err{(int)hipSuccess};
   const std::function<void(int)> run = [&](int s) {
-    for (long c = next++; c < nchunks && err == (int)hipSuccess; c = next++) {
+    for (long c = s; c < nchunks && err == (int)hipSuccess; c = next++) {
       const hipError_t e = body(c, slots[s]);
       if (e != hipSuccess) err = (int)e;
     }
   };
-  const int n = (int)std::min<long>({(long)nslots - 1, (long)pool.size(), nchunks - 1});
   if (n > 0) {
     {
       std::lock_guard<std::mutex> g(m);
@@ -150,6 +154,14 @@ hipError_t Staging::Set::each(long nchunks, const std::function<hipError_t(long,
   return (hipError_t)err.load();
 }
 
+// waits until no kernel is using the slot's buffer
+hipError_t Staging::Set::settle(Slot &s) {
+  if (!s.pending) return hipSuccess;
+  const hipError_t e = hipEventSynchronize(s.ev);
+  if (e == hipSuccess) s.pending = false;
+  return e;
+}
+
 hipError_t Staging::Set::upload(const double *src, long npts, int nv, hipStream_t st, const Kern &kernel) {
   const size_t bytes = (size_t)npts * nv * sizeof(double);
   if (!grow(bytes)) return hipErrorOutOfMemory;
@@ -159,11 +171,8 @@ hipError_t Staging::Set::upload(const double *src, long npts, int nv, hipStream_
   const long per = std::max<long>(1, (long)(chunk / (nv * sizeof(double))));
   return each((npts + per - 1) / per, [&](long c, Slot &s) {
     const long q0 = c * per, np = std::min(per, npts - q0);
-    if (s.pending) {
-      const hipError_t e = hipEventSynchronize(s.ev);
-      if (e != hipSuccess) return e;
-      s.pending = false;
-    }
+    const hipError_t e = settle(s);
+    if (e != hipSuccess) return e;
     memcpy(s.buf, src + q0 * nv, (size_t)np * nv * sizeof(double));
     kernel(q0, np, s.buf);
     s.pending = true;
@@ -178,17 +187,27 @@ hipError_t Staging::Set::download(double *dst, long npts, int nv, hipStream_t st
   size_t chunk;
   int n;
   shape(bytes, chunk, n);
-  const long per = std::max<long>(1, (long)(chunk / (nv * sizeof(double))));
-  return each((npts + per - 1) / per, [&](long c, Slot &s) {
+  const long per = std::max<long>(1, (long)(chunk / (nv * sizeof(double)))), nchunks = (npts + per - 1) / per;
+  auto fetch = [&](long c, Slot &s) {
     const long q0 = c * per, np = std::min(per, npts - q0);
-    if (s.pending) {
-      const hipError_t e = hipEventSynchronize(s.ev);
-      if (e != hipSuccess) return e;
-      s.pending = false;
-    }
+    const hipError_t e = settle(s);
+    if (e != hipSuccess) return e;
     kernel(q0, np, s.buf);
-    hipError_t e = hipEventRecord(s.ev, st);
-    if (e == hipSuccess) e = hipEventSynchronize(s.ev);
+    s.pending = true;
+    s.on = st;
+    return hipEventRecord(s.ev, st);
+  };
+  // the first chunk of every thread is asked for from here, and the threads wake
+  // when the first is there: until then one thread waits for the stream's work
+  const int ahead = threads(nchunks);
+  hipError_t e = hipSuccess;
+  for (int c = 0; c < ahead && e == hipSuccess; c++) e = fetch(c, slots[c]);
+  if (e == hipSuccess) e = settle(slots[0]);
+  if (e != hipSuccess) return e;
+  return each(nchunks, [&](long c, Slot &s) {
+    const long q0 = c * per, np = std::min(per, npts - q0);
+    hipError_t e = c < ahead ? hipSuccess : fetch(c, s);
+    if (e == hipSuccess) e = settle(s);
     if (e == hipSuccess) memcpy(dst + q0 * nv, s.buf, (size_t)np * nv * sizeof(double));
     return e;
   });

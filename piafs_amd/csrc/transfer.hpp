@@ -82,6 +82,8 @@ class Staging {
     bool grow(size_t bytes);
     void release();
     void worker(int id);
+    int threads(long nchunks) const;  // that move nchunks chunks
+    hipError_t settle(Slot &s);
     hipError_t each(long nchunks, const std::function<hipError_t(long, Slot &)> &body);
     hipError_t upload(const double *src, long npts, int nv, hipStream_t st, const Kern &kernel);
     hipError_t download(double *dst, long npts, int nv, hipStream_t st, const Kern &kernel);

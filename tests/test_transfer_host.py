@@ -13,6 +13,7 @@ CSRC = os.path.join(ROOT, "piafs_amd", "csrc")
 
 RUNTIME = r"""
 #pragma once
+#include <atomic>
 #include <condition_variable>
 #include <cstddef>
 #include <cstdlib>
@@ -97,8 +98,13 @@ inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
   e->n = s->queued;
   return hipSuccess;
 }
+inline std::atomic<int> waiting{0}, waiting_most{0};  // threads in hipEventSynchronize
 inline hipError_t hipEventSynchronize(hipEvent_t e) {
+  const int n = ++waiting;
+  for (int m = waiting_most; n > m && !waiting_most.compare_exchange_weak(m, n);) {
+  }
   if (e->s) e->s->wait(e->n);
+  --waiting;
   return hipSuccess;
 }
 inline hipError_t hipEventQuery(hipEvent_t e) {
@@ -192,6 +198,25 @@ int main(int, char **argv) {
 }
 """
 
+WAITERS = r"""
+// a download behind a computation keeps one thread waiting for it, not one a chunk
+int main() {
+  Staging s(0);
+  Stream a;
+  Gate gate;
+  Vec da = state(1.0), ha(NP * NV);
+  a.push([&] { gate.wait(); });
+  hipError_t e = hipSuccess;
+  std::thread t([&] { e = to_host(s, ha, da, a); });
+  std::this_thread::sleep_for(std::chrono::milliseconds(500));
+  const int most = waiting_most;
+  gate.release();
+  t.join();
+  if (e != hipSuccess || ha != da) return 2;
+  return most == 1 ? 0 : 1;
+}
+"""
+
 
 def _build(tmp_path, main):
     gxx = shutil.which("g++")
@@ -211,3 +236,7 @@ def _build(tmp_path, main):
 def test_a_transfer_does_not_wait_for_other_handles_work(tmp_path, direction):
     exe = _build(tmp_path, INDEPENDENT)
     assert subprocess.run([exe, direction], timeout=60).returncode == 0
+
+
+def test_one_thread_waits_for_queued_work(tmp_path):
+    assert subprocess.run([_build(tmp_path, WAITERS)], timeout=60).returncode == 0
