@@ -2375,14 +2375,16 @@ void launch_dev_planar(const Grid &G, const double *a, double *nat, double *tr, 
   hipLaunchKernelGGL(k_dev_planar, dim3(nblk(n)), dim3(TB), 0, s, G, a, nat, tr, to_planar, ghosts_only, out);
 }
 
-void launch_pack(const Grid &G, const double *host, long q0, long np, double *u, hipStream_t s) {
+hipError_t launch_pack(const Grid &G, const double *host, long q0, long np, double *u, hipStream_t s) {
   const long n = np * G.nv;
   hipLaunchKernelGGL(k_pack, dim3(nblk(n)), dim3(TB), 0, s, G, host, q0, (unsigned)n, u);
+  return hipGetLastError();
 }
 
-void launch_unpack(const Grid &G, const double *u, long q0, long np, double *host, hipStream_t s) {
+hipError_t launch_unpack(const Grid &G, const double *u, long q0, long np, double *host, hipStream_t s) {
   const long n = np * G.nv;
   hipLaunchKernelGGL(k_unpack, dim3(nblk(n)), dim3(TB), 0, s, G, u, q0, (unsigned)n, host);
+  return hipGetLastError();
 }
 
 void launch_set_time(double *time, double t, hipStream_t s) {

@@ -319,9 +319,10 @@ void launch_dev_weno(const AosGrid &A, int model, double gamma, const ReconParam
 void launch_dev_planar(const Grid &G, const double *a, double *nat, double *tr, int to_planar, int ghosts_only,
                        double *out, hipStream_t s);
 // Interior points q0 .. q0+np-1 (x fastest) of a state: point-major values in
-// pinned host memory -> the planar ghosted layout, and back.
-void launch_pack(const Grid &G, const double *host, long q0, long np, double *u, hipStream_t s);
-void launch_unpack(const Grid &G, const double *u, long q0, long np, double *host, hipStream_t s);
+// pinned host memory -> the planar ghosted layout, and back.  Both say whether the
+// launch failed.
+hipError_t launch_pack(const Grid &G, const double *host, long q0, long np, double *u, hipStream_t s);
+hipError_t launch_unpack(const Grid &G, const double *u, long q0, long np, double *host, hipStream_t s);
 void launch_set_time(double *time, double t, hipStream_t s);
 // one sweep's interface array: line-major -> reference layout
 void launch_dev_iface(int ndims, int dir, int nx, int N, int nl, int nv, const double *src, double *dst,

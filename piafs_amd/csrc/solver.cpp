@@ -343,20 +343,18 @@ Case::~Case() {
 // point-major interior (WriteBinary order) <-> natural planar ghosted
 int Case::upload(const double *uh, hipStream_t st) {
   const hipError_t e = staging->upload(uh, cfg.npts_int, cfg.nvars, st, [&](long q0, long np, double *buf) {
-    launch_pack(h.G, buf, q0, np, h.u, st);
+    return launch_pack(h.G, buf, q0, np, h.u, st);
   });
   if (e != hipSuccess) return fail(-1, std::string("state upload: ") + hipGetErrorString(e));
-  HIPCHK(hipGetLastError());
   return 0;
 }
 
 int Case::download(double *uh, hipStream_t st, const double *src) {
   const double *from = src ? src : h.u;
   const hipError_t e = staging->download(uh, cfg.npts_int, cfg.nvars, st, [&](long q0, long np, double *buf) {
-    launch_unpack(h.G, from, q0, np, buf, st);
+    return launch_unpack(h.G, from, q0, np, buf, st);
   });
   if (e != hipSuccess) return fail(-1, std::string("state download: ") + hipGetErrorString(e));
-  HIPCHK(hipGetLastError());
   return 0;
 }
 

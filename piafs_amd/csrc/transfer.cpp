@@ -162,6 +162,18 @@ hipError_t Staging::Set::settle(Slot &s) {
   return e;
 }
 
+// A chunk's device side.  Launch errors are kept by thread, so the thread that
+// launches reports them (kernel's result).
+hipError_t Staging::Set::enqueue(long q0, long np, Slot &s, hipStream_t st, const Kern &kernel) {
+  hipError_t e = kernel(q0, np, s.buf);
+  if (e != hipSuccess) return e;
+  s.on = st;
+  e = hipEventRecord(s.ev, st);
+  if (e == hipSuccess) s.pending = true;
+  else hipStreamSynchronize(st);  // no event to wait for: the buffer is given back idle
+  return e;
+}
+
 hipError_t Staging::Set::upload(const double *src, long npts, int nv, hipStream_t st, const Kern &kernel) {
   const size_t bytes = (size_t)npts * nv * sizeof(double);
   if (!grow(bytes)) return hipErrorOutOfMemory;
@@ -174,10 +186,7 @@ hipError_t Staging::Set::upload(const double *src, long npts, int nv, hipStream_
     const hipError_t e = settle(s);
     if (e != hipSuccess) return e;
     memcpy(s.buf, src + q0 * nv, (size_t)np * nv * sizeof(double));
-    kernel(q0, np, s.buf);
-    s.pending = true;
-    s.on = st;
-    return hipEventRecord(s.ev, st);
+    return enqueue(q0, np, s, st, kernel);
   });
 }
 
@@ -192,10 +201,7 @@ hipError_t Staging::Set::download(double *dst, long npts, int nv, hipStream_t st
     const long q0 = c * per, np = std::min(per, npts - q0);
     const hipError_t e = settle(s);
     if (e != hipSuccess) return e;
-    kernel(q0, np, s.buf);
-    s.pending = true;
-    s.on = st;
-    return hipEventRecord(s.ev, st);
+    return enqueue(q0, np, s, st, kernel);
   };
   // the first chunk of every thread is asked for from here, and the threads wake
   // when the first is there: until then one thread waits for the stream's work

@@ -47,9 +47,9 @@ class Staging {
   bool reserve(size_t bytes);
   // n doubles from `src` (host) / to `dst` (host) in chunks of whole points of
   // nv doubles: kernel(first point, points, buffer) enqueues the device side of
-  // a chunk on st.  upload returns when src is no longer needed (the kernels
+  // a chunk on st and says whether that failed.  upload returns when src is no longer needed (the kernels
   // may still run), download when dst is complete.
-  typedef std::function<void(long q0, long np, double *buf)> Kern;
+  typedef std::function<hipError_t(long q0, long np, double *buf)> Kern;
   hipError_t upload(const double *src, long npts, int nv, hipStream_t st, const Kern &kernel);
   hipError_t download(double *dst, long npts, int nv, hipStream_t st, const Kern &kernel);
 
@@ -84,6 +84,7 @@ class Staging {
     void worker(int id);
     int threads(long nchunks) const;  // that move nchunks chunks
     hipError_t settle(Slot &s);
+    hipError_t enqueue(long q0, long np, Slot &s, hipStream_t st, const Kern &kernel);
     hipError_t each(long nchunks, const std::function<hipError_t(long, Slot &)> &body);
     hipError_t upload(const double *src, long npts, int nv, hipStream_t st, const Kern &kernel);
     hipError_t download(double *dst, long npts, int nv, hipStream_t st, const Kern &kernel);

@@ -217,6 +217,38 @@ int main() {
 }
 """
 
+ERRORS = r"""
+// the launch of the last chunk fails (an upload's is a helper's), first in an
+// upload, then in a download; after that the buffers serve as before
+int main() {
+  Staging s(0);
+  Stream a;
+  const Vec h = state(1.0);
+  Vec d(NP * NV), back(NP * NV);
+  for (int pass = 0; pass < 4; pass++) {
+    auto kernel = [&](bool up) {
+      return [&, up](long q0, long np, double *buf) {
+        if (q0 + np == NP && pass == (up ? 0 : 1)) {
+          last_error = hipErrorLaunchFailure;  // of this thread; nothing is queued
+        } else {
+          a.push([=, &d] {
+            if (up) memcpy(&d[q0 * NV], buf, np * NV * sizeof(double));
+            else memcpy(buf, &d[q0 * NV], np * NV * sizeof(double));
+          });
+        }
+        return hipGetLastError();
+      };
+    };
+    const hipError_t eu = s.upload(h.data(), NP, NV, &a, kernel(true));
+    const hipError_t ed = s.download(back.data(), NP, NV, &a, kernel(false));
+    if (eu != (pass == 0 ? hipErrorLaunchFailure : hipSuccess)) return 1;
+    if (ed != (pass == 1 ? hipErrorLaunchFailure : hipSuccess)) return 2;
+    if (pass > 1 && back != h) return 3;
+  }
+  return 0;
+}
+"""
+
 
 def _build(tmp_path, main):
     gxx = shutil.which("g++")
@@ -240,3 +272,7 @@ def test_a_transfer_does_not_wait_for_other_handles_work(tmp_path, direction):
 
 def test_one_thread_waits_for_queued_work(tmp_path):
     assert subprocess.run([_build(tmp_path, WAITERS)], timeout=60).returncode == 0
+
+
+def test_failed_launches_are_reported(tmp_path):
+    assert subprocess.run([_build(tmp_path, ERRORS)], timeout=60).returncode == 0
