@@ -947,6 +947,7 @@ int piafs_download_state(piafs_case *pc, double *u) {
 int piafs_set_time(piafs_case *pc, double t) {
   if (!pc || !pc->c) return 1;  // no case
   pc->c->t = t;
+  hipSetDevice(pc->eng.device);
   launch_set_time(pc->c->h.time, t, pc->eng.stream);
   if (hipGetLastError() != hipSuccess) {
     pc->err = "set_time failed";

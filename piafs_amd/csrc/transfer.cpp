@@ -91,6 +91,7 @@ bool Staging::Set::settled(hipStream_t st) {
 }
 
 bool Staging::reserve(size_t bytes) {
+  hipSetDevice(ahead.device);
   std::unique_lock<std::mutex> g(ahead.use, std::try_to_lock);
   const bool first = g.owns_lock() && ahead.settled(nullptr);
   if (!first) g = std::unique_lock<std::mutex>(after.use);
@@ -222,6 +223,8 @@ hipError_t Staging::Set::download(double *dst, long npts, int nv, hipStream_t st
 // move(set) with a set that this transfer has
 template <class F>
 hipError_t Staging::on_a_set(hipStream_t st, F move) {
+  const hipError_t set = hipSetDevice(ahead.device);  // launches, and events that may be made, are the stream's device's
+  if (set != hipSuccess) return set;
   {
     std::unique_lock<std::mutex> g(ahead.use, std::try_to_lock);
     if (g.owns_lock() && ahead.settled(st)) return move(ahead);

@@ -21,8 +21,9 @@ RUNTIME = r"""
 #include <functional>
 #include <mutex>
 #include <thread>
-enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorNotReady = 600, hipErrorLaunchFailure = 719 };
+enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorNotReady = 600, hipErrorInvalidHandle = 400, hipErrorLaunchFailure = 719 };
 struct Stream {  // works in order; done counts what it has finished
+  int device = 0;
   std::mutex m;
   std::condition_variable cv;
   std::deque<std::function<void()>> q;
@@ -63,6 +64,7 @@ struct Stream {  // works in order; done counts what it has finished
   }
 };
 struct Event {
+  int device = 0;
   Stream *s = nullptr;
   long n = 0;
 };
@@ -75,7 +77,11 @@ inline hipError_t hipGetLastError() {
   last_error = hipSuccess;
   return e;
 }
-inline hipError_t hipSetDevice(int) { return hipSuccess; }
+inline thread_local int current_device = 0;
+inline hipError_t hipSetDevice(int d) {
+  current_device = d;
+  return hipSuccess;
+}
 inline hipError_t hipHostMalloc(void **p, size_t n, int) {
   *p = calloc(n, 1);
   return *p ? hipSuccess : hipErrorOutOfMemory;
@@ -86,6 +92,7 @@ inline hipError_t hipHostFree(void *p) {
 }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t *e, int) {
   *e = new Event;
+  (*e)->device = current_device;
   return hipSuccess;
 }
 inline hipError_t hipEventDestroy(hipEvent_t e) {
@@ -93,6 +100,7 @@ inline hipError_t hipEventDestroy(hipEvent_t e) {
   return hipSuccess;
 }
 inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  if (e->device != s->device) return hipErrorInvalidHandle;
   std::lock_guard<std::mutex> g(s->m);
   e->s = s;
   e->n = s->queued;
@@ -249,6 +257,34 @@ int main() {
 }
 """
 
+DEVICES = r"""
+// a thread whose current device is another one moves a case's state
+int main() {
+  Staging s(1);
+  Stream a;
+  a.device = 1;
+  const Vec h = state(1.0);
+  Vec d(NP * NV), back(NP * NV);
+  auto kernel = [&](bool up) {
+    return [&, up](long q0, long np, double *buf) {
+      if (current_device != a.device) return hipErrorLaunchFailure;
+      a.push([=, &d] {
+        if (up) memcpy(&d[q0 * NV], buf, np * NV * sizeof(double));
+        else memcpy(buf, &d[q0 * NV], np * NV * sizeof(double));
+      });
+      return hipSuccess;
+    };
+  };
+  for (int k = 0; k < 2; k++) {
+    hipSetDevice(0);
+    if (s.upload(h.data(), NP, NV, &a, kernel(true)) != hipSuccess) return 1;
+    hipSetDevice(0);
+    if (s.download(back.data(), NP, NV, &a, kernel(false)) != hipSuccess || back != h) return 2;
+  }
+  return 0;
+}
+"""
+
 
 def _build(tmp_path, main):
     gxx = shutil.which("g++")
@@ -276,3 +312,7 @@ def test_one_thread_waits_for_queued_work(tmp_path):
 
 def test_failed_launches_are_reported(tmp_path):
     assert subprocess.run([_build(tmp_path, ERRORS)], timeout=60).returncode == 0
+
+
+def test_the_callers_current_device_does_not_matter(tmp_path):
+    assert subprocess.run([_build(tmp_path, DEVICES)], timeout=60).returncode == 0
