@@ -211,10 +211,13 @@ int  piafs_conservation_errors(piafs_case *c, double *errors);
 int  piafs_kernel_times(piafs_case *c, int enable, const char **names, double *ms, int *n);
 
 /* Tile-shape autotuner (no counterpart in the reference): times the
- * reconstruction launch for line-solve segments of 4, 8, 12 and 16 rows per
- * lane on this case and keeps the fastest.  Results do not depend on the
- * choice (the line solves are exact).  Optional outputs: the chosen rows per
- * lane and its reconstruction time in ms. */
+ * reconstruction launches on this case with the segment lengths the library
+ * has chosen by size, which may differ from line to line, and with 4, 8, 12 and
+ * 16 rows per lane (lines that have no team of that many keep theirs), and
+ * keeps the fastest.  Results do not depend on the choice (the line solves are
+ * exact).  Optional outputs: the rows per lane -- where the library's own choice
+ * stays, the first of the four that none of its segments exceeds -- and the
+ * reconstruction time in ms. */
 int  piafs_autotune(piafs_case *c, int *rows_per_lane, double *recon_ms);
 
 /* ---------------------------------------------------------------------------

@@ -53,9 +53,10 @@ struct Case {
                       hipStream_t st);
   // conservation errors per variable (CalculateConservationError.c:20-40); -1 when unchecked
   int conservation_errors(std::vector<double> &ce, hipStream_t st);
-  // rows per lane of the line systems, 0: chosen by size (descriptor only; the
-  // engine's plan must be rebuilt afterwards)
-  int set_team_rows(int rows);
+  // rows per lane of the line systems, 0: chosen by size, as for sweeps that have
+  // no team of that many; whether one has (descriptor only; the engine's plan must
+  // be rebuilt afterwards)
+  bool set_team_rows(int rows);
   bool rows_set = false;
   static size_t plan_bytes(const Config &c);
 };

@@ -131,7 +131,7 @@ int Case::setup(int dev, hipStream_t st) {
     D.Sy.N = G.ny; D.Sy.g = G.g; D.Sy.plane = G.plane;
     D.Sy.nlines = G.nx; D.Sy.base = (long)G.g * G.nyg + G.gy; D.Sy.line_stride = G.nyg;
   }
-  if (set_team_rows(0)) return 1;
+  set_team_rows(0);
   // boundary zones, in list order (ApplyBoundaryConditions.c:20-40)
   std::vector<double> zvals;
   D.nzones = 0;
@@ -310,29 +310,31 @@ int Case::setup(int dev, hipStream_t st) {
   return 0;
 }
 
-int Case::set_team_rows(int want) {
+bool Case::set_team_rows(int want) {
   CaseDev &D = h;
   if (cfg.characteristic || !cfg.crweno) {  // no line teams
     D.Sx.team = D.Sy.team = 1;
     D.Sx.rows = D.Sy.rows = 1;
-    return 0;
+    return false;
   }
+  rows_set = false;
   std::vector<SweepGeom *> sweeps;
   for (int d = 0; d < cfg.ndims; d++) {
     SweepGeom &S = d ? D.Sy : D.Sx;
     S.longl = S.N - 1 > 256 * kMaxRows ? 1 : 0;  // longer than a 256-lane team covers
     S.team = S.rows = 1;
     if (S.longl) continue;
-    sweeps.push_back(&S);
-    if (want <= 0) continue;
-    S.rows = want;
-    if (!line_shape(S.N, want, S.team))
-      return fail(1, "lines of " + std::to_string(S.N) + " points have no team shape with " + std::to_string(want) +
-                         " rows per lane");
+    int T;
+    if (want > 0 && line_shape(S.N, want, T)) {
+      S.rows = want;
+      S.team = T;
+      rows_set = true;
+    } else {
+      sweeps.push_back(&S);
+    }
   }
-  if (want <= 0) choose_rows(sweeps, std::vector<int>(sweeps.size(), cfg.nvars));
-  rows_set = want > 0;
-  return 0;
+  choose_rows(sweeps, std::vector<int>(sweeps.size(), cfg.nvars));
+  return rows_set;
 }
 
 Case::~Case() {
@@ -602,32 +604,42 @@ double Engine::time_classes(const std::vector<int> &cls, int reps) {
 }
 
 // Segment length of the line solves (rows per lane, which sets each case's
-// team size): every candidate is timed on the members themselves and the
-// fastest kept.
+// team size): the choice by size and every candidate are timed on the members
+// themselves and the fastest kept.
 int Engine::autotune(const int *cands, int ncand, int reps, int *best_rows, double *best_ms) {
   HIPCHK(hipSetDevice(device));
   if (cases.empty()) return 0;
   std::vector<int> recon = {K_WENO};
   for (int v = 0; v < kNRecon; v++) recon.push_back(K_RECON + v);
+  auto set = [&](int rows) {
+    bool any = false;
+    for (Case *c : cases) any = c->set_team_rows(rows) || any;
+    return any;
+  };
   int best = -1;
   double bms = 0.0;
-  for (int k = 0; k < ncand; k++) {
-    bool ok = true;
-    for (Case *c : cases) ok = ok && c->set_team_rows(cands[k]) == 0;
-    if (!ok) continue;
-    int rc = build();
+  for (int k = -1; k < ncand; k++) {
+    const int rows = k < 0 ? 0 : cands[k];  // 0: chosen by size
+    if (!set(rows) && k >= 0) continue;  // no line has it
+    const int rc = build();
     if (rc) return rc;
     time_classes(recon, 1);  // warm
     const double ms = time_classes(recon, reps);
     if (best < 0 || ms < bms) {
-      best = cands[k];
+      best = rows;
       bms = ms;
     }
   }
-  if (best < 0) return fail(1, "no candidate segment length fits the members' lines");
-  for (Case *c : cases) c->set_team_rows(best);
-  int rc = build();
+  set(best);
+  const int rc = build();
   if (rc) return rc;
+  if (best == 0) {  // lengths may differ: the first candidate that bounds them all
+    int longest = 0;
+    for (int v = 0; v < kNRecon; v++)
+      if (plan.nblocks[K_RECON + v] > 0) longest = std::max(longest, kRecon[v].rows);
+    best = cands[ncand - 1];
+    for (int k = ncand - 1; k >= 0 && cands[k] >= longest; k--) best = cands[k];
+  }
   if (best_rows) *best_rows = best;
   if (best_ms) *best_ms = bms;
   return 0;

@@ -85,3 +85,17 @@ def test_species_fluxes_in_the_teams(tmp_path, nx, ny, upwinding):
     want = orc.OCase(d).rhs(u, 0.45)
     with piafs_amd.Case(d) as c:
         _close(c.rhs(u, 0.45), want)
+
+
+def test_autotuning_tries_the_choice_by_size(tmp_path):
+    """Lines of 896 and 448 rows fill teams of 14 rows a lane, which is not among
+    the uniform candidates, where 16 rows a lane would leave an eighth idle:
+    tuning keeps them."""
+    d = _deck(897, 449, n_iter=2).write(str(tmp_path))
+    with piafs_amd.Case(d) as c:
+        rows, ms = c.autotune()
+        c.profile(True)
+        c.step(1)
+        c.sync()
+        assert "recon_14" in c.kernel_times()
+    assert rows == 16 and ms > 0.0
