@@ -240,6 +240,9 @@ __host__ __device__ constexpr int recon_only(int dir, int r) { return (1 | (r & 
 KernFn weno_kernel();        // k_weno (weno.hip)
 constexpr int kWenoTile = 64;  // interfaces of a block
 
+// per-class timing: called before and after each launch with the stream it goes to
+typedef void (*MarkFn)(void *ctx, int cls, bool begin, hipStream_t st);
+
 // 1D cases advanced by whole steps: the class that can take a case (-1: none;
 // such a case takes the kernels of a stage), and n steps of a plan whose members
 // all have one.
@@ -249,7 +252,7 @@ constexpr size_t kLineLdsMax = 150 * 1024;
 __host__ __device__ constexpr int tube_core(int nstages) { return 63 - 6 * (nstages - 1); }
 int line_class(const CaseDev &c);
 hipError_t launch_lines(const CaseDev *d_cases, const Plan &plan, const std::vector<CaseDev> &cases, int n,
-                        hipStream_t st);
+                        hipStream_t st, MarkFn mark, void *mark_ctx);
 
 // Host side: blocks each case needs for each kernel class (0 = class unused).
 void case_blocks(const CaseDev &c, int blocks[K_NCLASS]);
@@ -274,9 +277,7 @@ int cw_back_fields(int nflow, int nv);
 
 // Stage s of the RK step for every case in the plan: stage state + BCs,
 // fluxes and viscous terms, reconstruction, upwinding, assembly of Udot[s].
-// Times: stage time = *time + c[s]*dt of each case.  `mark` (per-class timing)
-// is called before and after each launch with the stream the launch goes to.
-typedef void (*MarkFn)(void *ctx, int cls, bool begin, hipStream_t st);
+// Times: stage time = *time + c[s]*dt of each case.
 // With `last` < K_NCLASS only the work up to that class is done (in launch
 // order, which is the order of KClass), for the per-operator entry points:
 // K_GHOST ends with the stage state, K_FLUX with the cell fluxes.

@@ -271,7 +271,8 @@ int line_class(const CaseDev &c) {
   return K_TUBE;
 }
 
-hipError_t launch_lines(const CaseDev *d, const Plan &pl, const std::vector<CaseDev> &cases, int n, hipStream_t st) {
+hipError_t launch_lines(const CaseDev *d, const Plan &pl, const std::vector<CaseDev> &cases, int n, hipStream_t st,
+                        MarkFn mark, void *ctx) {
   if (n <= 0) return hipSuccess;  // as the stage kernels' loops take it
   for (int cls = K_LINE4; cls <= K_LINE8; cls++) {
     if (!pl.nblocks[cls]) continue;
@@ -281,17 +282,21 @@ hipError_t launch_lines(const CaseDev *d, const Plan &pl, const std::vector<Case
     const KernFn k = cls == K_LINE4 ? k_line<4> : k_line<8>;
     const hipError_t e = hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLineLdsMax);
     if (e != hipSuccess) return e;
-    for (int left = n; left > 0; left -= 256)  // a launch of bounded length
+    for (int left = n; left > 0; left -= 256) {  // a launch of bounded length
+      if (mark) mark(ctx, cls, true, st);
       hipLaunchKernelGGL(k, dim3(pl.nblocks[cls]), dim3(kLineThreads), bytes, st, d, pl.blockcase[cls],
                          pl.firstblock[cls], left < 256 ? left : 256);
+      if (mark) mark(ctx, cls, false, st);
+    }
   }
   if (pl.nblocks[K_TUBE]) {
-    for (int i = 0; i < n; i++)
-      hipLaunchKernelGGL(k_tube, dim3(pl.nblocks[K_TUBE]), dim3(256), 0, st, d, pl.blockcase[K_TUBE],
-                         pl.firstblock[K_TUBE], i & 1);
-    if (n & 1)
-      hipLaunchKernelGGL(k_tube_back, dim3(pl.nblocks[K_TUBEBACK]), dim3(256), 0, st, d, pl.blockcase[K_TUBEBACK],
-                         pl.firstblock[K_TUBEBACK], 0);
+    auto run = [&](int cls, KernFn k, int arg) {
+      if (mark) mark(ctx, cls, true, st);
+      hipLaunchKernelGGL(k, dim3(pl.nblocks[cls]), dim3(256), 0, st, d, pl.blockcase[cls], pl.firstblock[cls], arg);
+      if (mark) mark(ctx, cls, false, st);
+    };
+    for (int i = 0; i < n; i++) run(K_TUBE, k_tube, i & 1);
+    if (n & 1) run(K_TUBEBACK, k_tube_back, 0);
   }
   return hipGetLastError();
 }

@@ -559,8 +559,8 @@ int Engine::step(int n) {
   HIPCHK(hipSetDevice(device));
   if (!built) return fail(-1, "the ensemble plan is not built");
   if (cases.empty()) return 0;
-  if (!lines.empty() && !profiling) {
-    HIPCHK(launch_lines(d_cases, plan, lines, n, stream));
+  if (!lines.empty()) {
+    HIPCHK(launch_lines(d_cases, plan, lines, n, stream, profiling ? mark_cb : nullptr, this));
   } else if (use_graph && !profiling) {
     if (!gexec) {
       int rc = prepare();

@@ -92,3 +92,48 @@ def test_no_steps(tmp_path, scheme, interp):
                 c.step(none)
                 assert np.array_equal(c.solution(), u), none
                 assert c.info.t == t
+
+
+@pytest.mark.parametrize("N,scheme,interp,names", [(128, "crweno5", "components", {"line_4"}),
+                                                   (300, "crweno5", "components", {"line_8"}),
+                                                   (90, "weno5", "characteristic", {"tube", "tube_back"})])
+def test_profiled_steps_are_the_steps(tmp_path, N, scheme, interp, names):
+    """A profiled case takes the launches that it takes otherwise."""
+    with piafs_amd.Case(_deck(N, "mirror", scheme, interp, "roe", "44").write(str(tmp_path))) as c:
+        c.profile(True)
+        c.step(3)
+        c.sync()
+        times = c.kernel_times()
+    assert set(times) == names and all(t > 0.0 for t in times.values())
+
+
+def _beside_2d(tmp_path, decks_1d, steps, finite=True):
+    """Lines that step together with a 2D member go through the kernels of a
+    stage: alone they give the same bits."""
+    dirs = [dk.write(str(tmp_path / str(k))) for k, dk in enumerate(decks_1d)]
+    two = decks.ns2d_photochem(nx=20, ny=12, n_iter=sum(steps)).write(str(tmp_path / "two"))
+    with piafs_amd.Batch(dirs + [two]) as b:
+        for n in steps:
+            b.step(n)
+        want = [b.solution(k) for k in b.slots[:-1]]
+    for d, w, dk in zip(dirs, want, decks_1d):
+        with piafs_amd.Case(d) as c:
+            for n in steps:
+                c.step(n)
+            assert np.all(np.isfinite(w)) or not finite, dk.u.shape
+            assert np.array_equal(c.solution(), w, equal_nan=True), dk.u.shape
+
+
+@pytest.mark.parametrize("ends", sorted(ENDS))
+@pytest.mark.parametrize("interp,upwinding,rk", [("characteristic", "roe", "ssprk3"), ("components", "rf-char", "44"),
+                                                 ("characteristic", "llf-char", "44"), ("components", "rusanov", "1fe")])
+def test_windows_against_stage_kernels(tmp_path, ends, interp, upwinding, rk):
+    mem = [_deck(N, ends, "weno5", interp, upwinding, rk) for N in (8, 45, 51, 52, 90, 300)]
+    _beside_2d(tmp_path, mem, (1, 4, 3), ends != "reflect")
+
+
+@pytest.mark.parametrize("ends,upwinding", [("mirror", "roe"), ("periodic", "rf-char"), ("walls", "llf-char"),
+                                            ("reflect", "rusanov")])
+def test_line_systems_against_stage_kernels(tmp_path, ends, upwinding):
+    mem = [_deck(N, ends, "crweno5", "components", upwinding, "44", weights=N & 1) for N in (8, 33, 128, 257, 258, 513)]
+    _beside_2d(tmp_path, mem, (1, 6), ends != "reflect")
