@@ -246,7 +246,7 @@ typedef void (*MarkFn)(void *ctx, int cls, bool begin, hipStream_t st);
 // 1D cases advanced by whole steps: the class that can take a case (-1: none;
 // such a case takes the kernels of a stage), and n steps of a plan whose members
 // all have one.
-constexpr int kTubeVars = 8;
+constexpr int kLineVars = 3;  // species come with the chemistry, which these steps leave to the others
 constexpr size_t kLineLdsMax = 150 * 1024;
 // points of its window a k_tube block keeps
 __host__ __device__ constexpr int tube_core(int nstages) { return 63 - 6 * (nstages - 1); }

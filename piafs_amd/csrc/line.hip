@@ -70,7 +70,8 @@ template <int MR>
 __global__ void __launch_bounds__(kLineThreads) k_line(CASE_ARGS) {
   extern __shared__ double lds[];
   const CaseDev &C = cases[blockcase ? blockcase[blockIdx.x] : 0];
-  const int N = C.Sx.N, nv = C.G.nv, ns = C.nstages, g = C.G.g, P = N + 6, tid = threadIdx.x;
+  constexpr int nv = kLineVars;
+  const int N = C.Sx.N, ns = C.nstages, g = C.G.g, P = N + 6, tid = threadIdx.x;
   const double gam = C.P.gamma;
   double *u = lds, *U = u + nv * N + 3, *F = U + nv * P, *Ud = F + nv * P - 3, *io = Ud + ns * nv * N;
   // U, F: position i of variable v at v*P + i, i = -3 .. N+2; the interface
@@ -122,7 +123,7 @@ __global__ void __launch_bounds__(kLineThreads) k_line(CASE_ARGS) {
       }
       __syncthreads();
       for (int k = tid; k <= N; k += kLineThreads) {
-        double uLc[3], uRc[3], a[4][3], fo[3], e[3], c = 0.0;
+        double uLc[3], uRc[3], a[4][3], fo[3], e[3];
 #pragma unroll
         for (int m = 0; m < 3; m++) {
           uLc[m] = U[m * P + k - 1];
@@ -138,18 +139,16 @@ __global__ void __launch_bounds__(kLineThreads) k_line(CASE_ARGS) {
             ud[m] = 0.5 * (a[1][m] - a[0][m]);
             fs[m] = 0.5 * (a[2][m] + a[3][m]);
           }
-          c = mode == 0 ? roe_e1d(gam, uLc, uRc, ud, fs, fo) : rusanov_e1d(gam, uLc, uRc);
-          if (mode == 3)
+          if (mode == 0) {
+            roe_e1d(gam, uLc, uRc, ud, fs, fo);
+          } else {
+            const double c = rusanov_e1d(gam, uLc, uRc);
             for (int m = 0; m < 3; m++) fo[m] = fs[m] - c * ud[m];
+          }
         } else {
           rf_e1d(gam, mode == 2, uLc, uRc, a[0], a[1], a[2], a[3], fo, e);
         }
         for (int m = 0; m < 3; m++) F[m * P + k] = fo[m];
-        for (int m = 3; m < nv; m++) {
-          const double uL = at(0, m)[k], uR = at(1, m)[k], fL = at(2, m)[k], fR = at(3, m)[k];
-          F[m * P + k] = mode == 0 || mode == 3 ? 0.5 * (fL + fR) - c * (0.5 * (uR - uL))
-                                                : rf_pick(e[0], e[1], e[2], uL, uR, fL, fR, mode == 2);
-        }
       }
       __syncthreads();
       for (int q = tid; q < nv * N; q += kLineThreads) {
@@ -181,8 +180,9 @@ __global__ void __launch_bounds__(256) k_tube(CASE_ARGS) {
   CASE_PREAMBLE
   (void)t;
   __shared__ Rows rows;
-  __shared__ double u0[kTubeVars][kWin], U[kTubeVars][kWin + 6], Ud[4][kTubeVars][kWin], f[kTubeVars][64];
-  const int N = C.Sx.N, nv = C.G.nv, ns = C.nstages, g = C.G.g, tid = threadIdx.x;
+  constexpr int nv = kLineVars;
+  __shared__ double u0[nv][kWin], U[nv][kWin + 6], Ud[4][nv][kWin], f[nv][64];
+  const int N = C.Sx.N, ns = C.nstages, g = C.G.g, tid = threadIdx.x;
   const int lost = 3 * (ns - 1), core = tube_core(ns), bid = (int)(int)blockIdx.x - first;
   const int c0 = bid * core - lost;  // the window's first point
   const bool wraps = C.nzones > 0 && C.zones[0].kind == Z_PERIODIC;
@@ -252,13 +252,13 @@ __global__ void __launch_bounds__(256) k_tube_back(CASE_ARGS) {
 }
 
 size_t line_lds(const CaseDev &c) {
-  return sizeof(double) * c.G.nv * ((size_t)(1 + c.nstages) * c.G.nx + 2 * (c.G.nx + 6) + 4 * (c.G.nx + 1));
+  return sizeof(double) * kLineVars * ((size_t)(1 + c.nstages) * c.G.nx + 2 * (c.G.nx + 6) + 4 * (c.G.nx + 1));
 }
 
 }  // namespace
 
 int line_class(const CaseDev &c) {
-  if (c.G.ndims != 1 || c.model != 1 || c.G.nv > kTubeVars || c.cons || c.sponge || c.P.chem || c.terms != 7 || c.G.nx < 8)
+  if (c.G.ndims != 1 || c.model != 1 || c.G.nv != kLineVars || c.cons || c.sponge || c.P.chem || c.terms != 7 || c.G.nx < 8)
     return -1;
   if (c.R.crweno) {
     if (c.R.characteristic || line_lds(c) > kLineLdsMax) return -1;
