@@ -1,8 +1,10 @@
-"""1D cases advanced by whole steps (one launch for many steps, or one a step)
-against the kernels of a stage, which a profiled case runs: the same bits."""
+"""1D cases advanced by whole steps (one launch for many steps, or one a step):
+the same bits with timing marks around the launches, from the kernels of a
+stage, which lines beside a 2D member take, and the oracle's values."""
 import numpy as np
 import pytest
 
+import _oracle as orc
 import piafs_amd
 from piafs_amd import decks
 
@@ -137,3 +139,35 @@ def test_windows_against_stage_kernels(tmp_path, ends, interp, upwinding, rk):
 def test_line_systems_against_stage_kernels(tmp_path, ends, upwinding):
     mem = [_deck(N, ends, "crweno5", "components", upwinding, "44", weights=N & 1) for N in (8, 33, 128, 257, 258, 513)]
     _beside_2d(tmp_path, mem, (1, 6), ends != "reflect")
+
+
+def _scheme(dk, weights):
+    dk.weno.update(mapped=0, borges=int(weights == "z"), yc=int(weights == "yc"), no_limiting=int(weights == "none"))
+    return dk
+
+
+@pytest.mark.parametrize("weights", ["z", "yc", "none"])
+def test_other_weights(tmp_path, weights):
+    """Every weight rule is a kernel of its own: both kinds of lines, and upw5."""
+    mem = [_scheme(_deck(N, "mirror", *how, "44"), weights)
+           for N, how in [(61, ("weno5", "characteristic", "roe")), (62, ("weno5", "components", "rf-char")),
+                          (63, ("upw5", "components", "roe")), (64, ("upw5", "characteristic", "llf-char")),
+                          (100, ("crweno5", "components", "roe")), (300, ("crweno5", "components", "rf-char"))]]
+    _beside_2d(tmp_path, mem, (1, 5))
+
+
+@pytest.mark.parametrize("scheme,interp,weights", [("weno5", "characteristic", "z"), ("weno5", "components", "yc"),
+                                                   ("weno5", "components", "none"), ("upw5", "components", "none"),
+                                                   ("crweno5", "components", "z"), ("crweno5", "components", "yc"),
+                                                   ("crweno5", "components", "none")])
+def test_weights_against_the_oracle(tmp_path, scheme, interp, weights):
+    """10 steps; relative L2 norm of the difference per variable, the bound of the
+    other parity tests."""
+    dk = _scheme(_deck(100, "periodic", scheme, interp, "roe", "44"), weights)
+    dk.u[:] = dk.u[0] * (1.0 + 0.05 * np.sin(2 * np.pi * np.arange(100)[:, None] / 100))
+    d = dk.write(str(tmp_path))
+    o = orc.OCase(d)
+    o.step(10)
+    with piafs_amd.Case(d) as c:
+        c.step(10)
+        assert np.all(decks.rel_l2_per_var(c.solution(), o.solution()) <= 1e-11)

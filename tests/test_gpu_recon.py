@@ -99,3 +99,23 @@ def test_autotuning_tries_the_choice_by_size(tmp_path):
         c.sync()
         assert "recon_14" in c.kernel_times()
     assert rows == 16 and ms > 0.0
+
+
+# the segment length chosen for each of these lines, on 32 to 64, 128 and 256
+# lanes, the last one a row short
+@pytest.mark.parametrize("n,across,cls", [(128, 9, "4"), (384, 9, "6"), (512, 9, "8"), (640, 9, "10"), (768, 9, "12"),
+                                          (896, 9, "14"), (1024, 9, "16"), (1280, 9, "w10"), (1536, 17, "w12"),
+                                          (2048, 33, "w16"), (2560, 5, "w10"), (3072, 5, "w12"), (4096, 5, "w16")])
+@pytest.mark.parametrize("weights", ["js", "mapped", "z", "yc", "none"])
+def test_every_variant_with_every_weight(tmp_path, n, across, cls, weights):
+    nx, ny = (n, across) if weights in ("js", "z", "none") else (across, n)
+    dk = _deck(nx, ny, weights=weights, n_iter=1, dt=1e-5)
+    u = dk.u * (1.0 + 1e-2 * np.random.default_rng(n).uniform(-1, 1, dk.u.shape))
+    d = dk.write(str(tmp_path))
+    want = orc.OCase(d).rhs(u, 0.45)
+    with piafs_amd.Case(d) as c:
+        _close(c.rhs(u, 0.45), want)
+        c.profile(True)
+        c.step(1)
+        c.sync()
+        assert "recon_" + cls in c.kernel_times()
