@@ -36,39 +36,48 @@ HBM_PEAK_GBS = 8000.0
 STEP_BYTES_PER_CELL = lambda nv, ns: 40 * nv * ns  # noqa: E731
 
 
-def species_fused(nx, ny, nv, paired):
+def line_rows(kernels):
+    """Rows per lane of the line solves, from the kernel classes that ran (a
+    square grid's two sweeps have the same); None where there are none."""
+    rows = [int(m.group(1)) for m in (re.fullmatch(r"recon_w?(\d+)", k) for k in kernels) if m]
+    return max(rows) if rows else None
+
+
+def species_fused(n, nv, paired, rows):
     """Whether the library's reconstruction writes the species' Roe fluxes
-    itself: NS2D with species, paired Roe, and line teams of 32 to 128 lanes in
-    both sweeps (lines of 258 .. 2049 rows)."""
-    return paired and nv > 4 and 258 <= nx <= 2049 and 258 <= ny <= 2049
+    itself: NS2D with species, paired Roe, and line teams of 32 to 128 lanes
+    (a power of two of lanes whose segments of `rows` cover the n - 1 rows)."""
+    if not (paired and nv > 4 and rows):
+        return False
+    lanes = 1
+    while lanes * rows < n - 1:
+        lanes *= 2
+    return 32 <= lanes <= 128
 
 
-def kernel_algorithmic_bytes(name, nx, ny, nv, g, nstages, crweno, paired=True):
+def kernel_algorithmic_bytes(name, n, nv, g, paired=True, rows=None):
     """Compulsory bytes of one launch of a kernel class (its inputs read once
-    and outputs written once).  One launch covers both sweeps (x and y) of an
-    nx x ny grid; per sweep the counts below are for `lines` lines of N
-    interior points (the two sweeps have the same counts on a square grid).
-    paired: component-wise interpolation with Roe or Rusanov, where the
-    reconstruction writes only the two combinations 0.5 (uR - uL) and
-    0.5 (fL + fR) that the upwinding reads, instead of uL, uR, fL and fR."""
-    lines, N = ny, nx
-    pos = N + 2 * g
-    sweeps = 2
+    and outputs written once) on an n x n grid.  One launch covers both sweeps,
+    n lines of n interior points each.
+    paired: component-wise interpolation with Roe, where the reconstruction
+    writes only the two combinations 0.5 (uR - uL) and 0.5 (fL + fR) that the
+    upwinding reads, instead of uL, uR, fL and fR.  From 2^15 cells on the
+    species' cell fluxes are formed in the line teams, from their values and one
+    plane of velocities."""
+    pos, faces = (n + 2 * g) * n, (n + 1) * n
     nio = 2 if paired else 4
-    fused = species_fused(nx, ny, nv, paired)
-    if name.startswith("recon_") and name != "recon_ends":  # u and f at every position of every line; the interface arrays
-        if fused:  # flow: the two combinations; species: their flux, from |v_n| (one value per interface)
-            # (the state, the flow's fluxes and the velocity, from which the species' fluxes are formed)
-            return sweeps * 8 * ((nv + 4 + 1) * pos * lines + (2 * 4 + (nv - 4) + 1) * (N + 1) * lines)
-        return sweeps * 8 * (2 * nv * pos * lines + nio * nv * (N + 1) * lines)
+    fused = species_fused(n, nv, paired, rows)
+    fluxes = 4 + 1 if nv > 4 and rows and n * n >= 1 << 15 else nv
+    if re.fullmatch(r"recon_w?\d+", name):  # u and f at every position of every line; the interface arrays
+        # fused: the two combinations of the flow; the species' flux, from |v_n| (one value per interface)
+        return 2 * 8 * ((nv + fluxes) * pos + (2 * 4 + (nv - 4) + 1 if fused else nio * nv) * faces)
     if name == "upwind":  # the interface arrays + 4 flow vars at the two cells; fI
-        if fused:  # the flow variables only
-            return sweeps * 8 * (nio * 4 * (N + 1) * lines + 2 * 4 * (N + 1) * lines + 4 * (N + 1) * lines)
-        return sweeps * 8 * (nio * nv * (N + 1) * lines + 2 * 4 * (N + 1) * lines + nv * (N + 1) * lines)
-    if name == "flux":  # the flow's variables and fluxes and the velocity at every position; |v_n| per interface when fused
-        return sweeps * 8 * ((4 + 5) * pos * lines + ((N + 1) * lines if fused else 0))
+        m = 4 if fused else nv  # fused: the flow variables only
+        return 2 * 8 * (nio * m + 2 * 4 + m) * faces
+    if name == "flux":  # the variables that the fluxes are of, the fluxes; |v_n| per interface when fused
+        return 2 * 8 * (((4 if fluxes < nv else nv) + fluxes) * pos + (faces if fused else 0))
     if name == "stage_bc":  # u + up to one Udot read, U and UT written (ghosted)
-        return 8 * nv * (nx + 2 * g) * (ny + 2 * g) * 4
+        return 8 * nv * (n + 2 * g) ** 2 * 4
     return None
 
 
@@ -442,7 +451,7 @@ def main():
             share = {k: v * per_step.get(k, ns) for k, v in ktimes.items()}
             dom = max(share.items(), key=lambda kv: kv[1])[0]
             paired = (not inf.characteristic) and dk.physics["upwinding"] in ("roe", "rusanov")
-            io_byts = kernel_algorithmic_bytes(dom, nx, nx, nv, g, inf.nstages, True, paired)
+            io_byts = kernel_algorithmic_bytes(dom, nx, nv, g, paired, line_rows(ktimes))
             ms = ktimes[dom]
             # algorithmic bytes of one stage of a stage-fused RK step, 40 nv B per
             # cell (read the stage state and u_n, read and write the accumulator,

@@ -258,6 +258,13 @@ hipError_t launch_lines(const CaseDev *d_cases, const Plan &plan, const std::vec
 void case_blocks(const CaseDev &c, int blocks[K_NCLASS]);
 // Whether the reconstruction can write the species' Roe interface fluxes
 // itself (NS2D, paired Roe, teams of 32 to 128 lanes, |v_n| buffers present).
+// Lanes follow the segment length: a square case alone has such teams from 98 to
+// 129 and from 162 to 2049 points a side.  A step with k_upwind writing all fluxes / with the
+// reconstruction writing the species': 100 x 100 178 / 168 us, 128 x 97 185 / 173,
+// 192^2 250 / 243, 256^2 338 / 332, 320^2 484 / 479, 512^2 988 / 955, 700^2 2.12 /
+// 2.01 ms, 1024^2 4.10 / 3.90, 1531^2 11.62 / 11.28, 2048 x 1531 14.91 / 14.41.
+// Teams of 16 lanes lost 1.4 % (256^2 with 16 rows a lane); a team of 256 lanes has
+// a block to itself, without its partner.
 bool species_in_recon(const CaseDev &c);
 // Whether the reconstruction can form the species' cell fluxes itself, and from how
 // many cells of a plan on it does: it saves k_flux traffic (1024 x 1024 133 -> 77
