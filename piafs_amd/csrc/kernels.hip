@@ -2119,6 +2119,11 @@ bool line_shape(int N, int rows, int &team) {
 // (teams are powers of two, so a row count serves some lengths better than
 // others; short segments have more waves to hide their chains, long ones less
 // overhead per row).  Rows 16 only, the choice before, is the last column.
+// Teams of 128 and 256 lanes (rows 10 12 16; - : more than 256 lanes):
+//   N 1100: 1364 1406 1578     N 1281: 1596 1679 1872     N 1400: 3195 1852 2055     N 1537: 3531 2034 2311
+//   N 1800: 4213 4370 2774     N 2049: 4852 5022 3141     N 2561: 6160 6452 7251     N 3073:   -  7837 8865
+// and 10720 at 3600, 12420 at 4096, both 16 rows.  The fit gives 1631 at 1281 (10
+// rows), 2087 at 1537 (12), 3276 at 2049 (16) and the fastest of each line above.
 void choose_rows(const std::vector<SweepGeom *> &sweeps, const std::vector<int> &nvars) {
   static const double per_row[kNRecon] = {1.25, 1.10, 1.00, 1.06, 1.11, 1.10, 1.06, 1.44, 1.28, 1.13};
   auto latency = [](int v) { return 10.0 + 0.75 * kRecon[v].rows; };

@@ -29,7 +29,11 @@ __device__ __forceinline__ double advance(const CaseDev &C, int s, double u, F u
 // CRWENO5 by components: the line couples all of its points, so one block takes
 // a case, `stage` steps of it.  Bound by latency: four barriers a stage, of
 // which the line solves (a wave or part of one per system, MR rows a lane) are
-// the longest.  A line of 128 took 108 us a step in 21 launches.
+// the longest.  A step (RK4, Roe) in 21 launches of a graph and in this kernel, us:
+//   points     8    33   128   257   258   400   513
+//   launches  89    92   101   104   108   117   119
+//   here      21    22    30    42    52    54    56
+// The last is the longest line whose lanes' rows (8) fit a wave a system.
 constexpr int kLineThreads = 768;
 
 template <int MR, int KIND, bool LEFT>
