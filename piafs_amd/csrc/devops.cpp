@@ -8,7 +8,9 @@
 // the points of the grid with dim[dir]+1 interfaces along dir and no ghosts,
 // in the same order.
 //
-// The reconstruction and upwinding run the step's own kernels on staged
+// The flux, the upwinding, the derivative, the weights and the interpolation of
+// the schemes without line systems run on the caller's arrays as they are.  The
+// boundary fill and the CRWENO5 interpolation run the step's own kernels on staged
 // copies: the case's stage-state buffers (natural and transposed), its flux
 // buffers and its interface buffers in split mode, all of which a step
 // rewrites from the solution before reading them.  The case's solution is

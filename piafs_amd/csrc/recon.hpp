@@ -35,16 +35,16 @@ __device__ __forceinline__ bool any_lane(bool p) { return WIDE ? __syncthreads_o
 // value xlast.
 //
 // The result is the sequential sweep of tridiagLU.c:133-150 and :243-255 bit
-// for bit (see teams.hpp): each lane runs the sweep over its rows from an
-// estimate of the state entering them, and entries are replaced by what the
-// neighbour ended with until none changes.  The estimates here use how the
-// systems contract.  A pivot forgets its predecessors by a factor of about 0.1
-// a row, so a lane's own rows give its last pivot to the last bits from any
-// start; they are run as continuants, p_k = b_k p_{k-1} - a_k c_{k-1} p_{k-2}
-// with b'_k = p_k / p_{k-1}, without divisions.  x' and x forget by 0.55 a row
-// or better, so the affine maps of the 64 rows before a segment fix its entry.
-// Elsewhere (weights far from optimal) the estimates are worse and the relays
-// take more passes, T at most.
+// for bit (see teams.hpp; for tiny numerators see the back substitution): each
+// lane runs the sweep over its rows from an estimate of the state entering them,
+// and entries are replaced by what the neighbour ended with until none changes.
+// The estimates here use how the systems contract.  A pivot forgets its
+// predecessors by a factor of about 0.1 a row, so a lane's own rows give its last
+// pivot to the last bits from any start; they are run as continuants, p_k = b_k
+// p_{k-1} - a_k c_{k-1} p_{k-2} with b'_k = p_k / p_{k-1}, without divisions.  x'
+// and x forget by 0.55 a row or better, so the affine maps of the 64 rows before a
+// segment fix its entry.  Elsewhere (weights far from optimal) the estimates are
+// worse and the relays take more passes, T at most.
 template <int MR, bool WIDE>
 __device__ __forceinline__ void line_solve(double (&A)[MR], double (&B)[MR], double (&C)[MR], double (&X)[MR],
                                            int lane, int T, double xfirst, double xlast, double *red, int *status,
@@ -188,9 +188,12 @@ __device__ __forceinline__ void line_solve(double (&A)[MR], double (&B)[MR], dou
     if (last) yin = xlast;
   }
   // The quotients take the reciprocals at hand (wdiv's last steps): the IEEE
-  // quotient's bits within its envelope.  Past the ends of the range it gives
-  // NaN where the IEEE quotient is infinite; a NaN runs on to the segment's
-  // first row, and then the team divides again with the full sequence.
+  // quotient's bits within its envelope.  Past the upper end of the range it
+  // gives NaN where the IEEE quotient is infinite; a NaN runs on to the segment's
+  // first row, and then the team divides again with the full sequence.  Numerators
+  // below 2^-969, as in the tail of a species that is zero elsewhere, are not
+  // looked for: there one unit in the last place can be missing (2 to 3 % of the
+  // quotients of numerators below 2^-1029), and -0 becomes +0.
   const double yin0 = yin;
   for (int it = 0; it <= T; it++) {
     double x = yin;
