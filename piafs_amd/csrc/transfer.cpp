@@ -32,10 +32,8 @@ void Staging::Set::release() {
     if (s.ev && s.pending) hipEventSynchronize(s.ev);
     if (s.ev) hipEventDestroy(s.ev);
     if (s.buf) hipHostFree(s.buf);
-    s = Slot();
   }
-  nslots = 0;
-  cap = 0;
+  for (int k = 0; k < nold; k++) hipHostFree(old[k]);
 }
 
 // Chunk size and buffers of a state: an eighth of it, within kMinChunk (below,
@@ -51,22 +49,34 @@ bool Staging::Set::grow(size_t bytes) {
   int n;
   shape(bytes, chunk, n);
   if (chunk > cap || n > nslots) {
-    const size_t c = std::max(chunk, cap);
+    size_t c = kMinChunk;  // doubled, so that buffers are replaced four times at most
+    while (c < chunk) c *= 2;
+    c = std::max(c, cap);
     const int want = std::max(n, nslots);
-    release();
-    for (int k = 0; k < want; k++) {
-      void *p = nullptr;
-      if (hipHostMalloc(&p, c, hipHostMallocDefault) != hipSuccess) break;
-      slots[k].buf = (double *)p;
-      if (hipEventCreateWithFlags(&slots[k].ev, hipEventDisableTiming) != hipSuccess) {
-        hipHostFree(p);
-        slots[k] = Slot();
+    int have = 0;
+    for (; have < want; have++) {
+      Slot &s = slots[have];
+      if (!s.ev && hipEventCreateWithFlags(&s.ev, hipEventDisableTiming) != hipSuccess) {
+        s.ev = nullptr;
         break;
       }
-      nslots = k + 1;
+      if (s.buf && c == cap) continue;
+      void *p = nullptr;
+      if (hipHostMalloc(&p, c, hipHostMallocDefault) != hipSuccess) break;
+      if (s.buf) old[nold++] = s.buf;
+      s.buf = (double *)p;
+      s.pending = false;
     }
-    if (nslots) cap = c;
-    hipGetLastError();  // a shortage of pinned memory leaves fewer buffers
+    hipGetLastError();  // a shortage of pinned memory leaves fewer buffers, or the smaller ones
+    if (have > 0) {
+      for (int k = have; k < nslots; k++) {
+        old[nold++] = slots[k].buf;
+        slots[k].buf = nullptr;
+        slots[k].pending = false;
+      }
+      nslots = have;
+      cap = c;
+    }
   }
   while ((int)pool.size() < nslots - 1) {
     const int id = (int)pool.size() + 1;
@@ -181,7 +191,7 @@ hipError_t Staging::Set::upload(const double *src, long npts, int nv, hipStream_
   size_t chunk;
   int n;
   shape(bytes, chunk, n);
-  const long per = std::max<long>(1, (long)(chunk / (nv * sizeof(double))));
+  const long per = std::max<long>(1, (long)(std::min(chunk, cap) / (nv * sizeof(double))));
   return each((npts + per - 1) / per, [&](long c, Slot &s) {
     const long q0 = c * per, np = std::min(per, npts - q0);
     const hipError_t e = settle(s);
@@ -197,7 +207,7 @@ hipError_t Staging::Set::download(double *dst, long npts, int nv, hipStream_t st
   size_t chunk;
   int n;
   shape(bytes, chunk, n);
-  const long per = std::max<long>(1, (long)(chunk / (nv * sizeof(double)))), nchunks = (npts + per - 1) / per;
+  const long per = std::max<long>(1, (long)(std::min(chunk, cap) / (nv * sizeof(double)))), nchunks = (npts + per - 1) / per;
   auto fetch = [&](long c, Slot &s) {
     const long q0 = c * per, np = std::min(per, npts - q0);
     const hipError_t e = settle(s);

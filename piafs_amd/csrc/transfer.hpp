@@ -25,8 +25,8 @@
 namespace piafs {
 
 // The pinned buffers and copy threads of one device, shared by all its cases and
-// given back with the last of them.  Two sets of at most kSlots * kSlotBytes of
-// pinned memory each.  A transfer takes the first if nobody has it, and queues its
+// given back with the last of them.  Two sets of at most 2 * kSlots * kSlotBytes of
+// pinned memory each (a state of the largest size, and the buffers it outgrew).  A transfer takes the first if nobody has it, and queues its
 // chunks behind whatever its stream holds.  Since that may be a long computation,
 // during which the set is taken, any other transfer then waits for its own stream
 // alone and takes the second set, which is never held, nor its buffers in use, for
@@ -69,6 +69,9 @@ class Staging {
     Slot slots[kSlots];
     int nslots = 0;
     size_t cap = 0;  // bytes of every slot's buffer
+    // outgrown buffers, kept: freeing pinned memory waits for all work on the device
+    void *old[4 * kSlots];
+    int nold = 0;
 
     std::vector<std::thread> pool;
     std::mutex m;

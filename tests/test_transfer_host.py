@@ -21,6 +21,7 @@ RUNTIME = r"""
 #include <functional>
 #include <mutex>
 #include <thread>
+#include <vector>
 enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorNotReady = 600, hipErrorInvalidHandle = 400, hipErrorLaunchFailure = 719 };
 struct Stream {  // works in order; done counts what it has finished
   int device = 0;
@@ -63,6 +64,7 @@ struct Stream {  // works in order; done counts what it has finished
     th.join();
   }
 };
+inline std::vector<Stream *> streams;  // every one a test has, for what waits for the device
 struct Event {
   int device = 0;
   Stream *s = nullptr;
@@ -85,10 +87,6 @@ inline hipError_t hipSetDevice(int d) {
 inline hipError_t hipHostMalloc(void **p, size_t n, int) {
   *p = calloc(n, 1);
   return *p ? hipSuccess : hipErrorOutOfMemory;
-}
-inline hipError_t hipHostFree(void *p) {
-  free(p);
-  return hipSuccess;
 }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t *e, int) {
   *e = new Event;
@@ -127,6 +125,11 @@ inline hipError_t hipStreamSynchronize(hipStream_t s) {
     n = s->queued;
   }
   s->wait(n);
+  return hipSuccess;
+}
+inline hipError_t hipHostFree(void *p) {  // waits for the device's work
+  for (Stream *s : streams) hipStreamSynchronize(s);
+  free(p);
   return hipSuccess;
 }
 """
@@ -285,6 +288,39 @@ int main() {
 }
 """
 
+GROWTH = r"""
+// larger buffers, for a new case beside one whose computation runs, do not wait
+// for that computation, and hold what is moved through them
+int main() {
+  Staging s(0);
+  Stream a, b;
+  streams = {&a, &b};
+  Gate gate;
+  const long few = 1000;  // one small chunk
+  Vec da(few * NV), ha = state(1.0), hs = state(3.0), db(NP * NV), hb(NP * NV);
+  if (s.upload(ha.data(), few, NV, &a, [&](long q0, long np, double *buf) {
+        a.push([=, &da] { memcpy(&da[q0 * NV], buf, np * NV * sizeof(double)); });
+        return hipGetLastError();
+      }) != hipSuccess)
+    return 2;
+  hipStreamSynchronize(&a);
+  a.push([&] { gate.wait(); });
+  std::atomic<int> other{0};
+  std::thread tb([&] {
+    if (!s.reserve(NP * NV * sizeof(double))) return;
+    if (to_device(s, hs, db, b) != hipSuccess || to_host(s, hb, db, b) != hipSuccess) return;
+    other = 1;
+  });
+  for (int i = 0; i < 100 && !other; i++) std::this_thread::sleep_for(std::chrono::milliseconds(50));
+  const bool passed = other == 1;
+  gate.release();
+  tb.join();
+  hipStreamSynchronize(&a);
+  if (other != 1 || hb != hs || memcmp(da.data(), ha.data(), few * NV * sizeof(double))) return 3;
+  return passed ? 0 : 1;
+}
+"""
+
 
 def _build(tmp_path, main):
     gxx = shutil.which("g++")
@@ -316,3 +352,7 @@ def test_failed_launches_are_reported(tmp_path):
 
 def test_the_callers_current_device_does_not_matter(tmp_path):
     assert subprocess.run([_build(tmp_path, DEVICES)], timeout=60).returncode == 0
+
+
+def test_larger_buffers_do_not_wait_for_the_device(tmp_path):
+    assert subprocess.run([_build(tmp_path, GROWTH)], timeout=60).returncode == 0
